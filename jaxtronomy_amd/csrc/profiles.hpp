@@ -81,6 +81,44 @@ __device__ __forceinline__ double rcp_refined(double v) {
   return (e == e) ? r : r0;
 }
 
+// 1/v and 1/sqrt(v) for finite normal v > 0 to the last place or two: the
+// hardware's v_rcp_f64 / v_rsq_f64 (2^-24.4 and 2^-24.2 off at worst, measured
+// over 2^20 arguments) with one third-order step, whose error e^3 is below
+// 2^-72 (the second-order step of rcp_refined leaves 2^-48).
+__device__ __forceinline__ double rcp_full(double v) {
+  const double r = __builtin_amdgcn_rcp(v);
+  const double e = fma(-v, r, 1.0);
+  return fma(fma(e, e, e), r, r);
+}
+__device__ __forceinline__ double rsq_full(double v) {
+  const double y = __builtin_amdgcn_rsq(v);
+  const double e = fma(-(v * y), y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// A float64 literal as a scalar register pair.  Left to itself the compiler
+// hoists a series' literals out of the ray loop into vector registers and,
+// the accumulating form of the FMA overwriting its addend, copies each one
+// before its step: one more vector instruction per step, and up to a hundred
+// registers (one wave per SIMD for the TNFW).  From a scalar pair the step is
+// the FMA alone; the two scalar moves issue beside other waves' vector work.
+// (Used where many series share a loop, as in the TNFW; in the compile-time
+// render the literals of the logarithm and the exponential fit the vector
+// registers without copies, and scalar ones measured 5% slower.)
+__device__ __forceinline__ double scalar_lit(double c) {
+  asm volatile("" : "+s"(c));
+  return c;
+}
+
+// p[0] + p[1] x + ... + p[N - 1] x^(N - 1)
+template <int N>
+__device__ __forceinline__ double poly(const double (&p)[N], double x) {
+  double q = fma(scalar_lit(p[N - 1]), x, scalar_lit(p[N - 2]));
+#pragma unroll
+  for (int i = N - 3; i >= 0; --i) q = fma(q, x, scalar_lit(p[i]));
+  return q;
+}
+
 // log2 x for finite x > 0 (the callers floor their arguments), to a few ulp
 // in about a third of the library log2's instructions: x = m 2^e with m in
 // [sqrt(1/2), sqrt(2)), ln m = 2 atanh(s), s = (m - 1) / (m + 1), |s| <=
@@ -236,7 +274,18 @@ enum : int { NFW_RS = 2, NFW_A, NFW_IRS };
 //          tau^2/(tau^2+1)^2, tau pi + (tau^2-1) ln tau, (tau^2-1)/tau, 0.001 Rs, tau^2+1, 1/Rs
 enum : int { TN_RS = 2, TN_A, TN_TAU, TN_TAU2, TN_PRE, TN_C0, TN_C1, TN_RMIN, TN_T2P1, TN_IRS,
               TN_K,      // pi (tau^2 + 1)^2 / 2
-              TN_T2M1 }; // tau^2 - 1
+              TN_T2M1,   // tau^2 - 1
+              // the FP64 form's (tnfw_core)
+              TN_AP,     // 4 rho0 Rs tau^2/(tau^2+1)^2
+              TN_UFAR,   // X^2 from which both far series converge: max(16, 16 tau^2)
+              // the gradient's (tnfw_ray_grad)
+              TN_D0,     // tau pi + 2 tau^2 ln tau
+              TN_E1,     // (tau^2 + 1) / tau
+              TN_PT,     // pi tau^2 (tau^2 + 1)
+              TN_DP,     // d ln(tau^2/(tau^2+1)^2) / d ln tau = 2 (1 - tau^2) / (1 + tau^2)
+              TN_A1,     // 4 rho0 Rs / alpha_Rs
+              TN_IRT };  // 1 / r_trunc
+static_assert(TN_IRT < kRec, "TNFW record exceeds kRec");
 // SHEAR   (shear.py:37-53): ra_0, dec_0 in the centre slots, gamma1, gamma2; the
 //          steps of w = theta - alpha_scaling alpha_shear(theta) (affine in theta)
 enum : int { SH_G1 = 2, SH_G2, SH_WSX, SH_WSY, SH_WRX, SH_WRY };
@@ -465,6 +514,14 @@ __device__ inline void prepare_record(int type, const double *p, double *rec, do
       rec[TN_IRS] = 1.0 / Rs;
       rec[TN_K] = 0.5 * M_PI * (tau2 + 1.0) * (tau2 + 1.0);
       rec[TN_T2M1] = tau2 - 1.0;
+      rec[TN_AP] = rec[TN_A] * rec[TN_PRE];
+      rec[TN_UFAR] = 16.0 * fmax(1.0, tau2);
+      rec[TN_D0] = tau * M_PI + 2.0 * tau2 * log(tau);
+      rec[TN_E1] = (tau2 + 1.0) / tau;
+      rec[TN_PT] = M_PI * tau2 * (tau2 + 1.0);
+      rec[TN_DP] = 2.0 * (1.0 - tau2) / (1.0 + tau2);
+      rec[TN_A1] = 1.0 / (Rs * (1.0 + log(1.0 / 2.0)));
+      rec[TN_IRT] = 1.0 / r_trunc;
       break;
     }
     case LENSIM_SHEAR: {
@@ -939,23 +996,135 @@ __device__ __forceinline__ void nfw_defl(const Rec<T> &r, double x, double y, do
   }
 }
 
-// TNFW.F, LensModel/Profiles/tnfw.py:288-304 (FP64 form; the division by
-// sqrt(v) as a refined reciprocal, within two ulp of it).
-__device__ __forceinline__ double tnfw_F(double x) {
-  if (x < 1.0) {
-    const double sv = ::sqrt(1.0 - x * x);
-    return atanh_dbl(sv) * rcp_refined(sv);
+// The TNFW's g (LensModel/Profiles/tnfw.py:329-349) in double, on u = X^2 (the
+// caller's floor: u >= 1e-6), with w = sqrt(tau^2 + u):
+//   g = pre B,  B = (tau^2 + 2 u - 1) F - pi w + C0 + w L C1,
+//   F = arctan(sqrt(u - 1)) / sqrt(u - 1) (arctanh below u = 1),  L = ln(X / (tau + w)),
+// and, for the gradient, X dB/dX and tau dB/dtau (GRAD):
+//   X dB/dX = 4 u F + (tau^2 + 2 u - 1) X F' + (u / w) (L C1 - pi) + tau^2 - 1,  X F' = (1 - u F) / (u - 1),
+//   tau dB/dtau = 2 tau^2 F + D0 + (tau^2 / w) (L C1 - pi) + w L E1
+// (X dL/dX = tau / w, tau dL/dtau = -tau / w).  Nothing but u is needed of the
+// ray: no root for R, no division; F and L are polynomials where they can be:
+//  * u >= 4: F = (pi / 2) / v - G(1/u) / u, v = sqrt(u - 1), G(z) =
+//    asin(sqrt z) / sqrt(z (1 - z)) (degree 13 over z <= 1/4).  The pi terms,
+//    which grow like X and cancel, are taken together: with w^2 - v^2 = tau^2 + 1
+//    they are K / (v (v + w)^2) in B, -K u (2 v + w) / (v^3 w (v + w)^2) in
+//    X dB/dX and pi tau^2 (tau^2 + 1) / (v w (v + w)) in tau dB/dtau;
+//  * 1/4 <= u < 4: F = 2 P(t) / (1 + X), t = (X - 1) / (X + 1), P(t) =
+//    arctan(sqrt t) / sqrt t over |t| <= 1/3 (degree 19; both sides of X = 1);
+//  * below: F = arctanh(s) / s, s = sqrt(1 - u) correctly rounded: s nears 1,
+//    where the reference's formula loses digits to the rounding of 1 - u and of
+//    s, and its values are these;
+//  * y2 = tau^2 / u <= 1/4: w L = -tau sqrt(1 + y2) asinh(y) / y (degree 11 in y2),
+//    else the logarithm;
+//  * u >= TN_UFAR (z and y2 <= 1/16; most rays of most subhalos): the same with
+//    degrees 8 and 7, and no other branch.
+// The fits' relative errors are below 7e-17 (60-digit arithmetic).  Bound by
+// the issue of the vector ALU: the far branch is about 80 instructions, where
+// the form with a root for R, library-style arctangent and logarithm took
+// about 250 (of a 400^2-ray line of sight: 8.9 -> 6.0 ms a call).
+template <bool GRAD>
+__device__ __forceinline__ void tnfw_core(const double *rd, double u, double &iu, double &B, double &XBX,
+                                          double &tBt) {
+  const double tau = rd[TN_TAU], tau2 = rd[TN_TAU2];
+  const double rX = rsq_full(u);
+  iu = rX * rX;
+  const double sw = tau2 + u;
+  const double iw = rsq_full(sw), w = sw * iw;
+  const double y2 = tau2 * iu;
+  double B0, X0 = 0.0, t0 = 0.0, wL;
+  auto outer = [&](double G) {  // u >= 4
+    const double e = u - 1.0;
+    const double iv = rsq_full(e), v = e * iv;
+    const double vw = v + w, r = rcp_full(vw * vw);
+    const double Kr = rd[TN_K] * r;
+    B0 = fma(Kr, iv, -(fma(rd[TN_T2M1], iu, 2.0) * G));
+    if constexpr (GRAD) {
+      const double iv2 = iv * iv;
+      X0 = fma(-Kr * u, (v + vw) * iv * iv2 * iw, fma(fma(2.0, u, rd[TN_T2M1]) * iv2, 1.0 + G, -4.0 * G));
+      t0 = fma(rd[TN_PT] * iv, iw * r * vw, -2.0 * y2 * G);
+    }
+  };
+  if (u >= rd[TN_UFAR]) {
+    constexpr double g8[9] = {1, 0.66666666666655927, 0.53333333337906674, 0.45714284965716129, 0.406349818765735,
+                              0.36938031616196654, 0.34174313656705135, 0.30667133979364775, 0.39348549697643637};
+    constexpr double a7[8] = {0.99999999999999989, -0.16666666666652991, 0.074999999953953234, -0.04464285122483598,
+                              0.030381569908054854, -0.02235922958054741, 0.017103352105079236,
+                              -0.011406154740420803};
+    outer(poly(g8, iu));
+    wL = -(w * tau * rX) * poly(a7, y2);
+  } else {
+    if (u >= 4.0) {
+      constexpr double g13[14] = {1, 0.66666666666673224, 0.53333333331635013, 0.45714285887196332,
+                                  0.40634911476368524, 0.36941126493138032, 0.3409332932493519, 0.31907228762239243,
+                                  0.29180058074110277, 0.33511256175349097, 0.035139155368524883, 0.97765555800227311,
+                                  -1.1132861271784307, 1.5537792943093436};
+      outer(poly(g13, iu));
+    } else {
+      double F;
+      const double X = u * rX;
+      if (u >= 0.25) {
+        constexpr double p19[20] = {1, -0.33333333333333331, 0.2000000000000407, -0.14285714285718173,
+                                    0.1111111110990561, -0.090909090897571695, 0.076923078305074097,
+                                    -0.066666667987215295, 0.058823449184073437, -0.052631502289141152,
+                                    0.047621712357723792, -0.043480806937435917, 0.039946430293369972,
+                                    -0.036985856369465865, 0.035142777271370877, -0.032888583414052187,
+                                    0.025482617337549689, -0.023967278167745611, 0.045592597260624118,
+                                    -0.043367164921101896};
+        const double q = rcp_full(1.0 + X);
+        F = 2.0 * q * poly(p19, (X - 1.0) * q);
+      } else {
+        const double s = ::sqrt(1.0 - u);
+        F = atanh_dbl(s) * rcp_refined(s);
+      }
+      B0 = fma(fma(2.0, u, rd[TN_T2M1]), F, -M_PI * w);
+      if constexpr (GRAD) {
+        const double e = u - 1.0;
+        double XF;
+        if (fabs(e) < 0.03) {  // 2 u dF/du, F = sum (-e)^n / (2 n + 1): the quotient cancels here
+          constexpr double d9[10] = {-1.0 / 3, 2.0 / 5, -3.0 / 7, 4.0 / 9, -5.0 / 11,
+                                     6.0 / 13, -7.0 / 15, 8.0 / 17, -9.0 / 19, 10.0 / 21};
+          XF = 2.0 * u * poly(d9, e);
+        } else {
+          XF = fma(-u, F, 1.0) / e;
+        }
+        X0 = fma(fma(2.0, u, rd[TN_T2M1]), XF, u * fma(4.0, F, -M_PI * iw));
+        t0 = tau2 * fma(2.0, F, -M_PI * iw);
+      }
+    }
+    if (y2 <= 0.25) {
+      constexpr double a11[12] = {1, -0.16666666666665123, 0.074999999997043848, -0.04464285692054213,
+                                  0.030381935774005903, -0.02237195860704631, 0.017349806102795153,
+                                  -0.013935825648041482, 0.011358946619800086, -0.0088917876993182109,
+                                  0.0057663572208138262, -0.0021645995498866606};
+      wL = -(w * tau * rX) * poly(a11, y2);
+    } else {
+      wL = w * (0.6931471805599453 * log2_pos(u * rX * rcp_full(tau + w)));
+    }
   }
-  if (x > 1.0) {
-    const double sv = ::sqrt(x * x - 1.0);
-    return atan_dbl(sv) * rcp_refined(sv);
+  B = fma(wL, rd[TN_C1], B0 + rd[TN_C0]);
+  if constexpr (GRAD) {
+    const double LC = wL * iw * rd[TN_C1] * iw;  // L C1 / w
+    XBX = fma(u, LC, X0 + rd[TN_T2M1]);
+    tBt = fma(tau2, LC, fma(wL, rd[TN_E1], t0 + rd[TN_D0]));
   }
-  return x;
 }
-__device__ __forceinline__ float tnfw_F(float x) { return nfw_h_f32(x); }
+
+// TNFW deflection, LensModel/Profiles/tnfw.py:67-87, :226-248, FP64 form:
+// alpha = 4 rho0 Rs g / X^2 (dx, dy); X = max(R, 0.001 Rs) / Rs.
+__device__ __forceinline__ void tnfw_defl_f64(const double *rd, double x, double y, double &ax, double &ay) {
+  const double dx = x - rd[R_CX], dy = y - rd[R_CY];
+  const double xs = dx * rd[TN_IRS], ys = dy * rd[TN_IRS];
+  const double u = fmax(fma(xs, xs, ys * ys), 1e-6);
+  double iu, B, d0, d1;
+  tnfw_core<false>(rd, u, iu, B, d0, d1);
+  const double a = rd[TN_AP] * B * iu;
+  ax = fma(a, dx, ax);
+  ay = fma(a, dy, ay);
+}
 
 // TNFW deflection, LensModel/Profiles/tnfw.py:67-87, :226-248, _g :329-349,
-// _L :276-286 (Baltz, Marshall & Oguri 2009).
+// _L :276-286 (Baltz, Marshall & Oguri 2009), float form (the double one: tnfw_defl_f64).
 template <typename T>
 __device__ __forceinline__ void tnfw_defl(const Rec<T> &r, double x, double y, double &ax, double &ay) {
   const double dxd = x - r.d[R_CX], dyd = y - r.d[R_CY];
@@ -965,7 +1134,7 @@ __device__ __forceinline__ void tnfw_defl(const Rec<T> &r, double x, double y, d
   R = R > rmin ? R : rmin;
   T X = R * r[TN_IRS];
   X = X > T(0.001) ? X : T(0.001);
-  if (sizeof(T) == sizeof(float) && X < T(1)) {
+  if (X < T(1)) {
     // Inside the scale radius the terms of g cancel to O(X^2 ln X).  With
     // s = sqrt(1 - X^2), w = sqrt(tau^2 + X^2) and F = atanh(s)/s, the bracket
     // of g equals X^2 C with
@@ -994,7 +1163,7 @@ __device__ __forceinline__ void tnfw_defl(const Rec<T> &r, double x, double y, d
     ay += double(a * float(dy));
     return;
   }
-  if (sizeof(T) == sizeof(float) && X >= T(1.5)) {
+  if (X >= T(1.5)) {
     // Outside the scale radius (2 X^2 + tau^2 - 1) F(X) and -pi sqrt(tau^2 + X^2)
     // both grow like pi X and cancel to O(1).  With v = sqrt(X^2 - 1),
     // w = sqrt(X^2 + tau^2) and F = (pi/2 - atan(1/v)) / v, their sum is
@@ -1026,19 +1195,20 @@ __device__ __forceinline__ void tnfw_defl(const Rec<T> &r, double x, double y, d
     ay += double(a * float(dy));
     return;
   }
-  const T tau = r[TN_TAU], tau2 = r[TN_TAU2];
-  const T X2 = X * X;
-  const T sqtx = Fn<T>::sqrt_(tau2 + X2);
-  // the FP64 form's divisions as refined reciprocals (within two ulp)
-  constexpr bool kDbl = sizeof(T) == sizeof(double);
-  // (the FP64 logarithm of the positive ratio by log2_pos)
-  const T L = kDbl ? T(log2_pos(double(X) * rcp_refined(double(tau + sqtx))) * 0.6931471805599453)
-                   : Fn<T>::log_(X / (tau + sqtx));
-  const T g = r[TN_PRE] * ((r[TN_T2P1] + T(2) * (X2 - T(1))) * tnfw_F(X) + r[TN_C0] +
-                           sqtx * (T(-M_PI) + L * r[TN_C1]));
-  const T a = kDbl ? r[TN_A] * g * T(rcp_refined(double(X2))) : r[TN_A] * g / X2;
+  const float tau = r[TN_TAU], tau2 = r[TN_TAU2];
+  const float X2 = X * X;
+  const float sqtx = Fn<float>::sqrt_(tau2 + X2);
+  const float L = Fn<float>::log_(X / (tau + sqtx));
+  const float g = r[TN_PRE] * ((r[TN_T2P1] + 2.f * (X2 - 1.f)) * nfw_h_f32(X) + r[TN_C0] +
+                               sqtx * (float(-M_PI) + L * r[TN_C1]));
+  const float a = r[TN_A] * g / X2;
   ax += double(a * dx);
   ay += double(a * dy);
+}
+
+template <>
+__device__ __forceinline__ void tnfw_defl<double>(const Rec<double> &r, double x, double y, double &ax, double &ay) {
+  tnfw_defl_f64(r.d, x, y, ax, ay);
 }
 
 // External shear, LensModel/Profiles/shear.py:37-53 (linear: kept in double).
