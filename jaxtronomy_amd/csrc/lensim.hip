@@ -222,6 +222,7 @@ struct Layout {
   size_t gpart_mp;             // gradient, several planes: per-block partials of the deflectors (0: none)
   size_t gpad, gext;           // edge-padded PSF adjoint: padded dlogL/dmodel and its correlation
   size_t gchr, glu;            // supersampled convolution adjoint buffers
+  size_t mp_tab;               // several planes: the plane runs (mp_runs_kernel)
   size_t hr, chr, lowu, lowc, psf_low;  // supersampled convolution: ray fluxes, their convolution,
                                         // pooled unconvolved image and its low-resolution convolution
   size_t total;
@@ -344,6 +345,16 @@ struct SSPlan {
   int kxl = 0, kyl = 0;  // low-resolution split kernel (0: none)
 };
 
+// The plane runs of a multi-plane model (mp_runs_kernel), int32 per set of
+// plane arrays (one for the batch when they are shared): [0] the number of
+// runs n, [1] whether a deflector is on several planes, [2] whether the bulk
+// list holds subhalos and linear deflectors only, then run starts
+// [n + 1 <= mp_n], the run of each plane [mp_n - 1], the plane of each
+// deflector [n_defl], and the deflector of each plane with its type
+// [mp_n - 1] (index + 2^24 type).
+__host__ __device__ inline int mp_tab_ints(const ModelArgs &m) { return 1 + 3 * m.mp_n + m.n_defl; }
+size_t mp_tab_sets(const ModelArgs &m, int n_img) { return m.mp_stride ? size_t(n_img) : 1; }
+
 Layout layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img, int precision,
               const SSPlan &ss = SSPlan()) {
   Layout L{};
@@ -393,6 +404,8 @@ Layout layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img, int
       off = align256(off + size_t(ss.kxl) * kyp_of(ss.kyl) * 8);
     }
   }
+  L.mp_tab = off;
+  if (m.mp_n > 0) off = align256(off + mp_tab_sets(m, n_img) * size_t(mp_tab_ints(m)) * 4);
   L.bfrag = off;  // int exponent (16 B slot) then the MFMA B fragments (float64 fragments in the FP64 form)
   if (precision == LENSIM_MIXED) off = align256(off + 16 + size_t(mfma_steps(kx, ky)) * 2 * 64 * 16);
   else off = align256(off + size_t(mf64_steps(kx, ky)) * 64 * sizeof(double));
@@ -665,54 +678,28 @@ __device__ __forceinline__ void deflect_all(const ModelArgs &m, const RecPtrs<T>
   deflect_bulk<T, HALO, DBL, DBL_TNFW>(m, rp, x, y, ax, ay);
 }
 
-// One deflector k (inline lens k < n_lens with its series coefficients, or bulk).
-template <typename T, bool HALO, bool DBL, bool DBL_TNFW = DBL>
-__device__ __forceinline__ void deflect_one(const ModelArgs &m, const RecPtrs<T> &rp, int img, int k, double x,
-                                            double y, double &ax, double &ay) {
+// One deflector k of type `type` (inline lens k < n_lens with its series coefficients, or bulk).
+template <typename T, bool HALO, bool DBL, bool DBL_TNFW = DBL, bool SUB = false>
+__device__ __forceinline__ void deflect_one(const ModelArgs &m, const RecPtrs<T> &rp, int img, int k, int type,
+                                            double x, double y, double &ax, double &ay) {
   const Rec<T> r{rp.recd + k * kRec, rp.rect + k * kRec};
-  if (k < m.n_lens) {
-    const int e = m.epl_index[k];
-    const size_t co = (e >= 0) ? (size_t(img) * m.n_epl + e) * LENSIM_EPL_NMAX : 0;
-    if (e >= 0) CHECK_SPAN(rp.coeft + co, LENSIM_EPL_NMAX * sizeof(T));
-    add_deflection<T, HALO, DBL, DBL_TNFW>(m.types[k], r, rp.coefd + co, rp.coeft + co, x, y, ax, ay);
-  } else {
-    const int type = m.bulk_type ? m.bulk_type : AT(m.bulk_types, k - m.n_lens);
-    add_deflection<T, HALO, DBL, DBL_TNFW>(type == LENSIM_EPL ? LENSIM_NULL : type, r, nullptr, nullptr, x, y, ax, ay);
+  size_t co = 0;
+  if (!SUB && type == LENSIM_EPL) {
+    co = (size_t(img) * m.n_epl + m.epl_index[k]) * LENSIM_EPL_NMAX;
+    CHECK_SPAN(rp.coeft + co, LENSIM_EPL_NMAX * sizeof(T));
   }
+  add_deflection<T, HALO, DBL, DBL_TNFW, SUB>(type, r, rp.coefd + co, rp.coeft + co, x, y, ax, ay);
 }
 
-// Source-plane position of the ray at angle (x, y): single plane
-// beta = theta - alpha_scaling * alpha, or the multi-plane recursion of
-// MultiPlaneBulk.ray_shooting (LensModel/MultiPlane/multi_plane_bulk.py:152-212).
+// Source-plane position of the ray at angle (x, y) on a single plane:
+// beta = theta - alpha_scaling * alpha.
 template <typename T, bool HALO, bool DBL, bool DBL_TNFW = DBL>
 __device__ __forceinline__ void trace_ray(const ModelArgs &m, const RecPtrs<T> &rp, int img, double x, double y,
                                           double &bx, double &by) {
-  if (m.mp_n == 0) {
-    double ax = 0.0, ay = 0.0;
-    deflect_all<T, HALO, DBL, DBL_TNFW>(m, rp, img, x, y, ax, ay);
-    bx = x - ax * m.alpha_scaling;
-    by = y - ay * m.alpha_scaling;
-    return;
-  }
-  const size_t o = size_t(img) * size_t(m.mp_stride);
-  double angx = x, angy = y, px = 0.0, py = 0.0, tz = 1.0;
-  for (int p = 0; p < m.mp_n; ++p) {
-    const double dt = AT(m.mp_tij, o + p);
-    tz = AT(m.mp_tz, o + p);
-    px += angx * dt;
-    py += angy * dt;
-    if (p + 1 < m.mp_n) {
-      double ax = 0.0, ay = 0.0;
-      int k = AT(m.mp_order, p);
-      k = k < 0 ? 0 : (k >= m.n_defl ? m.n_defl - 1 : k);  // a bad index cannot read outside the records
-      deflect_one<T, HALO, DBL, DBL_TNFW>(m, rp, img, k, px / tz, py / tz, ax, ay);
-      const double f = AT(m.mp_r2p, o + p);
-      angx -= ax * f;
-      angy -= ay * f;
-    }
-  }
-  bx = px / tz;
-  by = py / tz;
+  double ax = 0.0, ay = 0.0;
+  deflect_all<T, HALO, DBL, DBL_TNFW>(m, rp, img, x, y, ax, ay);
+  bx = x - ax * m.alpha_scaling;
+  by = y - ay * m.alpha_scaling;
 }
 
 template <typename T>
@@ -1109,24 +1096,21 @@ __global__ __launch_bounds__(256) void block_max_kernel(const T *__restrict__ v,
   block_max_store(a, blkmax + size_t(img) * gridDim.x + blockIdx.x);
 }
 
-// Lanes per ray of the multi-plane kernels that share a plane's deflectors
-// among a quad (raytrace_mp_kernel, render_mp_kernel).
-constexpr int kMpG = 4;
-
-template <typename T, bool HALO, bool DBL>
-__global__ __launch_bounds__(256) void render_mp_kernel(ModelArgs m, GridArgs g, const double *__restrict__ recd,
-                                                        const float *__restrict__ recf,
-                                                        const double *__restrict__ coefd,
-                                                        const float *__restrict__ coeff, unsigned flags,
-                                                        T *__restrict__ out);
+constexpr int kMpBlock = 64;  // rays of a block of the multi-plane kernels (a lane each)
+int launch_mp_runs(const ModelArgs &m, int *tab, int n_img, hipStream_t st);
+template <typename T>
+int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf, const double *coefd,
+                     const float *coeff, const int *tab, unsigned flags, T *out, int n_img, hipStream_t st);
 
 // Launches render_fast_kernel when the model is one of its compile-time lists
 // (EPL, SIE / NIE or NFW, each with or without SHEAR after it, NFW + SIE / NIE
-// in either order; one Sersic source, none or one Sersic lens light), else
+// in either order; one Sersic source, none or one Sersic lens light),
+// render_mp_kernel for several planes (tab: its plane runs), else
 // render_kernel.
 template <typename T>
 int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf, const double *coefd,
-                  const float *coeff, unsigned flags, T *out, float *blkmax, int n_img, hipStream_t st) {
+                  const float *coeff, const int *tab, unsigned flags, T *out, float *blkmax, int n_img,
+                  hipStream_t st) {
   const dim3 rgrid((g.nx * g.ny + 255) / 256, n_img);
   auto sersic = [](int t) { return t == LENSIM_SERSIC || t == LENSIM_SERSIC_ELLIPSE; };
   auto nie = [](int t) { return t == LENSIM_SIE ? LENSIM_NIE : t; };
@@ -1141,28 +1125,8 @@ int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, con
     fast = pair && (d0 != LENSIM_EPL || m.epl_index[0] == 0);
     for (int k = m.n_lens; fast && k < m.n_lens + m.n_source + m.n_light; ++k) fast = sersic(m.types[k]);
   }
-  // a multi-plane launch of fewer than 2 waves per SIMD at one lane per pixel
-  // takes a quad per pixel (render_mp_kernel; the block maxima for the MFMA
-  // convolution follow from the image in a second launch)
-  const bool quad = m.mp_n && size_t(g.nx) * g.ny * size_t(n_img) < 131072;
-  if (!fast && quad) {
-    const dim3 qgrid((unsigned)((size_t(g.nx) * g.ny * kMpG + 255) / 256), n_img);
-#define LENSIM_RENDER(H, D) \
-  render_mp_kernel<T, H, D><<<qgrid, 256, 0, st>>>(m, g, recd, recf, coefd, coeff, flags, out)
-    bool done = false;
-    if constexpr (sizeof(T) == sizeof(float)) {
-      if (m.has_nie_nfw) {
-        if (m.has_halo) LENSIM_RENDER(true, true);
-        else LENSIM_RENDER(false, true);
-        done = true;
-      }
-    }
-    if (!done) {
-      if (m.has_halo) LENSIM_RENDER(true, false);
-      else LENSIM_RENDER(false, false);
-    }
-#undef LENSIM_RENDER
-    int rc = check_launch("render_mp_kernel");
+  if (m.mp_n) {  // the block maxima for the MFMA convolution follow from the image in a second launch
+    int rc = launch_render_mp<T>(m, g, recd, recf, coefd, coeff, tab, flags, out, n_img, st);
     if (rc || !blkmax) return rc;
     block_max_kernel<T><<<rgrid, 256, 0, st>>>(out, g.nx * g.ny, blkmax);
     return check_launch("block_max_kernel");
@@ -1255,150 +1219,327 @@ __device__ __forceinline__ double wave_sum(double v) {
   return (row(0) + row(16)) + (row(32) + row(48));
 }
 
-// Multi-plane ray tracing (MultiPlaneBulk.ray_shooting,
-// LensModel/MultiPlane/multi_plane_bulk.py:152-212) with kMpG lanes per ray.
+// ---- several planes ----
 // Deflectors on one plane follow each other in the plane order with T_ij = 0
-// between them, so the ray's comoving position does not move across them and
-// they all deflect it at one position: lane j of the ray's quad evaluates
-// deflector p + j of such a run (up to kMpG at a time) and a quad sum adds the
-// r2p-weighted deflections, which the reference subtracts one after another.
-// The order and the T arrays are the same for every ray of an image, so the
-// runs are uniform across the wave (scalar loads and branches).  A ray's
-// solitary plane-by-plane chain of record loads and deflections is kMpG times
-// shorter, and an image of 400^2 rays fills 10 waves per SIMD instead of 2.5.
-// The float form takes it (the line-of-sight workload: 9.1 -> 8.5 ms); the
-// FP64 form's software transcendentals keep the vector ALU busy at 2.5 waves
-// per SIMD already, and the gathers and quad sums made it slower (10.8 ->
-// 11.9 ms), so it keeps one lane per ray.
+// between them: the ray does not move across them and they all deflect it at
+// one position.  A run is up to kMpRun consecutive planes with one position,
+// T_z and reduced-to-physical factor; it is the unit the kernels below work in.
+constexpr int kMpRun = 64;
 
-template <typename T, bool HALO, bool DBL>
-__global__ __launch_bounds__(256) void raytrace_mp_kernel(ModelArgs m, const double *__restrict__ recd,
-                                                          const float *__restrict__ recf,
-                                                          const double *__restrict__ coefd,
-                                                          const float *__restrict__ coeff,
-                                                          const double *__restrict__ xs,
-                                                          const double *__restrict__ ys, int64_t n_ray,
-                                                          double *__restrict__ bx, double *__restrict__ by) {
-  const int img = blockIdx.y;
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int slot = threadIdx.x & (kMpG - 1);
-  const int64_t ray0 = t / kMpG;
-  const bool active = ray0 < n_ray;
-  const int64_t ray = active ? ray0 : n_ray - 1;  // a quad past the end follows the last ray (for the sums)
-  const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
-  const size_t o = size_t(img) * size_t(m.mp_stride);
-  const double *tij = m.mp_tij + o, *tzs = m.mp_tz + o, *r2p = m.mp_r2p + o;
-  double angx = AT(xs, ray), angy = AT(ys, ray), px = 0.0, py = 0.0;
-  const int nd = m.mp_n - 1;  // planes with a deflector; the last one is the source's
-  int p = 0;
-  while (p < nd) {
-    const double dt = AT(tij, p);
-    px += angx * dt;
-    py += angy * dt;
-    // deflectors p .. p + mc - 1 see the same position
-    int mc = 1;
-    while (mc < kMpG && p + mc < nd && AT(tij, p + mc) == 0.0) ++mc;
-    double ax = 0.0, ay = 0.0;
-    if (slot < mc) {
-      const int q = p + slot;
-      int k = AT(m.mp_order, q);
-      k = k < 0 ? 0 : (k >= m.n_defl ? m.n_defl - 1 : k);  // a bad index cannot read outside the records
-      const double tz = AT(tzs, q);
-      double dx = 0.0, dy = 0.0;
-      deflect_one<T, HALO, DBL, false>(m, rp, img, k, px / tz, py / tz, dx, dy);
-      const double f = AT(r2p, q);
-      ax = dx * f;
-      ay = dy * f;
+struct MpTab {  // see mp_tab_ints
+  const int *start, *run_of, *plane_of, *who;
+  int n, dup, sub;
+};
+static_assert(LENSIM_CONVERGENCE < 128, "a deflector's type shares an int with its index");
+constexpr int kWhoBits = 24;
+
+__host__ __device__ constexpr bool sub_type(int t) {  // add_deflection's SUB
+  return t == LENSIM_NULL || t == LENSIM_TNFW || t == LENSIM_SHEAR || t == LENSIM_CONVERGENCE;
+}
+__device__ __forceinline__ MpTab mp_tab(const ModelArgs &m, const int *__restrict__ tab, int img) {
+  const int *t = tab + (m.mp_stride ? size_t(img) * mp_tab_ints(m) : 0);
+  CHECK_SPAN(t, size_t(mp_tab_ints(m)) * sizeof(int));
+  return MpTab{t + 3,    t + 3 + m.mp_n, t + 2 + 2 * m.mp_n, t + 2 + 2 * m.mp_n + m.n_defl, t[0],
+               t[1], t[2]};
+}
+
+// The runs of each set of plane arrays, one block per set: every thread takes
+// a contiguous piece of the planes; a maximum scan over the pieces gives the
+// plane the position last changed at, and so the planes that start a run
+// (there, and every kMpRun planes after), a sum scan their numbers.
+__global__ __launch_bounds__(1024) void mp_runs_kernel(ModelArgs m, int *__restrict__ tab_all) {
+  int *tab = tab_all + size_t(blockIdx.x) * mp_tab_ints(m);
+  const size_t o = size_t(blockIdx.x) * size_t(m.mp_stride);
+  const int nd = m.mp_n - 1, t = threadIdx.x, per = (nd + 1023) / 1024;
+  const int q0 = min(nd, t * per), q1 = min(nd, q0 + per);
+  int *start = tab + 3, *run_of = tab + 3 + m.mp_n, *plane_of = tab + 2 + 2 * m.mp_n;
+  int *who = plane_of + m.n_defl;
+  auto moved = [&](int q) {
+    return q == 0 || AT(m.mp_tij, o + q) != 0.0 || AT(m.mp_tz, o + q) != AT(m.mp_tz, o + q - 1) ||
+           AT(m.mp_r2p, o + q) != AT(m.mp_r2p, o + q - 1);
+  };
+  __shared__ int sc[2][1024];
+  __shared__ int dup, other;
+  auto scan = [&](int v, auto op) {  // inclusive, over the threads
+    sc[0][t] = v;
+    __syncthreads();
+    int b = 0;
+    for (int d = 1; d < 1024; d <<= 1, b ^= 1) {
+      sc[b ^ 1][t] = t >= d ? op(sc[b][t], sc[b][t - d]) : sc[b][t];
+      __syncthreads();
     }
-    angx -= quad_sum(ax);
-    angy -= quad_sum(ay);
-    p += mc;
+    const int r = sc[b][t];
+    const int before = t ? sc[b][t - 1] : -1;
+    __syncthreads();
+    return make_int2(r, before);
+  };
+  int last = -1;
+  for (int q = q0; q < q1; ++q)
+    if (moved(q)) last = q;
+  const int from = scan(last, [](int a, int b) { return a > b ? a : b; }).y;
+  int at = from, cnt = 0;
+  for (int q = q0; q < q1; ++q) {
+    if (moved(q)) at = q;
+    cnt += (q - at) % kMpRun == 0;
   }
-  const double dt = AT(tij, nd);
-  px += angx * dt;
-  py += angy * dt;
-  const double tz = AT(tzs, nd);
-  if (active && slot == 0) {
-    AT(bx, size_t(img) * n_ray + ray) = px / tz;
-    AT(by, size_t(img) * n_ray + ray) = py / tz;
+  const int2 s = scan(cnt, [](int a, int b) { return a + b; });
+  int idx = t ? s.y : 0;
+  at = from;
+  for (int q = q0; q < q1; ++q) {
+    if (moved(q)) at = q;
+    if ((q - at) % kMpRun == 0) AT(start, idx++) = q;
+    AT(run_of, q) = idx - 1;
+  }
+  for (int k = t; k < m.n_defl; k += 1024) AT(plane_of, k) = -1;
+  if (t == 0) dup = other = 0;
+  __syncthreads();
+  for (int k = t; m.n_bulk > 0 && !m.bulk_type && k < m.n_bulk; k += 1024)
+    if (!sub_type(AT(m.bulk_types, k))) other = 1;
+  for (int q = q0; q < q1; ++q) {
+    int k = AT(m.mp_order, q);
+    k = k < 0 ? 0 : (k >= m.n_defl ? m.n_defl - 1 : k);  // a bad index cannot read outside the records
+    if (atomicExch(&AT(plane_of, k), q) >= 0) dup = 1;
+    int type = k < m.n_lens ? m.types[k] : (m.bulk_type ? m.bulk_type : AT(m.bulk_types, k - m.n_lens));
+    if (k >= m.n_lens && !bulk_type_ok_dev(type)) type = LENSIM_NULL;
+    AT(who, q) = k | type << kWhoBits;
+  }
+  __syncthreads();
+  if (t == 1023) {
+    AT(start, s.x) = nd;
+    AT(tab, 0) = s.x;
+    AT(tab, 1) = dup;
+    AT(tab, 2) = !other;
   }
 }
 
-// render_kernel for multi-plane lists with a quad per pixel: the quad walks
-// the pixel's sub-rays together and shares each plane's deflectors among its
-// lanes as raytrace_mp_kernel does (with render_kernel's deflection
-// arithmetic, trace_ray's), so every lane ends with the sub-ray's beta; every
-// lane adds the light, lane 0 stores.  For launches too small to fill the
-// SIMDs at one lane per pixel (a gradient's image of one line-of-sight scene).
-template <typename T, bool HALO, bool DBL>
-__global__ __launch_bounds__(256) void render_mp_kernel(ModelArgs m, GridArgs g, const double *__restrict__ recd,
-                                                        const float *__restrict__ recf,
-                                                        const double *__restrict__ coefd,
-                                                        const float *__restrict__ coeff, unsigned flags,
-                                                        T *__restrict__ out) {
+int launch_mp_runs(const ModelArgs &m, int *tab, int n_img, hipStream_t st) {
+  mp_runs_kernel<<<(unsigned)mp_tab_sets(m, n_img), 1024, 0, st>>>(m, tab);
+  return check_launch("mp_runs_kernel");
+}
+
+// The sums of (vx, vy) over the block's waves (lane by lane), in wave order, in
+// every wave.  buf alternates between consecutive calls, so one barrier does.
+__device__ __forceinline__ void across_waves(double2 (*red)[16][64], int buf, int nw, double &vx, double &vy) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  red[buf][wave][lane] = double2{vx, vy};
+  __syncthreads();
+  vx = vy = 0.0;
+  for (int w = 0; w < nw; ++w) {
+    const double2 v = red[buf][w][lane];
+    vx += v.x;
+    vy += v.y;
+  }
+}
+
+// Multi-plane ray tracing (MultiPlaneBulk.ray_shooting,
+// LensModel/MultiPlane/multi_plane_bulk.py:152-212) of 64 rays, one per lane,
+// by the whole block: each of its waves holds the same rays and takes every
+// nw-th deflector of a run, and the waves' sums meet in LDS once per run.  The
+// deflector is then the same for all lanes of a wave (its record comes by
+// scalar loads), 1 / T_z is taken once per run, and the chain of
+// record loads and deflections a ray waits for is nw times shorter: one lane
+// per ray left 400^2 rays at 2.4 waves per SIMD, waiting on memory for most of
+// a deflector's 1100 cycles.  Every thread of the block reaches this call.
+// each(c, x, y): run c's position, for callers that keep it.
+template <typename T, bool HALO, bool DBL, bool DBL_TNFW, bool SUB, typename F>
+__device__ __forceinline__ void block_trace(const ModelArgs &m, const RecPtrs<T> &rp, const MpTab &tab,
+                                            const double *__restrict__ tij, const double *__restrict__ tzs,
+                                            const double *__restrict__ r2p, int img, double x, double y,
+                                            double2 (*red)[16][64], double &bx, double &by, F each) {
+  const int lane = threadIdx.x & 63, nw = int(blockDim.x) >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double angx = x, angy = y, px = 0.0, py = 0.0;
+  // the deflectors of a run, a lane each, loaded one run ahead
+  auto members = [&](int p0, int p1) { return p0 + lane < p1 ? AT(tab.who, p0 + lane) : 0; };
+  int p0 = 0, p1 = tab.n ? AT(tab.start, 1) : 0;
+  int ks = members(p0, p1);
+  double dt = AT(tij, 0), itz = rcp_full(AT(tzs, 0)), f = AT(r2p, 0);
+  for (int c = 0; c < tab.n; ++c) {
+    const int p2 = c + 1 < tab.n ? AT(tab.start, c + 2) : p1;
+    const int ks_next = members(p1, p2);
+    const double dt_next = AT(tij, p1), tz_next = AT(tzs, p1), f_next = AT(r2p, p1);  // p1 <= nd: the source's plane
+    px = fma(angx, dt, px);
+    py = fma(angy, dt, py);
+    const double xr = px * itz, yr = py * itz;
+    each(c, xr, yr);
+    double ax = 0.0, ay = 0.0;
+    for (int q = wave; q < p1 - p0; q += nw) {
+      const int k = __builtin_amdgcn_readlane(ks, q);
+      deflect_one<T, HALO, DBL, DBL_TNFW, SUB>(m, rp, img, k & ((1 << kWhoBits) - 1), k >> kWhoBits, xr, yr, ax, ay);
+    }
+    across_waves(red, c & 1, nw, ax, ay);
+    angx = fma(-ax, f, angx);
+    angy = fma(-ay, f, angy);
+    p0 = p1;
+    p1 = p2;
+    ks = ks_next;
+    dt = dt_next;
+    itz = rcp_full(tz_next);
+    f = f_next;
+  }
+  px = fma(angx, dt, px);  // the source's plane
+  py = fma(angy, dt, py);
+  bx = px * itz;
+  by = py * itz;
+}
+
+// The plane arrays of image img as restrict pointers.
+#define LENSIM_MP_ARRAYS(m, img)                                        \
+  const size_t mp_o = size_t(img) * size_t((m).mp_stride);              \
+  const double *tij = (m).mp_tij + mp_o, *tzs = (m).mp_tz + mp_o, *r2p = (m).mp_r2p + mp_o
+
+// Waves per block for n rays an image: enough that a launch of one image
+// puts four or more waves on each SIMD where its deflectors allow it, and no
+// more, since a run is cut into as many pieces.  It depends on the image
+// alone (not on the batch), as the order of the sums does.  Measured on the
+// line of sight (400^2 rays): 3.42 ms a call with 8 waves, 3.50 with 4, 4.16
+// with 6; 100^2 rays render in 0.49 ms with 16.  Past 2^28 rays two, which keeps a launch's
+// threads below 2^32.
+int mp_waves(size_t n_ray, bool sub) {
+  if (n_ray > (size_t(1) << 28)) return 2;
+  return sub && n_ray < 65536 ? 16 : 8;
+}
+
+template <typename T, bool HALO, bool DBL, bool SUB>
+__global__ __launch_bounds__(SUB ? 1024 : 512) void raytrace_mp_kernel(ModelArgs m, const double *__restrict__ recd,
+                                                           const float *__restrict__ recf,
+                                                           const double *__restrict__ coefd,
+                                                           const float *__restrict__ coeff,
+                                                           const int *__restrict__ tab_all,
+                                                           const double *__restrict__ xs,
+                                                           const double *__restrict__ ys, int64_t n_ray,
+                                                           int64_t first, bool both, double *__restrict__ bx,
+                                                           double *__restrict__ by) {
+  __shared__ double2 red[2][16][64];
+  const int img = blockIdx.y;
+  const int64_t ray0 = first + int64_t(blockIdx.x) * kMpBlock + (threadIdx.x & 63);
+  const bool active = ray0 < n_ray;
+  const int64_t ray = active ? ray0 : n_ray - 1;  // lanes past the end follow the last ray
+  const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
+  const MpTab tab = mp_tab(m, tab_all, img);
+  if (both && bool(tab.sub) != SUB) return;  // the other instantiation's launch takes it
+  LENSIM_MP_ARRAYS(m, img);
+  double tx, ty;
+  block_trace<T, HALO, DBL, false, SUB>(m, rp, tab, tij, tzs, r2p, img, AT(xs, ray), AT(ys, ray), red, tx,
+                                        ty, [](int, double, double) {});
+  if (active && threadIdx.x < 64) {
+    AT(bx, size_t(img) * n_ray + ray) = tx;
+    AT(by, size_t(img) * n_ray + ray) = ty;
+  }
+}
+
+// render_kernel for several planes: the block's waves walk the sub-rays of its
+// 64 pixels together (block_trace); the first wave adds the light and stores.
+template <typename T, bool HALO, bool DBL, bool SUB>
+__global__ __launch_bounds__(SUB ? 1024 : 512) void render_mp_kernel(ModelArgs m, GridArgs g, const double *__restrict__ recd,
+                                                         const float *__restrict__ recf,
+                                                         const double *__restrict__ coefd,
+                                                         const float *__restrict__ coeff,
+                                                         const int *__restrict__ tab_all, unsigned flags, bool both,
+                                                         T *__restrict__ out) {
+  __shared__ double2 red[2][16][64];
   const int img = blockIdx.y;
   const int npix = g.nx * g.ny;
-  const int slot = threadIdx.x & (kMpG - 1);
-  const int pix0 = int((size_t(blockIdx.x) * blockDim.x + threadIdx.x) / kMpG);
+  const int pix0 = blockIdx.x * kMpBlock + (threadIdx.x & 63);
   const bool active = pix0 < npix;
   const int pix = active ? pix0 : npix - 1;
   int i;
   const int j = div_by(pix, g.nx, g.inv_nx, i);
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
+  const MpTab tab = mp_tab(m, tab_all, img);
+  if (both && bool(tab.sub) != SUB) return;  // the other instantiation's launch takes it
+  LENSIM_MP_ARRAYS(m, img);
   const double ra_c = i * g.m00 + j * g.m01 + g.ra0;
   const double dec_c = i * g.m10 + j * g.m11 + g.dec0;
-  const double inv_s = g.inv_s;
-  const double o0 = g.o0;
   const bool do_src = (flags & LENSIM_IMAGE_SOURCE) && m.n_source > 0;
   const bool do_light = (flags & LENSIM_IMAGE_LENS_LIGHT) && m.n_light > 0;
   const int k_src0 = m.n_defl, k_src1 = m.n_defl + m.n_source, k_l1 = m.n_prof;
-  const size_t o = size_t(img) * size_t(m.mp_stride);
-  const double *tij = m.mp_tij + o, *tzs = m.mp_tz + o, *r2p = m.mp_r2p + o;
-  const int nd = m.mp_n - 1;  // planes with a deflector; the last one is the source's
   double acc = 0.0;
-  const bool eval = active && evaluated(g, i, j);  // one value per quad (one pixel)
-  for (int sy = 0; eval && sy < g.s; ++sy) {
-    const double oy = o0 + sy * inv_s;
+  const bool eval = active && evaluated(g, i, j);
+  const bool any = __any(eval);  // the same in every wave: they hold the same pixels
+  for (int sy = 0; any && sy < g.s; ++sy) {
+    const double oy = g.o0 + sy * g.inv_s;
     for (int sx = 0; sx < g.s; ++sx) {
-      const double ox = o0 + sx * inv_s;
+      const double ox = g.o0 + sx * g.inv_s;
       const double x = ra_c + g.m00 * ox + g.m01 * oy;
       const double y = dec_c + g.m10 * ox + g.m11 * oy;
+      double bx = x, by = y;
       if (do_src) {
-        double angx = x, angy = y, px = 0.0, py = 0.0;
-        int p = 0;
-        while (p < nd) {
-          const double dt = AT(tij, p);
-          px += angx * dt;
-          py += angy * dt;
-          int mc = 1;  // deflectors p .. p + mc - 1 see the same position
-          while (mc < kMpG && p + mc < nd && AT(tij, p + mc) == 0.0) ++mc;
-          double ax = 0.0, ay = 0.0;
-          if (slot < mc) {
-            const int q = p + slot;
-            int k = AT(m.mp_order, q);
-            k = k < 0 ? 0 : (k >= m.n_defl ? m.n_defl - 1 : k);  // a bad index cannot read outside the records
-            const double tz = AT(tzs, q);
-            double dx = 0.0, dy = 0.0;
-            deflect_one<T, HALO, DBL, DBL>(m, rp, img, k, px / tz, py / tz, dx, dy);
-            const double f = AT(r2p, q);
-            ax = dx * f;
-            ay = dy * f;
-          }
-          angx -= quad_sum(ax);
-          angy -= quad_sum(ay);
-          p += mc;
-        }
-        const double dt = AT(tij, nd);
-        px += angx * dt;
-        py += angy * dt;
-        const double tz = AT(tzs, nd);
-        acc += light_sum<T>(m, rp, k_src0, k_src1, px / tz, py / tz);
+        __syncthreads();  // the last sub-ray's sums are read
+        block_trace<T, HALO, DBL, DBL, SUB>(m, rp, tab, tij, tzs, r2p, img, x, y, red, bx, by,
+                                            [](int, double, double) {});
       }
-      if (do_light) acc += light_sum<T>(m, rp, k_src1, k_l1, x, y);
+      if (eval && threadIdx.x < 64) {
+        if (do_src) acc += light_sum<T>(m, rp, k_src0, k_src1, bx, by);
+        if (do_light) acc += light_sum<T>(m, rp, k_src1, k_l1, x, y);
+      }
     }
   }
   const T v = T(acc * (g.scale * m.flux_scaling));
-  if (active && slot == 0) AT(out, size_t(img) * npix + pix) = v;
+  if (active && threadIdx.x < 64) AT(out, size_t(img) * npix + pix) = v;
+}
+
+// Whether every deflector is a subhalo or linear (add_deflection's SUB): 1
+// yes, 0 no, 2 when only the device knows (bulk deflectors of several types:
+// both instantiations are launched then, and mp_runs_kernel's flag ends one).
+int sub_list(const ModelArgs &m) {
+  for (int k = 0; k < m.n_lens; ++k)
+    if (!sub_type(m.types[k])) return 0;
+  if (m.n_bulk == 0) return 1;
+  return m.bulk_type ? int(sub_type(m.bulk_type)) : 2;
+}
+
+template <typename T>
+int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf, const double *coefd,
+                     const float *coeff, const int *tab, unsigned flags, T *out, int n_img, hipStream_t st) {
+  const size_t npix = size_t(g.nx) * g.ny;
+  const dim3 grid((unsigned)((npix + kMpBlock - 1) / kMpBlock), n_img);
+  const int sub = sub_list(m);
+#define LENSIM_RENDER(H, D, S)                                                                                \
+  render_mp_kernel<T, H, D, S><<<grid, 64 * mp_waves(npix, S), 0, st>>>(m, g, recd, recf, coefd, coeff, tab, \
+                                                                       flags, sub == 2, out)
+  // the float form deflects SIE / NIE and the NFW family in double
+  constexpr bool kF32 = sizeof(T) == sizeof(float);
+  if (sub) LENSIM_RENDER(true, kF32, true);
+  if (sub != 1) {
+    if (kF32 && m.has_nie_nfw && m.has_halo) LENSIM_RENDER(true, kF32, false);
+    else if (kF32 && m.has_nie_nfw) LENSIM_RENDER(false, kF32, false);
+    else if (m.has_halo) LENSIM_RENDER(true, false, false);
+    else LENSIM_RENDER(false, false, false);
+  }
+#undef LENSIM_RENDER
+  return check_launch("render_mp_kernel");
+}
+
+// raytrace_mp_kernel's launches for a call, in pieces of 2^28 rays (a launch's
+// threads stay below 2^32).
+template <typename T>
+int launch_raytrace_mp(const ModelArgs &m, const double *recd, const float *recf, const double *coefd,
+                       const float *coeff, const int *tab, const double *x, const double *y, int64_t n_ray, int n_img,
+                       double *bx, double *by, hipStream_t st) {
+  const int sub = sub_list(m);
+  constexpr bool kF32 = sizeof(T) == sizeof(float);
+  constexpr int64_t kPiece = int64_t(1) << 28;
+  for (int64_t r0 = 0; r0 < n_ray; r0 += kPiece) {
+    const int64_t nr = n_ray - r0 < kPiece ? n_ray - r0 : kPiece;
+    const dim3 grid((unsigned)((nr + kMpBlock - 1) / kMpBlock), n_img);
+#define LENSIM_TRACE(H, D, S)                                                                              \
+  raytrace_mp_kernel<T, H, D, S><<<grid, 64 * mp_waves(size_t(n_ray), S), 0, st>>>(                        \
+      m, recd, recf, coefd, coeff, tab, x, y, n_ray, r0, sub == 2, bx, by)
+    // the float form keeps the float TNFW of a list without SIE / NIE or NFW
+    // (rays within 2e-6 of FP64); those deflect in double (see nie_defl)
+    if (sub) LENSIM_TRACE(true, false, true);
+    if (sub != 1) {
+      if (kF32 && m.has_nie_nfw && m.has_halo) LENSIM_TRACE(true, kF32, false);
+      else if (kF32 && m.has_nie_nfw) LENSIM_TRACE(false, kF32, false);
+      else if (m.has_halo) LENSIM_TRACE(true, false, false);
+      else LENSIM_TRACE(false, false, false);
+    }
+#undef LENSIM_TRACE
+    const int rc = check_launch("raytrace_mp_kernel");
+    if (rc) return rc;
+  }
+  return LENSIM_OK;
 }
 
 template <typename T>
@@ -2894,7 +3035,9 @@ __global__ __launch_bounds__(256) void mp_grad_kernel(ModelArgs m, GridArgs g, G
           double ax = 0.0, ay = 0.0;
           int k = AT(m.mp_order, p);
           k = k < 0 ? 0 : (k >= m.n_defl ? m.n_defl - 1 : k);
-          deflect_one<T, HALO, true>(m, rp, img, k, Px / tz, Py / tz, ax, ay);
+          int type = type_of(m, k);
+          if (k >= m.n_lens && type == LENSIM_EPL) type = LENSIM_NULL;
+          deflect_one<T, HALO, true>(m, rp, img, k, type, Px / tz, Py / tz, ax, ay);
           const double f = AT(m.mp_r2p, o + p);
           Ax -= ax * f;
           Ay -= ay * f;
@@ -3289,12 +3432,14 @@ int run_image(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, i
   T *lowres = reinterpret_cast<T *>(ws + L.lowres);
   float *blkmax = mfma ? reinterpret_cast<float *>(ws + L.blkmax) : nullptr;
   const int npix = g.nx * g.ny;
+  int *tab = reinterpret_cast<int *>(ws + L.mp_tab);
+  if (m.mp_n && (rc = launch_mp_runs(m, tab, n_img, st))) return rc;
   timing_mark(0, st);
   const double *recd = reinterpret_cast<const double *>(ws + L.recd);
   const float *recf = reinterpret_cast<const float *>(ws + L.recf);
   const double *coefd = reinterpret_cast<const double *>(ws + L.coefd);
   const float *coeff = reinterpret_cast<const float *>(ws + L.coeff);
-  rc = launch_render<T>(m, g, recd, recf, coefd, coeff, flags, lowres, blkmax, n_img, st);
+  rc = launch_render<T>(m, g, recd, recf, coefd, coeff, tab, flags, lowres, blkmax, n_img, st);
   if (rc) return rc;
   timing_mark(1, st);
   ConvArgs c{};
@@ -3495,8 +3640,10 @@ int run_image_ss(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf
   const float *recf = reinterpret_cast<const float *>(ws + L.recf);
   const double *coefd = reinterpret_cast<const double *>(ws + L.coefd);
   const float *coeff = reinterpret_cast<const float *>(ws + L.coeff);
+  int *tab = reinterpret_cast<int *>(ws + L.mp_tab);
+  if (m.mp_n && (rc = launch_mp_runs(m, tab, n_img, st))) return rc;
   timing_mark(0, st);
-  rc = launch_render<T>(m, gh, recd, recf, coefd, coeff, flags, hr, blkmax, n_img, st);
+  rc = launch_render<T>(m, gh, recd, recf, coefd, coeff, tab, flags, hr, blkmax, n_img, st);
   if (rc) return rc;
   timing_mark(1, st);
   if (mfma) {
@@ -4216,16 +4363,17 @@ int lensim_raytrace(const lensim_model *model, const double *d_params, int32_t n
   const float *recf = reinterpret_cast<const float *>(w + L.recf);
   const double *coefd = reinterpret_cast<const double *>(w + L.coefd);
   const float *coeff = reinterpret_cast<const float *>(w + L.coeff);
-  const dim3 grid_mp((unsigned)((n_ray * kMpG + 255) / 256), n_img);
-#define LENSIM_TRACE(T, H, D)                                                                                      \
-  do {                                                                                                             \
-    if (m.mp_n && sizeof(T) == sizeof(float))                                                                      \
-      raytrace_mp_kernel<T, H, D><<<grid_mp, 256, 0, st>>>(m, recd, recf, coefd, coeff, d_x, d_y, n_ray, d_beta_x, \
-                                                           d_beta_y);                                             \
-    else                                                                                                           \
-      raytrace_kernel<T, H, D><<<grid, 256, 0, st>>>(m, recd, recf, coefd, coeff, d_x, d_y, n_ray, d_beta_x,       \
-                                                     d_beta_y);                                                   \
-  } while (0)
+  if (m.mp_n) {
+    int *tab = reinterpret_cast<int *>(w + L.mp_tab);
+    if ((rc = launch_mp_runs(m, tab, n_img, st))) return cr.end(st, rc);
+    rc = precision == LENSIM_FP64 ? launch_raytrace_mp<double>(m, recd, recf, coefd, coeff, tab, d_x, d_y, n_ray, n_img,
+                                                               d_beta_x, d_beta_y, st)
+                                  : launch_raytrace_mp<float>(m, recd, recf, coefd, coeff, tab, d_x, d_y, n_ray, n_img,
+                                                              d_beta_x, d_beta_y, st);
+    return cr.end(st, rc);
+  }
+#define LENSIM_TRACE(T, H, D)                                                                                     \
+  raytrace_kernel<T, H, D><<<grid, 256, 0, st>>>(m, recd, recf, coefd, coeff, d_x, d_y, n_ray, d_beta_x, d_beta_y)
   if (precision == LENSIM_FP64) {
     if (m.has_halo) LENSIM_TRACE(double, true, false);
     else LENSIM_TRACE(double, false, false);

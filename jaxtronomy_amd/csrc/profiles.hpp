@@ -270,14 +270,22 @@ enum : int { NIE_C = 2, NIE_S, NIE_Q, NIE_Q2, NIE_SS, NIE_BSQ, NIE_SQ, NIE_Q2S, 
               NIE_YRR, NIE_AC, NIE_AS };
 // NFW     (nfw.py:86-105, :257-279, :384-395): Rs (floored), 4 rho0 Rs, 1/Rs
 enum : int { NFW_RS = 2, NFW_A, NFW_IRS };
-// TNFW    (tnfw.py:67-87, :226-248, :329-349): Rs, 4 rho0 Rs, tau, tau^2,
-//          tau^2/(tau^2+1)^2, tau pi + (tau^2-1) ln tau, (tau^2-1)/tau, 0.001 Rs, tau^2+1, 1/Rs
-enum : int { TN_RS = 2, TN_A, TN_TAU, TN_TAU2, TN_PRE, TN_C0, TN_C1, TN_RMIN, TN_T2P1, TN_IRS,
+// TNFW    (tnfw.py:67-87, :226-248, :329-349).  The first slots are the FP64
+//          form's (tnfw_core), together so that they come by one or two
+//          scalar loads
+enum : int { TN_IRS = 2, // 1/Rs (0 for a negative Rs: X is then at its floor)
+              TN_TAU, TN_TAU2,
+              TN_UFAR,   // X^2 from which both far series converge: 16 max(1, tau^2)
               TN_K,      // pi (tau^2 + 1)^2 / 2
               TN_T2M1,   // tau^2 - 1
-              // the FP64 form's (tnfw_core)
               TN_AP,     // 4 rho0 Rs tau^2/(tau^2+1)^2
-              TN_UFAR,   // X^2 from which both far series converge: max(16, 16 tau^2)
+              TN_C0,     // tau pi + (tau^2-1) ln tau
+              TN_C1,     // (tau^2-1)/tau
+              // the float form's
+              TN_A,      // 4 rho0 Rs
+              TN_PRE,    // tau^2/(tau^2+1)^2
+              TN_RMIN,   // 0.001 Rs
+              TN_T2P1,   // tau^2+1
               // the gradient's (tnfw_ray_grad)
               TN_D0,     // tau pi + 2 tau^2 ln tau
               TN_E1,     // (tau^2 + 1) / tau
@@ -502,7 +510,6 @@ __device__ inline void prepare_record(int type, const double *p, double *rec, do
       const double tau = r_trunc / Rs, tau2 = tau * tau;
       rec[R_CX] = p[3];
       rec[R_CY] = p[4];
-      rec[TN_RS] = Rs;
       rec[TN_A] = 4.0 * rho0 * Rs;
       rec[TN_TAU] = tau;
       rec[TN_TAU2] = tau2;
@@ -511,7 +518,7 @@ __device__ inline void prepare_record(int type, const double *p, double *rec, do
       rec[TN_C1] = (tau2 - 1.0) / tau;
       rec[TN_RMIN] = 0.001 * Rs;
       rec[TN_T2P1] = tau2 + 1.0;
-      rec[TN_IRS] = 1.0 / Rs;
+      rec[TN_IRS] = Rs < 0.0 ? 0.0 : 1.0 / Rs;
       rec[TN_K] = 0.5 * M_PI * (tau2 + 1.0) * (tau2 + 1.0);
       rec[TN_T2M1] = tau2 - 1.0;
       rec[TN_AP] = rec[TN_A] * rec[TN_PRE];
@@ -1023,10 +1030,30 @@ __device__ __forceinline__ void nfw_defl(const Rec<T> &r, double x, double y, do
 // the issue of the vector ALU: the far branch is about 80 instructions, where
 // the form with a root for R, library-style arctangent and logarithm took
 // about 250 (of a 400^2-ray line of sight: 8.9 -> 6.0 ms a call).
+//
+// The record is one for the wave (a scalar load) and is read whole before the
+// first use of any of it: read where they are used, its constants cost five
+// waits for memory in a row, half of a deflector's time.
+__device__ __forceinline__ double wave_uniform(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+struct TnfwRec {
+  double cx, cy, irs, tau, tau2, ufar, K, t2m1, ap, c0, c1;
+  __device__ __forceinline__ explicit TnfwRec(const double *rd)
+      : cx(wave_uniform(rd[R_CX])), cy(wave_uniform(rd[R_CY])), irs(wave_uniform(rd[TN_IRS])),
+        tau(wave_uniform(rd[TN_TAU])), tau2(wave_uniform(rd[TN_TAU2])), ufar(wave_uniform(rd[TN_UFAR])),
+        K(wave_uniform(rd[TN_K])), t2m1(wave_uniform(rd[TN_T2M1])), ap(wave_uniform(rd[TN_AP])),
+        c0(wave_uniform(rd[TN_C0])), c1(wave_uniform(rd[TN_C1])) {
+    asm volatile("" : "+s"(cx), "+s"(cy), "+s"(irs), "+s"(tau), "+s"(tau2), "+s"(ufar), "+s"(K), "+s"(t2m1), "+s"(ap),
+                      "+s"(c0), "+s"(c1));
+  }
+};
+
 template <bool GRAD>
-__device__ __forceinline__ void tnfw_core(const double *rd, double u, double &iu, double &B, double &XBX,
-                                          double &tBt) {
-  const double tau = rd[TN_TAU], tau2 = rd[TN_TAU2];
+__device__ __forceinline__ void tnfw_core(const TnfwRec &r, const double *rd, double u, double &iu, double &B,
+                                          double &XBX, double &tBt) {
+  const double tau = r.tau, tau2 = r.tau2;
   const double rX = rsq_full(u);
   iu = rX * rX;
   const double sw = tau2 + u;
@@ -1036,16 +1063,16 @@ __device__ __forceinline__ void tnfw_core(const double *rd, double u, double &iu
   auto outer = [&](double G) {  // u >= 4
     const double e = u - 1.0;
     const double iv = rsq_full(e), v = e * iv;
-    const double vw = v + w, r = rcp_full(vw * vw);
-    const double Kr = rd[TN_K] * r;
-    B0 = fma(Kr, iv, -(fma(rd[TN_T2M1], iu, 2.0) * G));
+    const double vw = v + w, rvw = rcp_full(vw * vw);
+    const double Kr = r.K * rvw;
+    B0 = fma(Kr, iv, -(fma(r.t2m1, iu, 2.0) * G));
     if constexpr (GRAD) {
       const double iv2 = iv * iv;
-      X0 = fma(-Kr * u, (v + vw) * iv * iv2 * iw, fma(fma(2.0, u, rd[TN_T2M1]) * iv2, 1.0 + G, -4.0 * G));
-      t0 = fma(rd[TN_PT] * iv, iw * r * vw, -2.0 * y2 * G);
+      X0 = fma(-Kr * u, (v + vw) * iv * iv2 * iw, fma(fma(2.0, u, r.t2m1) * iv2, 1.0 + G, -4.0 * G));
+      t0 = fma(rd[TN_PT] * iv, iw * rvw * vw, -2.0 * y2 * G);
     }
   };
-  if (u >= rd[TN_UFAR]) {
+  if (u >= r.ufar) {
     constexpr double g8[9] = {1, 0.66666666666655927, 0.53333333337906674, 0.45714284965716129, 0.406349818765735,
                               0.36938031616196654, 0.34174313656705135, 0.30667133979364775, 0.39348549697643637};
     constexpr double a7[8] = {0.99999999999999989, -0.16666666666652991, 0.074999999953953234, -0.04464285122483598,
@@ -1077,7 +1104,7 @@ __device__ __forceinline__ void tnfw_core(const double *rd, double u, double &iu
         const double s = ::sqrt(1.0 - u);
         F = atanh_dbl(s) * rcp_refined(s);
       }
-      B0 = fma(fma(2.0, u, rd[TN_T2M1]), F, -M_PI * w);
+      B0 = fma(fma(2.0, u, r.t2m1), F, -M_PI * w);
       if constexpr (GRAD) {
         const double e = u - 1.0;
         double XF;
@@ -1088,7 +1115,7 @@ __device__ __forceinline__ void tnfw_core(const double *rd, double u, double &iu
         } else {
           XF = fma(-u, F, 1.0) / e;
         }
-        X0 = fma(fma(2.0, u, rd[TN_T2M1]), XF, u * fma(4.0, F, -M_PI * iw));
+        X0 = fma(fma(2.0, u, r.t2m1), XF, u * fma(4.0, F, -M_PI * iw));
         t0 = tau2 * fma(2.0, F, -M_PI * iw);
       }
     }
@@ -1102,10 +1129,10 @@ __device__ __forceinline__ void tnfw_core(const double *rd, double u, double &iu
       wL = w * (0.6931471805599453 * log2_pos(u * rX * rcp_full(tau + w)));
     }
   }
-  B = fma(wL, rd[TN_C1], B0 + rd[TN_C0]);
+  B = fma(wL, r.c1, B0 + r.c0);
   if constexpr (GRAD) {
-    const double LC = wL * iw * rd[TN_C1] * iw;  // L C1 / w
-    XBX = fma(u, LC, X0 + rd[TN_T2M1]);
+    const double LC = wL * iw * r.c1 * iw;  // L C1 / w
+    XBX = fma(u, LC, X0 + r.t2m1);
     tBt = fma(tau2, LC, fma(wL, rd[TN_E1], t0 + rd[TN_D0]));
   }
 }
@@ -1113,12 +1140,13 @@ __device__ __forceinline__ void tnfw_core(const double *rd, double u, double &iu
 // TNFW deflection, LensModel/Profiles/tnfw.py:67-87, :226-248, FP64 form:
 // alpha = 4 rho0 Rs g / X^2 (dx, dy); X = max(R, 0.001 Rs) / Rs.
 __device__ __forceinline__ void tnfw_defl_f64(const double *rd, double x, double y, double &ax, double &ay) {
-  const double dx = x - rd[R_CX], dy = y - rd[R_CY];
-  const double xs = dx * rd[TN_IRS], ys = dy * rd[TN_IRS];
+  const TnfwRec r(rd);
+  const double dx = x - r.cx, dy = y - r.cy;
+  const double xs = dx * r.irs, ys = dy * r.irs;
   const double u = fmax(fma(xs, xs, ys * ys), 1e-6);
   double iu, B, d0, d1;
-  tnfw_core<false>(rd, u, iu, B, d0, d1);
-  const double a = rd[TN_AP] * B * iu;
+  tnfw_core<false>(r, rd, u, iu, B, d0, d1);
+  const double a = r.ap * B * iu;
   ax = fma(a, dx, ax);
   ay = fma(a, dy, ay);
 }
@@ -1233,23 +1261,24 @@ __device__ __forceinline__ void convergence_defl(const double *rd, double x, dou
 // SIE / NIE or NFW, or halos on several planes; see nie_defl and nfw_defl);
 // DBL_TNFW: TNFW too (the render and gradient kernels; the ray-shooting
 // kernels keep the float TNFW, whose rays stay within 2e-6 of the FP64 form's).
-template <typename T, bool HALO, bool DBL = false, bool DBL_TNFW = DBL>
+// SUB: the list holds subhalos and linear deflectors only (TNFW, SHEAR,
+// CONVERGENCE): the other types' branches, and their registers, are left out.
+template <typename T, bool HALO, bool DBL = false, bool DBL_TNFW = DBL, bool SUB = false>
 __device__ __forceinline__ void add_deflection(int type, const Rec<T> &r, const double *__restrict__ coef_d,
                                                const T *__restrict__ coef_t, double x, double y, double &ax,
                                                double &ay) {
   switch (type) {
     case LENSIM_EPL:
-      if constexpr (sizeof(T) == sizeof(float))
-        epl_defl_f32(r, coef_t, coef_d, x, y, ax, ay);
-      else
-        epl_defl_f64(r, coef_d, x, y, ax, ay);
+      if constexpr (SUB) break;
+      else if constexpr (sizeof(T) == sizeof(float)) epl_defl_f32(r, coef_t, coef_d, x, y, ax, ay);
+      else epl_defl_f64(r, coef_d, x, y, ax, ay);
       break;
     case LENSIM_SIE:
     case LENSIM_NIE:
-      nie_defl<T, DBL>(r, x, y, ax, ay);
+      if constexpr (!SUB) nie_defl<T, DBL>(r, x, y, ax, ay);
       break;
     case LENSIM_NFW:
-      if constexpr (HALO) nfw_defl<T, DBL>(r, x, y, ax, ay);
+      if constexpr (HALO && !SUB) nfw_defl<T, DBL>(r, x, y, ax, ay);
       break;
     case LENSIM_TNFW:
       if constexpr (HALO) {
