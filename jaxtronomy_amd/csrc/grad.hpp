@@ -245,27 +245,6 @@ __device__ void nfw_g(const S *p, const S &x, const S &y, S &ax, S &ay) {
   ay = ay + a * dy;
 }
 
-// TNFW, tnfw.py:67-87, :226-248, :276-349.  p: Rs, alpha_Rs, r_trunc, center_x, center_y.
-template <typename T, typename S>
-__device__ void tnfw_g(const S *p, const S &x, const S &y, S &ax, S &ay) {
-  const S Rs = p[0];
-  const S rho0 = p[1] / (T(4) * Rs * Rs * (T(1) + T(::log(0.5))));
-  const S dx = x - p[3], dy = y - p[4];
-  S R = sqrt(dx * dx + dy * dy);
-  R = val(R) >= val(Rs) * T(0.001) ? R : Rs * T(0.001);
-  const S X = fmax(R / Rs, T(0.001));
-  const S tau = p[2] / Rs;
-  const S t2 = tau * tau;
-  const S F = nfw_F_g<T>(X);
-  const S L = log(X / (tau + sqrt(t2 + X * X)));
-  const S g = t2 / ((t2 + T(1)) * (t2 + T(1))) *
-              ((t2 + T(1) + T(2) * (X * X - T(1))) * F + tau * T(M_PI) + (t2 - T(1)) * log(tau) +
-               sqrt(t2 + X * X) * (L * (t2 - T(1)) / tau - T(M_PI)));
-  const S a = T(4) * rho0 * Rs * g / (X * X);
-  ax = ax + a * dx;
-  ay = ay + a * dy;
-}
-
 // One deflector from its raw slot.
 template <typename T, typename S>
 __device__ __forceinline__ void defl_g(int type, const S *p, const T *c, const T *dc, int nser, const S &x,
@@ -282,9 +261,6 @@ __device__ __forceinline__ void defl_g(int type, const S *p, const T *c, const T
       break;
     case LENSIM_NFW:
       nfw_g<T>(p, x, y, ax, ay);
-      break;
-    case LENSIM_TNFW:
-      tnfw_g<T>(p, x, y, ax, ay);
       break;
     case LENSIM_SHEAR: {
       const S dx = x - p[2], dy = y - p[3];

@@ -219,7 +219,8 @@ struct Layout {
   size_t recd, recf, coefd, coeff, dcoefd, dcoeff, psf, lowres, partial, blkmax, bfrag;
   size_t gmodel, glow, gpart;  // gradient: dlogL/dmodel, dlogL/dlowres, per-block partial gradients
   size_t gbeta;                // gradient: dS/dbeta of the sources at every ray (0: none)
-  size_t gpart_mp;             // gradient, several planes: per-block partials of the deflectors (0: none)
+  size_t beta;                 // gradient of a bulk or multi-plane list: beta at every ray (0: none)
+  size_t gpart_mp, gstate;     // ... its deflectors' partial sums and the rays' adjoints (0: none)
   size_t gpad, gext;           // edge-padded PSF adjoint: padded dlogL/dmodel and its correlation
   size_t gchr, glu;            // supersampled convolution adjoint buffers
   size_t mp_tab;               // several planes: the plane runs (mp_runs_kernel)
@@ -413,17 +414,37 @@ Layout layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img, int
   return L;
 }
 
-// Layout of lensim_loglike_grad: the image layout plus the gradient buffers
-// (on the ray grid when the convolution is supersampled).
-// Blocks per image of the multi-plane gradient: one 256-ray sweep each where
-// that keeps the whole launch near 2048 blocks, else several sweeps per block
-// (so that the per-block partials of every deflector stay bounded).
-int mp_grad_blocks(size_t rays, int n_img) {
-  const long sweeps = long((rays + 255) / 256);
-  const long want = (2048 + n_img - 1) / n_img;
-  return int(sweeps < want ? sweeps : (want > 0 ? want : 1));
+// Work plan of the gradient of a bulk or multi-plane deflector list over
+// `rays` rays an image (adjoint kernels, then defl_grad_kernel).  The adjoint
+// kernels keep four doubles per ray and run: per_img of them an image, at most
+// 2^25 (1 GiB) a call as long as that holds 64 rays of every run.  The host
+// knows the number of runs only as "at most one per plane", so it launches as
+// many rounds of rays as that could take; the kernels take as many rays a
+// round as the runs there are allow, usually all in the first, and the other
+// rounds' blocks end at once.  splits: pieces a deflector's rays are cut into
+// (a partial sum each), so that about 8192 waves share the deflectors.
+struct DeflGradPlan {
+  size_t per_img;
+  int rounds, splits, n;  // n: deflectors (planes, or the bulk list)
+  int slots() const { return rounds * splits; }
+};
+DeflGradPlan defl_grad_plan(const ModelArgs &m, size_t rays, int n_img) {
+  DeflGradPlan p{0, 1, 1, m.mp_n ? m.mp_n - 1 : m.n_bulk};
+  if (p.n == 0) return p;
+  const size_t runs = m.mp_n ? size_t(p.n) : 1, all = (rays + 63) / 64 * 64 * runs;
+  size_t share = (size_t(1) << 25) / n_img;
+  if (share < 64 * runs) share = 64 * runs;
+  p.per_img = all < share ? all : share;
+  const size_t cap = p.per_img / runs / 64 * 64;
+  p.rounds = int((rays + cap - 1) / cap);
+  const size_t pairs = size_t((p.n + 1) / 2) * n_img;
+  size_t sp = (8192 + pairs - 1) / pairs, most = (rays + 511) / 512;
+  p.splits = int(sp < most ? sp : most);
+  return p;
 }
 
+// Layout of lensim_loglike_grad: the image layout plus the gradient buffers
+// (on the ray grid when the convolution is supersampled).
 Layout grad_layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img, int precision, int edge,
                    const SSPlan &ss, int s) {
   Layout L = layout(m, nx, ny, kx, ky, n_img, precision, ss);
@@ -439,16 +460,23 @@ Layout grad_layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img
   L.gpart = off;
   off = align256(off + size_t(n_img) * m.n_prof * ((npix_r + 256 * kGradPix - 1) / (256 * kGradPix)) *
                            LENSIM_NPARAM * 8);
-  L.gbeta = 0;
+  L.gbeta = L.beta = L.gpart_mp = L.gstate = 0;
   const size_t rays = npix_r * (ss.on ? 1 : size_t(s) * s);
-  if ((m.n_lens > 0 || m.mp_n > 0) && m.n_source > 0) {  // dS/dbeta or beta per ray (two values, compute type)
+  const bool list = m.mp_n > 0 || m.n_bulk > 0;
+  if (m.n_lens > 0 && m.mp_n == 0 && m.n_source > 0) {
     L.gbeta = off;
     off = align256(off + size_t(n_img) * rays * 2 * tsz);
   }
-  L.gpart_mp = 0;
-  if (m.mp_n > 0 && m.n_defl > 0) {
+  if (list && m.n_source > 0) {
+    L.beta = off;
+    off = align256(off + size_t(n_img) * rays * 2 * tsz);
+  }
+  if (list && m.n_defl > 0) {
+    const DeflGradPlan p = defl_grad_plan(m, rays, n_img);
     L.gpart_mp = off;
-    off = align256(off + size_t(n_img) * m.n_defl * mp_grad_blocks(rays, n_img) * LENSIM_NPARAM * 8);
+    off = align256(off + size_t(n_img) * p.n * p.slots() * LENSIM_NPARAM * 8);
+    L.gstate = off;
+    off = align256(off + size_t(n_img) * p.per_img * 32);
   }
   L.gpad = L.gext = L.gchr = L.glu = off;
   if (edge) {  // extended domain (ny cs + ky - 1) x (nx cs + kx - 1)
@@ -1097,10 +1125,18 @@ __global__ __launch_bounds__(256) void block_max_kernel(const T *__restrict__ v,
 }
 
 constexpr int kMpBlock = 64;  // rays of a block of the multi-plane kernels (a lane each)
+// What a gradient keeps of its multi-plane render for mp_adjoint_kernel, so
+// that the rays are not traced again: per ray and run the position, and beta.
+struct MpKeep {
+  double4 *store;
+  size_t per_img;
+  void *beta;
+};
 int launch_mp_runs(const ModelArgs &m, int *tab, int n_img, hipStream_t st);
 template <typename T>
 int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf, const double *coefd,
-                     const float *coeff, const int *tab, unsigned flags, T *out, int n_img, hipStream_t st);
+                     const float *coeff, const int *tab, unsigned flags, const MpKeep &keep, T *out, int n_img,
+                     hipStream_t st);
 
 // Launches render_fast_kernel when the model is one of its compile-time lists
 // (EPL, SIE / NIE or NFW, each with or without SHEAR after it, NFW + SIE / NIE
@@ -1109,8 +1145,8 @@ int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, 
 // render_kernel.
 template <typename T>
 int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf, const double *coefd,
-                  const float *coeff, const int *tab, unsigned flags, T *out, float *blkmax, int n_img,
-                  hipStream_t st) {
+                  const float *coeff, const int *tab, unsigned flags, const MpKeep &keep, T *out, float *blkmax,
+                  int n_img, hipStream_t st) {
   const dim3 rgrid((g.nx * g.ny + 255) / 256, n_img);
   auto sersic = [](int t) { return t == LENSIM_SERSIC || t == LENSIM_SERSIC_ELLIPSE; };
   auto nie = [](int t) { return t == LENSIM_SIE ? LENSIM_NIE : t; };
@@ -1126,7 +1162,7 @@ int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, con
     for (int k = m.n_lens; fast && k < m.n_lens + m.n_source + m.n_light; ++k) fast = sersic(m.types[k]);
   }
   if (m.mp_n) {  // the block maxima for the MFMA convolution follow from the image in a second launch
-    int rc = launch_render_mp<T>(m, g, recd, recf, coefd, coeff, tab, flags, out, n_img, st);
+    int rc = launch_render_mp<T>(m, g, recd, recf, coefd, coeff, tab, flags, keep, out, n_img, st);
     if (rc || !blkmax) return rc;
     block_max_kernel<T><<<rgrid, 256, 0, st>>>(out, g.nx * g.ny, blkmax);
     return check_launch("block_max_kernel");
@@ -1208,10 +1244,14 @@ __device__ __forceinline__ double quad_sum(double v) {
 // The sum over a wave (every lane active), uniform: the quads' sums, then
 // the row's (row_ror 4 and 8 within each row of 16 lanes), then the four rows'
 // sums read from their first lanes and added in order.
-__device__ __forceinline__ double wave_sum(double v) {
+__device__ __forceinline__ double row_sum(double v) {  // over each row of 16 lanes, in all of them
   v = quad_sum(v);
   v += dpp_quad_f64<0x124>(v);  // row_ror:4
   v += dpp_quad_f64<0x128>(v);  // row_ror:8
+  return v;
+}
+__device__ __forceinline__ double wave_sum(double v) {
+  v = row_sum(v);
   auto row = [&](int l) {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
                             __builtin_amdgcn_readlane(__double2loint(v), l));
@@ -1317,15 +1357,33 @@ int launch_mp_runs(const ModelArgs &m, int *tab, int n_img, hipStream_t st) {
   return check_launch("mp_runs_kernel");
 }
 
-// The sums of (vx, vy) over the block's waves (lane by lane), in wave order, in
-// every wave.  buf alternates between consecutive calls, so one barrier does.
-__device__ __forceinline__ void across_waves(double2 (*red)[16][64], int buf, int nw, double &vx, double &vy) {
+// The sums of (vx, vy) over the block's waves, lane by lane, in every wave.
+// buf alternates between consecutive calls, so that no barrier is needed before
+// the write.  Up to eight waves each read all the waves' values (in wave
+// order); sixteen would each read 16 KB of LDS that way (2000 cycles a call),
+// so there a row of 16 lanes sums one ray's values and every wave reads the
+// sums, at the price of a second barrier.
+struct WaveSums {
+  double2 part[2][16][65];  // rows of 65: the 16 values of a ray lie on distinct banks
+  double2 sum[2][64];
+};
+__device__ __forceinline__ void across_waves(WaveSums &red, int buf, int nw, double &vx, double &vy) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  red[buf][wave][lane] = double2{vx, vy};
+  red.part[buf][wave][lane] = double2{vx, vy};
   __syncthreads();
+  if (nw == 16) {
+    const int ray = threadIdx.x >> 4, w = threadIdx.x & 15;
+    const double2 v = red.part[buf][w][ray];
+    const double2 s{row_sum(v.x), row_sum(v.y)};
+    if (w == 0) red.sum[buf][ray] = s;
+    __syncthreads();
+    vx = red.sum[buf][lane].x;
+    vy = red.sum[buf][lane].y;
+    return;
+  }
   vx = vy = 0.0;
   for (int w = 0; w < nw; ++w) {
-    const double2 v = red[buf][w][lane];
+    const double2 v = red.part[buf][w][lane];
     vx += v.x;
     vy += v.y;
   }
@@ -1345,7 +1403,7 @@ template <typename T, bool HALO, bool DBL, bool DBL_TNFW, bool SUB, typename F>
 __device__ __forceinline__ void block_trace(const ModelArgs &m, const RecPtrs<T> &rp, const MpTab &tab,
                                             const double *__restrict__ tij, const double *__restrict__ tzs,
                                             const double *__restrict__ r2p, int img, double x, double y,
-                                            double2 (*red)[16][64], double &bx, double &by, F each) {
+                                            WaveSums &red, double &bx, double &by, F each) {
   const int lane = threadIdx.x & 63, nw = int(blockDim.x) >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   double angx = x, angy = y, px = 0.0, py = 0.0;
@@ -1410,7 +1468,7 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void raytrace_mp_kernel(ModelArgs
                                                            const double *__restrict__ ys, int64_t n_ray,
                                                            int64_t first, bool both, double *__restrict__ bx,
                                                            double *__restrict__ by) {
-  __shared__ double2 red[2][16][64];
+  __shared__ WaveSums red;
   const int img = blockIdx.y;
   const int64_t ray0 = first + int64_t(blockIdx.x) * kMpBlock + (threadIdx.x & 63);
   const bool active = ray0 < n_ray;
@@ -1428,6 +1486,12 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void raytrace_mp_kernel(ModelArgs
   }
 }
 
+// Rays a round takes of image img's adjoint store, from its runs (all of them
+// where there is no deflector and so nothing to store).
+__device__ __forceinline__ int64_t round_rays(size_t per_img, int runs) {
+  return runs > 0 ? int64_t(per_img / size_t(runs) / 64 * 64) : int64_t(1) << 31;
+}
+
 // render_kernel for several planes: the block's waves walk the sub-rays of its
 // 64 pixels together (block_trace); the first wave adds the light and stores.
 template <typename T, bool HALO, bool DBL, bool SUB>
@@ -1436,8 +1500,8 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void render_mp_kernel(ModelArgs m
                                                          const double *__restrict__ coefd,
                                                          const float *__restrict__ coeff,
                                                          const int *__restrict__ tab_all, unsigned flags, bool both,
-                                                         T *__restrict__ out) {
-  __shared__ double2 red[2][16][64];
+                                                         MpKeep keep, T *__restrict__ out) {
+  __shared__ WaveSums red;
   const int img = blockIdx.y;
   const int npix = g.nx * g.ny;
   const int pix0 = blockIdx.x * kMpBlock + (threadIdx.x & 63);
@@ -1457,6 +1521,8 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void render_mp_kernel(ModelArgs m
   double acc = 0.0;
   const bool eval = active && evaluated(g, i, j);
   const bool any = __any(eval);  // the same in every wave: they hold the same pixels
+  const int64_t cap = keep.store ? round_rays(keep.per_img, tab.n) : 0;
+  const bool keeps = active && threadIdx.x < 64 && cap >= int64_t(npix) * g.s * g.s;
   for (int sy = 0; any && sy < g.s; ++sy) {
     const double oy = g.o0 + sy * g.inv_s;
     for (int sx = 0; sx < g.s; ++sx) {
@@ -1466,8 +1532,16 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void render_mp_kernel(ModelArgs m
       double bx = x, by = y;
       if (do_src) {
         __syncthreads();  // the last sub-ray's sums are read
-        block_trace<T, HALO, DBL, DBL, SUB>(m, rp, tab, tij, tzs, r2p, img, x, y, red, bx, by,
-                                            [](int, double, double) {});
+        const size_t ray = size_t(pix) * (g.s * g.s) + size_t(sy * g.s + sx);
+        block_trace<T, HALO, DBL, DBL, SUB>(
+            m, rp, tab, tij, tzs, r2p, img, x, y, red, bx, by, [&](int c, double xr, double yr) {
+              if (keeps) AT(keep.store, size_t(img) * keep.per_img + ray + size_t(c) * cap) = double4{xr, yr, 0.0, 0.0};
+            });
+        if (keeps && keep.beta) {
+          T *b = static_cast<T *>(keep.beta) + (size_t(img) * npix * size_t(g.s * g.s) + ray) * 2;
+          AT(b, 0) = T(bx);
+          AT(b, 1) = T(by);
+        }
       }
       if (eval && threadIdx.x < 64) {
         if (do_src) acc += light_sum<T>(m, rp, k_src0, k_src1, bx, by);
@@ -1491,13 +1565,14 @@ int sub_list(const ModelArgs &m) {
 
 template <typename T>
 int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf, const double *coefd,
-                     const float *coeff, const int *tab, unsigned flags, T *out, int n_img, hipStream_t st) {
+                     const float *coeff, const int *tab, unsigned flags, const MpKeep &keep, T *out, int n_img,
+                     hipStream_t st) {
   const size_t npix = size_t(g.nx) * g.ny;
   const dim3 grid((unsigned)((npix + kMpBlock - 1) / kMpBlock), n_img);
   const int sub = sub_list(m);
 #define LENSIM_RENDER(H, D, S)                                                                                \
   render_mp_kernel<T, H, D, S><<<grid, 64 * mp_waves(npix, S), 0, st>>>(m, g, recd, recf, coefd, coeff, tab, \
-                                                                       flags, sub == 2, out)
+                                                                       flags, sub == 2, keep, out)
   // the float form deflects SIE / NIE and the NFW family in double
   constexpr bool kF32 = sizeof(T) == sizeof(float);
   if (sub) LENSIM_RENDER(true, kF32, true);
@@ -2228,6 +2303,7 @@ struct GradArgs {
   const void *glow;       // [n_img][ny][nx] dlogL / d(unconvolved image), compute type
   double *gpart;          // [n_img][n_prof][nblk][8]
   void *gbeta;            // [n_img][ny][nx][s][s][2] dS/dbeta of the sources' sum, compute type, or NULL
+  void *beta;             // same shape: beta (bulk and multi-plane lists, by the adjoint kernels), or NULL
 };
 
 // A light profile's flux and its derivatives in its own kwargs (the N seeds
@@ -2279,12 +2355,14 @@ __device__ __forceinline__ gm::Dual<T, 2> sources_at(const ModelArgs &m, const G
 // Contribution of one ray to d flux / d(kwargs of profile k), with the
 // profile's own kwargs as N dual seeds; w = dlogL / d(ray flux).
 // gb: this ray's dS/dbeta of the sources' sum (two values), when the model
-// has lenses and sources: the first source's launch writes it, the lens
+// has inline lenses and sources: the first source's launch writes it, the lens
 // launches (which run after it) read it instead of deflecting by the other
-// deflectors and evaluating the sources again.
+// deflectors and evaluating the sources again.  bt: this ray's beta, where an
+// adjoint kernel stored it (and gb) before.
 template <typename T, int N, bool HALO>
 __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga, const RecPtrs<T> &rp, int img,
-                                         int k, int type, double x, double y, double w, double *acc, T *gb) {
+                                         int k, int type, double x, double y, double w, double *acc, T *gb,
+                                         const T *bt) {
   using S = gm::Dual<T, N>;
   const double *pk = ga.params + (size_t(img) * m.n_prof + k) * LENSIM_NPARAM;
   CHECK_SPAN(pk, LENSIM_NPARAM * sizeof(double));
@@ -2351,9 +2429,9 @@ __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga,
   } else if (k < m.n_defl + m.n_source) {
     // d/d(source kwargs) at the deflected position
     T bxs, bys;
-    if (m.mp_n) {  // multi-plane: mp_grad_kernel stored beta at every ray
-      bxs = AT(gb, 0);
-      bys = AT(gb, 1);
+    if (bt) {
+      bxs = AT(bt, 0);
+      bys = AT(bt, 1);
     } else {
       double ax = 0.0, ay = 0.0;
       deflect_all<T, HALO>(m, rp, img, x, y, ax, ay);
@@ -2361,7 +2439,7 @@ __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga,
       bys = T(y - ay * m.alpha_scaling);
     }
     bool done = false;
-    if (gb && !m.mp_n) {  // the first source's launch: also dS/dbeta of the sources' sum for the lens launches
+    if (gb && !bt) {  // the first source's launch: also dS/dbeta of the sources' sum for the lens launches
       if constexpr (N == 7) {
         if (m.n_source == 1 && type == LENSIM_SERSIC_ELLIPSE) {  // one evaluation gives both
           T gp[7], gx, gy;
@@ -2388,7 +2466,7 @@ __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga,
   for (int i = 0; i < N; ++i) acc[i] += w * double(flux.d[i]);
 }
 
-// ray_grad for an inline NFW or TNFW deflector k: the other deflectors in the
+// ray_grad for an inline NFW deflector k: the other deflectors in the
 // forward form, this one's duals in double in both forms (the float closed
 // forms of the NFW family cancel, as for the bulk list's duals).
 template <typename T, int N, bool HALO>
@@ -2650,27 +2728,34 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
       const double ox = o0 + sx * inv_s;
       const double x = ra_c + g.m00 * ox + g.m01 * oy;
       const double y = dec_c + g.m10 * ox + g.m11 * oy;
-      // this ray's slot: dS/dbeta, written by the first source's launch and read by the inline lens
-      // launches; with several planes, beta, written by mp_grad_kernel and read by the source launches
-      T *gb = (gbeta && (k < m.n_lens || k == m.n_defl || (m.mp_n && k < m.n_defl + m.n_source)))
-                  ? gbeta + ((size_t(img) * npix + pix) * size_t(g.s * g.s) + size_t(sy * g.s + sx)) * 2
-                  : nullptr;
+      // this ray's slots: dS/dbeta, written by the first source's launch (or an adjoint kernel) and read by
+      // the inline lens launches; beta, written by an adjoint kernel and read by the source launches
+      const size_t slot = ((size_t(img) * npix + pix) * size_t(g.s * g.s) + size_t(sy * g.s + sx)) * 2;
+      T *gb = (gbeta && (k < m.n_lens || k == m.n_defl)) ? gbeta + slot : nullptr;
+      const T *bt = (ga.beta && k >= m.n_defl && k < m.n_defl + m.n_source) ? static_cast<const T *>(ga.beta) + slot
+                                                                            : nullptr;
       if (gb) CHECK_SPAN(gb, 2 * sizeof(T));
+      if (bt) CHECK_SPAN(bt, 2 * sizeof(T));
       if constexpr (type == LENSIM_EPL) lens_ray_grad<T, HALO>(m, ga, rp, img, k, x, y, w, acc, gb);
       else if constexpr (type == LENSIM_SIE) lens_ray_grad<T, HALO, LENSIM_SIE>(m, ga, rp, img, k, x, y, w, acc, gb);
       else if constexpr (type == LENSIM_NIE) lens_ray_grad<T, HALO, LENSIM_NIE>(m, ga, rp, img, k, x, y, w, acc, gb);
       else if constexpr (type == LENSIM_NFW) halo_ray_grad<T, 4, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb);
-      else if constexpr (type == LENSIM_TNFW) halo_ray_grad<T, 5, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb);
-      else if constexpr (type == LENSIM_SHEAR) ray_grad<T, 4, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb);
+      else if constexpr (type == LENSIM_TNFW) {  // live and a lens: gb is there
+        const double lw = -m.alpha_scaling * w;
+        tnfw_ray_grad(TnfwRec(rp.recd + k * kRec), rp.recd + k * kRec, x, y, lw * double(AT(gb, 0)),
+                      lw * double(AT(gb, 1)), acc);
+      }
+      else if constexpr (type == LENSIM_SHEAR) ray_grad<T, 4, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb, bt);
       else if constexpr (type == LENSIM_CONVERGENCE)
-        ray_grad<T, 3, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb);
-      else if constexpr (type == LENSIM_SERSIC) ray_grad<T, 5, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb);
+        ray_grad<T, 3, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb, bt);
+      else if constexpr (type == LENSIM_SERSIC) ray_grad<T, 5, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb, bt);
       else if constexpr (type == LENSIM_SERSIC_ELLIPSE)
-        ray_grad<T, 7, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb);
-      else if constexpr (type == LENSIM_GAUSSIAN) ray_grad<T, 4, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb);
+        ray_grad<T, 7, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb, bt);
+      else if constexpr (type == LENSIM_GAUSSIAN) ray_grad<T, 4, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb, bt);
     }
   }
   }
+  if constexpr (type == LENSIM_TNFW) tnfw_grad_scale(rp.recd + k * kRec, acc);
   // block sum of the 8 accumulators in a fixed order
   __shared__ double red[256 / 64][LENSIM_NPARAM];
 #pragma unroll
@@ -2713,170 +2798,6 @@ int launch_grad_profile(const ModelArgs &m, const GridArgs &g, const GradArgs &g
   }
 #undef LENSIM_GRAD
   return check_launch("grad_kernel");
-}
-
-// d flux / d(kwargs) of the bulk deflectors (LensModelBulk lists, records
-// n_lens .. n_defl - 1).  With beta = theta - alpha_scaling sum_j alpha_j,
-// d(ray flux)/d p_k = -alpha_scaling grad S(beta) . d alpha_k / d p_k, so a
-// ray's total deflection and source gradient are needed once, and then each
-// deflector's own deflection in duals.  Block (b, img, c): the rays of pixels
-// [b kGradPix 256, (b + 1) kGradPix 256) of image img and deflectors
-// n_lens + c dpb + d, d < dpb (dpb = 64, 128 or 256 threads per deflector
-// group, 256 / dpb groups of whole waves).  Per tile of 256 rays each thread
-// traces one ray into LDS: (x, y) and g = w (-alpha_scaling) dS/dbeta; then
-// group grp's thread d runs its deflector's duals over the tile's rays grp,
-// grp + 256/dpb, ... (the same ray for every lane of a wave: the zero-weight
-// skip is uniform), and the groups' sums are added in a fixed order.
-// TYPE is the list's common type, or LENSIM_NULL for a list of several types
-// (a switch per deflector, outside the ray loop).
-// The deflectors' duals run in double in both forms: the NFW family's closed
-// forms cancel inside and outside the scale radius (the float forward
-// rewrites them; their duals would not follow), which costs a float dual all
-// its precision in the derivative by the centre.
-template <int TYPE, int N>
-__device__ __forceinline__ void bulk_tile_duals(const double *pk, const double *rd, const double *lx,
-                                                const double *ly, const double *lgx, const double *lgy, int r0,
-                                                int step, int r1, double *acc) {
-  if constexpr (TYPE == LENSIM_SIE || TYPE == LENSIM_NIE) {  // orientation from the record (nie_dalpha)
-    for (int r = r0; r < r1; r += step) {
-      const double gx = lgx[r], gy = lgy[r];
-      if (gx == 0.0 && gy == 0.0) continue;
-      double a_x, a_y, dax[6], day[6];
-      nie_dalpha<double, TYPE>(rd, pk, lx[r], ly[r], a_x, a_y, dax, day);
-#pragma unroll
-      for (int i = 0; i < N; ++i) acc[i] += gx * dax[i] + gy * day[i];
-    }
-    return;
-  }
-  using S = gm::Dual<double, N>;
-  S ps[LENSIM_NPARAM];
-#pragma unroll
-  for (int i = 0; i < LENSIM_NPARAM; ++i) ps[i] = i < N ? S::seed(pk[i], i) : S(pk[i]);
-  for (int r = r0; r < r1; r += step) {
-    const double gx = lgx[r], gy = lgy[r];
-    if (gx == 0.0 && gy == 0.0) continue;
-    S ax = S(0.0), ay = S(0.0);
-    gm::defl_g<double, S>(TYPE, ps, static_cast<const double *>(nullptr), static_cast<const double *>(nullptr), 1,
-                          S(lx[r]), S(ly[r]), ax, ay);
-#pragma unroll
-    for (int i = 0; i < N; ++i) acc[i] += gx * ax.d[i] + gy * ay.d[i];
-  }
-}
-
-template <typename T, bool HALO, int TYPE>
-__global__ __launch_bounds__(256) void bulk_grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
-                                                        const double *__restrict__ recd,
-                                                        const float *__restrict__ recf,
-                                                        const double *__restrict__ coefd,
-                                                        const float *__restrict__ coeff, int dpb) {
-  const int img = blockIdx.y;
-  const int npix = g.nx * g.ny, ss = g.s * g.s;
-  const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
-  const int t = threadIdx.x, d = t % dpb, grp = t / dpb, ngrp = blockDim.x / dpb;
-  const int k = m.n_lens + blockIdx.z * dpb + d;
-  const bool mine = k < m.n_defl;
-  int type = LENSIM_NULL;
-  if (mine) type = TYPE != LENSIM_NULL ? TYPE : AT(m.bulk_types, k - m.n_lens);
-  double pk[LENSIM_NPARAM], acc[LENSIM_NPARAM];
-#pragma unroll
-  for (int q = 0; q < LENSIM_NPARAM; ++q) {
-    pk[q] = mine ? AT(ga.params, (size_t(img) * m.n_prof + k) * LENSIM_NPARAM + q) : 0.0;
-    acc[q] = 0.0;
-  }
-  const double *rdk = rp.recd + (mine ? k : 0) * kRec;  // this deflector's record (SIE / NIE orientation)
-  __shared__ double lx[256], ly[256], lgx[256], lgy[256];
-  __shared__ double red[256][LENSIM_NPARAM];
-  const int p0 = blockIdx.x * kGradPix * 256, p1 = min(npix, p0 + kGradPix * 256);
-  const int r_end = (p1 - p0) * ss;  // rays of the block, pixel-major, s x s sub-rays per pixel
-  const double inv_s = g.inv_s, o0 = g.o0, as = m.alpha_scaling;
-  for (int base = 0; base < r_end; base += 256) {
-    // one ray per thread: position, weight and the source gradient at its beta
-    {
-      const int rr = base + t;
-      const bool active = rr < r_end;
-      int sub0;
-      const int q = div_by(active ? rr : 0, ss, g.inv_ss, sub0);
-      const int pix = p0 + q, sub = sub0;
-      int i, sx;
-      const int j = div_by(pix, g.nx, g.inv_nx, i), sy = div_by(sub, g.s, g.inv_s, sx);
-      const double ox = o0 + sx * inv_s, oy = o0 + sy * inv_s;
-      const double x = i * g.m00 + j * g.m01 + g.ra0 + g.m00 * ox + g.m01 * oy;
-      const double y = i * g.m10 + j * g.m11 + g.dec0 + g.m10 * ox + g.m11 * oy;
-      const double w = active ? double(AT(static_cast<const T *>(ga.glow), size_t(img) * npix + pix)) * g.scale *
-                                    m.flux_scaling
-                              : 0.0;
-      double gx = 0.0, gy = 0.0;
-      if (w != 0.0 && m.n_source > 0 && evaluated(g, i, j)) {
-        double ax = 0.0, ay = 0.0;
-        deflect_all<T, HALO>(m, rp, img, x, y, ax, ay);
-        const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, T(x - ax * as), T(y - ay * as));
-        gx = -as * w * double(f2.d[0]);
-        gy = -as * w * double(f2.d[1]);
-      }
-      lx[t] = x;
-      ly[t] = y;
-      lgx[t] = gx;
-      lgy[t] = gy;
-    }
-    __syncthreads();
-    const int r1 = min(256, r_end - base);
-    if constexpr (TYPE != LENSIM_NULL) {
-      if (mine) bulk_tile_duals<TYPE, n_params_of(TYPE)>(pk, rdk, lx, ly, lgx, lgy, grp, ngrp, r1, acc);
-    } else {
-      switch (type) {
-        case LENSIM_SIE: bulk_tile_duals<LENSIM_SIE, 5>(pk, rdk, lx, ly, lgx, lgy, grp, ngrp, r1, acc); break;
-        case LENSIM_NIE: bulk_tile_duals<LENSIM_NIE, 6>(pk, rdk, lx, ly, lgx, lgy, grp, ngrp, r1, acc); break;
-        case LENSIM_NFW:
-          if constexpr (HALO) bulk_tile_duals<LENSIM_NFW, 4>(pk, rdk, lx, ly, lgx, lgy, grp, ngrp, r1, acc);
-          break;
-        case LENSIM_TNFW:
-          if constexpr (HALO) bulk_tile_duals<LENSIM_TNFW, 5>(pk, rdk, lx, ly, lgx, lgy, grp, ngrp, r1, acc);
-          break;
-        case LENSIM_SHEAR: bulk_tile_duals<LENSIM_SHEAR, 4>(pk, rdk, lx, ly, lgx, lgy, grp, ngrp, r1, acc); break;
-        case LENSIM_CONVERGENCE:
-          bulk_tile_duals<LENSIM_CONVERGENCE, 3>(pk, rdk, lx, ly, lgx, lgy, grp, ngrp, r1, acc);
-          break;
-        default: break;  // no kwargs: zero partials
-      }
-    }
-    __syncthreads();
-  }
-  // the groups' sums in group order
-#pragma unroll
-  for (int q = 0; q < LENSIM_NPARAM; ++q) red[t][q] = acc[q];
-  __syncthreads();
-  if (grp == 0 && mine) {
-#pragma unroll
-    for (int q = 0; q < LENSIM_NPARAM; ++q) {
-      double v = 0.0;
-      for (int gi = 0; gi < ngrp; ++gi) v += red[gi * dpb + d][q];
-      AT(ga.gpart, ((size_t(img) * m.n_prof + k) * gridDim.x + blockIdx.x) * LENSIM_NPARAM + q) = v;
-    }
-  }
-}
-
-template <typename T, bool HALO>
-int launch_bulk_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, const double *recd,
-                     const float *recf, int nblk, int n_img, hipStream_t st) {
-  const int dpb = m.n_bulk <= 64 ? 64 : (m.n_bulk <= 128 ? 128 : 256);
-  const dim3 grid(nblk, n_img, (m.n_bulk + dpb - 1) / dpb);
-#define LENSIM_BULK_GRAD(TY) \
-  bulk_grad_kernel<T, HALO, TY><<<grid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, dpb)
-  switch (m.bulk_type) {
-    case LENSIM_SIE: LENSIM_BULK_GRAD(LENSIM_SIE); break;
-    case LENSIM_NIE: LENSIM_BULK_GRAD(LENSIM_NIE); break;
-    case LENSIM_NFW:
-      if constexpr (HALO) LENSIM_BULK_GRAD(LENSIM_NFW);
-      break;
-    case LENSIM_TNFW:
-      if constexpr (HALO) LENSIM_BULK_GRAD(LENSIM_TNFW);
-      break;
-    case LENSIM_SHEAR: LENSIM_BULK_GRAD(LENSIM_SHEAR); break;
-    case LENSIM_CONVERGENCE: LENSIM_BULK_GRAD(LENSIM_CONVERGENCE); break;
-    default: LENSIM_BULK_GRAD(LENSIM_NULL); break;  // several types: d_bulk_types per deflector
-  }
-#undef LENSIM_BULK_GRAD
-  return check_launch("bulk_grad_kernel");
 }
 
 // Deflector k's deflection at (x, y) and its derivatives by its kwargs,
@@ -2954,194 +2875,437 @@ __device__ __forceinline__ void deflector_dalpha(const ModelArgs &m, const GradA
     case LENSIM_NFW:
       if constexpr (HALO) dalpha_duals<LENSIM_NFW, 4>(pk, x, y, ax, ay, dax, day, dcen);
       break;
-    case LENSIM_TNFW:
-      if constexpr (HALO) dalpha_duals<LENSIM_TNFW, 5>(pk, x, y, ax, ay, dax, day, dcen);
-      break;
-    case LENSIM_SHEAR: dalpha_duals<LENSIM_SHEAR, 4>(pk, x, y, ax, ay, dax, day, dcen); break;
-    case LENSIM_CONVERGENCE: dalpha_duals<LENSIM_CONVERGENCE, 3>(pk, x, y, ax, ay, dax, day, dcen); break;
-    default: break;
+    default: break;  // TNFW, SHEAR and CONVERGENCE: their callers' closed forms
   }
 }
 
-// d flux / d(kwargs) of every deflector of a multi-plane model, the
-// recursion of trace_ray (MultiPlaneBulk.ray_shooting,
+// ---- gradient of bulk and multi-plane deflector lists ----
+// d flux / d(kwargs) of every deflector takes two steps.  An adjoint kernel
+// traces each ray and stores, per run of deflectors on one plane (one run for
+// a single-plane list), the ray's position (x, y) and the adjoint (lx, ly) of
+// the deflection there; then defl_grad_kernel sums lambda . d alpha_k /
+// d kwargs_k over the rays, deflector by deflector.  So the serial part (the
+// planes) holds no parameter sums, and those are taken with a lane per ray, in
+// registers, with one wave sum per deflector at the end.  (One kernel that did
+// both summed five parameters over each block at every deflector: 23.5 ms for
+// 5256 deflectors and 100^2 rays, where the two steps take 0.52 and 0.28 ms.)
+
+// A ray of image img: its index on the grid, position and the weight w =
+// dlogL / d(ray flux); live: whether it has a weight and a source to hit.
+struct GradRay {
+  size_t slot;
+  double x, y, w;
+  bool live;
+};
+template <typename T>
+__device__ __forceinline__ GradRay grad_ray(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, int img, int rr,
+                                            bool active) {
+  const int npix = g.nx * g.ny, ss = g.s * g.s;
+  int sub, i, sx;
+  const int pix = div_by(rr, ss, g.inv_ss, sub);
+  const int j = div_by(pix, g.nx, g.inv_nx, i), sy = div_by(sub, g.s, g.inv_s, sx);
+  const double ox = g.o0 + sx * g.inv_s, oy = g.o0 + sy * g.inv_s;
+  GradRay r;
+  r.x = i * g.m00 + j * g.m01 + g.ra0 + g.m00 * ox + g.m01 * oy;
+  r.y = i * g.m10 + j * g.m11 + g.dec0 + g.m10 * ox + g.m11 * oy;
+  r.w = active ? double(AT(static_cast<const T *>(ga.glow), size_t(img) * npix + pix)) * g.scale * m.flux_scaling : 0.0;
+  r.live = r.w != 0.0 && m.n_source > 0 && evaluated(g, i, j);
+  r.slot = ((size_t(img) * npix + pix) * size_t(ss) + size_t(sub)) * 2;
+  return r;
+}
+
+// (d alpha_k / dx)^T l of one deflector added to (jx, jy).
+template <typename T, bool HALO, bool SUB>
+__device__ __forceinline__ void adjoint_one(const ModelArgs &m, const GradArgs &ga, const RecPtrs<T> &rp, int img,
+                                            int k, int type, double x, double y, double lx, double ly, double &jx,
+                                            double &jy) {
+  const double *rd = rp.recd + k * kRec;
+  switch (type) {
+    case LENSIM_TNFW:
+      if constexpr (HALO) tnfw_adjoint(TnfwRec(rd), rd, x, y, lx, ly, jx, jy);
+      break;
+    case LENSIM_CONVERGENCE:
+      jx = fma(rd[CV_KAPPA], lx, jx);
+      jy = fma(rd[CV_KAPPA], ly, jy);
+      break;
+    case LENSIM_SHEAR:
+      jx += rd[SH_G1] * lx + rd[SH_G2] * ly;
+      jy += rd[SH_G2] * lx - rd[SH_G1] * ly;
+      break;
+    case LENSIM_NULL:
+      break;
+    default:
+      if constexpr (!SUB) {
+        double ax = 0.0, ay = 0.0, dax[LENSIM_NPARAM], day[LENSIM_NPARAM], dcen[4] = {0.0, 0.0, 0.0, 0.0};
+        deflector_dalpha<T, HALO>(m, ga, rp, img, k, type, x, y, ax, ay, dax, day, dcen);
+        jx -= lx * dcen[0] + ly * dcen[1];
+        jy -= lx * dcen[2] + ly * dcen[3];
+      }
+      break;
+  }
+}
+
+// The adjoint of the multi-plane recursion (MultiPlaneBulk.ray_shooting,
 // LensModel/MultiPlane/multi_plane_bulk.py:152-212)
 //   P_p = P_{p-1} + T_p A_{p-1},  A_p = A_{p-1} - f_p alpha_p(P_p / Tz_p),
-//   beta = P_n / Tz_n  (P_{-1} = 0, A_{-1} = the ray's angle)
-// differentiated in reverse.  From the adjoints (gP, gA) of (P_p, A_p):
-//   lambda = -f_p gA  (the adjoint of alpha_p),
-//   d flux / d kwargs_p = lambda . d alpha_p / d kwargs_p,
-//   gP += (d alpha_p / d x)^T lambda / Tz_p,  then gA += T_p gP,
-// starting from gP = w dS/dbeta / Tz_n, gA = 0 at the source plane.  The
-// plane states are not stored: each backward step inverts its forward one,
-// A_{p-1} = A_p + f_p alpha_p and P_{p-1} = P_p - T_p A_{p-1}, with alpha_p
-// the value of the duals the step evaluates anyway.  (d alpha / d x)^T lambda
-// is minus lambda's product with the centre's derivative.
-// Block (b, img) takes sweeps [b spb, (b + 1) spb) of 256 rays of image img
-// (the rays pixel-major, s x s sub-rays per pixel), one ray per thread per
-// sweep; all threads sweep the planes together, so a plane's contributions
-// are summed over the block (waves, then the waves in order) and added to its
-// deflector's partial in gpart_mp, which the block owns; mp_partial_reduce
-// sums the blocks in order.  Each ray's beta is also stored (ga.gbeta) for
-// the source profiles' launches.
-template <typename T, bool HALO>
-__global__ __launch_bounds__(256) void mp_grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
-                                                      const double *__restrict__ recd,
-                                                      const float *__restrict__ recf,
-                                                      const double *__restrict__ coefd,
-                                                      const float *__restrict__ coeff, double *__restrict__ gpart_mp,
-                                                      int spb) {
-  const int img = blockIdx.y;
-  const int npix = g.nx * g.ny, ss = g.s * g.s;
+//   beta = P_n / Tz_n  (P_{-1} = 0, A_{-1} = the ray's angle):
+// from gP = w dS/dbeta / Tz_n and gA = 0 at the source plane backwards,
+//   lambda_p = -f_p gA  (the adjoint of alpha_p),
+//   gP += (d alpha_p / dx)^T lambda_p / Tz_p,  then gA += T_p gP.
+// Forwards nothing is left to do where the render kept its rays (MpKeep); when
+// they take more than a round, block_trace again, storing each run's position.
+// Backwards the same split of a run's deflectors over the block's waves (they
+// share position and lambda: gA does not change where T is 0).  Each ray's beta
+// is stored too, for the source profiles' launches.  Bound by the runs' serial chain at few rays
+// (a barrier and the deflectors' records per run), by the vector ALU at many.
+template <typename T, bool HALO, bool SUB>
+__global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
+    ModelArgs m, GridArgs g, GradArgs ga, const double *__restrict__ recd, const float *__restrict__ recf,
+    const double *__restrict__ coefd, const float *__restrict__ coeff, const int *__restrict__ tab_all, bool both,
+    double4 *store, size_t per_img, int round, const double *__restrict__ all_tij,
+    const double *__restrict__ all_tz, const double *__restrict__ all_r2p) {
+  __shared__ WaveSums red;
+  const int img = blockIdx.y, lane = threadIdx.x & 63, nw = int(blockDim.x) >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const MpTab tab = mp_tab(m, tab_all, img);
+  if (both && bool(tab.sub) != SUB) return;  // the other instantiation's launch takes it
+  const int r_all = g.nx * g.ny * g.s * g.s;
+  const int64_t cap = round_rays(per_img, tab.n), in = int64_t(blockIdx.x) * 64;
+  if (in >= cap || round * cap + in >= r_all) return;
+  const int64_t rr = round * cap + in + lane;
+  const bool active = rr < r_all;
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
-  const int t = threadIdx.x;
+  const GradRay ray = grad_ray<T>(m, g, ga, img, int(active ? rr : r_all - 1), active);
+  double4 *st = store + size_t(img) * per_img + in + lane;  // this ray's entry of run c at st[c * cap]
+  if (!__any(ray.live)) {  // the same in every wave: they hold the same rays
+    for (int c = wave; c < tab.n; c += nw) AT(st, c * cap) = double4{0.0, 0.0, 0.0, 0.0};
+    return;
+  }
   const size_t o = size_t(img) * size_t(m.mp_stride);
-  const int nd = m.mp_n - 1;  // deflector planes; plane nd is the source's
-  auto slot = [&](int k) {
-    return ((size_t(img) * m.n_defl + k) * gridDim.x + blockIdx.x) * LENSIM_NPARAM;
-  };
-  // this block's partials of every deflector start at zero
-  for (int q = t; q < m.n_defl * LENSIM_NPARAM; q += blockDim.x)
-    AT(gpart_mp, slot(q / LENSIM_NPARAM) + q % LENSIM_NPARAM) = 0.0;
-  __syncthreads();
-  __shared__ double red[2][256 / 64][LENSIM_NPARAM];
-  const int r_all = npix * ss;
-  const int r0 = min(r_all, int(blockIdx.x) * spb * 256), r_end = min(r_all, r0 + spb * 256);
-  int step = 0;  // plane steps so far: consecutive ones alternate between the two halves of red
-  for (int base = r0; base < r_end; base += 256) {
-    const int rr = base + t;
-    const bool active = rr < r_end;
-    int sub;
-    const int pix = div_by(active ? rr : r0, ss, g.inv_ss, sub);
-    int i, sx;
-    const int j = div_by(pix, g.nx, g.inv_nx, i), sy = div_by(sub, g.s, g.inv_s, sx);
-    const double ox = g.o0 + sx * g.inv_s, oy = g.o0 + sy * g.inv_s;
-    const double x = i * g.m00 + j * g.m01 + g.ra0 + g.m00 * ox + g.m01 * oy;
-    const double y = i * g.m10 + j * g.m11 + g.dec0 + g.m10 * ox + g.m11 * oy;
-    const double w = active ? double(AT(static_cast<const T *>(ga.glow), size_t(img) * npix + pix)) * g.scale *
-                                  m.flux_scaling
-                            : 0.0;
-    const bool live = w != 0.0 && m.n_source > 0 && evaluated(g, i, j);
-    // forwards to the source plane
-    double Ax = x, Ay = y, Px = 0.0, Py = 0.0;
-    double gPx = 0.0, gPy = 0.0, gAx = 0.0, gAy = 0.0;
-    if (live) {
-      for (int p = 0; p <= nd; ++p) {
-        const double dt = AT(m.mp_tij, o + p);
-        Px += Ax * dt;
-        Py += Ay * dt;
-        if (p < nd) {
-          const double tz = AT(m.mp_tz, o + p);
-          double ax = 0.0, ay = 0.0;
-          int k = AT(m.mp_order, p);
-          k = k < 0 ? 0 : (k >= m.n_defl ? m.n_defl - 1 : k);
-          int type = type_of(m, k);
-          if (k >= m.n_lens && type == LENSIM_EPL) type = LENSIM_NULL;
-          deflect_one<T, HALO, true>(m, rp, img, k, type, Px / tz, Py / tz, ax, ay);
-          const double f = AT(m.mp_r2p, o + p);
-          Ax -= ax * f;
-          Ay -= ay * f;
+  const double *tij = all_tij + o, *tzs = all_tz + o, *r2p = all_r2p + o;
+  T bx = T(0), by = T(0), *b = static_cast<T *>(ga.beta) + ray.slot;
+  if (cap >= r_all) {  // the render kept the positions and beta (MpKeep)
+    if (ray.live) {
+      bx = AT(b, 0);
+      by = AT(b, 1);
+    }
+  } else {
+    double bxd, byd;
+    block_trace<T, HALO, true, true, SUB>(m, rp, tab, tij, tzs, r2p, img, ray.x, ray.y, red, bxd, byd,
+                                          [&](int c, double x, double y) {
+                                            if (wave == 0) AT(st, c * cap) = double4{x, y, 0.0, 0.0};
+                                          });
+    bx = T(bxd);
+    by = T(byd);
+    if (ray.live && wave == 0) {
+      AT(b, 0) = bx;
+      AT(b, 1) = by;
+    }
+  }
+  if (tab.n == 0) return;
+  const int nd = m.mp_n - 1;
+  double gPx = 0.0, gPy = 0.0, gAx = 0.0, gAy = 0.0;
+  if (ray.live) {
+    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, bx, by);
+    const double tzn = AT(tzs, nd), dt = AT(tij, nd);
+    gPx = ray.w * double(f2.d[0]) / tzn;
+    gPy = ray.w * double(f2.d[1]) / tzn;
+    gAx = dt * gPx;
+    gAy = dt * gPy;
+  }
+  __syncthreads();  // the positions are stored, the last sums read
+  auto members = [&](int p0, int p1) { return p0 + lane < p1 ? AT(tab.who, p0 + lane) : 0; };
+  int c = tab.n - 1, p0 = AT(tab.start, c), p1 = AT(tab.start, c + 1);
+  int ks = members(p0, p1);
+  double4 at = AT(st, c * cap);
+  double dt = AT(tij, p0), itz = rcp_full(AT(tzs, p0)), f = AT(r2p, p0);
+  for (; c >= 0; --c) {
+    const int cn = c > 0 ? c - 1 : 0, q0 = AT(tab.start, cn);
+    const int ks_next = members(q0, p0);
+    const double4 at_next = AT(st, cn * cap);
+    const double dt_next = AT(tij, q0), tz_next = AT(tzs, q0), f_next = AT(r2p, q0);
+    const double lx = -f * gAx, ly = -f * gAy;
+    double jx = 0.0, jy = 0.0;
+    for (int q = wave; q < p1 - p0; q += nw) {
+      const int k = __builtin_amdgcn_readlane(ks, q);
+      adjoint_one<T, HALO, SUB>(m, ga, rp, img, k & ((1 << kWhoBits) - 1), k >> kWhoBits, at.x, at.y, lx, ly, jx, jy);
+    }
+    if (wave == 0) AT(st, c * cap) = double4{at.x, at.y, ray.live ? lx : 0.0, ray.live ? ly : 0.0};
+    across_waves(red, c & 1, nw, jx, jy);
+    gPx = fma(jx, itz, gPx);
+    gPy = fma(jy, itz, gPy);
+    gAx = fma(dt, gPx, gAx);
+    gAy = fma(dt, gPy, gAy);
+    p1 = p0;
+    p0 = q0;
+    ks = ks_next;
+    at = at_next;
+    dt = dt_next;
+    itz = rcp_full(tz_next);
+    f = f_next;
+  }
+}
+
+// The same for a single-plane list: with beta = theta - alpha_scaling sum_j
+// alpha_j the adjoint of every deflection is l = -alpha_scaling w dS/dbeta.
+// The block's waves share the bulk list of its 64 rays (the first takes the
+// inline deflectors too).  Stores (x, y, l), beta, and dS/dbeta for the inline
+// deflectors' launches.
+constexpr int kBulkWaves = 8;
+template <typename T, bool HALO>
+__global__ __launch_bounds__(64 * kBulkWaves) void bulk_adjoint_kernel(
+    ModelArgs m, GridArgs g, GradArgs ga, const double *__restrict__ recd, const float *__restrict__ recf,
+    const double *__restrict__ coefd, const float *__restrict__ coeff, double4 *__restrict__ store, size_t per_img,
+    int round) {
+  __shared__ WaveSums red;
+  const int img = blockIdx.y, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r_all = g.nx * g.ny * g.s * g.s;
+  const int64_t cap = round_rays(per_img, 1), in = int64_t(blockIdx.x) * 64;
+  if (in >= cap || round * cap + in >= r_all) return;
+  const int64_t rr = round * cap + in + lane;
+  const bool active = rr < r_all;
+  const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
+  const GradRay ray = grad_ray<T>(m, g, ga, img, int(active ? rr : r_all - 1), active);
+  double ax = 0.0, ay = 0.0;
+  if (__any(ray.live)) {  // the same in every wave
+    if (wave == 0)
+      for (int k = 0; k < m.n_lens; ++k) deflect_one<T, HALO, false>(m, rp, img, k, m.types[k], ray.x, ray.y, ax, ay);
+    for (int k = m.n_lens + wave; k < m.n_defl; k += kBulkWaves) {
+      const int type = m.bulk_type ? m.bulk_type : AT(m.bulk_types, k - m.n_lens);
+      deflect_one<T, HALO, false>(m, rp, img, k, type == LENSIM_EPL ? LENSIM_NULL : type, ray.x, ray.y, ax, ay);
+    }
+    across_waves(red, 0, kBulkWaves, ax, ay);
+  }
+  if (wave != 0) return;
+  double lx = 0.0, ly = 0.0;
+  if (ray.live) {
+    const double as = m.alpha_scaling;
+    const T bx = T(ray.x - ax * as), by = T(ray.y - ay * as);
+    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, bx, by);
+    lx = -as * ray.w * double(f2.d[0]);
+    ly = -as * ray.w * double(f2.d[1]);
+    T *b = static_cast<T *>(ga.beta) + ray.slot;
+    AT(b, 0) = bx;
+    AT(b, 1) = by;
+    if (ga.gbeta) {
+      T *gb = static_cast<T *>(ga.gbeta) + ray.slot;
+      AT(gb, 0) = f2.d[0];
+      AT(gb, 1) = f2.d[1];
+    }
+  }
+  AT(store, size_t(img) * per_img + in + lane) = double4{ray.x, ray.y, lx, ly};
+}
+
+// One deflector's (or, of TNFW, a pair's) sums over rays [r0, r1) of `st`: a
+// lane per ray, each entry read once for the pair.
+template <int D>
+__device__ __forceinline__ void tnfw_sums(const double *const (&rd)[2], const double4 *st, int64_t r0, int64_t r1,
+                                          int lane, double (&acc)[2][LENSIM_NPARAM]) {
+  const TnfwRec ra(rd[0]), rb(rd[D - 1]);
+  for (int64_t r = r0 + lane; r < r1; r += 64) {
+    const double4 s = AT(st, r);
+    if (s.z == 0.0 && s.w == 0.0) continue;
+    tnfw_ray_grad(ra, rd[0], s.x, s.y, s.z, s.w, acc[0]);
+    if constexpr (D == 2) tnfw_ray_grad(rb, rd[1], s.x, s.y, s.z, s.w, acc[1]);
+  }
+}
+
+// Partial sums [img][plane or bulk index][slot][8] of lambda . d alpha /
+// d kwargs over a round's rays: a wave takes two planes' (or bulk) deflectors
+// q, q + 1 and one of the splits of the rays.  REST: the deflectors that are
+// not subhalos or linear (their duals' registers would cost the others waves);
+// each launch leaves the other's deflectors alone.
+template <typename T, bool HALO, bool REST>
+__global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
+                                                        const double *__restrict__ recd,
+                                                        const float *__restrict__ recf,
+                                                        const double *__restrict__ coefd,
+                                                        const float *__restrict__ coeff,
+                                                        const int *__restrict__ tab_all,
+                                                        const double4 *__restrict__ store, size_t per_img, int n,
+                                                        int round, int n_slots, bool both,
+                                                        double *__restrict__ gpart_mp) {
+  const int img = blockIdx.y, lane = threadIdx.x & 63;
+  if (REST && both && m.mp_n && mp_tab(m, tab_all, img).sub) return;  // no such deflector
+  const int q = 2 * __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (q >= n) return;
+  const int nq = min(2, n - q), slot = round * int(gridDim.z) + int(blockIdx.z);
+  const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
+  int k[2], type[2], run[2], runs = 1;
+  if (m.mp_n) {
+    const MpTab tab = mp_tab(m, tab_all, img);
+    runs = tab.n;
+    for (int d = 0; d < nq; ++d) {
+      const int v = __builtin_amdgcn_readfirstlane(AT(tab.who, q + d));
+      k[d] = v & ((1 << kWhoBits) - 1);
+      type[d] = v >> kWhoBits;
+      run[d] = __builtin_amdgcn_readfirstlane(AT(tab.run_of, q + d));
+    }
+  } else {
+    for (int d = 0; d < nq; ++d) {
+      k[d] = m.n_lens + q + d;
+      type[d] = __builtin_amdgcn_readfirstlane(m.bulk_type ? m.bulk_type : AT(m.bulk_types, q + d));
+      if (!bulk_type_ok_dev(type[d])) type[d] = LENSIM_NULL;
+      run[d] = 0;
+    }
+  }
+  // the round's rays and this split's share of them (whole waves)
+  const int64_t cap = round_rays(per_img, runs), left = int64_t(g.nx) * g.ny * g.s * g.s - round * cap;
+  const int64_t n_ray = left < 0 ? 0 : (left < cap ? left : cap);
+  const int64_t len = ((n_ray + 63) / 64 + gridDim.z - 1) / gridDim.z * 64;
+  const int64_t r0 = min(n_ray, len * blockIdx.z), r1 = min(n_ray, r0 + len);
+  if (!REST && r0 == r1) {  // nothing of this round (REST's deflectors are stored over by its own launch, after)
+    if (lane < nq * LENSIM_NPARAM)
+      AT(gpart_mp, ((size_t(img) * n + q + lane / LENSIM_NPARAM) * n_slots + slot) * LENSIM_NPARAM +
+                       lane % LENSIM_NPARAM) = 0.0;
+    return;
+  }
+  const double4 *st[2];
+  const double *rd[2];
+  for (int d = 0; d < 2; ++d) {
+    st[d] = store + size_t(img) * per_img + size_t(run[d < nq ? d : 0]) * cap;
+    rd[d] = rp.recd + k[d < nq ? d : 0] * kRec;
+  }
+  double acc[2][LENSIM_NPARAM];
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int i = 0; i < LENSIM_NPARAM; ++i) acc[d][i] = 0.0;
+  const bool pair = nq == 2 && type[0] == LENSIM_TNFW && type[1] == LENSIM_TNFW && run[0] == run[1];
+  if (!REST && pair) {
+    if constexpr (HALO) tnfw_sums<2>(rd, st[0], r0, r1, lane, acc);
+  } else {
+    for (int d = 0; d < nq; ++d) {
+      double a[2][LENSIM_NPARAM];
+#pragma unroll
+      for (int i = 0; i < LENSIM_NPARAM; ++i) a[0][i] = 0.0;
+      if (!REST && type[d] == LENSIM_TNFW) {
+        if constexpr (HALO) {
+          const double *const r[2] = {rd[d], rd[d]};
+          tnfw_sums<1>(r, st[d], r0, r1, lane, a);
+        }
+      } else if (!REST && (type[d] == LENSIM_CONVERGENCE || type[d] == LENSIM_SHEAR)) {
+        const double cx = rd[d][R_CX], cy = rd[d][R_CY], c2 = rd[d][2], c3 = rd[d][3];
+        const bool conv = type[d] == LENSIM_CONVERGENCE;
+        for (int64_t r = r0 + lane; r < r1; r += 64) {
+          const double4 s = AT(st[d], r);
+          if (s.z == 0.0 && s.w == 0.0) continue;
+          const double dx = s.x - cx, dy = s.y - cy;
+          if (conv) {  // alpha = kappa (dx, dy)
+            a[0][0] += s.z * dx + s.w * dy;
+            a[0][1] -= c2 * s.z;
+            a[0][2] -= c2 * s.w;
+          } else {  // alpha = (g1 dx + g2 dy, g2 dx - g1 dy)
+            a[0][0] += s.z * dx - s.w * dy;
+            a[0][1] += s.z * dy + s.w * dx;
+            a[0][2] -= c2 * s.z + c3 * s.w;
+            a[0][3] -= c3 * s.z - c2 * s.w;
+          }
+        }
+      } else if (REST && !sub_type(type[d])) {
+        for (int64_t r = r0 + lane; r < r1; r += 64) {
+          const double4 s = AT(st[d], r);
+          if (s.z == 0.0 && s.w == 0.0) continue;
+          double ax = 0.0, ay = 0.0, dax[LENSIM_NPARAM], day[LENSIM_NPARAM], dcen[4];
+          deflector_dalpha<T, HALO>(m, ga, rp, img, k[d], type[d], s.x, s.y, ax, ay, dax, day, dcen);
+#pragma unroll
+          for (int i = 0; i < LENSIM_NPARAM; ++i) a[0][i] += s.z * dax[i] + s.w * day[i];
         }
       }
-      const double tzn = AT(m.mp_tz, o + nd);
-      const T bx = T(Px / tzn), by = T(Py / tzn);
-      if (ga.gbeta) {  // beta for the source launches
-        T *gb = static_cast<T *>(ga.gbeta) + ((size_t(img) * npix + pix) * size_t(ss) + size_t(sub)) * 2;
-        AT(gb, 0) = bx;
-        AT(gb, 1) = by;
+#pragma unroll
+      for (int i = 0; i < LENSIM_NPARAM; ++i) {
+        if (d == 0) acc[0][i] = a[0][i];
+        else acc[1][i] = a[0][i];
       }
-      const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, bx, by);
-      gPx = w * double(f2.d[0]) / tzn;
-      gPy = w * double(f2.d[1]) / tzn;
-      // the source plane's step (no deflector): A_{nd-1} = A_nd
-      const double dt = AT(m.mp_tij, o + nd);
-      gAx += dt * gPx;
-      gAy += dt * gPy;
-      Px -= dt * Ax;
-      Py -= dt * Ay;
     }
-    // backwards over the deflector planes
-    for (int p = nd - 1; p >= 0; --p) {
-      int k = AT(m.mp_order, p);
-      k = k < 0 ? 0 : (k >= m.n_defl ? m.n_defl - 1 : k);
-      const int type = k < m.n_lens ? m.types[k] : (m.bulk_type ? m.bulk_type : AT(m.bulk_types, k - m.n_lens));
-      const int n = (type == LENSIM_EPL && k >= m.n_lens) ? 0 : n_params_of(type);  // bulk EPL: NULL
-      double c[LENSIM_NPARAM];
+  }
+  for (int d = 0; d < nq; ++d) {
+    if (REST == sub_type(type[d])) continue;
+    double v[LENSIM_NPARAM];
 #pragma unroll
-      for (int q = 0; q < LENSIM_NPARAM; ++q) c[q] = 0.0;
-      if (live && n > 0) {
-        const double tz = AT(m.mp_tz, o + p), f = AT(m.mp_r2p, o + p), dt = AT(m.mp_tij, o + p);
-        double ax = 0.0, ay = 0.0, dax[LENSIM_NPARAM], day[LENSIM_NPARAM], dcen[4];
-        deflector_dalpha<T, HALO>(m, ga, rp, img, k, type, Px / tz, Py / tz, ax, ay, dax, day, dcen);
-        const double lx = -f * gAx, ly = -f * gAy;
+    for (int i = 0; i < LENSIM_NPARAM; ++i) v[i] = wave_sum(d == 0 ? acc[0][i] : acc[1][i]);
+    if (type[d] == LENSIM_TNFW) tnfw_grad_scale(rd[d], v);
+    if (lane < LENSIM_NPARAM) {
+      double mine = 0.0;
 #pragma unroll
-        for (int q = 0; q < LENSIM_NPARAM; ++q) c[q] = lx * dax[q] + ly * day[q];
-        gPx -= (lx * dcen[0] + ly * dcen[1]) / tz;
-        gPy -= (lx * dcen[2] + ly * dcen[3]) / tz;
-        Ax += f * ax;
-        Ay += f * ay;
-        gAx += dt * gPx;
-        gAy += dt * gPy;
-        Px -= dt * Ax;
-        Py -= dt * Ay;
-      } else if (live) {  // a deflector without kwargs deflects by zero
-        const double dt = AT(m.mp_tij, o + p);
-        gAx += dt * gPx;
-        gAy += dt * gPy;
-        Px -= dt * Ax;
-        Py -= dt * Ay;
-      }
-      // the plane's sum over the block, added to deflector k's partial
-      const int buf = step++ & 1;
-#pragma unroll
-      for (int q = 0; q < LENSIM_NPARAM; ++q) {
-        const double v = wave_sum(c[q]);
-        if ((t & 63) == 0) red[buf][t >> 6][q] = v;
-      }
-      __syncthreads();
-      if (t < n) {
-        double v = 0.0;
-        for (int wv = 0; wv < int(blockDim.x >> 6); ++wv) v += red[buf][wv][t];
-        // the block's first sweep stores (no wait for a load), later ones add
-        if (base == r0)
-          AT(gpart_mp, slot(k) + t) = v;
-        else
-          AT(gpart_mp, slot(k) + t) += v;
-      }
+      for (int i = 0; i < LENSIM_NPARAM; ++i) mine = lane == i ? v[i] : mine;
+      AT(gpart_mp, ((size_t(img) * n + q + d) * n_slots + slot) * LENSIM_NPARAM + lane) = mine;
     }
   }
 }
 
-// The deflectors' partials of the nb_mp blocks of mp_grad_kernel summed in
-// block order into the first of the nblk slots grad_reduce_kernel reads (the
-// others zero).
-__global__ void mp_partial_reduce(const double *__restrict__ gpart_mp, int nb_mp, int n_img, int n_defl, int n_prof,
-                                  int nblk, double *__restrict__ gpart) {
+// The list's partial sums added up in slot order into the first of the nblk
+// slots grad_reduce_kernel reads (the others zero).  A deflector that the
+// caller's order names on several planes gets the sum over them, one that it
+// does not name zero.
+__global__ void defl_partial_reduce(ModelArgs m, const int *__restrict__ tab_all, const double *__restrict__ gpart_mp,
+                                    int n, int n_slots, int n_img, int nblk, double *__restrict__ gpart) {
+  const int k0 = m.mp_n ? 0 : m.n_lens, nk = m.n_defl - k0;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_img * n_defl * LENSIM_NPARAM) return;
-  const int q = i % LENSIM_NPARAM, r = i / LENSIM_NPARAM, k = r % n_defl, img = r / n_defl;
+  if (i >= n_img * nk * LENSIM_NPARAM) return;
+  const int p = i % LENSIM_NPARAM, r = i / LENSIM_NPARAM, k = k0 + r % nk, img = r / nk;
   double v = 0.0;
-  for (int b = 0; b < nb_mp; ++b) v += AT(gpart_mp, (size_t(r) * nb_mp + b) * LENSIM_NPARAM + q);
-  const size_t o = (size_t(img) * n_prof + k) * nblk;
-  for (int b = 0; b < nblk; ++b) AT(gpart, (o + b) * LENSIM_NPARAM + q) = b == 0 ? v : 0.0;
+  auto add = [&](int q) {
+    for (int b = 0; b < n_slots; ++b)
+      v += AT(gpart_mp, ((size_t(img) * n + q) * n_slots + b) * LENSIM_NPARAM + p);
+  };
+  if (!m.mp_n) {
+    add(k - k0);
+  } else {
+    const MpTab tab = mp_tab(m, tab_all, img);
+    if (!tab.dup) {
+      if (AT(tab.plane_of, k) >= 0) add(AT(tab.plane_of, k));
+    } else {
+      for (int q = 0; q < n; ++q)
+        if ((AT(tab.who, q) & ((1 << kWhoBits) - 1)) == k) add(q);
+    }
+  }
+  const size_t o = (size_t(img) * m.n_prof + k) * nblk;
+  for (int b = 0; b < nblk; ++b) AT(gpart, (o + b) * LENSIM_NPARAM + p) = b == 0 ? v : 0.0;
 }
 
-template <typename T>
-int launch_mp_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, const double *recd, const float *recf,
-                   double *gpart_mp, int nblk, int n_img, hipStream_t st) {
+// The gradient of the multi-plane or bulk list into ga.gpart, and beta (and
+// dS/dbeta) at every ray for the launches that follow.
+template <typename T, bool HALO>
+int launch_defl_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, const double *recd, const float *recf,
+                     const int *tab, double *gpart_mp, double4 *store, int nblk, int n_img, hipStream_t st) {
   const size_t rays = size_t(g.nx) * g.ny * g.s * g.s;
-  const int nb_mp = mp_grad_blocks(rays, n_img);
-  const int spb = int(((rays + 255) / 256 + nb_mp - 1) / nb_mp);
-  const dim3 grid(nb_mp, n_img);
-  if (m.has_halo)
-    mp_grad_kernel<T, true><<<grid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, gpart_mp, spb);
-  else
-    mp_grad_kernel<T, false><<<grid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, gpart_mp, spb);
-  int rc = check_launch("mp_grad_kernel");
-  if (rc || m.n_defl == 0) return rc;
-  const int n = n_img * m.n_defl * LENSIM_NPARAM;
-  mp_partial_reduce<<<(n + 255) / 256, 256, 0, st>>>(gpart_mp, nb_mp, n_img, m.n_defl, m.n_prof, nblk, ga.gpart);
-  return check_launch("mp_partial_reduce");
+  const DeflGradPlan p = defl_grad_plan(m, rays, n_img);
+  const dim3 grid((unsigned)((rays + 63) / 64), n_img);
+  const dim3 dgrid((p.n + 7) / 8, n_img, p.splits);
+  int sub = sub_list(m);
+  if (!m.mp_n && sub == 0) sub = m.bulk_type ? int(sub_type(m.bulk_type)) : 2;  // of the bulk list alone
+  for (int r = 0; r < p.rounds; ++r) {
+    if (!m.mp_n) {
+      bulk_adjoint_kernel<T, HALO><<<grid, 64 * kBulkWaves, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, store,
+                                                                     p.per_img, r);
+    } else {
+#define LENSIM_ADJOINT(H, S)                                                                                         \
+  mp_adjoint_kernel<T, H, S><<<grid, 64 * mp_waves(rays, S), 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, \
+                                                                      sub == 2, store, p.per_img, r, m.mp_tij,       \
+                                                                      m.mp_tz, m.mp_r2p)
+      if (sub) LENSIM_ADJOINT(true, true);
+      if (sub != 1) LENSIM_ADJOINT(HALO, false);
+#undef LENSIM_ADJOINT
+    }
+    int rc = check_launch("adjoint kernel");
+    if (rc) return rc;
+    if (p.n == 0) return LENSIM_OK;  // no deflector: beta alone
+    // of an inline list the types are known: a launch for the kinds it holds
+    bool any_sub = m.n_bulk > 0 && sub != 0, any_rest = sub != 1;
+    for (int k = 0; m.mp_n && k < m.n_lens; ++k) any_sub = any_sub || sub_type(m.types[k]);
+    if (any_sub || m.n_bulk > 0)
+      defl_grad_kernel<T, HALO, false><<<dgrid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, store,
+                                                              p.per_img, p.n, r, p.slots(), sub == 2, gpart_mp);
+    if (any_rest)
+      defl_grad_kernel<T, HALO, true><<<dgrid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, store,
+                                                             p.per_img, p.n, r, p.slots(), sub == 2, gpart_mp);
+    if ((rc = check_launch("defl_grad_kernel"))) return rc;
+  }
+  const int nt = n_img * (m.n_defl - (m.mp_n ? 0 : m.n_lens)) * LENSIM_NPARAM;
+  defl_partial_reduce<<<(nt + 255) / 256, 256, 0, st>>>(m, tab, gpart_mp, p.n, p.slots(), n_img, nblk, ga.gpart);
+  return check_launch("defl_partial_reduce");
 }
 
 __global__ void grad_reduce_kernel(const double *__restrict__ gpart, int nblk, int n, double *__restrict__ grad) {
@@ -3392,7 +3556,8 @@ int launch_conv_mfma(ConvArgs c, const MfmaPlan &pl, int n_img, const float *in,
 template <typename T>
 int run_image(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, int kx, int ky, int edge,
               const lensim_data *data, const double *params, int n_img, unsigned flags, T *out, double *logl,
-              unsigned char *ws, const Layout &L, hipStream_t st, T *gout = nullptr) {
+              unsigned char *ws, const Layout &L, hipStream_t st, T *gout = nullptr,
+              const MpKeep &keep = MpKeep{}) {
   const ModelArgs m = with_grid(m_in, g);
   const bool identity = !psf || psf->type == LENSIM_PSF_NONE || (flags & LENSIM_IMAGE_UNCONVOLVED);
   const bool mfma = use_mfma<T>(identity, kx, ky);
@@ -3439,7 +3604,7 @@ int run_image(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, i
   const float *recf = reinterpret_cast<const float *>(ws + L.recf);
   const double *coefd = reinterpret_cast<const double *>(ws + L.coefd);
   const float *coeff = reinterpret_cast<const float *>(ws + L.coeff);
-  rc = launch_render<T>(m, g, recd, recf, coefd, coeff, tab, flags, lowres, blkmax, n_img, st);
+  rc = launch_render<T>(m, g, recd, recf, coefd, coeff, tab, flags, keep, lowres, blkmax, n_img, st);
   if (rc) return rc;
   timing_mark(1, st);
   ConvArgs c{};
@@ -3611,7 +3776,8 @@ __global__ void unpool_kernel(const T *__restrict__ in, int nx, int ny, int s, i
 template <typename T>
 int run_image_ss(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, int kx, int ky, int edge,
                  const SSPlan &ss, const lensim_data *data, const double *params, int n_img, unsigned flags, T *out,
-                 double *logl, unsigned char *ws, const Layout &L, hipStream_t st, T *gout = nullptr) {
+                 double *logl, unsigned char *ws, const Layout &L, hipStream_t st, T *gout = nullptr,
+                 const MpKeep &keep = MpKeep{}) {
   const int s = ss.s;
   const GridArgs gh = ray_grid(g);
   const ModelArgs m = with_grid(m_in, gh);
@@ -3643,7 +3809,7 @@ int run_image_ss(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf
   int *tab = reinterpret_cast<int *>(ws + L.mp_tab);
   if (m.mp_n && (rc = launch_mp_runs(m, tab, n_img, st))) return rc;
   timing_mark(0, st);
-  rc = launch_render<T>(m, gh, recd, recf, coefd, coeff, tab, flags, hr, blkmax, n_img, st);
+  rc = launch_render<T>(m, gh, recd, recf, coefd, coeff, tab, flags, keep, hr, blkmax, n_img, st);
   if (rc) return rc;
   timing_mark(1, st);
   if (mfma) {
@@ -3762,9 +3928,16 @@ int run_grad(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int k
              unsigned char *ws, const Layout &L, hipStream_t st) {
   T *gmodel = reinterpret_cast<T *>(ws + L.gmodel);
   const unsigned flags = LENSIM_IMAGE_SOURCE | LENSIM_IMAGE_LENS_LIGHT;
+  MpKeep keep{};
+  if (m.mp_n && m.n_source > 0) {
+    const size_t rays = size_t(g.nx) * g.ny * g.s * g.s;
+    keep.store = reinterpret_cast<double4 *>(ws + L.gstate);
+    keep.per_img = defl_grad_plan(m, rays, n_img).per_img;
+    keep.beta = ws + L.beta;
+  }
   int rc = ss.on ? run_image_ss<T>(m, g, psf, kx, ky, edge, ss, data, params, n_img, flags, nullptr, logl, ws, L, st,
-                                   gmodel)
-                 : run_image<T>(m, g, psf, kx, ky, edge, data, params, n_img, flags, nullptr, logl, ws, L, st, gmodel);
+                                   gmodel, keep)
+                 : run_image<T>(m, g, psf, kx, ky, edge, data, params, n_img, flags, nullptr, logl, ws, L, st, gmodel, keep);
   if (rc) return rc;
   const bool identity = !psf || psf->type == LENSIM_PSF_NONE;
   const int kyp = kyp_of(ky);
@@ -3804,26 +3977,26 @@ int run_grad(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int k
   ga.glow = glow;
   ga.gpart = reinterpret_cast<double *>(ws + L.gpart);
   ga.gbeta = L.gbeta ? static_cast<void *>(ws + L.gbeta) : nullptr;
+  ga.beta = L.beta ? static_cast<void *>(ws + L.beta) : nullptr;
   const int npix = gg.nx * gg.ny, nblk = (npix + 256 * kGradPix - 1) / (256 * kGradPix);
   const double *recd = reinterpret_cast<const double *>(ws + L.recd);
   const float *recf = reinterpret_cast<const float *>(ws + L.recf);
-  // multi-plane: every deflector in one launch, which also stores beta at every
-  // ray (ga.gbeta) for the source launches
-  if (m.mp_n && (rc = launch_mp_grad<T>(m, gg, ga, recd, recf, reinterpret_cast<double *>(ws + L.gpart_mp), nblk,
-                                        n_img, st)))
-    return rc;
-  // the sources first: the first source's launch stores dS/dbeta at every ray
+  // a multi-plane or bulk list first: it also stores beta (and dS/dbeta) at
+  // every ray for the launches below
+  if (m.mp_n || m.n_bulk > 0) {
+    const int *tab = reinterpret_cast<const int *>(ws + L.mp_tab);
+    double *gpart_mp = reinterpret_cast<double *>(ws + L.gpart_mp);
+    double4 *store = reinterpret_cast<double4 *>(ws + L.gstate);
+    rc = m.has_halo ? launch_defl_grad<T, true>(m, gg, ga, recd, recf, tab, gpart_mp, store, nblk, n_img, st)
+                    : launch_defl_grad<T, false>(m, gg, ga, recd, recf, tab, gpart_mp, store, nblk, n_img, st);
+    if (rc) return rc;
+  }
+  // then the sources: the first source's launch stores dS/dbeta at every ray
   // (ga.gbeta), which the inline lens launches after it read
   for (int q = 0; q < m.n_prof; ++q) {
     const int k = q < m.n_source ? m.n_defl + q : (q < m.n_source + m.n_defl ? q - m.n_source : q);
-    if (m.mp_n && k < m.n_defl) continue;  // multi-plane: mp_grad_kernel above
-    if (k == m.n_lens && m.n_bulk > 0) {  // the bulk list in one launch
-      rc = m.has_halo ? launch_bulk_grad<T, true>(m, gg, ga, recd, recf, nblk, n_img, st)
-                      : launch_bulk_grad<T, false>(m, gg, ga, recd, recf, nblk, n_img, st);
-      if (rc) return rc;
-      q += m.n_bulk - 1;
-      continue;
-    }
+    if (m.mp_n && k < m.n_defl) continue;            // done above
+    if (k >= m.n_lens && k < m.n_defl) continue;     // the bulk list, done above
     rc = m.has_halo ? launch_grad_profile<T, true>(m, gg, ga, recd, recf, nblk, n_img, k, st)
                     : launch_grad_profile<T, false>(m, gg, ga, recd, recf, nblk, n_img, k, st);
     if (rc) return rc;

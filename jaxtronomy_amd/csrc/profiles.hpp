@@ -1007,7 +1007,7 @@ __device__ __forceinline__ void nfw_defl(const Rec<T> &r, double x, double y, do
 // caller's floor: u >= 1e-6), with w = sqrt(tau^2 + u):
 //   g = pre B,  B = (tau^2 + 2 u - 1) F - pi w + C0 + w L C1,
 //   F = arctan(sqrt(u - 1)) / sqrt(u - 1) (arctanh below u = 1),  L = ln(X / (tau + w)),
-// and, for the gradient, X dB/dX and tau dB/dtau (GRAD):
+// and, for the gradient, X dB/dX and tau dB/dtau:
 //   X dB/dX = 4 u F + (tau^2 + 2 u - 1) X F' + (u / w) (L C1 - pi) + tau^2 - 1,  X F' = (1 - u F) / (u - 1),
 //   tau dB/dtau = 2 tau^2 F + D0 + (tau^2 / w) (L C1 - pi) + w L E1
 // (X dL/dX = tau / w, tau dL/dtau = -tau / w).  Nothing but u is needed of the
@@ -1050,7 +1050,8 @@ struct TnfwRec {
   }
 };
 
-template <bool GRAD>
+// GRAD: 0 B alone, 1 X dB/dX too, 2 tau dB/dtau too
+template <int GRAD>
 __device__ __forceinline__ void tnfw_core(const TnfwRec &r, const double *rd, double u, double &iu, double &B,
                                           double &XBX, double &tBt) {
   const double tau = r.tau, tau2 = r.tau2;
@@ -1066,9 +1067,11 @@ __device__ __forceinline__ void tnfw_core(const TnfwRec &r, const double *rd, do
     const double vw = v + w, rvw = rcp_full(vw * vw);
     const double Kr = r.K * rvw;
     B0 = fma(Kr, iv, -(fma(r.t2m1, iu, 2.0) * G));
-    if constexpr (GRAD) {
+    if constexpr (GRAD > 0) {
       const double iv2 = iv * iv;
       X0 = fma(-Kr * u, (v + vw) * iv * iv2 * iw, fma(fma(2.0, u, r.t2m1) * iv2, 1.0 + G, -4.0 * G));
+    }
+    if constexpr (GRAD > 1) {
       t0 = fma(rd[TN_PT] * iv, iw * rvw * vw, -2.0 * y2 * G);
     }
   };
@@ -1105,7 +1108,7 @@ __device__ __forceinline__ void tnfw_core(const TnfwRec &r, const double *rd, do
         F = atanh_dbl(s) * rcp_refined(s);
       }
       B0 = fma(fma(2.0, u, r.t2m1), F, -M_PI * w);
-      if constexpr (GRAD) {
+      if constexpr (GRAD > 0) {
         const double e = u - 1.0;
         double XF;
         if (fabs(e) < 0.03) {  // 2 u dF/du, F = sum (-e)^n / (2 n + 1): the quotient cancels here
@@ -1116,7 +1119,7 @@ __device__ __forceinline__ void tnfw_core(const TnfwRec &r, const double *rd, do
           XF = fma(-u, F, 1.0) / e;
         }
         X0 = fma(fma(2.0, u, r.t2m1), XF, u * fma(4.0, F, -M_PI * iw));
-        t0 = tau2 * fma(2.0, F, -M_PI * iw);
+        if constexpr (GRAD > 1) t0 = tau2 * fma(2.0, F, -M_PI * iw);
       }
     }
     if (y2 <= 0.25) {
@@ -1130,10 +1133,10 @@ __device__ __forceinline__ void tnfw_core(const TnfwRec &r, const double *rd, do
     }
   }
   B = fma(wL, r.c1, B0 + r.c0);
-  if constexpr (GRAD) {
+  if constexpr (GRAD > 0) {
     const double LC = wL * iw * r.c1 * iw;  // L C1 / w
     XBX = fma(u, LC, X0 + r.t2m1);
-    tBt = fma(tau2, LC, fma(wL, rd[TN_E1], t0 + rd[TN_D0]));
+    if constexpr (GRAD > 1) tBt = fma(tau2, LC, fma(wL, rd[TN_E1], t0 + rd[TN_D0]));
   }
 }
 
@@ -1145,10 +1148,58 @@ __device__ __forceinline__ void tnfw_defl_f64(const double *rd, double x, double
   const double xs = dx * r.irs, ys = dy * r.irs;
   const double u = fmax(fma(xs, xs, ys * ys), 1e-6);
   double iu, B, d0, d1;
-  tnfw_core<false>(r, rd, u, iu, B, d0, d1);
+  tnfw_core<0>(r, rd, u, iu, B, d0, d1);
   const double a = r.ap * B * iu;
   ax = fma(a, dx, ax);
   ay = fma(a, dy, ay);
+}
+
+// With alpha = a d, d = (x, y) - centre, a = 4 rho0 Rs g / X^2 and (lx, ly) the
+// adjoint of alpha: the Jacobian d alpha / dx = a I + (X da/dX / R^2) d d^T
+// (X da/dX = 4 rho0 Rs pre X dB/dX / X^2 - 2 a; 0 at X's floor), so
+//   (d alpha / dx)^T l = a l + (X da/dX / R^2) (l . d) d,
+// whose negative is the product with the centre's derivative.
+__device__ __forceinline__ void tnfw_adjoint(const TnfwRec &r, const double *rd, double x, double y, double lx,
+                                             double ly, double &jx, double &jy) {
+  const double dx = x - r.cx, dy = y - r.cy;
+  const double xs = dx * r.irs, ys = dy * r.irs;
+  const double u0 = fma(xs, xs, ys * ys), u = fmax(u0, 1e-6);
+  double iu, B, XBX, tBt;
+  tnfw_core<1>(r, rd, u, iu, B, XBX, tBt);
+  const double ai = r.ap * iu, a = ai * B;
+  const double q = u0 > 1e-6 ? fma(ai, XBX, -2.0 * a) * (iu * r.irs * r.irs) : 0.0;
+  const double qs = q * fma(lx, dx, ly * dy);
+  jx = fma(a, lx, fma(qs, dx, jx));
+  jy = fma(a, ly, fma(qs, dy, jy));
+}
+
+// l . d alpha / d(Rs, alpha_Rs, r_trunc, center_x, center_y) added to acc[0..4],
+// the first three up to the factors of tnfw_grad_scale: a is a function of
+// (Rs, X, tau) = (Rs, R / Rs, r_trunc / Rs), so
+//   Rs da/dRs = -(a + X da/dX + tau da/dtau),  r_trunc da/dr_trunc = tau da/dtau,
+// tau da/dtau = a d ln pre / d ln tau + 4 rho0 Rs pre tau dB/dtau / X^2.
+__device__ __forceinline__ void tnfw_ray_grad(const TnfwRec &r, const double *rd, double x, double y, double lx,
+                                              double ly, double *acc) {
+  const double dx = x - r.cx, dy = y - r.cy;
+  const double xs = dx * r.irs, ys = dy * r.irs;
+  const double u0 = fma(xs, xs, ys * ys), u = fmax(u0, 1e-6);
+  double iu, B, XBX, tBt;
+  tnfw_core<2>(r, rd, u, iu, B, XBX, tBt);
+  const double ai = r.ap * iu, a = ai * B;
+  const double aX = u0 > 1e-6 ? fma(ai, XBX, -2.0 * a) : 0.0;
+  const double at = fma(a, rd[TN_DP], ai * tBt);
+  const double sd = fma(lx, dx, ly * dy);
+  const double qs = aX * (iu * r.irs * r.irs) * sd;
+  acc[0] = fma(-sd, a + aX + at, acc[0]);
+  acc[1] = fma(sd, B * iu, acc[1]);
+  acc[2] = fma(sd, at, acc[2]);
+  acc[3] -= fma(a, lx, qs * dx);
+  acc[4] -= fma(a, ly, qs * dy);
+}
+__device__ __forceinline__ void tnfw_grad_scale(const double *rd, double *acc) {
+  acc[0] *= rd[TN_IRS];
+  acc[1] *= rd[TN_A1] * rd[TN_PRE];
+  acc[2] *= rd[TN_IRT];
 }
 
 // TNFW deflection, LensModel/Profiles/tnfw.py:67-87, :226-248, _g :329-349,
