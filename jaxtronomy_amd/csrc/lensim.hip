@@ -198,6 +198,7 @@ struct ModelArgs {
   int32_t has_nie_nfw;  // an SIE / NIE or NFW deflector (inline or bulk), or halos on several planes: the float
                         // form deflects SIE / NIE and the NFW family in double
   SubSteps sub;         // sub-ray steps of the call's grid, for the records (with_grid); zero without a grid
+  int32_t unit_amp;     // the light profiles' records take amp = 1 (the linear solve's responses)
   const int32_t *bulk_types;
   int32_t types[LENSIM_MAX_PROFILES];
   int32_t epl_index[LENSIM_MAX_PROFILES];
@@ -604,7 +605,10 @@ __device__ void prep_one(const ModelArgs &m, const double *__restrict__ params, 
       CHECK_SPAN(dcf, LENSIM_EPL_NMAX * sizeof(float));
     }
   }
-  prepare_record(type, p, rec, coef, m.sub, dcoef, cf, dcf);
+  double q[LENSIM_NPARAM];
+#pragma unroll
+  for (int i = 0; i < LENSIM_NPARAM; ++i) q[i] = (i == 0 && m.unit_amp && k >= m.n_defl) ? 1.0 : p[i];
+  prepare_record(type, q, rec, coef, m.sub, dcoef, cf, dcf);
   for (int i = 0; i < kRec; ++i) {
     AT(recd, size_t(ri) * kRec + i) = rec[i];
     AT(recf, size_t(ri) * kRec + i) = float(rec[i]);
@@ -1159,7 +1163,14 @@ int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, con
     const bool pair = ((d0 == LENSIM_EPL || d0 == LENSIM_NIE || d0 == LENSIM_NFW) && (d1 == 0 || d1 == LENSIM_SHEAR)) ||
                       (d0 == LENSIM_NFW && d1 == LENSIM_NIE) || (d0 == LENSIM_NIE && d1 == LENSIM_NFW);
     fast = pair && (d0 != LENSIM_EPL || m.epl_index[0] == 0);
-    for (int k = m.n_lens; fast && k < m.n_lens + m.n_source + m.n_light; ++k) fast = sersic(m.types[k]);
+    // a light profile that a response column of the linear solve leaves out
+    // (LENSIM_NULL) is no hindrance where nothing reads its record; in the
+    // float form, whose two renders round differently, the columns stay with
+    // render_kernel
+    const bool f64 = sizeof(T) == sizeof(double);
+    const int ts = m.types[m.n_lens], tl = m.n_light ? m.types[m.n_lens + 1] : LENSIM_NULL;
+    fast = fast && (sersic(ts) || (f64 && ts == LENSIM_NULL && !(flags & LENSIM_IMAGE_SOURCE))) &&
+           (sersic(tl) || m.n_light == 0 || (f64 && tl == LENSIM_NULL));
   }
   if (m.mp_n) {  // the block maxima for the MFMA convolution follow from the image in a second launch
     int rc = launch_render_mp<T>(m, g, recd, recf, coefd, coeff, tab, flags, keep, out, n_img, st);
@@ -1187,7 +1198,7 @@ int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, con
 #undef LENSIM_RENDER
     return check_launch("render_kernel");
   }
-  const bool ll = m.n_light == 1;
+  const bool ll = m.n_light == 1 && m.types[m.n_lens + 1] != LENSIM_NULL;
 #define LENSIM_FAST(A, B)                                                                                       \
   do {                                                                                                          \
     if (ll)                                                                                                     \
@@ -3320,14 +3331,15 @@ __global__ void grad_reduce_kernel(const double *__restrict__ gpart, int nblk, i
 // One wave per image: lane l sums partials l, l + 64, ... and a fixed
 // butterfly adds the 64 lane sums, so the order depends on n_tiles alone (not
 // on the batch); the partials of an image are read contiguously.
+// add: a term per image (the linear solve's marginalisation constant), or NULL.
 __global__ __launch_bounds__(64) void logl_kernel(const double *__restrict__ partial, int n_tiles,
-                                                  double *__restrict__ logl) {
+                                                  const double *__restrict__ add, double *__restrict__ logl) {
   const int img = blockIdx.x;
   const double *p = partial + size_t(img) * n_tiles;
   double s = 0.0;
   for (int t = threadIdx.x; t < n_tiles; t += 64) s += AT(p, t);
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (threadIdx.x == 0) AT(logl, img) = -s / 2.0;
+  if (threadIdx.x == 0) AT(logl, img) = -s / 2.0 + (add ? AT(add, img) : 0.0);
 }
 
 // ------------------------------------------------------------ launches ---
@@ -3552,6 +3564,67 @@ int launch_conv_mfma(ConvArgs c, const MfmaPlan &pl, int n_img, const float *in,
   }
 }
 
+// The PSF preparation of a call on the grid itself, and which convolution it is
+// for (at most one of mfma, mf64).
+template <typename T>
+struct ConvChoice {
+  bool mfma, mf64;
+  PsfJob job;
+  ConvChoice(const lensim_psf *psf, unsigned flags, int kx, int ky, unsigned char *ws, const Layout &L) {
+    const bool identity = !psf || psf->type == LENSIM_PSF_NONE || (flags & LENSIM_IMAGE_UNCONVOLVED);
+    mfma = use_mfma<T>(identity, kx, ky);
+    mf64 = use_mf64<T>(identity, kx, ky);
+    job = PsfJob{};
+    job.mode = mfma ? 2 : (mf64 ? 3 : 1);
+    job.k = identity ? nullptr : psf->d_kernel;
+    job.kx = kx;
+    job.ky = ky;
+    job.kyp = kyp_of(ky);
+    job.kt = reinterpret_cast<double *>(ws + (mf64 ? L.bfrag : L.psf));
+    job.hdr = reinterpret_cast<int *>(ws + L.bfrag);
+    job.frag = reinterpret_cast<half8 *>(ws + L.bfrag + 16);
+    if (mfma) {
+      job.nks = mfma_nks(kx);
+      job.n_steps = mfma_steps(kx, ky);
+    }
+    if (mf64) {
+      job.nks = mf64_nk4(kx);
+      job.n_steps = mf64_steps(kx, ky);
+    }
+  }
+};
+
+// The records (with EPL coefficients' derivatives when dc) and the PSF
+// preparation in one launch; the plane runs of a multi-plane model in another.
+int launch_prep_psf(const ModelArgs &m, const double *params, int n_img, const PsfJob &pj, bool dc, unsigned char *ws,
+                    const Layout &L, hipStream_t st) {
+  const int nb_prep = (n_img * m.n_prof + 255) / 256;
+  prep_psf_kernel<<<nb_prep + psf_job_blocks(pj), 256, 0, st>>>(
+      m, params, n_img, reinterpret_cast<double *>(ws + L.recd), reinterpret_cast<float *>(ws + L.recf),
+      reinterpret_cast<double *>(ws + L.coefd), reinterpret_cast<float *>(ws + L.coeff),
+      dc ? reinterpret_cast<double *>(ws + L.dcoefd) : nullptr, dc ? reinterpret_cast<float *>(ws + L.dcoeff) : nullptr,
+      pj, nb_prep);
+  int rc = check_launch("prep_psf_kernel");
+  if (!rc && m.mp_n) rc = launch_mp_runs(m, reinterpret_cast<int *>(ws + L.mp_tab), n_img, st);
+  return rc;
+}
+
+// 'Same' convolution of n_img pooled images with the prepared PSF; with data
+// in c also their chi^2 partials (n_tiles an image).
+template <typename T>
+int launch_conv(const ConvArgs &c, const ConvChoice<T> &cc, int n_img, const T *in, const float *blkmax, T *out,
+                double *partial, int *n_tiles, hipStream_t st) {
+  if (!cc.mfma && !cc.mf64) return launch_conv_kernel<T>(c, n_img, in, cc.job.kt, out, partial, n_tiles, st);
+  *n_tiles = n16_tiles(c.nx, c.ny);  // chi^2 partials of the 16 x 16 output tiles
+  if (cc.mfma)
+    return launch_conv_mfma(c, mfma_plan(c.nx, c.ny, n_img, c.kx, c.ky), n_img, reinterpret_cast<const float *>(in),
+                            cc.job.hdr, cc.job.frag, blkmax, (c.nx * c.ny + 255) / 256, reinterpret_cast<float *>(out),
+                            partial, st);
+  return launch_conv_mf64(c, mfma_plan(c.nx, c.ny, n_img, c.kx, c.ky, true), n_img,
+                          reinterpret_cast<const double *>(in), cc.job.kt, reinterpret_cast<double *>(out), partial,
+                          st);
+}
+
 // The image pipeline shared by lensim_image and lensim_loglike.
 template <typename T>
 int run_image(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, int kx, int ky, int edge,
@@ -3559,46 +3632,12 @@ int run_image(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, i
               unsigned char *ws, const Layout &L, hipStream_t st, T *gout = nullptr,
               const MpKeep &keep = MpKeep{}) {
   const ModelArgs m = with_grid(m_in, g);
-  const bool identity = !psf || psf->type == LENSIM_PSF_NONE || (flags & LENSIM_IMAGE_UNCONVOLVED);
-  const bool mfma = use_mfma<T>(identity, kx, ky);
-  const bool mf64 = use_mf64<T>(identity, kx, ky);
-  const int kyp = kyp_of(ky);
-  double *kf = reinterpret_cast<double *>(ws + L.psf);
-  int *hdr = reinterpret_cast<int *>(ws + L.bfrag);
-  half8 *frag = reinterpret_cast<half8 *>(ws + L.bfrag + 16);
-  double *frag64 = reinterpret_cast<double *>(ws + L.bfrag);
-  // records and the PSF preparation in one launch
-  PsfJob pj{};
-  pj.mode = mfma ? 2 : (mf64 ? 3 : 1);
-  pj.k = identity ? nullptr : psf->d_kernel;
-  pj.kx = kx;
-  pj.ky = ky;
-  pj.kyp = kyp;
-  pj.kt = mf64 ? frag64 : kf;
-  pj.hdr = hdr;
-  pj.frag = frag;
-  if (mfma) {
-    pj.nks = mfma_nks(kx);
-    pj.n_steps = mfma_steps(kx, ky);
-  }
-  if (mf64) {
-    pj.nks = mf64_nk4(kx);
-    pj.n_steps = mf64_steps(kx, ky);
-  }
-  const int nb_prep = (n_img * m.n_prof + 255) / 256;
-  const bool dc = gout != nullptr;
-  prep_psf_kernel<<<nb_prep + psf_job_blocks(pj), 256, 0, st>>>(
-      m, params, n_img, reinterpret_cast<double *>(ws + L.recd), reinterpret_cast<float *>(ws + L.recf),
-      reinterpret_cast<double *>(ws + L.coefd), reinterpret_cast<float *>(ws + L.coeff),
-      dc ? reinterpret_cast<double *>(ws + L.dcoefd) : nullptr, dc ? reinterpret_cast<float *>(ws + L.dcoeff) : nullptr,
-      pj, nb_prep);
-  int rc = check_launch("prep_psf_kernel");
+  const ConvChoice<T> cc(psf, flags, kx, ky, ws, L);
+  int rc = launch_prep_psf(m, params, n_img, cc.job, gout != nullptr, ws, L, st);
   if (rc) return rc;
   T *lowres = reinterpret_cast<T *>(ws + L.lowres);
-  float *blkmax = mfma ? reinterpret_cast<float *>(ws + L.blkmax) : nullptr;
-  const int npix = g.nx * g.ny;
-  int *tab = reinterpret_cast<int *>(ws + L.mp_tab);
-  if (m.mp_n && (rc = launch_mp_runs(m, tab, n_img, st))) return rc;
+  float *blkmax = cc.mfma ? reinterpret_cast<float *>(ws + L.blkmax) : nullptr;
+  const int *tab = reinterpret_cast<const int *>(ws + L.mp_tab);
   timing_mark(0, st);
   const double *recd = reinterpret_cast<const double *>(ws + L.recd);
   const float *recf = reinterpret_cast<const float *>(ws + L.recf);
@@ -3612,7 +3651,7 @@ int run_image(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, i
   c.ny = g.ny;
   c.kx = kx;
   c.ky = ky;
-  c.kyp = kyp;
+  c.kyp = cc.job.kyp;
   c.edge = edge;
   double *partial = nullptr;
   if (data) {
@@ -3628,23 +3667,11 @@ int run_image(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, i
     partial = reinterpret_cast<double *>(ws + L.partial);
   }
   int n_tiles;
-  if (mfma) {
-    const MfmaPlan pl = mfma_plan(g.nx, g.ny, n_img, kx, ky);
-    n_tiles = n16_tiles(g.nx, g.ny);  // chi^2 partials of the 16 x 16 output tiles
-    rc = launch_conv_mfma(c, pl, n_img, reinterpret_cast<const float *>(lowres), hdr, frag, blkmax,
-                          (npix + 255) / 256, reinterpret_cast<float *>(out), partial, st);
-  } else if (mf64) {
-    const MfmaPlan pl = mfma_plan(g.nx, g.ny, n_img, kx, ky, true);
-    n_tiles = n16_tiles(g.nx, g.ny);
-    rc = launch_conv_mf64(c, pl, n_img, reinterpret_cast<const double *>(lowres), frag64,
-                          reinterpret_cast<double *>(out), partial, st);
-  } else {
-    rc = launch_conv_kernel<T>(c, n_img, lowres, kf, out, partial, &n_tiles, st);
-  }
+  rc = launch_conv<T>(c, cc, n_img, lowres, blkmax, out, partial, &n_tiles, st);
   if (rc) return rc;
   timing_mark(2, st);
   if (data) {
-    logl_kernel<<<n_img, 64, 0, st>>>(partial, n_tiles, logl);
+    logl_kernel<<<n_img, 64, 0, st>>>(partial, n_tiles, nullptr, logl);
     rc = check_launch("logl_kernel");
     if (rc) return rc;
   }
@@ -3859,7 +3886,7 @@ int run_image_ss(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf
   combine_kernel<T><<<dim3(nblk, n_img), 256, 0, st>>>(cc, chr, lowc, s, out, partial);
   if ((rc = check_launch("combine_kernel"))) return rc;
   if (data) {
-    logl_kernel<<<n_img, 64, 0, st>>>(partial, nblk, logl);
+    logl_kernel<<<n_img, 64, 0, st>>>(partial, nblk, nullptr, logl);
     return check_launch("logl_kernel");
   }
   return LENSIM_OK;
@@ -4013,29 +4040,23 @@ int run_grad(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int k
 // (de_lens.get_param_WLS, ImSim/de_lens.py:10-36) and the likelihood of the
 // solved model (:229-340).
 constexpr int kMaxLin = 8;  // linear amplitudes per model
-constexpr int kLinAcc = kMaxLin * (kMaxLin + 1) / 2 + kMaxLin;  // M (upper triangle) and R
-
-// params with the amplitude (slot 0) of every light profile set to 1
-__global__ void amp_one_kernel(const double *__restrict__ params, int n_img, int n_prof, int k_light0,
-                               double *__restrict__ out) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n_img * n_prof * LENSIM_NPARAM) return;
-  const int q = idx % LENSIM_NPARAM, k = (idx / LENSIM_NPARAM) % n_prof;
-  AT(out, idx) = (k >= k_light0 && q == 0) ? 1.0 : AT(params, idx);
-}
+constexpr int lin_acc(int n) { return n * (n + 1) / 2 + n; }  // M (upper triangle) and R
 
 // Weights mask / C_D(data) (ImageModel.error_response, image_model.py:577-596:
 // Data.C_D, the variance estimated from the data) and per-block partial sums
-// of M = A W A^T (upper triangle) and R = A W d.  A is [n_lin][n_img][npix].
-template <typename T>
-__global__ __launch_bounds__(256) void normal_kernel(ConvArgs c, const T *__restrict__ A, int n_lin, int n_img,
+// of M = A W A^T (upper triangle) and R = A W d.  A is [N][n_img][npix].  N is
+// fixed at compile time: the sums of eight amplitudes (44) cost two of them
+// 22 us where their own five take 4.6 us (99^2, 16 images).
+template <typename T, int N>
+__global__ __launch_bounds__(256) void normal_kernel(ConvArgs c, const T *__restrict__ A, int n_img,
                                                      double *__restrict__ part) {
+  constexpr int NA = lin_acc(N);
   const int img = blockIdx.y;
   const int npix = c.nx * c.ny;
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc[kLinAcc];
+  double acc[NA];
 #pragma unroll
-  for (int q = 0; q < kLinAcc; ++q) acc[q] = 0.0;
+  for (int q = 0; q < NA; ++q) acc[q] = 0.0;
   if (p < npix) {
     const size_t pd = p + size_t(img) * size_t(c.dstride);
     const double d = AT(c.data, pd);
@@ -4047,166 +4068,223 @@ __global__ __launch_bounds__(256) void normal_kernel(ConvArgs c, const T *__rest
       var = (d >= 0.0 ? d : 0.0) / t + c.bkg2;
     }
     const double w = (c.mask ? AT(c.mask, p) : 1.0) / var;
-    double a[kMaxLin];
+    double a[N];
 #pragma unroll
-    for (int l = 0; l < kMaxLin; ++l) a[l] = l < n_lin ? double(AT(A, (size_t(l) * n_img + img) * npix + p)) : 0.0;
+    for (int l = 0; l < N; ++l) a[l] = double(AT(A, (size_t(l) * n_img + img) * npix + p));
     if (w != 0.0) {
       int q = 0;
 #pragma unroll
-      for (int i = 0; i < kMaxLin; ++i) {
+      for (int i = 0; i < N; ++i) {
 #pragma unroll
-        for (int j = i; j < kMaxLin; ++j) acc[q++] = a[i] * w * a[j];
+        for (int j = i; j < N; ++j) acc[q++] = a[i] * w * a[j];
       }
 #pragma unroll
-      for (int i = 0; i < kMaxLin; ++i) acc[q++] = a[i] * w * d;
+      for (int i = 0; i < N; ++i) acc[q++] = a[i] * w * d;
     }
   }
-  __shared__ double red[4][kLinAcc];
+  __shared__ double red[4][NA];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
-  for (int q = 0; q < kLinAcc; ++q) {
-    double v = acc[q];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  for (int q = 0; q < NA; ++q) {
+    const double v = wave_sum(acc[q]);
     if (lane == 0) red[wave][q] = v;
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < kLinAcc; q += blockDim.x)
-    AT(part, (size_t(img) * gridDim.x + blockIdx.x) * kLinAcc + q) = red[0][q] + red[1][q] + red[2][q] + red[3][q];
+  if (threadIdx.x < NA) {
+    const int q = threadIdx.x;
+    AT(part, (size_t(img) * gridDim.x + blockIdx.x) * NA + q) = red[0][q] + red[1][q] + red[2][q] + red[3][q];
+  }
 }
 
-// Eigenvalues of a symmetric n x n matrix (cyclic Jacobi rotations).
-__device__ void sym_eigenvalues(double (*a)[kMaxLin], int n, double *ev) {
+// Eigenvalues of a symmetric N x N matrix (cyclic Jacobi rotations), in registers.
+template <int N>
+__device__ void sym_eigenvalues(double (&a)[N][N], double *ev) {
   for (int sweep = 0; sweep < 30; ++sweep) {
     double off = 0.0;
-    for (int i = 0; i < n; ++i)
-      for (int j = i + 1; j < n; ++j) off += a[i][j] * a[i][j];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int j = i + 1; j < N; ++j) off += a[i][j] * a[i][j];
     if (off == 0.0) break;
-    for (int p = 0; p < n; ++p)
-      for (int q = p + 1; q < n; ++q) {
+#pragma unroll
+    for (int p = 0; p < N; ++p)
+#pragma unroll
+      for (int q = p + 1; q < N; ++q) {
         if (a[p][q] == 0.0) continue;
         const double theta = (a[q][q] - a[p][p]) / (2.0 * a[p][q]);
         const double t = (theta >= 0.0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
         const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
-        for (int k = 0; k < n; ++k) {  // columns p, q
+#pragma unroll
+        for (int k = 0; k < N; ++k) {  // columns p, q
           const double akp = a[k][p], akq = a[k][q];
           a[k][p] = c * akp - s * akq;
           a[k][q] = s * akp + c * akq;
         }
-        for (int k = 0; k < n; ++k) {  // rows p, q
+#pragma unroll
+        for (int k = 0; k < N; ++k) {  // rows p, q
           const double apk = a[p][k], aqk = a[q][k];
           a[p][k] = c * apk - s * aqk;
           a[q][k] = s * apk + c * aqk;
         }
       }
   }
-  for (int i = 0; i < n; ++i) ev[i] = a[i][i];
+#pragma unroll
+  for (int i = 0; i < N; ++i) ev[i] = a[i][i];
 }
 
 // LU factorisation with partial pivoting in place; returns the permutation
-// parity (+1 / -1), 0 if a pivot is exactly zero.
-__device__ int lu_factor(double (*a)[kMaxLin], int n, int *piv) {
+// parity (+1 / -1), 0 if a pivot is exactly zero.  The row exchanges are
+// selections over the (compile-time) rows, so that the matrix stays in registers.
+template <int N>
+__device__ int lu_factor(double (&a)[N][N], int (&piv)[N]) {
   int parity = 1;
-  for (int k = 0; k < n; ++k) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
     int pr = k;
-    for (int i = k + 1; i < n; ++i)
-      if (fabs(a[i][k]) > fabs(a[pr][k])) pr = i;
-    piv[k] = pr;
-    if (pr != k) {
-      parity = -parity;
-      for (int j = 0; j < n; ++j) {
-        const double t = a[k][j];
-        a[k][j] = a[pr][j];
-        a[pr][j] = t;
+    double best = fabs(a[k][k]);
+#pragma unroll
+    for (int i = k + 1; i < N; ++i)
+      if (fabs(a[i][k]) > best) {
+        best = fabs(a[i][k]);
+        pr = i;
       }
-    }
+    piv[k] = pr;
+    if (pr != k) parity = -parity;
+#pragma unroll
+    for (int i = k + 1; i < N; ++i)
+      if (pr == i) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const double t = a[k][j];
+          a[k][j] = a[i][j];
+          a[i][j] = t;
+        }
+      }
     if (a[k][k] == 0.0) return 0;
-    for (int i = k + 1; i < n; ++i) {
+#pragma unroll
+    for (int i = k + 1; i < N; ++i) {
       a[i][k] /= a[k][k];
-      for (int j = k + 1; j < n; ++j) a[i][j] -= a[i][k] * a[k][j];
+#pragma unroll
+      for (int j = k + 1; j < N; ++j) a[i][j] -= a[i][k] * a[k][j];
     }
   }
   return parity;
 }
 
-__device__ void lu_solve(const double (*lu)[kMaxLin], const int *piv, int n, double *b) {
-  for (int k = 0; k < n; ++k) {
-    const double t = b[k];
-    b[k] = b[piv[k]];
-    b[piv[k]] = t;
+template <int N>
+__device__ void lu_solve(const double (&lu)[N][N], const int (&piv)[N], double (&b)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+#pragma unroll
+    for (int i = k + 1; i < N; ++i)
+      if (piv[k] == i) {
+        const double t = b[k];
+        b[k] = b[i];
+        b[i] = t;
+      }
   }
-  for (int i = 1; i < n; ++i)
+#pragma unroll
+  for (int i = 1; i < N; ++i)
+#pragma unroll
     for (int j = 0; j < i; ++j) b[i] -= lu[i][j] * b[j];
-  for (int i = n - 1; i >= 0; --i) {
-    for (int j = i + 1; j < n; ++j) b[i] -= lu[i][j] * b[j];
+#pragma unroll
+  for (int i = N - 1; i >= 0; --i) {
+#pragma unroll
+    for (int j = i + 1; j < N; ++j) b[i] -= lu[i][j] * b[j];
     b[i] /= lu[i][i];
   }
 }
 
-// One thread per image: sums the partials, checks cond(M) < 5 / eps, solves
+// One wave per image: its lanes sum the partials (lane l blocks l, l + 64, ...,
+// then the fixed wave sum), then every lane checks cond(M) < 5 / eps, solves
 // M B = R (B = 0 when unstable or not finite), optionally inverts M
 // (nan_to_num'ed, zero when unstable) and the marginalisation constant
-// (de_lens.marginalisation_const / marginalization_new, de_lens.py:40-77).
-__global__ void lin_solve_kernel(const double *__restrict__ part, int nblk, int n_lin, int n_img, int source_marg,
-                                 double d_prior, double *__restrict__ amp, double *__restrict__ cov,
-                                 double *__restrict__ marg) {
-  const int img = blockIdx.x * blockDim.x + threadIdx.x;
-  if (img >= n_img) return;
-  double acc[kLinAcc];
-  for (int q = 0; q < kLinAcc; ++q) acc[q] = 0.0;
-  for (int b = 0; b < nblk; ++b)
-    for (int q = 0; q < kLinAcc; ++q) acc[q] += AT(part, (size_t(img) * nblk + b) * kLinAcc + q);
-  double M[kMaxLin][kMaxLin], W[kMaxLin][kMaxLin], R[kMaxLin];
-  int q = 0;
-  for (int i = 0; i < kMaxLin; ++i)
-    for (int j = i; j < kMaxLin; ++j) {
-      M[i][j] = M[j][i] = acc[q];
-      ++q;
-    }
-  for (int i = 0; i < kMaxLin; ++i) R[i] = acc[q++];
-  const int n = n_lin;
-  for (int i = 0; i < n; ++i)
-    for (int j = 0; j < n; ++j) W[i][j] = M[i][j];
-  double ev[kMaxLin];
-  sym_eigenvalues(W, n, ev);
+// (de_lens.marginalisation_const / marginalization_new, de_lens.py:40-77) in
+// registers, and the first stores.  One thread per image with its matrices in
+// scratch memory and 44 serial sums took 171 us for 16 images, this 11.
+template <int N>
+__global__ __launch_bounds__(64) void lin_solve_kernel(const double *__restrict__ part, int nblk, int source_marg,
+                                                       double d_prior, double *__restrict__ amp,
+                                                       double *__restrict__ amp_out, double *__restrict__ cov,
+                                                       double *__restrict__ marg) {
+  constexpr int NA = lin_acc(N);
+  const int img = blockIdx.x, lane = threadIdx.x;
+  double acc[NA];
+#pragma unroll
+  for (int q = 0; q < NA; ++q) acc[q] = 0.0;
+  for (int b = lane; b < nblk; b += 64)
+#pragma unroll
+    for (int q = 0; q < NA; ++q) acc[q] += AT(part, (size_t(img) * nblk + b) * NA + q);
+#pragma unroll
+  for (int q = 0; q < NA; ++q) acc[q] = wave_sum(acc[q]);
+  double M[N][N], W[N][N], B[N];
+  {
+    int q = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int j = i; j < N; ++j) M[i][j] = M[j][i] = acc[q++];
+#pragma unroll
+    for (int i = 0; i < N; ++i) B[i] = acc[q++];
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < N; ++j) W[i][j] = M[i][j];
+  double ev[N];
+  sym_eigenvalues<N>(W, ev);
   double emax = 0.0, emin = INFINITY;
-  for (int i = 0; i < n; ++i) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
     emax = fmax(emax, fabs(ev[i]));
     emin = fmin(emin, fabs(ev[i]));
   }
   const double eps = 2.220446049250313e-16;
   const bool stable = emin > 0.0 && emax / emin < 5.0 / eps;
-  int piv[kMaxLin];
-  for (int i = 0; i < n; ++i)
-    for (int j = 0; j < n; ++j) W[i][j] = M[i][j];
-  const int parity = lu_factor(W, n, piv);
-  double B[kMaxLin];
-  for (int i = 0; i < n; ++i) B[i] = R[i];
-  bool finite = stable && parity != 0;
-  if (finite) {
-    lu_solve(W, piv, n, B);
-    for (int i = 0; i < n; ++i) finite = finite && isfinite(B[i]);
+  int piv[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    piv[i] = i;
+#pragma unroll
+    for (int j = 0; j < N; ++j) W[i][j] = M[i][j];
   }
-  for (int i = 0; i < n; ++i) AT(amp, size_t(img) * n + i) = finite ? B[i] : 0.0;
+  const int parity = lu_factor<N>(W, piv);
+  const bool ok = stable && parity != 0;
+  bool finite = ok;
+  if (finite) {
+    lu_solve<N>(W, piv, B);
+#pragma unroll
+    for (int i = 0; i < N; ++i) finite = finite && isfinite(B[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (lane == 0) {
+      const double v = finite ? B[i] : 0.0;
+      AT(amp, size_t(img) * N + i) = v;
+      if (amp_out) AT(amp_out, size_t(img) * N + i) = v;
+    }
   if (cov) {
-    for (int j = 0; j < n; ++j) {
-      double e[kMaxLin];
-      for (int i = 0; i < n; ++i) e[i] = i == j ? 1.0 : 0.0;
-      if (stable && parity != 0) lu_solve(W, piv, n, e);
-      for (int i = 0; i < n; ++i) {
-        const double v = (stable && parity != 0 && isfinite(e[i])) ? e[i] : 0.0;
-        AT(cov, (size_t(img) * n + i) * n + j) = v;
-      }
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      double e[N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) e[i] = i == j ? 1.0 : 0.0;
+      if (ok) lu_solve<N>(W, piv, e);
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (lane == 0) AT(cov, (size_t(img) * N + i) * N + j) = (ok && isfinite(e[i])) ? e[i] : 0.0;
     }
   }
   double mc = 0.0;
   if (source_marg) {
-    if (!(stable && parity != 0)) {
+    if (!ok) {
       mc = -1e15;  // slogdet / eig of a zero covariance
     } else if (!(d_prior > 0.0)) {
       // 1/2 log det(M^-1) = -1/2 sum log|U_ii| with the sign of det(M)
       double logdet = 0.0;
       int sign = parity;
-      for (int i = 0; i < n; ++i) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
         logdet += log(fabs(W[i][i]));
         if (W[i][i] < 0.0) sign = -sign;
       }
@@ -4214,16 +4292,33 @@ __global__ void lin_solve_kernel(const double *__restrict__ part, int nblk, int 
     } else {
       // eigenvalues of M^-1 = 1 / eigenvalues of M, clipped at d_prior^2
       double ld = 0.0, sgn = 1.0;
-      for (int i = 0; i < n; ++i) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
         const double v = 1.0 / ev[i];
         sgn *= v > 0.0 ? 1.0 : (v < 0.0 ? -1.0 : 0.0);
         ld += log(fmin(fabs(v), d_prior * d_prior));
       }
       const double log_det = ld * sgn;
-      mc = isnan(log_det) ? -1e15 : log_det / 2.0 + n / 2.0 * log(M_PI / 2.0) - n * log(d_prior);
+      mc = isnan(log_det) ? -1e15 : log_det / 2.0 + N / 2.0 * log(M_PI / 2.0) - N * log(d_prior);
     }
   }
-  AT(marg, img) = mc;
+  if (lane == 0) AT(marg, img) = mc;
+}
+
+// normal_kernel and lin_solve_kernel for n_lin amplitudes (1 .. kMaxLin).
+template <typename T, int N = kMaxLin>
+int launch_normal_solve(const ConvArgs &c, const T *A, int n_lin, int n_img, int nblk, double *part, int source_marg,
+                        double d_prior, double *amp, double *amp_out, double *cov, double *marg, hipStream_t st) {
+  if constexpr (N > 1) {
+    if (n_lin < N)
+      return launch_normal_solve<T, N - 1>(c, A, n_lin, n_img, nblk, part, source_marg, d_prior, amp, amp_out, cov, marg,
+                                           st);
+  }
+  normal_kernel<T, N><<<dim3(nblk, n_img), 256, 0, st>>>(c, A, n_img, part);
+  int rc = check_launch("normal_kernel");
+  if (rc) return rc;
+  lin_solve_kernel<N><<<n_img, 64, 0, st>>>(part, nblk, source_marg, d_prior, amp, amp_out, cov, marg);
+  return check_launch("lin_solve_kernel");
 }
 
 // Solved model (zero outside the likelihood mask, array_masked2image) and its chi^2.
@@ -4251,16 +4346,12 @@ __global__ __launch_bounds__(256) void lin_model_kernel(ConvArgs c, const T *__r
   if (threadIdx.x == 0) AT(partial, size_t(img) * gridDim.x + blockIdx.x) = red[0] + red[1] + red[2] + red[3];
 }
 
-__global__ void add_kernel(double *__restrict__ x, const double *__restrict__ y, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) AT(x, i) += AT(y, i);
-}
-
-// Workspace of the linear solve: the image layout of one column, then the
-// columns A, the amp = 1 parameters, partials, amplitudes and constants.
+// Workspace of the linear solve: the image layout of one column, the columns A
+// with their pooled images and block maxima (all columns are convolved in one
+// launch), partials, amplitudes and constants.
 struct LinLayout {
   Layout img;
-  size_t A, params1, part, chi, amp, marg, total;
+  size_t A, low, blkmax, part, chi, amp, marg, total;
 };
 
 LinLayout lin_layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img, int precision, const SSPlan &ss,
@@ -4272,10 +4363,14 @@ LinLayout lin_layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_i
   size_t off = L.img.total;
   L.A = off;
   off = align256(off + size_t(n_lin) * n_img * npix * tsz);
-  L.params1 = off;
-  off = align256(off + size_t(n_img) * m.n_prof * LENSIM_NPARAM * 8);
+  L.low = L.blkmax = off;
+  if (!ss.on) {
+    off = align256(off + size_t(n_lin) * n_img * npix * tsz);
+    L.blkmax = off;
+    off = align256(off + size_t(n_lin) * n_img * nblk * 4);
+  }
   L.part = off;
-  off = align256(off + size_t(n_img) * nblk * kLinAcc * 8);
+  off = align256(off + size_t(n_img) * nblk * lin_acc(n_lin) * 8);
   L.chi = off;
   off = align256(off + size_t(n_img) * nblk * 8);
   L.amp = off;
@@ -4286,30 +4381,75 @@ LinLayout lin_layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_i
   return L;
 }
 
+// The response columns of run_linear without supersampled convolution: the
+// records (at amp = 1) and the PSF prepared once, a render per light profile
+// (every other one left out), one convolution over all columns' images.
 template <typename T>
-int run_linear(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int kx, int ky, int edge,
+int run_responses(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, int kx, int ky, int edge,
+                  const double *params, int n_img, int n_lin, T *A, unsigned char *ws, const LinLayout &LL,
+                  hipStream_t st) {
+  const Layout &L = LL.img;
+  ModelArgs m = with_grid(m_in, g);
+  const ConvChoice<T> cc(psf, 0, kx, ky, ws, L);
+  int rc = launch_prep_psf(m, params, n_img, cc.job, false, ws, L, st);
+  if (rc) return rc;
+  const size_t npix = size_t(g.nx) * g.ny, nblk = (npix + 255) / 256;
+  T *low = reinterpret_cast<T *>(ws + LL.low);
+  float *blkmax = cc.mfma ? reinterpret_cast<float *>(ws + LL.blkmax) : nullptr;
+  for (int l = 0; l < n_lin; ++l) {
+    ModelArgs mc = m;
+    for (int k = 0; k < n_lin; ++k)
+      if (k != l) mc.types[m.n_lens + k] = LENSIM_NULL;
+    rc = launch_render<T>(mc, g, reinterpret_cast<const double *>(ws + L.recd),
+                          reinterpret_cast<const float *>(ws + L.recf),
+                          reinterpret_cast<const double *>(ws + L.coefd),
+                          reinterpret_cast<const float *>(ws + L.coeff), reinterpret_cast<const int *>(ws + L.mp_tab),
+                          l < m.n_source ? LENSIM_IMAGE_SOURCE : LENSIM_IMAGE_LENS_LIGHT, MpKeep{},
+                          low + size_t(l) * n_img * npix, blkmax ? blkmax + size_t(l) * n_img * nblk : nullptr, n_img,
+                          st);
+    if (rc) return rc;
+  }
+  ConvArgs c{};
+  c.nx = g.nx;
+  c.ny = g.ny;
+  c.kx = kx;
+  c.ky = ky;
+  c.kyp = cc.job.kyp;
+  c.edge = edge;
+  const int all = n_img * n_lin, most = 65535;  // images a launch's grid holds
+  for (int i = 0; i < all; i += most) {
+    int n_tiles;
+    rc = launch_conv<T>(c, cc, all - i < most ? all - i : most, low + i * npix, blkmax ? blkmax + i * nblk : nullptr,
+                        A + i * npix, nullptr, &n_tiles, st);
+    if (rc) return rc;
+  }
+  return LENSIM_OK;
+}
+
+template <typename T>
+int run_linear(const ModelArgs &m_in, const GridArgs &g, const lensim_psf *psf, int kx, int ky, int edge,
                const SSPlan &ss, const lensim_data *data, const double *params, int n_img, int source_marg,
                double d_prior, double *amp_out, double *logl, T *model_out, double *cov, T *resp_out,
                unsigned char *ws, const LinLayout &LL, hipStream_t st) {
+  ModelArgs m = m_in;
+  m.unit_amp = 1;
   const int n_lin = m.n_source + m.n_light;
   const int npix = g.nx * g.ny, nblk = (npix + 255) / 256;
-  double *params1 = reinterpret_cast<double *>(ws + LL.params1);
-  const int ntot = n_img * m.n_prof * LENSIM_NPARAM;
-  amp_one_kernel<<<(ntot + 255) / 256, 256, 0, st>>>(params, n_img, m.n_prof, m.n_defl, params1);
-  int rc = check_launch("amp_one_kernel");
-  if (rc) return rc;
   T *A = resp_out ? resp_out : reinterpret_cast<T *>(ws + LL.A);
-  // one column per linear profile: the model with every other light profile off
-  for (int l = 0; l < n_lin; ++l) {
-    ModelArgs mc = m;
-    for (int k = m.n_lens; k < m.n_lens + n_lin; ++k)
-      if (k - m.n_lens != l) mc.types[k] = LENSIM_NULL;
-    const unsigned flags = l < m.n_source ? LENSIM_IMAGE_SOURCE : LENSIM_IMAGE_LENS_LIGHT;
-    T *col = A + size_t(l) * n_img * npix;
-    rc = ss.on ? run_image_ss<T>(mc, g, psf, kx, ky, edge, ss, nullptr, params1, n_img, flags, col, nullptr, ws,
-                                 LL.img, st)
-               : run_image<T>(mc, g, psf, kx, ky, edge, nullptr, params1, n_img, flags, col, nullptr, ws, LL.img, st);
-    if (rc) return rc;
+  int rc = LENSIM_OK;
+  if (!ss.on) {
+    if ((rc = run_responses<T>(m, g, psf, kx, ky, edge, params, n_img, n_lin, A, ws, LL, st))) return rc;
+  } else {
+    // one column per linear profile: the model with every other light profile off
+    for (int l = 0; l < n_lin; ++l) {
+      ModelArgs mc = m;
+      for (int k = m.n_lens; k < m.n_lens + n_lin; ++k)
+        if (k - m.n_lens != l) mc.types[k] = LENSIM_NULL;
+      const unsigned flags = l < m.n_source ? LENSIM_IMAGE_SOURCE : LENSIM_IMAGE_LENS_LIGHT;
+      rc = run_image_ss<T>(mc, g, psf, kx, ky, edge, ss, nullptr, params, n_img, flags, A + size_t(l) * n_img * npix,
+                           nullptr, ws, LL.img, st);
+      if (rc) return rc;
+    }
   }
   ConvArgs c{};
   c.nx = g.nx;
@@ -4322,25 +4462,16 @@ int run_linear(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int
   c.bkg2 = data->background_rms * data->background_rms;
   c.inv_t = 1.0 / data->exposure_time;
   c.dstride = data->image_stride;
-  double *part = reinterpret_cast<double *>(ws + LL.part);
-  normal_kernel<T><<<dim3(nblk, n_img), 256, 0, st>>>(c, A, n_lin, n_img, part);
-  if ((rc = check_launch("normal_kernel"))) return rc;
   double *amp = reinterpret_cast<double *>(ws + LL.amp);
   double *marg = reinterpret_cast<double *>(ws + LL.marg);
-  lin_solve_kernel<<<(n_img + 63) / 64, 64, 0, st>>>(part, nblk, n_lin, n_img, source_marg, d_prior, amp, cov, marg);
-  if ((rc = check_launch("lin_solve_kernel"))) return rc;
+  rc = launch_normal_solve<T>(c, A, n_lin, n_img, nblk, reinterpret_cast<double *>(ws + LL.part), source_marg, d_prior,
+                              amp, amp_out, cov, marg, st);
+  if (rc) return rc;
   double *chi = reinterpret_cast<double *>(ws + LL.chi);
   lin_model_kernel<T><<<dim3(nblk, n_img), 256, 0, st>>>(c, A, amp, n_lin, n_img, model_out, chi);
   if ((rc = check_launch("lin_model_kernel"))) return rc;
-  logl_kernel<<<n_img, 64, 0, st>>>(chi, nblk, logl);
-  if ((rc = check_launch("logl_kernel"))) return rc;
-  add_kernel<<<(n_img + 255) / 256, 256, 0, st>>>(logl, marg, n_img);
-  if ((rc = check_launch("add_kernel"))) return rc;
-  if (amp_out) {
-    const hipError_t e = hipMemcpyAsync(amp_out, amp, size_t(n_img) * n_lin * 8, hipMemcpyDeviceToDevice, st);
-    if (e != hipSuccess) return hip_fail(e, "hipMemcpyAsync(amp)");
-  }
-  return LENSIM_OK;
+  logl_kernel<<<n_img, 64, 0, st>>>(chi, nblk, marg, logl);
+  return check_launch("logl_kernel");
 }
 
 // ------------------------------------------- allocation-free entry point --
@@ -4753,7 +4884,7 @@ int lensim_data_loglike(const lensim_data *data, int32_t nx, int32_t ny, const v
   else
     data_chi2_kernel<float><<<dim3(nblk, n_img), 256, 0, st>>>(c, static_cast<const float *>(d_model), partial);
   if ((rc = check_launch("data_chi2_kernel"))) return cr.end(st, rc);
-  logl_kernel<<<n_img, 64, 0, st>>>(partial, nblk, d_logl);
+  logl_kernel<<<n_img, 64, 0, st>>>(partial, nblk, nullptr, d_logl);
   return cr.end(st, check_launch("logl_kernel"));
 }
 
