@@ -198,53 +198,6 @@ __device__ void nie_g(const S &theta_E, const S &e1, const S &e2, const S &s_sca
   nie_g_geo<T>(theta_E, q, cos(phi), sin(phi), s_scale, cx, cy, x, y, ax, ay);
 }
 
-// F(X) of the NFW family: arctanh(sqrt(1 - X^2)) / sqrt(1 - X^2) = arccosh(1/X)
-// / sqrt(1 - X^2) below X = 1, arctan(sqrt(X^2 - 1)) / sqrt(X^2 - 1) = arccos(1/X)
-// / sqrt(X^2 - 1) above, 1 at X = 1 (nfw.py:345-365, tnfw.py:288-304).  Both
-// sides are the one series sum_n (-u)^n / (2n + 1) in u = X^2 - 1, used for
-// |u| < u0: there the closed forms' derivatives are differences of two terms
-// that agree to O(u), so their duals lose (epsilon / |u|) relative precision
-// (all of it in float within a few 1e-7 of X = 1); the series carries the
-// derivative with no cancellation.  u0 = 0.1 (float) leaves a truncation of
-// 0.1^9 / 19 after nine terms, u0 = 0.01 (double) 0.01^9 / 19.
-template <typename T, typename S>
-__device__ __forceinline__ S nfw_F_g(const S &X) {
-  const S u = X * X - T(1);
-  const T u0 = sizeof(T) == sizeof(float) ? T(0.1) : T(0.01);
-  if (val(u) < u0 && val(u) > -u0) {
-    S f = lift(T(1) / T(17), u);
-#pragma unroll
-    for (int n = 7; n >= 0; --n) f = T(1) / T(2 * n + 1) - u * f;
-    return f;
-  }
-  if (val(u) < T(0)) {
-    const S r = sqrt(-u);
-    return atanh(r) / r;
-  }
-  const S r = sqrt(u);
-  return atan(r) / r;
-}
-
-// NFW.g, nfw.py:345-365: log(X/2) + F(X)
-template <typename T, typename S>
-__device__ __forceinline__ S nfw_g_g(S X) {
-  X = fmax(X, T(0.000001));
-  return log(X * T(0.5)) + nfw_F_g<T>(X);
-}
-
-// NFW, nfw.py:86-105, :257-279, :384-395.  p: Rs, alpha_Rs, center_x, center_y.
-template <typename T, typename S>
-__device__ void nfw_g(const S *p, const S &x, const S &y, S &ax, S &ay) {
-  const S rho0 = p[1] / (T(4) * p[0] * p[0] * (T(1) + T(::log(0.5))));
-  const S Rs = fmax(p[0], T(0.0000001));
-  const S dx = x - p[2], dy = y - p[3];
-  const S R = fmax(sqrt(dx * dx + dy * dy), T(0.00000001));
-  const S X = R / Rs;
-  const S a = T(4) * rho0 * Rs * nfw_g_g<T>(X) / (X * X);
-  ax = ax + a * dx;
-  ay = ay + a * dy;
-}
-
 // One deflector from its raw slot.
 template <typename T, typename S>
 __device__ __forceinline__ void defl_g(int type, const S *p, const T *c, const T *dc, int nser, const S &x,
@@ -258,9 +211,6 @@ __device__ __forceinline__ void defl_g(int type, const S *p, const T *c, const T
       break;
     case LENSIM_NIE:
       nie_g<T>(p[0], p[1], p[2], p[3], p[4], p[5], x, y, ax, ay);
-      break;
-    case LENSIM_NFW:
-      nfw_g<T>(p, x, y, ax, ay);
       break;
     case LENSIM_SHEAR: {
       const S dx = x - p[2], dy = y - p[3];
@@ -340,6 +290,262 @@ __device__ __forceinline__ T sersic_ellipse_grad(const double *p, T x, T y, T *g
   gp[5] = -gx;
   gp[6] = -gy;
   return amp * E;
+}
+
+// ---- FP64 closed forms ----
+// The float gradient kernels differentiate with duals; in double those took
+// 3000 vector instructions a ray for the EPL (every dual division, root and
+// logarithm on library functions).  The FP64 kernels use the derivatives
+// written out below, on the records' constants, the library's own log2, exp2,
+// atan and atanh and third-order reciprocals.
+
+// The EPL's alpha at (x, y) and its derivatives by (theta_E, gamma, e1, e2,
+// center_x, center_y).  With Z = q x + i y (major-axis frame), R = |Z|, z = -f
+// Z / conj(Z), F = 2F1(1, t/2; 2 - t/2; z) and s = 2/(1+q) (b/R)^t, alpha = s Z F.
+//  * F = 1 + delta, delta = (w P(w) + z/2) / (1 - z/2), w = z/(z - 2), P = sum_n>=1
+//    F_n w^(n-1) (the Lopez-Temme series of epl_major_f64).  With its first
+//    parameter 1, F obeys the first-order equation
+//      z F' = [b z + (b z + 1 - c) delta] / (1 - z),  b = t/2, c = 2 - t/2,
+//    so no second series is needed for dF/dz;
+//  * d/dt: ln(b/R) alpha + s Z dF/dt, dF/dt = (sum dF_n/dt w^n) / (1 - z/2);
+//  * d/dq at fixed frame: dZ = x dq, dz/z = df/f - 2 i x y dq / R^2, ds/s =
+//    (-1/(1+q) + t (1/(2q) - q x^2/R^2)) dq;
+//  * theta_E, the centre and the orientation as in epl_dalpha's comment, the
+//    Hessian with 1/r^2 alone.
+__device__ __forceinline__ void epl_dalpha_f64(const double *rd, const double *__restrict__ c,
+                                               const double *__restrict__ dc, const double *pk, double x, double y,
+                                               double &a_x, double &a_y, double *dax, double *day) {
+  const double q = rd[EPL_Q], t = rd[EPL_T], f = rd[EPL_F], cs = rd[EPL_C], sn = rd[EPL_S];
+  const double dx = x - rd[R_CX], dy = y - rd[R_CY];
+  const double xr = dx * cs + dy * sn, yr = dy * cs - dx * sn;
+  const double Zr = q * xr, Zi = yr;
+  const double R2 = Zr * Zr + Zi * Zi;
+  a_x = a_y = 0.0;
+#pragma unroll
+  for (int i = 0; i < 6; ++i) dax[i] = day[i] = 0.0;
+  if (R2 == 0.0) return;  // the reference's NaN at Z = 0 becomes 0 (epl.py:391-392)
+  const bool rfree = R2 >= 1e-18;  // the floor R >= 1e-9 passes no derivative
+  const double R2c = rfree ? R2 : 1e-18;
+  const double iR2 = rcp_full(R2);
+  double Fr = 1.0, Fi = 0.0, tr = 0.0, ti = 0.0, gr = 0.0, gi = 0.0;  // F, dF/dt, z F' (dz/dq)/z
+  if (f != 0.0) {
+    const double zr = -f * (Zr * Zr - Zi * Zi) * iR2, zi = -2.0 * f * (Zr * Zi) * iR2;
+    const double er = fma(-0.5, zr, 1.0), ei = -0.5 * zi;
+    const double ed = rcp_full(fma(er, er, ei * ei));
+    const double vr = er * ed, vi = -ei * ed;  // 1 / (1 - z/2)
+    const double wr = -0.5 * (zr * vr - zi * vi), wi = -0.5 * (zr * vi + zi * vr);
+    const int n = (int)rd[EPL_NMAX];
+    double Pr, Pi, Ur, Ui;
+    real_poly_at_complex<double>(c + 1, n - 1, wr, wi, Pr, Pi);
+    real_poly_at_complex<double>(dc + 1, n - 1, wr, wi, Ur, Ui);
+    const double nr = fma(wr, Pr, fma(-wi, Pi, 0.5 * zr)), ni = fma(wr, Pi, fma(wi, Pr, 0.5 * zi));
+    const double er2 = nr * vr - ni * vi, ei2 = nr * vi + ni * vr;  // delta
+    Fr = 1.0 + er2;
+    Fi = ei2;
+    const double ur = wr * Ur - wi * Ui, ui = wr * Ui + wi * Ur;
+    tr = ur * vr - ui * vi;
+    ti = ur * vi + ui * vr;
+    // z F'
+    const double b = 0.5 * t, mr = fma(b, zr, b - 1.0), mi = b * zi;
+    const double kr = fma(b, zr, mr * er2 - mi * ei2), ki = fma(b, zi, mr * ei2 + mi * er2);
+    const double or_ = 1.0 - zr, od = rcp_full(fma(or_, or_, zi * zi));
+    const double hr = (kr * or_ - ki * zi) * od, hi = (kr * zi + ki * or_) * od;
+    // times (dz/dq) / z
+    const double qr = -2.0 / ((1.0 + q) * (1.0 + q) * f), qi = -2.0 * xr * yr * iR2;
+    gr = hr * qr - hi * qi;
+    gi = hr * qi + hi * qr;
+  }
+  const double lb2 = rd[EPL_LB2] - 0.5 * log2_pos(R2c);  // log2(b / R)
+  const double pw = exp2_fin(t * lb2), s = rd[EPL_PREF] * pw;
+  const double sZr = s * Zr, sZi = s * Zi;
+  const double fr = sZr * Fr - sZi * Fi, fi = sZr * Fi + sZi * Fr;
+  const double lnbr = pw > 0.0 ? 0.6931471805599453 * lb2 : 0.0;
+  const double atr = fma(lnbr, fr, sZr * tr - sZi * ti), ati = fma(lnbr, fi, sZr * ti + sZi * tr);
+  const double ls = -1.0 / (1.0 + q) + t * (0.5 / q - (rfree ? q * xr * xr * iR2 : 0.0));
+  const double sx = s * xr;
+  const double aqr = fma(ls, fr, fma(sx, Fr, sZr * gr - sZi * gi)), aqi = fma(ls, fi, fma(sx, Fi, sZr * gi + sZi * gr));
+  a_x = fr * cs - fi * sn;
+  a_y = fr * sn + fi * cs;
+  const double thetaE = pk[0], dth = thetaE != 0.0 ? t / thetaE : 0.0;
+  dax[0] = a_x * dth;
+  day[0] = a_y * dth;
+  dax[1] = atr * cs - ati * sn;
+  day[1] = atr * sn + ati * cs;
+  const double qx = aqr * cs - aqi * sn, qy = aqr * sn + aqi * cs;
+  // Hessian: kappa and the shear of EPLMajorAxis.hessian, rotated back
+  const double x2 = xr * xr, y2 = yr * yr, ir2 = rcp_full(x2 + y2);
+  const double kappa = 0.5 * (2.0 - t) * pw;
+  const double g1 = ((1.0 - t) * (fr * xr - fi * yr) - kappa * (x2 - y2)) * ir2;
+  const double g2 = ((1.0 - t) * (fi * xr + fr * yr) - kappa * (2.0 * xr * yr)) * ir2;
+  const double c2p = cs * cs - sn * sn, s2p = 2.0 * sn * cs;
+  const double G1 = c2p * g1 - s2p * g2, fxy = s2p * g1 + c2p * g2;
+  const double fxx = kappa + G1, fyy = kappa - G1;
+  const double dphx = fxx * dy - fxy * dx - a_y, dphy = fxy * dy - fyy * dx + a_x;
+  const double e1 = pk[2], e2 = pk[3], c2 = e1 * e1 + e2 * e2, ce = ::sqrt(c2);
+  const double h = 0.5 / c2, dp1 = -e2 * h, dp2 = e1 * h;
+  const double dqdc = ce < 0.9999 ? -2.0 / ((1.0 + ce) * (1.0 + ce)) : 0.0;
+  const double dq1 = dqdc * e1 / ce, dq2 = dqdc * e2 / ce;
+  dax[2] = qx * dq1 + dphx * dp1;
+  day[2] = qy * dq1 + dphy * dp1;
+  dax[3] = qx * dq2 + dphx * dp2;
+  day[3] = qy * dq2 + dphy * dp2;
+  dax[4] = -fxx;
+  day[4] = -fxy;
+  dax[5] = -fxy;
+  day[5] = -fyy;
+}
+
+// The SIE / NIE's alpha at (x, y) and its derivatives by (theta_E, e1, e2[,
+// s_scale], center_x, center_y).  In the major-axis frame alpha = k (A, B), k = b
+// / sq, sq = sqrt(1 - q^2), A = arctan(sq x / D1), B = arctanh(sq y / D2), D1 =
+// psi + s, D2 = psi + q^2 s, psi^2 = q^2 (s^2 + x^2) + y^2, with b = theta_E
+// sqrt(q) and s = s_scale / sqrt(q) (nie.py:182-200, :280-295).
+template <int TYPE>
+__device__ __forceinline__ void nie_dalpha_f64(const double *rd, const double *pk, double x, double y, double &a_x,
+                                               double &a_y, double *dax, double *day) {
+  constexpr bool kNie = TYPE == LENSIM_NIE;
+  constexpr int kc = kNie ? 4 : 3;  // the centre's slots
+  const double q = rd[NIE_Q], q2 = rd[NIE_Q2], s = rd[NIE_SS], sq = rd[NIE_SQ], k = rd[NIE_BSQ], cs = rd[NIE_C],
+               sn = rd[NIE_S];
+  const double e1 = pk[1], e2 = pk[2], c2 = e1 * e1 + e2 * e2, ce = ::sqrt(c2);
+  const double cc = ce < 0.9999 ? ce : 0.9999, q0 = (1.0 - cc) / (1.0 + cc);  // unclamped q: b, s
+  const bool qfree = q0 < 1.0;                                              // else the frame's q is a constant
+  const double dx = x - rd[R_CX], dy = y - rd[R_CY];
+  const double xr = dx * cs + dy * sn, yr = dy * cs - dx * sn;
+  const double p2 = fma(q2, fma(s, s, xr * xr), yr * yr);
+  const double ip = p2 > 0.0 ? rsq_full(p2) : 0.0, psi = p2 * ip;
+  const double D1 = psi + s, D2 = fma(q2, s, psi);
+  const double i1 = rcp_full(D1), i2 = rcp_full(D2);
+  const double u1 = sq * xr * i1, u2 = sq * yr * i2;
+  const double A = atan_dbl(u1), B = atanh_dbl(u2);
+  const double fx = k * A, fy = k * B;
+  a_x = fx * cs - fy * sn;
+  a_y = fx * sn + fy * cs;
+  // k dA = k1 d(x / D1 sq) and k dB = k2 d(y / D2 sq)
+  const double k1 = k * rcp_full(fma(u1, u1, 1.0)), k2 = k * rcp_full(fma(-u2, u2, 1.0));
+  const double px = q2 * xr * ip, py = yr * ip, ps = q2 * s * ip, pq = q * fma(s, s, xr * xr) * ip;
+  const double w1 = k1 * sq * i1, w2 = k2 * sq * i2;
+  const double axx = w1 * (1.0 - xr * px * i1), axy = -w1 * xr * py * i1;
+  const double ayx = -w2 * yr * px * i2, ayy = w2 * (1.0 - yr * py * i2);
+  const double axs = -w1 * xr * (ps + 1.0) * i1, ays = -w2 * yr * (ps + q2) * i2;
+  // q: through k, sq and psi (the frame's q), and through b and s = s_scale / sqrt(q)
+  const double isq2 = 1.0 / (sq * sq), iq0 = 0.5 / q0;
+  double qxr = iq0 * fma(-s, axs, fx), qyr = iq0 * fma(-s, ays, fy);
+  if (qfree) {
+    qxr += q * isq2 * (fx - w1 * xr) - w1 * xr * pq * i1;
+    qyr += q * isq2 * (fy - w2 * yr) - w2 * yr * fma(2.0 * q, s, pq) * i2;
+  }
+  const double ith = pk[0] != 0.0 ? 1.0 / pk[0] : 0.0;
+  dax[0] = a_x * ith;
+  day[0] = a_y * ith;
+  // H = R (d alpha / d(xr, yr)) R^T
+  const double mxx = axx * cs - ayx * sn, mxy = axy * cs - ayy * sn, myx = axx * sn + ayx * cs,
+               myy = axy * sn + ayy * cs;
+  const double hxx = mxx * cs - mxy * sn, hxy = mxx * sn + mxy * cs, hyx = myx * cs - myy * sn,
+               hyy = myx * sn + myy * cs;
+  const double dphx = hxx * dy - hxy * dx - a_y, dphy = hyx * dy - hyy * dx + a_x;
+  const double h = 0.5 / c2, dp1 = -e2 * h, dp2 = e1 * h;
+  const double dqdc = ce < 0.9999 ? -2.0 / ((1.0 + ce) * (1.0 + ce)) : 0.0;
+  const double dq1 = dqdc * e1 / ce, dq2 = dqdc * e2 / ce;
+  const double qx = qxr * cs - qyr * sn, qy = qxr * sn + qyr * cs;
+  dax[1] = qx * dq1 + dphx * dp1;
+  day[1] = qy * dq1 + dphy * dp1;
+  dax[2] = qx * dq2 + dphx * dp2;
+  day[2] = qy * dq2 + dphy * dp2;
+  if constexpr (kNie) {  // s = s_scale / sqrt(q)
+    const double isq = rsq_full(q0);
+    const double sx = axs * isq, sy = ays * isq;
+    dax[3] = sx * cs - sy * sn;
+    day[3] = sx * sn + sy * cs;
+  }
+  dax[kc] = -hxx;
+  day[kc] = -hyx;
+  dax[kc + 1] = -hxy;
+  day[kc + 1] = -hyy;
+}
+
+// The NFW's alpha = a (dx, dy) at (x, y), a = 4 rho0 Rs g / u, u = X^2, and its
+// derivatives by (Rs, alpha_Rs, center_x, center_y): X dg/dX = 1 + X F' = u (1 -
+// F) / (u - 1), so X da/dX = 4 rho0 Rs X dg/dX / u - 2 a, Rs da/dRs = -(a + X
+// da/dX), and the Jacobian a I + (X da/dX / R^2) d d^T.  Floors as nfw.py:86-105
+// (R >= 1e-8, X >= 1e-6 in g, Rs >= 1e-7), which pass no derivative.
+__device__ __forceinline__ void nfw_dalpha_f64(const double *rd, const double *pk, double x, double y, double &a_x,
+                                               double &a_y, double *dax, double *day) {
+  const double dx = x - rd[R_CX], dy = y - rd[R_CY], irs = rd[NFW_IRS];
+  const double R2 = fma(dx, dx, dy * dy);
+  const bool rfree = R2 >= 1e-16;
+  const double u = (rfree ? R2 : 1e-16) * irs * irs;
+  const bool xfree = u >= 1e-12;
+  const double uc = xfree ? u : 1e-12, rX = rsq_full(uc), iu = xfree ? rX * rX : 1.0 / u;
+  const double F = halo_F(uc, rX);
+  const double l = fma(0.34657359027997264, log2_pos(uc), -0.6931471805599453);  // ln(X / 2)
+  double g = l + F;
+  if (uc < 0.0025) {
+    // the sum cancels to u: with F = arccosh(1 / X) / sqrt(1 - u) by its series,
+    // g = -u (l P(u) + Q(u)) to 2e-16 here
+    constexpr double kP[6] = {0.5, 0.375, 0.3125, 0.2734375, 0.24609375, 0.2255859375};
+    constexpr double kQ[6] = {0.25, 0.21875, 0.19270833333333334, 0.17350260416666666, 0.15888671875,
+                              0.14735514322916668};
+    g = -uc * fma(l, poly(kP, uc), poly(kQ, uc));
+  }
+  const double e = uc - 1.0;
+  const double xg = fabs(e) < 0.03 ? 1.0 + halo_XdF(uc, F) : uc * (1.0 - F) * rcp_full(e);
+  const double A = rd[NFW_A], a = A * g * iu;
+  const double aX = rfree ? fma(A * iu, xfree ? xg : 0.0, -2.0 * a) : 0.0;
+  const double rs0 = pk[0];
+  const double aR = rs0 >= 0.0000001 ? -(a + aX) * irs : -2.0 * a / rs0;
+  const double aA = rd[NFW_RS] / (rs0 * rs0 * (1.0 + ::log(0.5))) * g * iu;
+  const double q = aX * rcp_full(rfree ? R2 : 1.0);
+  a_x = a * dx;
+  a_y = a * dy;
+  dax[0] = aR * dx;
+  day[0] = aR * dy;
+  dax[1] = aA * dx;
+  day[1] = aA * dy;
+  dax[2] = -fma(q * dx, dx, a);
+  day[2] = dax[3] = -(q * dx) * dy;
+  day[3] = -fma(q * dy, dy, a);
+}
+
+// sersic_ellipse_grad in double from the profile's record rd and kwargs p.
+__device__ __forceinline__ double sersic_ellipse_grad_f64(const double *rd, const double *p, double x, double y,
+                                                          double *gp, double &gx, double &gy) {
+  const double amp = rd[SE_AMP], p1 = p[1], e1 = p[3], e2 = p[4], invn = rd[SE_INVN];
+  const double dx = x - rd[R_CX], dy = y - rd[R_CY];
+  const double v = 1.0 - e1 * e1 - e2 * e2, sq = ::sqrt(fabs(v));
+  const bool nfree = sq >= 0.000001, sfree = p1 >= 0.0001, bfree = 1.9992 * p[2] - 0.3271 >= 0.00001;
+  const double inorm = 1.0 / (nfree ? sq : 0.000001);
+  const double sg = v >= 0.0 ? 1.0 : -1.0;
+  const double dn1 = nfree ? -sg * e1 * inorm : 0.0, dn2 = nfree ? -sg * e2 * inorm : 0.0;
+  const double xe = rd[SE_M00] * dx + rd[SE_M01] * dy, ye = rd[SE_M01] * dx + rd[SE_M11] * dy;
+  const double R2 = fma(xe, xe, ye * ye);
+  const bool rfree = R2 >= 1e-8;
+  const double R2c = rfree ? R2 : 1e-8;
+#pragma unroll
+  for (int i = 0; i < 7; ++i) gp[i] = 0.0;
+  gx = gy = 0.0;
+  if (!(R2c <= rd[SE_R2MAX])) return 0.0;
+  const double l2 = (0.5 * log2_pos(R2c) - rd[SE_LNRS] * 1.4426950408889634) * invn;  // log2(frac) / n
+  const double u = exp2_fin(l2);
+  const double E = exp2_fin(rd[SE_K2] * (1.0 - u)), aE = amp * E;
+  const double c = -aE * rd[SE_BN] * u * invn;  // d flux / d ln(frac)
+  gp[0] = E;
+  gp[1] = sfree ? -c * rd[SE_IRS] : 0.0;
+  gp[2] = -c * (0.6931471805599453 * l2) - (bfree ? aE * (u - 1.0) * 1.9992 : 0.0);
+  const double k = rfree ? c * rcp_full(R2c) : 0.0;
+  const double gxe = k * xe, gye = k * ye;
+  gp[3] = (gxe * (-dx - xe * dn1) + gye * (dy - ye * dn1)) * inorm;
+  gp[4] = (gxe * (-dy - xe * dn2) + gye * (-dx - ye * dn2)) * inorm;
+  gx = gxe * rd[SE_M00] + gye * rd[SE_M01];
+  gy = gye * rd[SE_M11] + gxe * rd[SE_M01];
+  gp[5] = -gx;
+  gp[6] = -gy;
+  return aE;
+}
+template <typename T>
+__device__ __forceinline__ T sersic_ellipse_grad_rec(const double *rd, const double *p, T x, T y, T *gp, T &gx, T &gy) {
+  if constexpr (sizeof(T) == sizeof(double)) return sersic_ellipse_grad_f64(rd, p, x, y, gp, gx, gy);
+  else return sersic_ellipse_grad<T>(p, x, y, gp, gx, gy);
 }
 
 // One light profile from its raw slot at (x, y).

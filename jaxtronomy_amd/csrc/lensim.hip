@@ -2320,14 +2320,14 @@ struct GradArgs {
 // A light profile's flux and its derivatives in its own kwargs (the N seeds
 // of ps) at (x, y): closed form for SERSIC_ELLIPSE, duals otherwise.
 template <typename T, int N>
-__device__ __forceinline__ gm::Dual<T, N> light_grad(int type, const gm::Dual<T, N> *ps, const double *pk, T x,
-                                                     T y) {
+__device__ __forceinline__ gm::Dual<T, N> light_grad(int type, const gm::Dual<T, N> *ps, const double *rd,
+                                                     const double *pk, T x, T y) {
   using S = gm::Dual<T, N>;
   if constexpr (N == 7) {
     if (type == LENSIM_SERSIC_ELLIPSE) {
       T gp[7], gx, gy;
       S r;
-      r.v = gm::sersic_ellipse_grad<T>(pk, x, y, gp, gx, gy);
+      r.v = gm::sersic_ellipse_grad_rec<T>(rd, pk, x, y, gp, gx, gy);
 #pragma unroll
       for (int i = 0; i < 7; ++i) r.d[i] = gp[i];
       return r;
@@ -2340,7 +2340,8 @@ __device__ __forceinline__ gm::Dual<T, N> light_grad(int type, const gm::Dual<T,
 // tangents d[0], d[1]): closed form for SERSIC_ELLIPSE, two dual seeds
 // otherwise.
 template <typename T>
-__device__ __forceinline__ gm::Dual<T, 2> sources_at(const ModelArgs &m, const GradArgs &ga, int img, T bx, T by) {
+__device__ __forceinline__ gm::Dual<T, 2> sources_at(const ModelArgs &m, const GradArgs &ga, const RecPtrs<T> &rp,
+                                                     int img, T bx, T by) {
   using S2 = gm::Dual<T, 2>;
   const S2 bx2 = S2::seed(bx, 0), by2 = S2::seed(by, 1);
   S2 f2 = S2(T(0));
@@ -2350,7 +2351,7 @@ __device__ __forceinline__ gm::Dual<T, 2> sources_at(const ModelArgs &m, const G
     const int tj = m.types[j - m.n_bulk];
     if (tj == LENSIM_SERSIC_ELLIPSE) {
       T gp[7], gx, gy;
-      f2.v += gm::sersic_ellipse_grad<T>(pj, bx, by, gp, gx, gy);
+      f2.v += gm::sersic_ellipse_grad_rec<T>(rp.recd + j * kRec, pj, bx, by, gp, gx, gy);
       f2.d[0] += gx;
       f2.d[1] += gy;
       continue;
@@ -2381,6 +2382,7 @@ __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga,
 #pragma unroll
   for (int i = 0; i < LENSIM_NPARAM; ++i) ps[i] = i < N ? S::seed(T(pk[i]), i) : S(T(pk[i]));
   S flux;
+  if constexpr (sizeof(T) == sizeof(double)) __builtin_assume(k >= m.n_lens || gb);
   if (k < m.n_lens && gb) {
     // d flux = dS/dbeta . d beta, d beta = -alpha_scaling d alpha_k
     S ax = S(T(0)), ay = S(T(0));
@@ -2433,7 +2435,7 @@ __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga,
     const S bx = xs - ax * T(m.alpha_scaling), by = ys - ay * T(m.alpha_scaling);
     // the sources' gradient in beta, chained into this deflector's kwargs:
     // d flux = dS/dbeta_x d beta_x + dS/dbeta_y d beta_y
-    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, bx.v, by.v);
+    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, rp, img, bx.v, by.v);
     flux.v = f2.v;
 #pragma unroll
     for (int i = 0; i < N; ++i) flux.d[i] = f2.d[0] * bx.d[i] + f2.d[1] * by.d[i];
@@ -2454,7 +2456,7 @@ __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga,
       if constexpr (N == 7) {
         if (m.n_source == 1 && type == LENSIM_SERSIC_ELLIPSE) {  // one evaluation gives both
           T gp[7], gx, gy;
-          flux.v = gm::sersic_ellipse_grad<T>(pk, bxs, bys, gp, gx, gy);
+          flux.v = gm::sersic_ellipse_grad_rec<T>(rp.recd + k * kRec, pk, bxs, bys, gp, gx, gy);
 #pragma unroll
           for (int i = 0; i < 7; ++i) flux.d[i] = gp[i];
           AT(gb, 0) = gx;
@@ -2463,61 +2465,32 @@ __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga,
         }
       }
       if (!done) {
-        const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, bxs, bys);
+        const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, rp, img, bxs, bys);
         AT(gb, 0) = f2.d[0];
         AT(gb, 1) = f2.d[1];
       }
     }
-    if (!done) flux = light_grad<T, N>(type, ps, pk, bxs, bys);
+    if (!done) flux = light_grad<T, N>(type, ps, rp.recd + k * kRec, pk, bxs, bys);
   } else {
     // d/d(lens light kwargs) at the ray
-    flux = light_grad<T, N>(type, ps, pk, T(x), T(y));
+    flux = light_grad<T, N>(type, ps, rp.recd + k * kRec, pk, T(x), T(y));
   }
 #pragma unroll
   for (int i = 0; i < N; ++i) acc[i] += w * double(flux.d[i]);
 }
 
-// ray_grad for an inline NFW deflector k: the other deflectors in the
-// forward form, this one's duals in double in both forms (the float closed
-// forms of the NFW family cancel, as for the bulk list's duals).
-template <typename T, int N, bool HALO>
-__device__ __forceinline__ void halo_ray_grad(const ModelArgs &m, const GradArgs &ga, const RecPtrs<T> &rp, int img,
-                                              int k, int type, double x, double y, double w, double *acc,
-                                              const T *gb) {
-  using S = gm::Dual<double, N>;
+// ray_grad for an inline NFW deflector k, its closed forms in double in both
+// forms (the NFW family's float ones cancel); gb: dS/dbeta.
+template <typename T>
+__device__ __forceinline__ void nfw_ray_grad(const ModelArgs &m, const GradArgs &ga, const RecPtrs<T> &rp, int img,
+                                             int k, double x, double y, double w, double *acc, const T *gb) {
   const double *pk = ga.params + (size_t(img) * m.n_prof + k) * LENSIM_NPARAM;
   CHECK_SPAN(pk, LENSIM_NPARAM * sizeof(double));
-  if (gb) {  // dS/dbeta from the first source's launch
-    S ps[LENSIM_NPARAM];
+  double a_x, a_y, dax[4], day[4];
+  gm::nfw_dalpha_f64(rp.recd + k * kRec, pk, x, y, a_x, a_y, dax, day);
+  const double gx = double(AT(gb, 0)), gy = double(AT(gb, 1)), as = m.alpha_scaling;
 #pragma unroll
-    for (int i = 0; i < LENSIM_NPARAM; ++i) ps[i] = i < N ? S::seed(pk[i], i) : S(pk[i]);
-    S ax = S(0.0), ay = S(0.0);
-    gm::defl_g<double, S>(type, ps, static_cast<const double *>(nullptr), static_cast<const double *>(nullptr), 1,
-                          S(x), S(y), ax, ay);
-    const double gx = double(AT(gb, 0)), gy = double(AT(gb, 1)), as = m.alpha_scaling;
-#pragma unroll
-    for (int i = 0; i < N; ++i) acc[i] += w * (-as * (gx * ax.d[i] + gy * ay.d[i]));
-    return;
-  }
-  double axp = 0.0, ayp = 0.0;
-  for (int j = 0; j < m.n_lens; ++j) {
-    if (j == k) continue;
-    const int e = m.epl_index[j];
-    const size_t co = (e >= 0) ? (size_t(img) * m.n_epl + e) * LENSIM_EPL_NMAX : 0;
-    add_deflection<T, HALO>(m.types[j], Rec<T>{rp.recd + j * kRec, rp.rect + j * kRec}, rp.coefd + co,
-                            rp.coeft + co, x, y, axp, ayp);
-  }
-  deflect_bulk<T, HALO>(m, rp, x, y, axp, ayp);
-  S ps[LENSIM_NPARAM];
-#pragma unroll
-  for (int i = 0; i < LENSIM_NPARAM; ++i) ps[i] = i < N ? S::seed(pk[i], i) : S(pk[i]);
-  S ax = S(axp), ay = S(ayp);
-  gm::defl_g<double, S>(type, ps, static_cast<const double *>(nullptr), static_cast<const double *>(nullptr), 1,
-                        S(x), S(y), ax, ay);
-  const S bx = S(x) - ax * m.alpha_scaling, by = S(y) - ay * m.alpha_scaling;
-  const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, T(bx.v), T(by.v));
-#pragma unroll
-  for (int i = 0; i < N; ++i) acc[i] += w * (double(f2.d[0]) * bx.d[i] + double(f2.d[1]) * by.d[i]);
+  for (int i = 0; i < 4; ++i) acc[i] += w * (-as * (gx * dax[i] + gy * day[i]));
 }
 
 // The deflection of the EPL deflector k at (x, y) and its derivatives by the
@@ -2538,6 +2511,13 @@ template <typename T>
 __device__ __forceinline__ void epl_dalpha(const ModelArgs &m, const GradArgs &ga, const RecPtrs<T> &rp, int img,
                                            int k, const double *pk, double x, double y, T &a_x, T &a_y, T *dax,
                                            T *day) {
+  if constexpr (sizeof(T) == sizeof(double)) {
+    const size_t co = (size_t(img) * m.n_epl + m.epl_index[k]) * LENSIM_EPL_NMAX;
+    CHECK_SPAN(ga.coefd + co, LENSIM_EPL_NMAX * sizeof(double));
+    CHECK_SPAN(ga.dcoefd + co, LENSIM_EPL_NMAX * sizeof(double));
+    gm::epl_dalpha_f64(rp.recd + k * kRec, ga.coefd + co, ga.dcoefd + co, pk, x, y, a_x, a_y, dax, day);
+    return;
+  }
   using S = gm::Dual<T, 2>;
   S ps[LENSIM_NPARAM];
 #pragma unroll
@@ -2612,6 +2592,10 @@ __device__ __forceinline__ void epl_dalpha(const ModelArgs &m, const GradArgs &g
 template <typename T, int TYPE>
 __device__ __forceinline__ void nie_dalpha(const double *rd, const double *pk, double x, double y, T &a_x, T &a_y,
                                            T *dax, T *day) {
+  if constexpr (sizeof(T) == sizeof(double)) {
+    gm::nie_dalpha_f64<TYPE>(rd, pk, x, y, a_x, a_y, dax, day);
+    return;
+  }
   using S = gm::Dual<T, 4>;  // q, s_scale, center_x, center_y
   constexpr bool kNie = TYPE == LENSIM_NIE;
   const T e1 = T(pk[1]), e2 = T(pk[2]);
@@ -2658,6 +2642,7 @@ __device__ __forceinline__ void lens_ray_grad(const ModelArgs &m, const GradArgs
                                              int k, double x, double y, double w, double *acc, const T *gb) {
   const double *pk = ga.params + (size_t(img) * m.n_prof + k) * LENSIM_NPARAM;
   CHECK_SPAN(pk, LENSIM_NPARAM * sizeof(double));
+  if constexpr (sizeof(T) == sizeof(double)) __builtin_assume(gb != nullptr);
   double axp = 0.0, ayp = 0.0;  // the other deflectors in the forward form (not needed with gb)
   if (!gb) {
     for (int j = 0; j < m.n_lens; ++j) {
@@ -2682,7 +2667,7 @@ __device__ __forceinline__ void lens_ray_grad(const ModelArgs &m, const GradArgs
     gy = AT(gb, 1);
   } else {
     const T bxv = T(x) - (T(axp) + a_x) * as, byv = T(y) - (T(ayp) + a_y) * as;
-    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, bxv, byv);
+    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, rp, img, bxv, byv);
     gx = f2.d[0];
     gy = f2.d[1];
   }
@@ -2697,7 +2682,10 @@ __device__ __forceinline__ void lens_ray_grad(const ModelArgs &m, const GradArgs
 // kGradPix pixels' rays.
 // The float form is held to 128 VGPRs (four waves per SIMD instead of three
 // for the EPL's duals; no spills): 239k -> 250k gradients/s.  The FP64 form,
-// and the NFW / TNFW kernels with their double duals, would spill.
+// and the double closed forms of NFW / TNFW, would spill.  What bounds it in
+// FP64 is the vector unit's instructions: the closed forms of grad.hpp in place
+// of duals took 64 images of 120^2 (EPL + SHEAR, Sersic source and light) from
+// 620 to 411 us a call.
 template <typename T, int TYPE>
 constexpr int grad_waves_per_eu() {
   return (sizeof(T) == sizeof(float) && TYPE != LENSIM_NFW && TYPE != LENSIM_TNFW) ? 4 : 1;
@@ -2750,7 +2738,7 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
       if constexpr (type == LENSIM_EPL) lens_ray_grad<T, HALO>(m, ga, rp, img, k, x, y, w, acc, gb);
       else if constexpr (type == LENSIM_SIE) lens_ray_grad<T, HALO, LENSIM_SIE>(m, ga, rp, img, k, x, y, w, acc, gb);
       else if constexpr (type == LENSIM_NIE) lens_ray_grad<T, HALO, LENSIM_NIE>(m, ga, rp, img, k, x, y, w, acc, gb);
-      else if constexpr (type == LENSIM_NFW) halo_ray_grad<T, 4, HALO>(m, ga, rp, img, k, type, x, y, w, acc, gb);
+      else if constexpr (type == LENSIM_NFW) nfw_ray_grad<T>(m, ga, rp, img, k, x, y, w, acc, gb);
       else if constexpr (type == LENSIM_TNFW) {  // live and a lens: gb is there
         const double lw = -m.alpha_scaling * w;
         tnfw_ray_grad(TnfwRec(rp.recd + k * kRec), rp.recd + k * kRec, x, y, lw * double(AT(gb, 0)),
@@ -2812,41 +2800,13 @@ int launch_grad_profile(const ModelArgs &m, const GridArgs &g, const GradArgs &g
 }
 
 // Deflector k's deflection at (x, y) and its derivatives by its kwargs,
-// slots 0 .. N-1 (N returned; 0 for a type without kwargs): the EPL's closed
-// forms in the compute type, the other types' duals in double (as in the bulk
-// list's gradient).  The last two slots of every deflector type are its
-// centre, whose derivative is minus the column of d alpha / d(x, y).
-template <int TYPE, int N>
-__device__ __forceinline__ void dalpha_duals(const double *pk, double x, double y, double &ax, double &ay,
-                                             double *dax, double *day, double *dcen) {
-  using S = gm::Dual<double, N>;
-  S ps[LENSIM_NPARAM];
-#pragma unroll
-  for (int i = 0; i < LENSIM_NPARAM; ++i) ps[i] = i < N ? S::seed(pk[i], i) : S(pk[i]);
-  S sx = S(0.0), sy = S(0.0);
-  gm::defl_g<double, S>(TYPE, ps, static_cast<const double *>(nullptr), static_cast<const double *>(nullptr), 1,
-                        S(x), S(y), sx, sy);
-  ax = sx.v;
-  ay = sy.v;
-#pragma unroll
-  for (int i = 0; i < LENSIM_NPARAM; ++i) {
-    dax[i] = i < N ? sx.d[i] : 0.0;
-    day[i] = i < N ? sy.d[i] : 0.0;
-  }
-  // the centre's derivatives (slots N-2, N-1): minus d alpha / dx and d alpha / dy
-  dcen[0] = sx.d[N - 2];
-  dcen[1] = sy.d[N - 2];
-  dcen[2] = sx.d[N - 1];
-  dcen[3] = sy.d[N - 1];
-}
-
-// nie_dalpha in double, laid out as dalpha_duals'.
-template <int TYPE>
-__device__ __forceinline__ void nie_dalpha_mp(const double *rd, const double *pk, double x, double y, double &ax,
-                                              double &ay, double *dax, double *day, double *dcen) {
-  constexpr int N = n_params_of(TYPE);
-  double dx[6], dy[6];
-  nie_dalpha<double, TYPE>(rd, pk, x, y, ax, ay, dx, dy);
+// slots 0 .. N-1: the EPL's in the compute type, the other types' closed forms
+// in double.  The last two slots of every deflector type are its centre, whose
+// derivative is minus the column of d alpha / d(x, y).
+// N = n_params_of(TYPE) derivatives of a closed form, laid out for deflector_dalpha.
+template <int N>
+__device__ __forceinline__ void spread_dalpha(const double *dx, const double *dy, double *dax, double *day,
+                                              double *dcen) {
 #pragma unroll
   for (int i = 0; i < LENSIM_NPARAM; ++i) {
     dax[i] = i < N ? dx[i] : 0.0;
@@ -2881,10 +2841,24 @@ __device__ __forceinline__ void deflector_dalpha(const ModelArgs &m, const GradA
       dcen[3] = day[5];
       break;
     }
-    case LENSIM_SIE: nie_dalpha_mp<LENSIM_SIE>(rp.recd + k * kRec, pk, x, y, ax, ay, dax, day, dcen); break;
-    case LENSIM_NIE: nie_dalpha_mp<LENSIM_NIE>(rp.recd + k * kRec, pk, x, y, ax, ay, dax, day, dcen); break;
+    case LENSIM_SIE: {
+      double dx[6], dy[6];
+      nie_dalpha<double, LENSIM_SIE>(rp.recd + k * kRec, pk, x, y, ax, ay, dx, dy);
+      spread_dalpha<5>(dx, dy, dax, day, dcen);
+      break;
+    }
+    case LENSIM_NIE: {
+      double dx[6], dy[6];
+      nie_dalpha<double, LENSIM_NIE>(rp.recd + k * kRec, pk, x, y, ax, ay, dx, dy);
+      spread_dalpha<6>(dx, dy, dax, day, dcen);
+      break;
+    }
     case LENSIM_NFW:
-      if constexpr (HALO) dalpha_duals<LENSIM_NFW, 4>(pk, x, y, ax, ay, dax, day, dcen);
+      if constexpr (HALO) {
+        double dx[4], dy[4];
+        gm::nfw_dalpha_f64(rp.recd + k * kRec, pk, x, y, ax, ay, dx, dy);
+        spread_dalpha<4>(dx, dy, dax, day, dcen);
+      }
       break;
     default: break;  // TNFW, SHEAR and CONVERGENCE: their callers' closed forms
   }
@@ -3017,7 +2991,7 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
   const int nd = m.mp_n - 1;
   double gPx = 0.0, gPy = 0.0, gAx = 0.0, gAy = 0.0;
   if (ray.live) {
-    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, bx, by);
+    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, rp, img, bx, by);
     const double tzn = AT(tzs, nd), dt = AT(tij, nd);
     gPx = ray.w * double(f2.d[0]) / tzn;
     gPy = ray.w * double(f2.d[1]) / tzn;
@@ -3093,7 +3067,7 @@ __global__ __launch_bounds__(64 * kBulkWaves) void bulk_adjoint_kernel(
   if (ray.live) {
     const double as = m.alpha_scaling;
     const T bx = T(ray.x - ax * as), by = T(ray.y - ay * as);
-    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, img, bx, by);
+    const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, rp, img, bx, by);
     lx = -as * ray.w * double(f2.d[0]);
     ly = -as * ray.w * double(f2.d[1]);
     T *b = static_cast<T *>(ga.beta) + ray.slot;

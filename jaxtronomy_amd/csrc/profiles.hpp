@@ -1003,6 +1003,48 @@ __device__ __forceinline__ void nfw_defl(const Rec<T> &r, double x, double y, do
   }
 }
 
+// F(X) of the NFW family in double, on u = X^2: arctan(sqrt(u - 1)) / sqrt(u - 1)
+// above u = 1, arctanh(sqrt(1 - u)) / sqrt(1 - u) below, by the series listed at
+// tnfw_core.  halo_G: G of F = (pi / 2) / v - G(1/u) / u (1/u <= 1/4); halo_P:
+// F from 1/4 to 4 (either side of X = 1).
+__device__ __forceinline__ double halo_G(double iu) {
+  constexpr double g13[14] = {1, 0.66666666666673224, 0.53333333331635013, 0.45714285887196332, 0.40634911476368524,
+                              0.36941126493138032, 0.3409332932493519, 0.31907228762239243, 0.29180058074110277,
+                              0.33511256175349097, 0.035139155368524883, 0.97765555800227311, -1.1132861271784307,
+                              1.5537792943093436};
+  return poly(g13, iu);
+}
+__device__ __forceinline__ double halo_P(double X) {
+  constexpr double p19[20] = {1, -0.33333333333333331, 0.2000000000000407, -0.14285714285718173, 0.1111111110990561,
+                              -0.090909090897571695, 0.076923078305074097, -0.066666667987215295, 0.058823449184073437,
+                              -0.052631502289141152, 0.047621712357723792, -0.043480806937435917, 0.039946430293369972,
+                              -0.036985856369465865, 0.035142777271370877, -0.032888583414052187, 0.025482617337549689,
+                              -0.023967278167745611, 0.045592597260624118, -0.043367164921101896};
+  const double q = rcp_full(1.0 + X);
+  return 2.0 * q * poly(p19, (X - 1.0) * q);
+}
+// X dF/dX = (1 - u F) / (u - 1); near u = 1, where the quotient cancels, 2 u
+// dF/du of F = sum (-e)^n / (2 n + 1), e = u - 1.
+__device__ __forceinline__ double halo_XdF(double u, double F) {
+  const double e = u - 1.0;
+  if (fabs(e) < 0.03) {
+    constexpr double d9[10] = {-1.0 / 3, 2.0 / 5,   -3.0 / 7, 4.0 / 9,   -5.0 / 11,
+                               6.0 / 13, -7.0 / 15, 8.0 / 17, -9.0 / 19, 10.0 / 21};
+    return 2.0 * u * poly(d9, e);
+  }
+  return fma(-u, F, 1.0) * rcp_full(e);
+}
+// F itself from u and rX = 1 / X.
+__device__ __forceinline__ double halo_F(double u, double rX) {
+  if (u >= 4.0) {
+    const double iv = rsq_full(u - 1.0), iu = rX * rX;
+    return fma(1.5707963267948966, iv, -(iu * halo_G(iu)));
+  }
+  if (u >= 0.25) return halo_P(u * rX);
+  const double is = rsq_full(1.0 - u);  // ln((1 + s) / X) / s, s = sqrt(1 - u)
+  return 0.6931471805599453 * is * log2_pos(fma(1.0 - u, is, 1.0) * rX);
+}
+
 // The TNFW's g (LensModel/Profiles/tnfw.py:329-349) in double, on u = X^2 (the
 // caller's floor: u >= 1e-6), with w = sqrt(tau^2 + u):
 //   g = pre B,  B = (tau^2 + 2 u - 1) F - pi w + C0 + w L C1,
@@ -1085,40 +1127,19 @@ __device__ __forceinline__ void tnfw_core(const TnfwRec &r, const double *rd, do
     wL = -(w * tau * rX) * poly(a7, y2);
   } else {
     if (u >= 4.0) {
-      constexpr double g13[14] = {1, 0.66666666666673224, 0.53333333331635013, 0.45714285887196332,
-                                  0.40634911476368524, 0.36941126493138032, 0.3409332932493519, 0.31907228762239243,
-                                  0.29180058074110277, 0.33511256175349097, 0.035139155368524883, 0.97765555800227311,
-                                  -1.1132861271784307, 1.5537792943093436};
-      outer(poly(g13, iu));
+      outer(halo_G(iu));
     } else {
       double F;
       const double X = u * rX;
       if (u >= 0.25) {
-        constexpr double p19[20] = {1, -0.33333333333333331, 0.2000000000000407, -0.14285714285718173,
-                                    0.1111111110990561, -0.090909090897571695, 0.076923078305074097,
-                                    -0.066666667987215295, 0.058823449184073437, -0.052631502289141152,
-                                    0.047621712357723792, -0.043480806937435917, 0.039946430293369972,
-                                    -0.036985856369465865, 0.035142777271370877, -0.032888583414052187,
-                                    0.025482617337549689, -0.023967278167745611, 0.045592597260624118,
-                                    -0.043367164921101896};
-        const double q = rcp_full(1.0 + X);
-        F = 2.0 * q * poly(p19, (X - 1.0) * q);
+        F = halo_P(X);
       } else {
         const double s = ::sqrt(1.0 - u);
         F = atanh_dbl(s) * rcp_refined(s);
       }
       B0 = fma(fma(2.0, u, r.t2m1), F, -M_PI * w);
       if constexpr (GRAD > 0) {
-        const double e = u - 1.0;
-        double XF;
-        if (fabs(e) < 0.03) {  // 2 u dF/du, F = sum (-e)^n / (2 n + 1): the quotient cancels here
-          constexpr double d9[10] = {-1.0 / 3, 2.0 / 5, -3.0 / 7, 4.0 / 9, -5.0 / 11,
-                                     6.0 / 13, -7.0 / 15, 8.0 / 17, -9.0 / 19, 10.0 / 21};
-          XF = 2.0 * u * poly(d9, e);
-        } else {
-          XF = fma(-u, F, 1.0) / e;
-        }
-        X0 = fma(fma(2.0, u, r.t2m1), XF, u * fma(4.0, F, -M_PI * iw));
+        X0 = fma(fma(2.0, u, r.t2m1), halo_XdF(u, F), u * fma(4.0, F, -M_PI * iw));
         if constexpr (GRAD > 1) t0 = tau2 * fma(2.0, F, -M_PI * iw);
       }
     }
