@@ -674,22 +674,23 @@ __device__ __forceinline__ RecPtrs<T> rec_ptrs(const ModelArgs &m, const double 
   return r;
 }
 
-// The deflection of the bulk list (records n_lens .. n_defl - 1) added to (ax, ay).
+// The deflection of the bulk list (records n_lens .. n_defl - 1) added to (ax, ay):
+// every nw-th of them from the one `from`.
 template <typename T, bool HALO, bool DBL = false, bool DBL_TNFW = DBL>
 __device__ __forceinline__ void deflect_bulk(const ModelArgs &m, const RecPtrs<T> &rp, double x, double y,
-                                             double &ax, double &ay) {
+                                             double &ax, double &ay, int from = 0, int nw = 1) {
   if (m.n_bulk == 0) return;
   if (m.bulk_type == LENSIM_TNFW) {
     // common case of substructure: one profile type, no per-deflector switch
     if constexpr (HALO) {
-      for (int k = m.n_lens; k < m.n_defl; ++k) {
+      for (int k = m.n_lens + from; k < m.n_defl; k += nw) {
         if constexpr (DBL_TNFW) tnfw_defl<double>(Rec<double>{rp.recd + k * kRec, rp.recd + k * kRec}, x, y, ax, ay);
         else tnfw_defl<T>(Rec<T>{rp.recd + k * kRec, rp.rect + k * kRec}, x, y, ax, ay);
       }
     }
     return;
   }
-  for (int k = m.n_lens; k < m.n_defl; ++k) {
+  for (int k = m.n_lens + from; k < m.n_defl; k += nw) {
     const int type = m.bulk_type ? m.bulk_type : AT(m.bulk_types, k - m.n_lens);
     const Rec<T> r{rp.recd + k * kRec, rp.rect + k * kRec};
     add_deflection<T, HALO, DBL, DBL_TNFW>(type == LENSIM_EPL ? LENSIM_NULL : type, r, nullptr, nullptr, x, y, ax, ay);
@@ -1129,8 +1130,9 @@ __global__ __launch_bounds__(256) void block_max_kernel(const T *__restrict__ v,
 }
 
 constexpr int kMpBlock = 64;  // rays of a block of the multi-plane kernels (a lane each)
-// What a gradient keeps of its multi-plane render for mp_adjoint_kernel, so
-// that the rays are not traced again: per ray and run the position, and beta.
+// What a gradient keeps of its render for the adjoint kernels, so that the
+// rays are not traced again: several planes, per ray and run the position, and
+// beta; a bulk list that render_bulk_kernel takes, beta.
 struct MpKeep {
   double4 *store;
   size_t per_img;
@@ -1142,11 +1144,17 @@ int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, 
                      const float *coeff, const int *tab, unsigned flags, const MpKeep &keep, T *out, int n_img,
                      hipStream_t st);
 
+int bulk_waves(const ModelArgs &m, size_t npix);
+template <typename T>
+int launch_render_bulk(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf,
+                       const double *coefd, const float *coeff, unsigned flags, const MpKeep &keep, T *out, int n_img,
+                       hipStream_t st);
+
 // Launches render_fast_kernel when the model is one of its compile-time lists
 // (EPL, SIE / NIE or NFW, each with or without SHEAR after it, NFW + SIE / NIE
 // in either order; one Sersic source, none or one Sersic lens light),
-// render_mp_kernel for several planes (tab: its plane runs), else
-// render_kernel.
+// render_mp_kernel for several planes (tab: its plane runs),
+// render_bulk_kernel for a bulk list over few pixels, else render_kernel.
 template <typename T>
 int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf, const double *coefd,
                   const float *coeff, const int *tab, unsigned flags, const MpKeep &keep, T *out, float *blkmax,
@@ -1172,8 +1180,10 @@ int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, con
     fast = fast && (sersic(ts) || (f64 && ts == LENSIM_NULL && !(flags & LENSIM_IMAGE_SOURCE))) &&
            (sersic(tl) || m.n_light == 0 || (f64 && tl == LENSIM_NULL));
   }
-  if (m.mp_n) {  // the block maxima for the MFMA convolution follow from the image in a second launch
-    int rc = launch_render_mp<T>(m, g, recd, recf, coefd, coeff, tab, flags, keep, out, n_img, st);
+  const bool share = !m.mp_n && (flags & LENSIM_IMAGE_SOURCE) && bulk_waves(m, size_t(g.nx) * g.ny) > 1;
+  if (m.mp_n || share) {  // the block maxima for the MFMA convolution follow from the image in a second launch
+    int rc = share ? launch_render_bulk<T>(m, g, recd, recf, coefd, coeff, flags, keep, out, n_img, st)
+                   : launch_render_mp<T>(m, g, recd, recf, coefd, coeff, tab, flags, keep, out, n_img, st);
     if (rc || !blkmax) return rc;
     block_max_kernel<T><<<rgrid, 256, 0, st>>>(out, g.nx * g.ny, blkmax);
     return check_launch("block_max_kernel");
@@ -1374,15 +1384,18 @@ int launch_mp_runs(const ModelArgs &m, int *tab, int n_img, hipStream_t st) {
 // order); sixteen would each read 16 KB of LDS that way (2000 cycles a call),
 // so there a row of 16 lanes sums one ray's values and every wave reads the
 // sums, at the price of a second barrier.
-struct WaveSums {
-  double2 part[2][16][65];  // rows of 65: the 16 values of a ray lie on distinct banks
-  double2 sum[2][64];
+template <int W>  // waves at most: 8 or 16
+struct WaveSumsOf {
+  double2 part[2][W][65];  // rows of 65: the 16 values of a ray lie on distinct banks
+  double2 sum[W == 16 ? 2 : 1][64];
 };
-__device__ __forceinline__ void across_waves(WaveSums &red, int buf, int nw, double &vx, double &vy) {
+using WaveSums = WaveSumsOf<16>;
+template <int W>
+__device__ __forceinline__ void across_waves(WaveSumsOf<W> &red, int buf, int nw, double &vx, double &vy) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   red.part[buf][wave][lane] = double2{vx, vy};
   __syncthreads();
-  if (nw == 16) {
+  if (W == 16 && nw == 16) {
     const int ray = threadIdx.x >> 4, w = threadIdx.x & 15;
     const double2 v = red.part[buf][w][ray];
     const double2 s{row_sum(v.x), row_sum(v.y)};
@@ -1595,6 +1608,96 @@ int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, 
   }
 #undef LENSIM_RENDER
   return check_launch("render_mp_kernel");
+}
+
+// render_kernel for a bulk list over few pixels: the block's waves hold the
+// same 64 pixels and share the list (the first takes the inline deflectors
+// too), their sums meeting in LDS once per sub-ray; the first adds the light.
+// A lane per pixel alone leaves 4 images of 100^2 at less than one wave per
+// SIMD, each waiting out 200 deflectors' latency four times over (479 us; 275
+// so, and the adjoint kernel's 204 us of deflections fall away with the beta
+// kept here: a gradient 989 -> 605 us).  beta: see MpKeep.
+template <typename T, bool HALO, bool DBL>
+__global__ __launch_bounds__(512) void render_bulk_kernel(ModelArgs m, GridArgs g, const double *__restrict__ recd,
+                                                          const float *__restrict__ recf,
+                                                          const double *__restrict__ coefd,
+                                                          const float *__restrict__ coeff, unsigned flags,
+                                                          T *__restrict__ beta, T *__restrict__ out) {
+  __shared__ WaveSumsOf<8> red;
+  const int img = blockIdx.y, nw = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int npix = g.nx * g.ny;
+  const int pix0 = blockIdx.x * 64 + (threadIdx.x & 63);
+  const bool active = pix0 < npix;
+  const int pix = active ? pix0 : npix - 1;
+  int i;
+  const int j = div_by(pix, g.nx, g.inv_nx, i);
+  const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
+  const double ra_c = i * g.m00 + j * g.m01 + g.ra0;
+  const double dec_c = i * g.m10 + j * g.m11 + g.dec0;
+  const bool do_light = (flags & LENSIM_IMAGE_LENS_LIGHT) && m.n_light > 0;
+  const int k_src0 = m.n_defl, k_src1 = m.n_defl + m.n_source, k_l1 = m.n_prof;
+  double acc = 0.0;
+  const bool eval = active && evaluated(g, i, j);
+  const bool any = __any(eval);  // the same in every wave: they hold the same pixels
+  const int rays = any ? g.s * g.s : 0;
+  for (int r = 0; r < rays; ++r) {
+    const int sy = r / g.s, sx = r - sy * g.s;
+    const double oy = g.o0 + sy * g.inv_s, ox = g.o0 + sx * g.inv_s;
+    const double x = ra_c + g.m00 * ox + g.m01 * oy;
+    const double y = dec_c + g.m10 * ox + g.m11 * oy;
+    double ax = 0.0, ay = 0.0;
+    if (wave == 0)
+      for (int k = 0; k < m.n_lens; ++k) deflect_one<T, HALO, DBL>(m, rp, img, k, m.types[k], x, y, ax, ay);
+    deflect_bulk<T, HALO, DBL>(m, rp, x, y, ax, ay, wave, nw);
+    across_waves(red, r & 1, nw, ax, ay);
+    if (wave == 0 && eval) {
+      const double bx = x - ax * m.alpha_scaling, by = y - ay * m.alpha_scaling;
+      if (beta) {
+        T *b = beta + ((size_t(img) * npix + pix) * size_t(g.s * g.s) + size_t(r)) * 2;
+        AT(b, 0) = T(bx);
+        AT(b, 1) = T(by);
+      }
+      acc += light_sum<T>(m, rp, k_src0, k_src1, bx, by);
+      if (do_light) acc += light_sum<T>(m, rp, k_src1, k_l1, x, y);
+    }
+  }
+  if (active && wave == 0) AT(out, size_t(img) * npix + pix) = T(acc * (g.scale * m.flux_scaling));
+}
+
+// Waves that share a bulk list's pixels (render_bulk_kernel), 1 for
+// render_kernel: enough for one image to put four waves on each SIMD while
+// each takes eight deflectors or more.  It depends on the image alone (not on
+// the batch), as the order of the sums does.  BULK_WAVES_FIGURES
+int bulk_waves(const ModelArgs &m, size_t npix) {
+  int nw = 1;
+  while (m.mp_n == 0 && m.n_source > 0 && nw < 8 && npix * nw < 64 * 4096 && m.n_bulk >= 16 * nw) nw *= 2;
+  return nw;
+}
+
+// Whether a gradient's render_bulk_kernel keeps beta for bulk_adjoint_kernel:
+// not where the float form renders in double what the adjoint takes in float.
+template <typename T>
+bool bulk_keeps(const ModelArgs &m, size_t npix) {
+  return bulk_waves(m, npix) > 1 && (sizeof(T) == sizeof(double) || !m.has_nie_nfw);
+}
+
+template <typename T>
+int launch_render_bulk(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf,
+                       const double *coefd, const float *coeff, unsigned flags, const MpKeep &keep, T *out, int n_img,
+                       hipStream_t st) {
+  const size_t npix = size_t(g.nx) * g.ny;
+  const dim3 grid((unsigned)((npix + 63) / 64), n_img);
+#define LENSIM_RENDER(H, D)                                                                               \
+  render_bulk_kernel<T, H, D><<<grid, 64 * bulk_waves(m, npix), 0, st>>>(m, g, recd, recf, coefd, coeff, \
+                                                                         flags, static_cast<T *>(keep.beta), out)
+  constexpr bool kF32 = sizeof(T) == sizeof(float);  // as render_kernel's
+  if (kF32 && m.has_nie_nfw && m.has_halo) LENSIM_RENDER(true, kF32);
+  else if (kF32 && m.has_nie_nfw) LENSIM_RENDER(false, kF32);
+  else if (m.has_halo) LENSIM_RENDER(true, false);
+  else LENSIM_RENDER(false, false);
+#undef LENSIM_RENDER
+  return check_launch("render_bulk_kernel");
 }
 
 // raytrace_mp_kernel's launches for a call, in pieces of 2^28 rays (a launch's
@@ -3034,15 +3137,16 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
 // The same for a single-plane list: with beta = theta - alpha_scaling sum_j
 // alpha_j the adjoint of every deflection is l = -alpha_scaling w dS/dbeta.
 // The block's waves share the bulk list of its 64 rays (the first takes the
-// inline deflectors too).  Stores (x, y, l), beta, and dS/dbeta for the inline
+// inline deflectors too); kept: the render kept beta, and the block is one
+// wave.  Stores (x, y, l), beta, and dS/dbeta for the inline
 // deflectors' launches.
 constexpr int kBulkWaves = 8;
 template <typename T, bool HALO>
 __global__ __launch_bounds__(64 * kBulkWaves) void bulk_adjoint_kernel(
     ModelArgs m, GridArgs g, GradArgs ga, const double *__restrict__ recd, const float *__restrict__ recf,
     const double *__restrict__ coefd, const float *__restrict__ coeff, double4 *__restrict__ store, size_t per_img,
-    int round) {
-  __shared__ WaveSums red;
+    int round, bool kept) {
+  __shared__ WaveSumsOf<kBulkWaves> red;
   const int img = blockIdx.y, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r_all = g.nx * g.ny * g.s * g.s;
@@ -3053,7 +3157,7 @@ __global__ __launch_bounds__(64 * kBulkWaves) void bulk_adjoint_kernel(
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
   const GradRay ray = grad_ray<T>(m, g, ga, img, int(active ? rr : r_all - 1), active);
   double ax = 0.0, ay = 0.0;
-  if (__any(ray.live)) {  // the same in every wave
+  if (!kept && __any(ray.live)) {  // the same in every wave
     if (wave == 0)
       for (int k = 0; k < m.n_lens; ++k) deflect_one<T, HALO, false>(m, rp, img, k, m.types[k], ray.x, ray.y, ax, ay);
     for (int k = m.n_lens + wave; k < m.n_defl; k += kBulkWaves) {
@@ -3066,13 +3170,15 @@ __global__ __launch_bounds__(64 * kBulkWaves) void bulk_adjoint_kernel(
   double lx = 0.0, ly = 0.0;
   if (ray.live) {
     const double as = m.alpha_scaling;
-    const T bx = T(ray.x - ax * as), by = T(ray.y - ay * as);
+    T *b = static_cast<T *>(ga.beta) + ray.slot;
+    const T bx = kept ? AT(b, 0) : T(ray.x - ax * as), by = kept ? AT(b, 1) : T(ray.y - ay * as);
     const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, rp, img, bx, by);
     lx = -as * ray.w * double(f2.d[0]);
     ly = -as * ray.w * double(f2.d[1]);
-    T *b = static_cast<T *>(ga.beta) + ray.slot;
-    AT(b, 0) = bx;
-    AT(b, 1) = by;
+    if (!kept) {
+      AT(b, 0) = bx;
+      AT(b, 1) = by;
+    }
     if (ga.gbeta) {
       T *gb = static_cast<T *>(ga.gbeta) + ray.slot;
       AT(gb, 0) = f2.d[0];
@@ -3263,8 +3369,9 @@ int launch_defl_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, 
   if (!m.mp_n && sub == 0) sub = m.bulk_type ? int(sub_type(m.bulk_type)) : 2;  // of the bulk list alone
   for (int r = 0; r < p.rounds; ++r) {
     if (!m.mp_n) {
-      bulk_adjoint_kernel<T, HALO><<<grid, 64 * kBulkWaves, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, store,
-                                                                     p.per_img, r);
+      const bool kept = bulk_keeps<T>(m, size_t(g.nx) * g.ny);
+      bulk_adjoint_kernel<T, HALO><<<grid, kept ? 64 : 64 * kBulkWaves, 0, st>>>(
+          m, g, ga, recd, recf, ga.coefd, ga.coeff, store, p.per_img, r, kept);
     } else {
 #define LENSIM_ADJOINT(H, S)                                                                                         \
   mp_adjoint_kernel<T, H, S><<<grid, 64 * mp_waves(rays, S), 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, \
@@ -3934,6 +4041,8 @@ int run_grad(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int k
     const size_t rays = size_t(g.nx) * g.ny * g.s * g.s;
     keep.store = reinterpret_cast<double4 *>(ws + L.gstate);
     keep.per_img = defl_grad_plan(m, rays, n_img).per_img;
+    keep.beta = ws + L.beta;
+  } else if (bulk_keeps<T>(m, size_t(g.nx) * g.ny * (ss.on ? size_t(ss.s) * ss.s : 1))) {
     keep.beta = ws + L.beta;
   }
   int rc = ss.on ? run_image_ss<T>(m, g, psf, kx, ky, edge, ss, data, params, n_img, flags, nullptr, logl, ws, L, st,
