@@ -25,6 +25,7 @@
 #include <string.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "grad.hpp"
 #include "profiles.hpp"
@@ -273,24 +274,22 @@ size_t mfma_smem(int kx, int ky, int tl) {
   return size_t(kMfTY + ky - 1) * mfma_ls(kx, tl) * 2 * sizeof(_Float16);
 }
 
-// ---- float64 matrix-core convolution (FP64 form) ----
-// v_mfma_f64_16x16x4_f64 (lane l holds A[l % 16][l / 16] and B[l / 16][l % 16]
-// of a K-step): per kernel row a, D(16 x 16) += A(16 x 4 nk4) B(4 nk4 x 16)
-// with A = 16 image rows of the padded tile and B[k][n] = Kf[a][k - n]; nk4
-// K-steps of 4 cover 16 + kx - 1 columns.  The LDS row stride is 2 (mod 16)
-// doubles: the 32 lanes of each half of a ds_read_b64 (16 rows x 2 columns)
-// then fall on distinct banks.
-int mf64_nk4(int kx) { return (16 + kx - 1 + 3) / 4; }
-int mf64_tw(int kx, int tl) { return 16 * (tl - 1) + 4 * mf64_nk4(kx); }
-int mf64_ls(int kx, int tl) {
-  const int tw = mf64_tw(kx, tl);
-  return tw + ((2 - tw % 16) + 16) % 16;
+// ---- convolution of the FP64 form ----
+// conv_f64_kernel's LDS: rows of a tile (the register groups are read whole,
+// past the rows in use), doubles of the tile (later the waves' sums), and
+// with the weights in bytes.
+int conv_f64_rows(int ky, int r, int h) {
+  const int used = 2 * r * h + ky - 1, read = (2 * h - 1) * r + 24 + ky / 8 * 8;
+  return used > read ? used : read;
 }
-size_t mf64_smem(int kx, int ky, int tl) { return size_t(kMfTY + ky - 1) * mf64_ls(kx, tl) * sizeof(double); }
-// K-steps (kernel rows x nk4) padded with zero fragments to a multiple of the
-// kernel's prefetch depth, so its step loop has no partial group
-constexpr int kMf64B = 8;
-int mf64_steps(int kx, int ky) { return (ky * mf64_nk4(kx) + kMf64B - 1) / kMf64B * kMf64B; }
+__host__ __device__ inline int conv_f64_tile(int kx, int th, int r, int h, int cls) {
+  const int t = th * (32 + kx - 1) + 1, sums = 64 * cls * h * r;
+  return (t > sums ? t : sums) & ~1;
+}
+size_t conv_f64_smem(int kx, int ky, int r, int h, int cls, bool gw) {
+  return (size_t(conv_f64_tile(kx, conv_f64_rows(ky, r, h), r, h, cls)) + (gw ? 0 : size_t(kx) * kyp_of(ky))) *
+         sizeof(double);
+}
 
 // Blocks of 64 rows x 16 tl columns.  All of a call's blocks are resident at
 // once on this workload's sizes, so the time is that of the busiest CU:
@@ -313,12 +312,12 @@ int cu_count() {
   }
   return n;
 }
-MfmaPlan mfma_plan(int nx, int ny, int n_img, int kx, int ky, bool f64 = false) {
+MfmaPlan mfma_plan(int nx, int ny, int n_img, int kx, int ky) {
   MfmaPlan best{0, 0, 0};
   long best_load = 0;
   const int cus = cu_count();
   for (int tl = 4; tl >= 2; --tl) {
-    if ((f64 ? mf64_smem(kx, ky, tl) : mfma_smem(kx, ky, tl)) > kMaxLds) continue;
+    if (mfma_smem(kx, ky, tl) > kMaxLds) continue;
     const int ntx = (nx + 16 * tl - 1) / (16 * tl), nt = ntx * ((ny + kMfTY - 1) / kMfTY);
     const long blocks = long(nt) * n_img;
     const long load = (blocks + cus - 1) / cus * tl;
@@ -408,9 +407,8 @@ Layout layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img, int
   }
   L.mp_tab = off;
   if (m.mp_n > 0) off = align256(off + mp_tab_sets(m, n_img) * size_t(mp_tab_ints(m)) * 4);
-  L.bfrag = off;  // int exponent (16 B slot) then the MFMA B fragments (float64 fragments in the FP64 form)
+  L.bfrag = off;  // int exponent (16 B slot) then the MFMA B fragments
   if (precision == LENSIM_MIXED) off = align256(off + 16 + size_t(mfma_steps(kx, ky)) * 2 * 64 * 16);
-  else off = align256(off + size_t(mf64_steps(kx, ky)) * 64 * sizeof(double));
   L.total = off;
   return L;
 }
@@ -1668,7 +1666,9 @@ __global__ __launch_bounds__(512) void render_bulk_kernel(ModelArgs m, GridArgs 
 // Waves that share a bulk list's pixels (render_bulk_kernel), 1 for
 // render_kernel: enough for one image to put four waves on each SIMD while
 // each takes eight deflectors or more.  It depends on the image alone (not on
-// the batch), as the order of the sums does.  BULK_WAVES_FIGURES
+// the batch), as the order of the sums does.  Measured with 1 / 2 / 4 / 8
+// waves: 16 mixed images of 300^2 and 1000 subhalos 21.8 / 21.5 / 20.95 / 22.2
+// ms a call, 4 gradients of 100^2 and 200 in FP64 1010 / 684 / 605 / 604 us.
 int bulk_waves(const ModelArgs &m, size_t npix) {
   int nw = 1;
   while (m.mp_n == 0 && m.n_source > 0 && nw < 8 && npix * nw < 64 * 4096 && m.n_bulk >= 16 * nw) nw *= 2;
@@ -1937,6 +1937,193 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs c, const T *__restri
 }
 
 
+// The FP64 form's convolution: conv_kernel's sum on a tile of 32 columns x 2 R H
+// rows.  Each of the 4 H waves takes the kernel columns of one class (mod 4) for
+// 32 x 2 R pixels; the classes' sums meet in LDS and are added in class order,
+// so that neither the sum nor the chi^2 partials (of 32 x 16 pixels) depend on
+// the block's shape, which follows the batch.  A lane has R consecutive rows of
+// one column: of a kernel column it reads each image value once (consecutive
+// lanes, consecutive words) and holds 24 of them in three groups of eight that
+// rotate by name, so that no register is moved.  GW: the weights by scalar
+// loads, else from LDS (few blocks: there every step's loads would miss the
+// caches in turn).  The FP64 vector unit has the matrix unit's rate here, and no
+// band of zeros to multiply (a Toeplitz block on v_mfma_f64_16x16x4 spends 41 of
+// 56 columns at 41 x 41).  Measured: 71^2 with 21 x 21 22.3 -> 7.4 us, 60^2 with
+// 11 x 11 13.6 -> 6.2, 4 images of 100^2 with 21 x 21 30 -> 9, 64 of 180^2 with 41
+// x 41 184 -> 165 (42 TFLOP/s of the 65 a matrix product reaches; the rest is
+// the ragged edge tiles, 13%, halo loads and each column's first reads).
+template <int R, int H, int CLS, bool GW>
+__global__ __launch_bounds__(64 * CLS * H) void conv_f64_kernel(ConvArgs c, int th, const double *__restrict__ in,
+                                                       const double *__restrict__ kt, double *__restrict__ out,
+                                                       double *__restrict__ partial) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  double *tile = reinterpret_cast<double *>(smem_raw);
+  int img = blockIdx.y, tile_id = blockIdx.x;
+  {  // XCD-aware order, as conv_mfma_kernel
+    const int n_blk = gridDim.x * gridDim.y, lin = blockIdx.y * gridDim.x + blockIdx.x;
+    if ((n_blk & 7) == 0) {
+      const int logical = (lin & 7) * (n_blk >> 3) + (lin >> 3);
+      img = logical / gridDim.x;
+      tile_id = logical - img * gridDim.x;
+    }
+  }
+  const int tyi = tile_id / c.n_tiles_x, txi = tile_id - tyi * c.n_tiles_x;
+  const int y0 = tyi * 2 * R * H, x0 = txi * 32;
+  const int cy = (c.ky - 1) / 2, cx = (c.kx - 1) / 2;
+  const int TH = 2 * R * H + c.ky - 1, TW = 32 + c.kx - 1;
+  const double *src = in + size_t(img) * c.nx * c.ny;
+  const int tid = threadIdx.x;
+  double *wl = tile + conv_f64_tile(c.kx, th, R, H, CLS);
+  static_assert(R % CLS == 0 && R * H % 8 == 0, "");
+  // the weights and the tile, eight loads in flight per thread: every thread
+  // loads (from the nearest pixel of the image), zeros are chosen afterwards
+  constexpr int NT = 64 * CLS * H, kLd = 8, kLw = 2;
+  const int nt = TH * TW, nwt = c.kx * c.kyp;
+  const int dy = NT / TW, dx = NT - dy * TW;
+  double w0[kLw];
+  if constexpr (GW) CHECK_SPAN(kt, size_t(nwt) * sizeof(double));
+#pragma unroll
+  for (int u = 0; u < kLw; ++u) w0[u] = GW ? 0.0 : AT(kt, min(tid + u * NT, nwt - 1));
+  int ly = tid / TW, lx0 = tid - ly * TW;
+  auto some = [&](auto n, int base) {
+    constexpr int kN = decltype(n)::value;
+    double v[kN];
+    bool ok[kN];
+#pragma unroll
+    for (int u = 0; u < kN; ++u) {
+      const int gy = y0 - cy + ly, gx = x0 - cx + lx0;
+      const int py = min(max(gy, 0), c.ny - 1), px = min(max(gx, 0), c.nx - 1);
+      v[u] = AT(src, py * c.nx + px);
+      ok[u] = c.edge || (py == gy && px == gx);
+      lx0 += dx;
+      ly += dy;
+      const bool wrap = lx0 >= TW;
+      lx0 -= wrap ? TW : 0;
+      ly += wrap;
+    }
+#pragma unroll
+    for (int u = 0; u < kN; ++u)
+      if (base + tid + u * NT < nt) tile[base + tid + u * NT] = ok[u] ? v[u] : 0.0;
+  };
+  int base = 0;
+  for (; base + (kLd - 2) * NT < nt; base += NT * kLd) some(std::integral_constant<int, kLd>(), base);
+  for (; base < nt; base += NT * 2) some(std::integral_constant<int, 2>(), base);
+#pragma unroll
+  for (int u = 0; u < kLw; ++u)
+    if (!GW && tid + u * NT < nwt) wl[tid + u * NT] = w0[u];
+  for (int at = tid + kLw * NT; !GW && at < nwt; at += NT * kLd) {
+    double v[kLd];
+#pragma unroll
+    for (int u = 0; u < kLd; ++u) v[u] = AT(kt, min(at + u * NT, nwt - 1));
+#pragma unroll
+    for (int u = 0; u < kLd; ++u)
+      if (at + u * NT < nwt) wl[at + u * NT] = v[u];
+  }
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lx = lane & 31;
+  const int cls = wave % CLS, row0 = wave / CLS * 2 * R + (lane >> 5) * R;  // the lane's first row of the tile
+  double acc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = 0.0;
+  for (int cc = cls; cc < c.kx; cc += CLS) {
+    const double *col = tile + row0 * TW + lx + cc;
+    const double *w = (GW ? kt : wl) + cc * c.kyp;
+    double g0[8], g1[8], g2[8];
+    auto load = [&](double (&g)[8]) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) g[i] = col[i * TW];
+      col += 8 * TW;
+    };
+    // the next n taps of w: tap u reads rows u .. u + R - 1 of a, b, d
+    auto taps = [&](auto n, const double (&a)[8], const double (&b)[8], const double (&d)[8]) {
+#pragma unroll
+      for (int u = 0; u < decltype(n)::value; ++u) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int q = u + r;
+          acc[r] = fma(q < 8 ? a[q & 7] : (q < 16 ? b[q & 7] : d[q & 7]), w[u], acc[r]);
+        }
+      }
+      w += 8;
+    };
+    // a kernel has an odd number of rows: 1, 3, 5 or 7 in its last group
+    auto tail = [&](int n, const double (&a)[8], const double (&b)[8], const double (&d)[8]) {
+      if (n & 4) {
+        if (n & 2) taps(std::integral_constant<int, 7>(), a, b, d);
+        else taps(std::integral_constant<int, 5>(), a, b, d);
+      } else {
+        if (n & 2) taps(std::integral_constant<int, 3>(), a, b, d);
+        else taps(std::integral_constant<int, 1>(), a, b, d);
+      }
+    };
+    constexpr std::integral_constant<int, 8> k8;
+    load(g0);
+    load(g1);
+    if (R + c.ky - 1 > 16) load(g2);
+    int left = c.ky;
+    while (true) {
+      if (left < 8) {
+        tail(left, g0, g1, g2);
+        break;
+      }
+      taps(k8, g0, g1, g2);
+      load(g0);
+      if ((left -= 8) < 8) {
+        tail(left, g1, g2, g0);
+        break;
+      }
+      taps(k8, g1, g2, g0);
+      load(g1);
+      if ((left -= 8) < 8) {
+        tail(left, g2, g0, g1);
+        break;
+      }
+      taps(k8, g2, g0, g1);
+      load(g2);
+      left -= 8;
+    }
+  }
+  if constexpr (CLS > 1) {
+    __syncthreads();  // the tile is read: the classes' sums take its place
+#pragma unroll
+    for (int r = 0; r < R; ++r) tile[(wave * R + r) * 64 + lane] = acc[r];
+    __syncthreads();
+  }
+  const int x = x0 + lx;
+  double chi[R / CLS];
+#pragma unroll
+  for (int i = 0; i < R / CLS; ++i) {
+    const int r = cls + CLS * i, y = y0 + row0 + r;
+    double m = acc[i];
+    if constexpr (CLS > 1) {
+      const double *s = tile + (wave / CLS * CLS * R + r) * 64 + lane;
+      m = (s[0] + s[R * 64]) + (s[2 * R * 64] + s[3 * R * 64]);
+    }
+    chi[i] = 0.0;
+    if (x < c.nx && y < c.ny) {
+      const size_t p = size_t(y) * c.nx + x;
+      if (out) AT(out, size_t(img) * c.nx * c.ny + p) = m;
+      if (partial) chi[i] = chi2_pixel<double>(c, p, m, img);
+      if (c.gout) AT(static_cast<double *>(c.gout), size_t(img) * c.nx * c.ny + p) = dlogl_dm(c, p, m, img);
+    }
+  }
+  if (partial) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < R / CLS; ++i) tile[(row0 + cls + CLS * i) * 32 + lx] = chi[i];
+    __syncthreads();
+    for (int q = wave; q < R * H / 8; q += CLS * H) {
+      const int ty = (y0 >> 4) + q;
+      double v = 0.0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v += tile[q * 512 + i * 64 + lane];
+      v = wave_sum(v);
+      const int n = c.n_tiles_x * ((c.ny + 15) >> 4);
+      if (lane == 0 && 16 * ty < c.ny) AT(partial, size_t(img) * n + ty * c.n_tiles_x + txi) = v;
+    }
+  }
+}
+
 // ------------------------------------------------ MFMA convolution (mixed) --
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -2002,21 +2189,7 @@ struct PsfJob {
 int psf_job_blocks(const PsfJob &pj) {
   if (pj.mode == 1) return (pj.kyp * pj.kx + 255) / 256;
   if (pj.mode == 2) return (pj.n_steps * 2 * 64 + 255) / 256;
-  if (pj.mode == 3) return (pj.n_steps * 64 + 255) / 256;
   return 0;
-}
-
-// B fragments of the float64 matrix-core convolution, [a][kk][lane] in the
-// lane layout of v_mfma_f64_16x16x4_f64 (lane l holds B[l / 16][l % 16] of
-// K-step kk): B[k][n] = Kf[a][k - n], Kf = the flipped kernel, zero outside;
-// the n_steps - ky nk4 padding steps are zero.
-__device__ void psf_mf64_prep_one(const double *__restrict__ k, int kx, int ky, int nk4, int n_steps,
-                                  double *__restrict__ frag, int idx) {
-  if (idx >= n_steps * 64) return;
-  const int lane = idx & 63, step = idx >> 6;
-  const int a = step / nk4, kk = step - a * nk4;
-  const int c = 4 * kk + (lane >> 4) - (lane & 15);  // tap of the flipped row a
-  AT(frag, idx) = (a < ky && c >= 0 && c < kx) ? AT(k, size_t(ky - 1 - a) * kx + (kx - 1 - c)) : 0.0;
 }
 
 // Blocks [0, nb_prep): one thread per (image, profile) record; the rest: the PSF job.
@@ -2033,8 +2206,6 @@ __global__ __launch_bounds__(256) void prep_psf_kernel(ModelArgs m, const double
   const int b = blockIdx.x - nb_prep;
   if (pj.mode == 2) {
     psf_mfma_prep_block(pj.k, pj.kx, pj.ky, pj.nks, pj.n_steps, pj.hdr, pj.frag, b);
-  } else if (pj.mode == 3) {
-    psf_mf64_prep_one(pj.k, pj.kx, pj.ky, pj.nks, pj.n_steps, pj.kt, b * 256 + threadIdx.x);
   } else {
     const int idx = b * 256 + threadIdx.x;
     if (idx < pj.kyp * pj.kx) psf_prep_one(pj.k, pj.kx, pj.ky, pj.kyp, pj.kt, 1, idx);
@@ -2250,140 +2421,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 3))) voi
       for (int off = 32; off > 0; off >>= 1) chi += __shfl_xor(chi, off, 64);
       const int tx16 = (X0 >> 4) + t;
       // tiles past the image's edge hold no pixel and have no slot
-      if (lane == 0 && 16 * tx16 < c.nx && 16 * ty16 < c.ny)
-        AT(partial, size_t(img) * n16 + size_t(ty16) * n16x + tx16) = chi;
-    }
-  }
-}
-
-
-// Direct 'same' convolution in float64 on the matrix cores (FP64 form):
-// block = 64 rows x 16 TL columns (4 waves x TL tiles of 16 x 16), per
-// kernel row a and K-step kk one v_mfma_f64_16x16x4_f64 per tile; the padded
-// tile sits in LDS, the B fragments (psf_mf64_prep_one) come from L2 through
-// buffer loads.  Same outputs, chi^2 partials (per 16 x 16 tile) and
-// dlogL/dmodel as conv_mfma_kernel, all in float64.
-typedef double double4_t __attribute__((ext_vector_type(4)));
-
-template <int TL>
-__global__ __launch_bounds__(256) void conv_mf64_kernel(ConvArgs c, int ls, int nk4, const double *__restrict__ in,
-                                                        const double *__restrict__ frag, double *__restrict__ out,
-                                                        double *__restrict__ partial) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  double *tile = reinterpret_cast<double *>(smem_raw);
-  // XCD-aware order, as conv_mfma_kernel
-  int img = blockIdx.y, tile_id = blockIdx.x;
-  {
-    const int n_blk = gridDim.x * gridDim.y, lin = blockIdx.y * gridDim.x + blockIdx.x;
-    if ((n_blk & 7) == 0) {
-      const int logical = (lin & 7) * (n_blk >> 3) + (lin >> 3);
-      img = logical / gridDim.x;
-      tile_id = logical - img * gridDim.x;
-    }
-  }
-  const int tyi = tile_id / c.n_tiles_x, txi = tile_id - tyi * c.n_tiles_x;
-  const int Y0 = tyi * kMfTY, X0 = txi * 16 * TL;
-  const int cy = (c.ky - 1) / 2, cx = (c.kx - 1) / 2;
-  const int TH = kMfTY + c.ky - 1, TW = 16 * (TL - 1) + 4 * nk4;
-  const int tid = threadIdx.x;
-  const double *src = in + size_t(img) * c.nx * c.ny;
-  // padded tile: eight loads in flight per thread before the LDS stores
-  constexpr int kLd = 8;
-  for (int base = tid; base < TH * TW; base += 256 * kLd) {
-    double v[kLd];
-    int at[kLd];
-#pragma unroll
-    for (int u = 0; u < kLd; ++u) {
-      const int idx = base + u * 256;
-      const int ly = idx / TW, lx = idx - ly * TW;
-      int gy = Y0 - cy + ly, gx = X0 - cx + lx;
-      v[u] = 0.0;
-      at[u] = idx < TH * TW ? ly * ls + lx : -1;
-      if (idx >= TH * TW) {
-      } else if (c.edge) {
-        gy = gy < 0 ? 0 : (gy >= c.ny ? c.ny - 1 : gy);
-        gx = gx < 0 ? 0 : (gx >= c.nx ? c.nx - 1 : gx);
-        v[u] = AT(src, size_t(gy) * c.nx + gx);
-      } else if (gy >= 0 && gy < c.ny && gx >= 0 && gx < c.nx) {
-        v[u] = AT(src, size_t(gy) * c.nx + gx);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kLd; ++u)
-      if (at[u] >= 0) tile[at[u]] = v[u];
-  }
-  __syncthreads();
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, li = lane & 15, lg = lane >> 4;
-  // lane (li, lg) reads A[li][lg] of each K-step: tile row 16 wave + li + a,
-  // column 16 t + 4 kk + lg
-  const double *arow = tile + (16 * wave + li) * ls + lg;
-  // n_steps: a multiple of kMf64B; the steps past ky nk4 have zero B
-  // fragments and re-read A of the last kernel row (a stays at ky - 1)
-  const int n_steps = (c.ky * nk4 + kMf64B - 1) / kMf64B * kMf64B;
-  const __amdgpu_buffer_rsrc_t frs =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(frag), (short)0, n_steps * 512, 0x00020000);
-  const int voff = lane * 8;
-  CHECK_SPAN(frag, size_t(n_steps) * 512);
-  double4_t acc[TL];
-#pragma unroll
-  for (int t = 0; t < TL; ++t) acc[t] = double4_t{0.0, 0.0, 0.0, 0.0};
-  // the B fragments of kMf64B steps are requested ahead of their MFMAs
-  double bq[kMf64B];
-#pragma unroll
-  for (int p = 0; p < kMf64B; ++p)
-    bq[p] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(frs, voff, p * 512, 0));
-  // A of a step is read from LDS one step ahead, so its latency falls under
-  // the previous step's MFMAs (a block's LDS leaves room for one block per CU
-  // at the usual tile widths: no other wave hides it)
-  int a = 0, kk = 0;
-  double av[TL];
-#pragma unroll
-  for (int t = 0; t < TL; ++t) av[t] = arow[16 * t];
-  for (int s0 = 0; s0 < n_steps; s0 += kMf64B) {
-#pragma unroll
-    for (int p = 0; p < kMf64B; ++p) {
-      int a1 = a, kk1 = kk + 1;
-      if (kk1 == nk4) {
-        kk1 = 0;
-        if (a1 + 1 < c.ky) ++a1;
-      }
-      const double *apn = arow + a1 * ls + 4 * kk1;
-      double an[TL];
-#pragma unroll
-      for (int t = 0; t < TL; ++t) an[t] = apn[16 * t];
-#pragma unroll
-      for (int t = 0; t < TL; ++t) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[t], bq[p], acc[t], 0, 0, 0);
-#pragma unroll
-      for (int t = 0; t < TL; ++t) av[t] = an[t];
-      a = a1;
-      kk = kk1;
-      // refill slot p with step s0 + p + kMf64B (the refills past the end re-read the last step, unused)
-      const int q = __builtin_amdgcn_readfirstlane(s0 + p + kMf64B < n_steps ? s0 + p + kMf64B : n_steps - 1);
-      bq[p] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(frs, voff, q * 512, 0));
-    }
-  }
-  // result register j of lane l holds D[l / 16 + 4 j][l % 16] of each tile
-  // (measured on gfx950); chi^2 partials per 16 x 16 tile
-  const int n16x = (c.nx + 15) >> 4, n16 = n16x * ((c.ny + 15) >> 4);
-  const int ty16 = (Y0 >> 4) + wave;
-#pragma unroll
-  for (int t = 0; t < TL; ++t) {
-    const int x = X0 + 16 * t + li;
-    double chi = 0.0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int y = Y0 + 16 * wave + lg + 4 * j;
-      if (x < c.nx && y < c.ny) {
-        const size_t p = size_t(y) * c.nx + x;
-        const double m = acc[t][j];
-        if (out) AT(out, size_t(img) * c.nx * c.ny + p) = m;
-        if (partial) chi += chi2_pixel<double>(c, p, m, img);
-        if (c.gout) AT(static_cast<double *>(c.gout), size_t(img) * c.nx * c.ny + p) = dlogl_dm(c, p, m, img);
-      }
-    }
-    if (partial) {
-      for (int off = 32; off > 0; off >>= 1) chi += __shfl_xor(chi, off, 64);
-      const int tx16 = (X0 >> 4) + t;
       if (lane == 0 && 16 * tx16 < c.nx && 16 * ty16 < c.ny)
         AT(partial, size_t(img) * n16 + size_t(ty16) * n16x + tx16) = chi;
     }
@@ -3528,7 +3565,8 @@ size_t conv_smem(int kx, int kyp, int ty = ConvTile<T>::TY) {
 
 // conv_kernel over n_img images (c.n_tiles_x is set here, the tile count goes
 // to *n_tiles): 64-row tiles where their LDS fits (four waves a block, a
-// smaller share of halo rows), 32-row tiles otherwise.
+// smaller share of halo rows), 32-row tiles otherwise.  FP64 images go to
+// conv_f64_kernel as long as its tile fits the LDS.
 template <typename T, int TY, bool LW>
 int launch_conv_tile(const ConvArgs &c, dim3 grid, size_t smem, const T *in, const double *kf, T *out,
                      double *partial, hipStream_t st) {
@@ -3541,9 +3579,45 @@ int launch_conv_tile(const ConvArgs &c, dim3 grid, size_t smem, const T *in, con
   return check_launch("conv_kernel");
 }
 
+template <int R, int H, int CLS, bool GW>
+int launch_conv_f64(ConvArgs c, int n_img, const double *in, const double *kf, double *out, double *partial,
+                    int *n_tiles, hipStream_t st) {
+  const size_t smem = conv_f64_smem(c.kx, c.ky, R, H, CLS, GW);
+  c.n_tiles_x = (c.nx + 31) / 32;
+  *n_tiles = c.n_tiles_x * ((c.ny + 15) / 16);
+  if (smem > 65536) {  // dynamic LDS beyond 64 KB needs the kernel attribute raised first
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&conv_f64_kernel<R, H, CLS, GW>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, int(smem));
+    if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(conv_f64_kernel)");
+  }
+  const dim3 grid(c.n_tiles_x * ((c.ny + 2 * R * H - 1) / (2 * R * H)), n_img);
+  conv_f64_kernel<R, H, CLS, GW><<<grid, 64 * CLS * H, smem, st>>>(c, conv_f64_rows(c.ky, R, H), in, kf, out, partial);
+  return check_launch("conv_f64_kernel");
+}
+
 template <typename T>
 int launch_conv_kernel(ConvArgs c, int n_img, const T *in, const double *kf, T *out, double *partial,
                        int *n_tiles, hipStream_t st) {
+  if constexpr (sizeof(T) == sizeof(double)) {
+    // conv_f64_kernel by the number of 32 x 32 tiles (fewer than CUs: short
+    // tiles, weights in LDS) and its LDS; classes of kernel columns by the
+    // kernel alone, so that an image's sums are the same in any batch: below
+    // ten columns the split's barriers cost more than the work it shares (5 x
+    // 5, 64 images of 180^2, 57.5 against 67.7 us a call; 11 x 11 73 in both,
+    // one image of 60^2 19.4 against 21.5).  One block of 82 KB LDS or more
+    // fills a CU: there two row groups of waves (81 x 81, 743 against 918 us).
+    const bool few = size_t((c.nx + 31) / 32) * ((c.ny + 31) / 32) * n_img < 256;
+    auto fits = [&](int r, int h, int cls, bool gw, size_t lds) {
+      return conv_f64_smem(c.kx, c.ky, r, h, cls, gw) <= lds;
+    };
+#define LENSIM_CONV(R, H, CLS, GW) launch_conv_f64<R, H, CLS, GW>(c, n_img, in, kf, out, partial, n_tiles, st)
+    if (c.kx < 10 && fits(8, 4, 1, true, kMaxLds / 2) && fits(4, 4, 1, false, kMaxLds))
+      return few ? LENSIM_CONV(4, 4, 1, false) : LENSIM_CONV(8, 4, 1, true);
+    if (few && fits(4, 2, 4, false, kMaxLds)) return LENSIM_CONV(4, 2, 4, false);
+    if (fits(16, 1, 4, true, kMaxLds / 2)) return LENSIM_CONV(16, 1, 4, true);
+    if (fits(16, 2, 4, true, kMaxLds)) return LENSIM_CONV(16, 2, 4, true);
+#undef LENSIM_CONV
+  }
   constexpr int TX = ConvTile<T>::TX;
   int ty = ConvTile<T>::TY;
   if (conv_smem<T>(c.kx, c.kyp, 64) <= kMaxLds) ty = 64;
@@ -3595,40 +3669,6 @@ int launch_conv_mfma_tl(const ConvArgs &c, int tl, dim3 grid, const float *in, c
   }
 }
 
-// Whether the FP64 form convolves on the matrix cores (kernels of at least
-// 21 x 21 whose tile fits the LDS; smaller ones use the direct stencil).
-template <typename T>
-bool use_mf64(bool identity, int kx, int ky) {
-  if (sizeof(T) != sizeof(double) || identity) return false;
-  return kx >= 21 && ky >= 21 && mf64_smem(kx, ky, 2) <= kMaxLds;
-}
-
-template <int TL>
-int launch_conv_mf64_n(const ConvArgs &c, dim3 grid, const double *in, const double *frag, double *out,
-                       double *partial, hipStream_t st) {
-  const size_t smem = mf64_smem(c.kx, c.ky, TL);
-  if (smem > 65536) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&conv_mf64_kernel<TL>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, int(smem));
-    if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(conv_mf64_kernel)");
-  }
-  conv_mf64_kernel<TL><<<grid, 256, smem, st>>>(c, mf64_ls(c.kx, TL), mf64_nk4(c.kx), in, frag, out, partial);
-  return check_launch("conv_mf64_kernel");
-}
-
-int launch_conv_mf64(ConvArgs c, const MfmaPlan &pl, int n_img, const double *in, const double *frag, double *out,
-                     double *partial, hipStream_t st) {
-  if (pl.tl == 0) return fail(LENSIM_EUNSUPPORTED, "psf %dx%d exceeds the float64 matrix-core tile's LDS", c.ky, c.kx);
-  c.n_tiles_x = pl.n_tiles_x;
-  const dim3 grid(pl.n_tiles, n_img);
-  switch (pl.tl) {
-    case 2: return launch_conv_mf64_n<2>(c, grid, in, frag, out, partial, st);
-    case 3: return launch_conv_mf64_n<3>(c, grid, in, frag, out, partial, st);
-    case 4: return launch_conv_mf64_n<4>(c, grid, in, frag, out, partial, st);
-    default: return fail(LENSIM_EINVAL, "matrix-core tile width %d", pl.tl);
-  }
-}
-
 // The MFMA convolution of n_img images by plan pl (c.kx, c.ky, c.edge set;
 // c.n_tiles_x is set here).
 int launch_conv_mfma(ConvArgs c, const MfmaPlan &pl, int n_img, const float *in, const int *hdr, const half8 *frag,
@@ -3646,31 +3686,26 @@ int launch_conv_mfma(ConvArgs c, const MfmaPlan &pl, int n_img, const float *in,
 }
 
 // The PSF preparation of a call on the grid itself, and which convolution it is
-// for (at most one of mfma, mf64).
+// for.
 template <typename T>
 struct ConvChoice {
-  bool mfma, mf64;
+  bool mfma;
   PsfJob job;
   ConvChoice(const lensim_psf *psf, unsigned flags, int kx, int ky, unsigned char *ws, const Layout &L) {
     const bool identity = !psf || psf->type == LENSIM_PSF_NONE || (flags & LENSIM_IMAGE_UNCONVOLVED);
     mfma = use_mfma<T>(identity, kx, ky);
-    mf64 = use_mf64<T>(identity, kx, ky);
     job = PsfJob{};
-    job.mode = mfma ? 2 : (mf64 ? 3 : 1);
+    job.mode = mfma ? 2 : 1;
     job.k = identity ? nullptr : psf->d_kernel;
     job.kx = kx;
     job.ky = ky;
     job.kyp = kyp_of(ky);
-    job.kt = reinterpret_cast<double *>(ws + (mf64 ? L.bfrag : L.psf));
+    job.kt = reinterpret_cast<double *>(ws + L.psf);
     job.hdr = reinterpret_cast<int *>(ws + L.bfrag);
     job.frag = reinterpret_cast<half8 *>(ws + L.bfrag + 16);
     if (mfma) {
       job.nks = mfma_nks(kx);
       job.n_steps = mfma_steps(kx, ky);
-    }
-    if (mf64) {
-      job.nks = mf64_nk4(kx);
-      job.n_steps = mf64_steps(kx, ky);
     }
   }
 };
@@ -3695,15 +3730,11 @@ int launch_prep_psf(const ModelArgs &m, const double *params, int n_img, const P
 template <typename T>
 int launch_conv(const ConvArgs &c, const ConvChoice<T> &cc, int n_img, const T *in, const float *blkmax, T *out,
                 double *partial, int *n_tiles, hipStream_t st) {
-  if (!cc.mfma && !cc.mf64) return launch_conv_kernel<T>(c, n_img, in, cc.job.kt, out, partial, n_tiles, st);
+  if (!cc.mfma) return launch_conv_kernel<T>(c, n_img, in, cc.job.kt, out, partial, n_tiles, st);
   *n_tiles = n16_tiles(c.nx, c.ny);  // chi^2 partials of the 16 x 16 output tiles
-  if (cc.mfma)
-    return launch_conv_mfma(c, mfma_plan(c.nx, c.ny, n_img, c.kx, c.ky), n_img, reinterpret_cast<const float *>(in),
-                            cc.job.hdr, cc.job.frag, blkmax, (c.nx * c.ny + 255) / 256, reinterpret_cast<float *>(out),
-                            partial, st);
-  return launch_conv_mf64(c, mfma_plan(c.nx, c.ny, n_img, c.kx, c.ky, true), n_img,
-                          reinterpret_cast<const double *>(in), cc.job.kt, reinterpret_cast<double *>(out), partial,
-                          st);
+  return launch_conv_mfma(c, mfma_plan(c.nx, c.ny, n_img, c.kx, c.ky), n_img, reinterpret_cast<const float *>(in),
+                          cc.job.hdr, cc.job.frag, blkmax, (c.nx * c.ny + 255) / 256, reinterpret_cast<float *>(out),
+                          partial, st);
 }
 
 // The image pipeline shared by lensim_image and lensim_loglike.

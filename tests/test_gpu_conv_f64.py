@@ -1,0 +1,68 @@
+"""The FP64 form's convolution (conv_f64_kernel in csrc/lensim.hip) against the
+oracle at every remainder of its groups of eight kernel rows, at the kernel
+sizes where its block shape changes, on ragged tiles, in both PSF modes, and
+the same bits from a few images as from a large batch."""
+
+import numpy as np
+import pytest
+import torch
+
+from jaxtronomy_amd import backend
+from jaxtronomy_amd import workloads as W
+from jaxtronomy_amd.Data.imaging_data import ImageData
+from jaxtronomy_amd.Data.psf import PSF
+from jaxtronomy_amd.ImSim.image_model import ImageModel
+from jaxtronomy_amd.LensModel.lens_model import LensModel
+from jaxtronomy_amd.LightModel.light_model import LightModel
+from oracle import lensim_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+LENS = [dict(theta_E=0.9, e1=0.1, e2=-0.06, center_x=0.02, center_y=-0.01)]
+SOURCE = [dict(amp=20.0, R_sersic=0.4, n_sersic=1.5, center_x=0.05, center_y=0.03)]
+
+
+def model(num_pix, psf, data=None):
+    cfg = dict(W.EPL180, numPix=num_pix, deltaPix=3.2 / num_pix, supersampling=1)
+    return cfg, ImageModel(ImageData(**W.data_kwargs(cfg, data)), psf, LensModel(["SIE"]), LightModel(["SERSIC"]),
+                           kwargs_numerics={"supersampling_factor": 1})
+
+
+def batches(im, n):
+    params, _ = im.pack(LENS, SOURCE)
+    params = np.repeat(params, n, axis=0)
+    params[:, 0, 0] *= 1.0 + 0.001 * np.arange(n)
+    return backend.to_device_f64(params)
+
+
+@pytest.mark.parametrize("num_pix", [7, 33, 50])
+@pytest.mark.parametrize("ky,kx", [(k, k) for k in (1, 3, 5, 7, 9, 11, 13, 15, 17, 31, 41, 61, 83, 91)] +
+                         [(41, 5), (5, 41), (23, 9)])
+def test_pixel_kernel_vs_oracle(ky, kx, num_pix):
+    """Positive terms, at most 8281 of them: the sum rounds to 1e-12, the rays under it to the library's FP64 bar."""
+    k = max(ky, kx)
+    kernel = W.moffat_kernel(k, 3.0, 2.0) + 0.1 * np.random.default_rng(k).random((k, k)) / k**2
+    kernel = kernel[(k - ky) // 2:(k + ky) // 2, (k - kx) // 2:(k + kx) // 2]
+    kernel /= kernel.sum()
+    cfg, im = model(num_pix, PSF("PIXEL", kernel_point_source=kernel))
+    want = O.image(W.grid_dict(cfg), ["SIE"], LENS, ["SERSIC"], SOURCE, [], [], kernel=kernel)
+    few = im.image_batch(batches(im, 2), 2)
+    assert np.max(np.abs(few[0].cpu().numpy() - want)) <= 1e-10 * np.max(want)
+    im = model(num_pix, PSF("PIXEL", kernel_point_source=kernel), 1.01 * want)[1]
+    n = 256 // ((num_pix + 31) // 32) ** 2 + 3
+    params = batches(im, n)
+    many = im.image_batch(params, n)
+    logl = im.likelihood_batch(params, n)
+    for i in (0, 1):
+        assert torch.equal(many[i], few[i])
+    assert torch.equal(logl[:2], im.likelihood_batch(params[:2].contiguous(), 2))
+
+
+@pytest.mark.parametrize("num_pix", [5, 37])
+def test_gaussian_edge_mode_vs_oracle(num_pix):
+    psf = PSF("GAUSSIAN", fwhm=0.3, truncation=4)
+    cfg, im = model(num_pix, psf)
+    flat = model(num_pix, PSF("NONE"))[1].image_batch(batches(im, 1), 1)[0].cpu().numpy()
+    want = O.convolve_same(flat, im.kernel, mode="edge")
+    got = im.image_batch(batches(im, 1), 1)[0].cpu().numpy()
+    assert np.max(np.abs(got - want)) <= 1e-12 * np.max(want)
