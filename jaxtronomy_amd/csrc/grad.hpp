@@ -312,17 +312,41 @@ __device__ __forceinline__ T sersic_ellipse_grad(const double *p, T x, T y, T *g
 //    (-1/(1+q) + t (1/(2q) - q x^2/R^2)) dq;
 //  * theta_E, the centre and the orientation as in epl_dalpha's comment, the
 //    Hessian with 1/r^2 alone.
-__device__ __forceinline__ void epl_dalpha_f64(const double *rd, const double *__restrict__ c,
-                                               const double *__restrict__ dc, const double *pk, double x, double y,
-                                               double &a_x, double &a_y, double *dax, double *day) {
+// epl_basis_f64 gives alpha, d/dt and d/dq of it, its derivative by the angle
+// and by the centre (x and y components in ax[], ay[]); the kwargs' derivatives
+// are linear in these with factors of the kwargs alone (EllKw, epl_kw): sums
+// over rays are taken of the basis.
+struct EllKw {
+  double dp1, dp2, dq1, dq2;  // d phi and d q by e1 and e2
+  double q0;                  // the unclamped q
+  EllKw() = default;
+  __device__ __forceinline__ EllKw(double e1, double e2) {
+    const double c2 = e1 * e1 + e2 * e2, ce = ::sqrt(c2);
+    const double cc = ce < 0.9999 ? ce : 0.9999, h = 0.5 / c2;
+    q0 = (1.0 - cc) / (1.0 + cc);
+    dp1 = -e2 * h;
+    dp2 = e1 * h;
+    const double dqdc = ce < 0.9999 ? -2.0 / ((1.0 + ce) * (1.0 + ce)) : 0.0;
+    dq1 = dqdc * e1 / ce;
+    dq2 = dqdc * e2 / ce;
+  }
+};
+__device__ __forceinline__ void epl_kw(const EllKw &ek, const double *rd, const double *pk, double *v) {
+  const double q = v[2], ph = v[3];
+  v[0] *= pk[0] != 0.0 ? rd[EPL_T] / pk[0] : 0.0;
+  v[2] = q * ek.dq1 + ph * ek.dp1;
+  v[3] = q * ek.dq2 + ph * ek.dp2;
+}
+__device__ __forceinline__ void epl_basis_f64(const double *rd, const double *__restrict__ c,
+                                              const double *__restrict__ dc, double x, double y, double *ax,
+                                              double *ay) {
   const double q = rd[EPL_Q], t = rd[EPL_T], f = rd[EPL_F], cs = rd[EPL_C], sn = rd[EPL_S];
   const double dx = x - rd[R_CX], dy = y - rd[R_CY];
   const double xr = dx * cs + dy * sn, yr = dy * cs - dx * sn;
   const double Zr = q * xr, Zi = yr;
   const double R2 = Zr * Zr + Zi * Zi;
-  a_x = a_y = 0.0;
 #pragma unroll
-  for (int i = 0; i < 6; ++i) dax[i] = day[i] = 0.0;
+  for (int i = 0; i < 6; ++i) ax[i] = ay[i] = 0.0;
   if (R2 == 0.0) return;  // the reference's NaN at Z = 0 becomes 0 (epl.py:391-392)
   const bool rfree = R2 >= 1e-18;  // the floor R >= 1e-9 passes no derivative
   const double R2c = rfree ? R2 : 1e-18;
@@ -364,14 +388,12 @@ __device__ __forceinline__ void epl_dalpha_f64(const double *rd, const double *_
   const double ls = -1.0 / (1.0 + q) + t * (0.5 / q - (rfree ? q * xr * xr * iR2 : 0.0));
   const double sx = s * xr;
   const double aqr = fma(ls, fr, fma(sx, Fr, sZr * gr - sZi * gi)), aqi = fma(ls, fi, fma(sx, Fi, sZr * gi + sZi * gr));
-  a_x = fr * cs - fi * sn;
-  a_y = fr * sn + fi * cs;
-  const double thetaE = pk[0], dth = thetaE != 0.0 ? t / thetaE : 0.0;
-  dax[0] = a_x * dth;
-  day[0] = a_y * dth;
-  dax[1] = atr * cs - ati * sn;
-  day[1] = atr * sn + ati * cs;
-  const double qx = aqr * cs - aqi * sn, qy = aqr * sn + aqi * cs;
+  ax[0] = fr * cs - fi * sn;
+  ay[0] = fr * sn + fi * cs;
+  ax[1] = atr * cs - ati * sn;
+  ay[1] = atr * sn + ati * cs;
+  ax[2] = aqr * cs - aqi * sn;
+  ay[2] = aqr * sn + aqi * cs;
   // Hessian: kappa and the shear of EPLMajorAxis.hessian, rotated back
   const double x2 = xr * xr, y2 = yr * yr, ir2 = rcp_full(x2 + y2);
   const double kappa = 0.5 * (2.0 - t) * pw;
@@ -380,19 +402,21 @@ __device__ __forceinline__ void epl_dalpha_f64(const double *rd, const double *_
   const double c2p = cs * cs - sn * sn, s2p = 2.0 * sn * cs;
   const double G1 = c2p * g1 - s2p * g2, fxy = s2p * g1 + c2p * g2;
   const double fxx = kappa + G1, fyy = kappa - G1;
-  const double dphx = fxx * dy - fxy * dx - a_y, dphy = fxy * dy - fyy * dx + a_x;
-  const double e1 = pk[2], e2 = pk[3], c2 = e1 * e1 + e2 * e2, ce = ::sqrt(c2);
-  const double h = 0.5 / c2, dp1 = -e2 * h, dp2 = e1 * h;
-  const double dqdc = ce < 0.9999 ? -2.0 / ((1.0 + ce) * (1.0 + ce)) : 0.0;
-  const double dq1 = dqdc * e1 / ce, dq2 = dqdc * e2 / ce;
-  dax[2] = qx * dq1 + dphx * dp1;
-  day[2] = qy * dq1 + dphy * dp1;
-  dax[3] = qx * dq2 + dphx * dp2;
-  day[3] = qy * dq2 + dphy * dp2;
-  dax[4] = -fxx;
-  day[4] = -fxy;
-  dax[5] = -fxy;
-  day[5] = -fyy;
+  ax[3] = fxx * dy - fxy * dx - ay[0];
+  ay[3] = fxy * dy - fyy * dx + ax[0];
+  ax[4] = -fxx;
+  ax[5] = ay[4] = -fxy;
+  ay[5] = -fyy;
+}
+__device__ __forceinline__ void epl_dalpha_f64(const double *rd, const double *__restrict__ c,
+                                               const double *__restrict__ dc, const double *pk, double x, double y,
+                                               double &a_x, double &a_y, double *dax, double *day) {
+  epl_basis_f64(rd, c, dc, x, y, dax, day);
+  a_x = dax[0];
+  a_y = day[0];
+  const EllKw ek(pk[2], pk[3]);
+  epl_kw(ek, rd, pk, dax);
+  epl_kw(ek, rd, pk, day);
 }
 
 // The SIE / NIE's alpha at (x, y) and its derivatives by (theta_E, e1, e2[,
@@ -400,16 +424,24 @@ __device__ __forceinline__ void epl_dalpha_f64(const double *rd, const double *_
 // / sq, sq = sqrt(1 - q^2), A = arctan(sq x / D1), B = arctanh(sq y / D2), D1 =
 // psi + s, D2 = psi + q^2 s, psi^2 = q^2 (s^2 + x^2) + y^2, with b = theta_E
 // sqrt(q) and s = s_scale / sqrt(q) (nie.py:182-200, :280-295).
+// nie_basis_f64: alpha, d/dq, the derivative by the angle, for a NIE by s, and
+// by the centre; nie_kw as epl_kw.
 template <int TYPE>
-__device__ __forceinline__ void nie_dalpha_f64(const double *rd, const double *pk, double x, double y, double &a_x,
-                                               double &a_y, double *dax, double *day) {
+__device__ __forceinline__ void nie_kw(const EllKw &ek, const double *pk, double *v) {
+  const double q = v[1], ph = v[2];
+  v[0] *= pk[0] != 0.0 ? 1.0 / pk[0] : 0.0;
+  v[1] = q * ek.dq1 + ph * ek.dp1;
+  v[2] = q * ek.dq2 + ph * ek.dp2;
+  if constexpr (TYPE == LENSIM_NIE) v[3] *= rsq_full(ek.q0);  // s = s_scale / sqrt(q)
+}
+template <int TYPE>
+__device__ __forceinline__ void nie_basis_f64(const double *rd, double q0, double x, double y, double *ax,
+                                              double *ay) {
   constexpr bool kNie = TYPE == LENSIM_NIE;
   constexpr int kc = kNie ? 4 : 3;  // the centre's slots
   const double q = rd[NIE_Q], q2 = rd[NIE_Q2], s = rd[NIE_SS], sq = rd[NIE_SQ], k = rd[NIE_BSQ], cs = rd[NIE_C],
                sn = rd[NIE_S];
-  const double e1 = pk[1], e2 = pk[2], c2 = e1 * e1 + e2 * e2, ce = ::sqrt(c2);
-  const double cc = ce < 0.9999 ? ce : 0.9999, q0 = (1.0 - cc) / (1.0 + cc);  // unclamped q: b, s
-  const bool qfree = q0 < 1.0;                                              // else the frame's q is a constant
+  const bool qfree = q0 < 1.0;  // else the frame's q is a constant
   const double dx = x - rd[R_CX], dy = y - rd[R_CY];
   const double xr = dx * cs + dy * sn, yr = dy * cs - dx * sn;
   const double p2 = fma(q2, fma(s, s, xr * xr), yr * yr);
@@ -419,8 +451,8 @@ __device__ __forceinline__ void nie_dalpha_f64(const double *rd, const double *p
   const double u1 = sq * xr * i1, u2 = sq * yr * i2;
   const double A = atan_dbl(u1), B = atanh_dbl(u2);
   const double fx = k * A, fy = k * B;
-  a_x = fx * cs - fy * sn;
-  a_y = fx * sn + fy * cs;
+  ax[0] = fx * cs - fy * sn;
+  ay[0] = fx * sn + fy * cs;
   // k dA = k1 d(x / D1 sq) and k dB = k2 d(y / D2 sq)
   const double k1 = k * rcp_full(fma(u1, u1, 1.0)), k2 = k * rcp_full(fma(-u2, u2, 1.0));
   const double px = q2 * xr * ip, py = yr * ip, ps = q2 * s * ip, pq = q * fma(s, s, xr * xr) * ip;
@@ -429,39 +461,39 @@ __device__ __forceinline__ void nie_dalpha_f64(const double *rd, const double *p
   const double ayx = -w2 * yr * px * i2, ayy = w2 * (1.0 - yr * py * i2);
   const double axs = -w1 * xr * (ps + 1.0) * i1, ays = -w2 * yr * (ps + q2) * i2;
   // q: through k, sq and psi (the frame's q), and through b and s = s_scale / sqrt(q)
-  const double isq2 = 1.0 / (sq * sq), iq0 = 0.5 / q0;
+  const double isq2 = rcp_full(sq * sq), iq0 = 0.5 * rcp_full(q0);
   double qxr = iq0 * fma(-s, axs, fx), qyr = iq0 * fma(-s, ays, fy);
   if (qfree) {
     qxr += q * isq2 * (fx - w1 * xr) - w1 * xr * pq * i1;
     qyr += q * isq2 * (fy - w2 * yr) - w2 * yr * fma(2.0 * q, s, pq) * i2;
   }
-  const double ith = pk[0] != 0.0 ? 1.0 / pk[0] : 0.0;
-  dax[0] = a_x * ith;
-  day[0] = a_y * ith;
   // H = R (d alpha / d(xr, yr)) R^T
   const double mxx = axx * cs - ayx * sn, mxy = axy * cs - ayy * sn, myx = axx * sn + ayx * cs,
                myy = axy * sn + ayy * cs;
   const double hxx = mxx * cs - mxy * sn, hxy = mxx * sn + mxy * cs, hyx = myx * cs - myy * sn,
                hyy = myx * sn + myy * cs;
-  const double dphx = hxx * dy - hxy * dx - a_y, dphy = hyx * dy - hyy * dx + a_x;
-  const double h = 0.5 / c2, dp1 = -e2 * h, dp2 = e1 * h;
-  const double dqdc = ce < 0.9999 ? -2.0 / ((1.0 + ce) * (1.0 + ce)) : 0.0;
-  const double dq1 = dqdc * e1 / ce, dq2 = dqdc * e2 / ce;
-  const double qx = qxr * cs - qyr * sn, qy = qxr * sn + qyr * cs;
-  dax[1] = qx * dq1 + dphx * dp1;
-  day[1] = qy * dq1 + dphy * dp1;
-  dax[2] = qx * dq2 + dphx * dp2;
-  day[2] = qy * dq2 + dphy * dp2;
-  if constexpr (kNie) {  // s = s_scale / sqrt(q)
-    const double isq = rsq_full(q0);
-    const double sx = axs * isq, sy = ays * isq;
-    dax[3] = sx * cs - sy * sn;
-    day[3] = sx * sn + sy * cs;
+  ax[1] = qxr * cs - qyr * sn;
+  ay[1] = qxr * sn + qyr * cs;
+  ax[2] = hxx * dy - hxy * dx - ay[0];
+  ay[2] = hyx * dy - hyy * dx + ax[0];
+  if constexpr (kNie) {
+    ax[3] = axs * cs - ays * sn;
+    ay[3] = axs * sn + ays * cs;
   }
-  dax[kc] = -hxx;
-  day[kc] = -hyx;
-  dax[kc + 1] = -hxy;
-  day[kc + 1] = -hyy;
+  ax[kc] = -hxx;
+  ay[kc] = -hyx;
+  ax[kc + 1] = -hxy;
+  ay[kc + 1] = -hyy;
+}
+template <int TYPE>
+__device__ __forceinline__ void nie_dalpha_f64(const double *rd, const double *pk, double x, double y, double &a_x,
+                                               double &a_y, double *dax, double *day) {
+  const EllKw ek(pk[1], pk[2]);
+  nie_basis_f64<TYPE>(rd, ek.q0, x, y, dax, day);
+  a_x = dax[0];
+  a_y = day[0];
+  nie_kw<TYPE>(ek, pk, dax);
+  nie_kw<TYPE>(ek, pk, day);
 }
 
 // The NFW's alpha = a (dx, dy) at (x, y), a = 4 rho0 Rs g / u, u = X^2, and its
@@ -542,6 +574,66 @@ __device__ __forceinline__ double sersic_ellipse_grad_f64(const double *rd, cons
   gp[6] = -gy;
   return aE;
 }
+// Sums over rays of w times sersic_ellipse_grad_f64's derivatives, from a
+// profile's constants read once: with k = (d flux / d ln R) / R^2 the
+// derivatives by e1, e2 and the centre are linear in the moments of k about the
+// centre, and those by R_sersic and n in three sums, so a ray adds nine numbers
+// and the kwargs' factors are applied to the sums (kwargs()).
+struct SersicGrad {
+  double cx, cy, m00, m01, m11, a, b, c, amp, lnrs, invn, k2, bnin, r2max;
+  double se = 0.0, sc = 0.0, sl = 0.0, su = 0.0, kx = 0.0, ky = 0.0, kxx = 0.0, kxy = 0.0, kyy = 0.0;
+  __device__ __forceinline__ explicit SersicGrad(const double *rd)
+      : cx(wave_uniform(rd[R_CX])), cy(wave_uniform(rd[R_CY])), m00(wave_uniform(rd[SE_M00])),
+        m01(wave_uniform(rd[SE_M01])), m11(wave_uniform(rd[SE_M11])), amp(wave_uniform(rd[SE_AMP])),
+        lnrs(wave_uniform(rd[SE_LNRS] * 1.4426950408889634)), invn(wave_uniform(rd[SE_INVN])),
+        k2(wave_uniform(rd[SE_K2])), bnin(wave_uniform(rd[SE_BN] * rd[SE_INVN])), r2max(wave_uniform(rd[SE_R2MAX])) {
+    a = wave_uniform(m00 * m00 + m01 * m01);
+    b = wave_uniform(m01 * (m00 + m11));
+    c = wave_uniform(m01 * m01 + m11 * m11);
+  }
+  // the ray at (x, y) with weight w; (gx, gy): d flux / d(x, y)
+  __device__ __forceinline__ void add(double x, double y, double w, double &gx, double &gy) {
+    const double dx = x - cx, dy = y - cy;
+    const double xe = m00 * dx + m01 * dy, ye = m01 * dx + m11 * dy;
+    const double R2 = fma(xe, xe, ye * ye);
+    const bool rfree = R2 >= 1e-8;
+    const double R2c = rfree ? R2 : 1e-8;
+    gx = gy = 0.0;
+    if (!(R2c <= r2max)) return;
+    const double l2 = fma(0.5, log2_pos(R2c), -lnrs) * invn;  // log2(frac) / n
+    const double u = exp2_fin(l2);
+    const double E = exp2_fin(k2 * (1.0 - u)), aE = amp * E;
+    const double d = -aE * bnin * u, wd = w * d;  // d flux / d ln(frac)
+    se = fma(w, E, se);
+    sc += wd;
+    sl = fma(wd, l2, sl);
+    su = fma(w * aE, u - 1.0, su);
+    const double k = rfree ? d * rcp_full(R2c) : 0.0, wx = w * k * dx, wy = w * k * dy;
+    gx = k * fma(a, dx, b * dy);
+    gy = k * fma(b, dx, c * dy);
+    kx += wx;
+    ky += wy;
+    kxx = fma(wx, dx, kxx);
+    kxy = fma(wx, dy, kxy);
+    kyy = fma(wy, dy, kyy);
+  }
+  __device__ __forceinline__ void kwargs(const double *rd, const double *p, double *acc) const {
+    const double e1 = p[3], e2 = p[4], v = 1.0 - e1 * e1 - e2 * e2, sq = ::sqrt(fabs(v));
+    const bool nfree = sq >= 0.000001, sfree = p[1] >= 0.0001, bfree = 1.9992 * p[2] - 0.3271 >= 0.00001;
+    const double inorm = 1.0 / (nfree ? sq : 0.000001), sg = v >= 0.0 ? 1.0 : -1.0;
+    const double dn1 = nfree ? -sg * e1 * inorm : 0.0, dn2 = nfree ? -sg * e2 * inorm : 0.0;
+    const double sr = a * kxx + 2.0 * b * kxy + c * kyy;  // sum of k R^2
+    acc[0] = se;
+    acc[1] = sfree ? -sc * rd[SE_IRS] : 0.0;
+    acc[2] = -0.6931471805599453 * sl - (bfree ? 1.9992 * su : 0.0);
+    acc[3] = (m11 * kyy - m00 * kxx - dn1 * sr) * inorm;
+    acc[4] = (-(m00 * kxy + m01 * kyy) - (m01 * kxx + m11 * kxy) - dn2 * sr) * inorm;
+    acc[5] = -(a * kx + b * ky);
+    acc[6] = -(b * kx + c * ky);
+    acc[7] = 0.0;
+  }
+};
+
 template <typename T>
 __device__ __forceinline__ T sersic_ellipse_grad_rec(const double *rd, const double *p, T x, T y, T *gp, T &gx, T &gy) {
   if constexpr (sizeof(T) == sizeof(double)) return sersic_ellipse_grad_f64(rd, p, x, y, gp, gx, gy);

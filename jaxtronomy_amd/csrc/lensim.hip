@@ -2825,7 +2825,8 @@ __device__ __forceinline__ void lens_ray_grad(const ModelArgs &m, const GradArgs
 // and the double closed forms of NFW / TNFW, would spill.  What bounds it in
 // FP64 is the vector unit's instructions: the closed forms of grad.hpp in place
 // of duals took 64 images of 120^2 (EPL + SHEAR, Sersic source and light) from
-// 620 to 411 us a call.
+// 620 to 411 us a call, sums of their bases with the kwargs' factors applied
+// once a block (a square root and five divisions a ray less) from 391 to 351.
 template <typename T, int TYPE>
 constexpr int grad_waves_per_eu() {
   return (sizeof(T) == sizeof(float) && TYPE != LENSIM_NFW && TYPE != LENSIM_TNFW) ? 4 : 1;
@@ -2845,6 +2846,14 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
   double acc[LENSIM_NPARAM];
 #pragma unroll
   for (int q = 0; q < LENSIM_NPARAM; ++q) acc[q] = 0.0;
+  // FP64: sums of the closed forms' bases, whose factors of the kwargs alone are applied below
+  constexpr bool kF64 = sizeof(T) == sizeof(double);
+  constexpr bool kEll = kF64 && (type == LENSIM_EPL || type == LENSIM_SIE || type == LENSIM_NIE);
+  constexpr bool kSersic = kF64 && type == LENSIM_SERSIC_ELLIPSE;
+  const double *rd = rp.recd + k * kRec, *pk = ga.params + (size_t(img) * m.n_prof + k) * LENSIM_NPARAM;
+  CHECK_SPAN(pk, LENSIM_NPARAM * sizeof(double));
+  const gm::EllKw ek = kEll ? gm::EllKw(pk[type == LENSIM_EPL ? 2 : 1], pk[type == LENSIM_EPL ? 3 : 2]) : gm::EllKw();
+  std::conditional_t<kSersic, gm::SersicGrad, const double *> sersic(rd);
   for (int pp = 0; pp < kGradPix; ++pp) {
   const int pix0 = (blockIdx.x * kGradPix + pp) * blockDim.x + threadIdx.x;
   const bool active = pix0 < npix;
@@ -2875,7 +2884,41 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
                                                                             : nullptr;
       if (gb) CHECK_SPAN(gb, 2 * sizeof(T));
       if (bt) CHECK_SPAN(bt, 2 * sizeof(T));
-      if constexpr (type == LENSIM_EPL) lens_ray_grad<T, HALO>(m, ga, rp, img, k, x, y, w, acc, gb);
+      if constexpr (kEll) {
+        double bx[6], by[6];
+        const double lw = -m.alpha_scaling * w, lx = lw * double(AT(gb, 0)), ly = lw * double(AT(gb, 1));
+        if constexpr (type == LENSIM_EPL) {
+          const size_t co = (size_t(img) * m.n_epl + m.epl_index[k]) * LENSIM_EPL_NMAX;
+          CHECK_SPAN(ga.coefd + co, LENSIM_EPL_NMAX * sizeof(double));
+          CHECK_SPAN(ga.dcoefd + co, LENSIM_EPL_NMAX * sizeof(double));
+          gm::epl_basis_f64(rd, ga.coefd + co, ga.dcoefd + co, x, y, bx, by);
+        } else {
+          gm::nie_basis_f64<type>(rd, ek.q0, x, y, bx, by);
+        }
+#pragma unroll
+        for (int q = 0; q < n_params_of(type); ++q) acc[q] += fma(lx, bx[q], ly * by[q]);
+      } else if constexpr (kSersic) {
+        double px = x, py = y, gx, gy;
+        if (k < m.n_defl + m.n_source) {
+          if (bt) {
+            px = double(AT(bt, 0));
+            py = double(AT(bt, 1));
+          } else {
+            trace_ray<T, HALO, false>(m, rp, img, x, y, px, py);
+          }
+        }
+        sersic.add(px, py, w, gx, gy);
+        if (gb && !bt) {  // the first source's launch, for the lens launches
+          if (m.n_source > 1) {
+            const gm::Dual<T, 2> f2 = sources_at<T>(m, ga, rp, img, T(px), T(py));
+            gx = double(f2.d[0]);
+            gy = double(f2.d[1]);
+          }
+          AT(gb, 0) = T(gx);
+          AT(gb, 1) = T(gy);
+        }
+      }
+      else if constexpr (type == LENSIM_EPL) lens_ray_grad<T, HALO>(m, ga, rp, img, k, x, y, w, acc, gb);
       else if constexpr (type == LENSIM_SIE) lens_ray_grad<T, HALO, LENSIM_SIE>(m, ga, rp, img, k, x, y, w, acc, gb);
       else if constexpr (type == LENSIM_NIE) lens_ray_grad<T, HALO, LENSIM_NIE>(m, ga, rp, img, k, x, y, w, acc, gb);
       else if constexpr (type == LENSIM_NFW) nfw_ray_grad<T>(m, ga, rp, img, k, x, y, w, acc, gb);
@@ -2894,7 +2937,10 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
     }
   }
   }
-  if constexpr (type == LENSIM_TNFW) tnfw_grad_scale(rp.recd + k * kRec, acc);
+  if constexpr (type == LENSIM_TNFW) tnfw_grad_scale(rd, acc);
+  if constexpr (kEll && type == LENSIM_EPL) gm::epl_kw(ek, rd, pk, acc);
+  if constexpr (kEll && type != LENSIM_EPL) gm::nie_kw<type>(ek, pk, acc);
+  if constexpr (kSersic) sersic.kwargs(rd, pk, acc);
   // block sum of the 8 accumulators in a fixed order
   __shared__ double red[256 / 64][LENSIM_NPARAM];
 #pragma unroll
