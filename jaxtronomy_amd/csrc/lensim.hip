@@ -966,12 +966,12 @@ __device__ __forceinline__ void defl_fast(const Rec<T> &r, const T *coef_t, cons
 // other deflectors)).  The records hold the steps (prepare_record's
 // SubSteps).  In the float form each Sersic profile's values of a pixel are
 // summed in float and multiplied by its amplitude in double at the end.
-template <typename T, int D0, int D1, int NSRC, int NLL>
+template <typename T, int D0, int D1, int NSRC, int NLL, bool KEEP>
 __global__ __launch_bounds__(256) void render_fast_kernel(ModelArgs m, GridArgs g, const double *__restrict__ recd,
                                                           const float *__restrict__ recf,
                                                           const double *__restrict__ coefd,
                                                           const float *__restrict__ coeff, unsigned flags,
-                                                          T *__restrict__ out, float *__restrict__ blkmax) {
+                                                          double *__restrict__ beta, T *__restrict__ out, float *__restrict__ blkmax) {
   constexpr bool kF32 = sizeof(T) == sizeof(float);
   static_assert(NSRC == 1, "the compile-time render takes one source");
   const int img = blockIdx.y;
@@ -1060,6 +1060,11 @@ __global__ __launch_bounds__(256) void render_fast_kernel(ModelArgs m, GridArgs 
         defl_fast<T, D0>(r0, rp.coeft + co, rp.coefd + co, u0, asc, g, sr, bx, by);
         if constexpr (D1 == LENSIM_NIE || D1 == LENSIM_NFW)
           defl_fast<T, D1C>(r1, nullptr, nullptr, u1, asc, g, sr, bx, by);
+        if constexpr (KEEP) {  // for the gradient's source launch (MpKeep)
+          double *b = beta + ((size_t(img) * npix + pix) * size_t(g.s * g.s) + size_t(sy * g.s + sx)) * 2;
+          AT(b, 0) = bx + rds[R_CX];
+          AT(b, 1) = by + rds[R_CY];
+        }
         // (bx, by) = beta - c_source
         const double xs = fma(rds[SE_M00S], bx, rds[SE_M01S] * by);
         const double ys = fma(rds[SE_M01S], bx, rds[SE_M11S] * by);
@@ -1130,7 +1135,8 @@ __global__ __launch_bounds__(256) void block_max_kernel(const T *__restrict__ v,
 constexpr int kMpBlock = 64;  // rays of a block of the multi-plane kernels (a lane each)
 // What a gradient keeps of its render for the adjoint kernels, so that the
 // rays are not traced again: several planes, per ray and run the position, and
-// beta; a bulk list that render_bulk_kernel takes, beta.
+// beta; a bulk list that render_bulk_kernel takes, or in FP64 a model that
+// render_fast_kernel takes, beta.
 struct MpKeep {
   double4 *store;
   size_t per_img;
@@ -1148,21 +1154,14 @@ int launch_render_bulk(const ModelArgs &m, const GridArgs &g, const double *recd
                        const double *coefd, const float *coeff, unsigned flags, const MpKeep &keep, T *out, int n_img,
                        hipStream_t st);
 
-// Launches render_fast_kernel when the model is one of its compile-time lists
-// (EPL, SIE / NIE or NFW, each with or without SHEAR after it, NFW + SIE / NIE
-// in either order; one Sersic source, none or one Sersic lens light),
-// render_mp_kernel for several planes (tab: its plane runs),
-// render_bulk_kernel for a bulk list over few pixels, else render_kernel.
+// Whether render_fast_kernel has the model (see launch_render); its deflectors.
 template <typename T>
-int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf, const double *coefd,
-                  const float *coeff, const int *tab, unsigned flags, const MpKeep &keep, T *out, float *blkmax,
-                  int n_img, hipStream_t st) {
-  const dim3 rgrid((g.nx * g.ny + 255) / 256, n_img);
+bool fast_model(const ModelArgs &m, unsigned flags, int &d0, int &d1) {
   auto sersic = [](int t) { return t == LENSIM_SERSIC || t == LENSIM_SERSIC_ELLIPSE; };
   auto nie = [](int t) { return t == LENSIM_SIE ? LENSIM_NIE : t; };
   bool fast = m.mp_n == 0 && m.n_bulk == 0 && (m.n_lens == 1 || m.n_lens == 2) && m.n_source == 1 &&
               (m.n_light == 0 || m.n_light == 1);
-  int d0 = 0, d1 = 0;
+  d0 = d1 = 0;
   if (fast) {
     d0 = nie(m.types[0]);
     d1 = m.n_lens == 2 ? nie(m.types[1]) : 0;
@@ -1178,6 +1177,21 @@ int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, con
     fast = fast && (sersic(ts) || (f64 && ts == LENSIM_NULL && !(flags & LENSIM_IMAGE_SOURCE))) &&
            (sersic(tl) || m.n_light == 0 || (f64 && tl == LENSIM_NULL));
   }
+  return fast;
+}
+
+// Launches render_fast_kernel when the model is one of its compile-time lists
+// (EPL, SIE / NIE or NFW, each with or without SHEAR after it, NFW + SIE / NIE
+// in either order; one Sersic source, none or one Sersic lens light),
+// render_mp_kernel for several planes (tab: its plane runs),
+// render_bulk_kernel for a bulk list over few pixels, else render_kernel.
+template <typename T>
+int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf, const double *coefd,
+                  const float *coeff, const int *tab, unsigned flags, const MpKeep &keep, T *out, float *blkmax,
+                  int n_img, hipStream_t st) {
+  const dim3 rgrid((g.nx * g.ny + 255) / 256, n_img);
+  int d0, d1;
+  const bool fast = fast_model<T>(m, flags, d0, d1);
   const bool share = !m.mp_n && (flags & LENSIM_IMAGE_SOURCE) && bulk_waves(m, size_t(g.nx) * g.ny) > 1;
   if (m.mp_n || share) {  // the block maxima for the MFMA convolution follow from the image in a second launch
     int rc = share ? launch_render_bulk<T>(m, g, recd, recf, coefd, coeff, flags, keep, out, n_img, st)
@@ -1207,12 +1221,19 @@ int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, con
     return check_launch("render_kernel");
   }
   const bool ll = m.n_light == 1 && m.types[m.n_lens + 1] != LENSIM_NULL;
-#define LENSIM_FAST(A, B)                                                                                       \
-  do {                                                                                                          \
-    if (ll)                                                                                                     \
-      render_fast_kernel<T, A, B, 1, 1><<<rgrid, 256, 0, st>>>(m, g, recd, recf, coefd, coeff, flags, out, blkmax); \
-    else                                                                                                        \
-      render_fast_kernel<T, A, B, 1, 0><<<rgrid, 256, 0, st>>>(m, g, recd, recf, coefd, coeff, flags, out, blkmax); \
+  double *beta = sizeof(T) == sizeof(double) ? static_cast<double *>(keep.beta) : nullptr;
+  auto launch = [&](auto kernel) {
+    kernel<<<rgrid, 256, 0, st>>>(m, g, recd, recf, coefd, coeff, flags, beta, out, blkmax);
+  };
+#define LENSIM_FAST(A, B)                                                                             \
+  do {                                                                                                \
+    if constexpr (sizeof(T) == sizeof(double)) {                                                      \
+      if (beta) {                                                                                     \
+        launch(ll ? &render_fast_kernel<T, A, B, 1, 1, true> : &render_fast_kernel<T, A, B, 1, 0, true>); \
+        break;                                                                                        \
+      }                                                                                               \
+    }                                                                                                 \
+    launch(ll ? &render_fast_kernel<T, A, B, 1, 1, false> : &render_fast_kernel<T, A, B, 1, 0, false>); \
   } while (0)
   if (d0 == LENSIM_EPL && d1 == LENSIM_SHEAR) LENSIM_FAST(LENSIM_EPL, LENSIM_SHEAR);
   else if (d0 == LENSIM_EPL) LENSIM_FAST(LENSIM_EPL, 0);
@@ -2454,6 +2475,7 @@ struct GradArgs {
   const void *glow;       // [n_img][ny][nx] dlogL / d(unconvolved image), compute type
   double *gpart;          // [n_img][n_prof][nblk][8]
   void *gbeta;            // [n_img][ny][nx][s][s][2] dS/dbeta of the sources' sum, compute type, or NULL
+  bool kept;              // gbeta holds beta (from the render) until the source's launch puts dS/dbeta there
   void *beta;             // same shape: beta (bulk and multi-plane lists, by the adjoint kernels), or NULL
 };
 
@@ -2826,7 +2848,8 @@ __device__ __forceinline__ void lens_ray_grad(const ModelArgs &m, const GradArgs
 // FP64 is the vector unit's instructions: the closed forms of grad.hpp in place
 // of duals took 64 images of 120^2 (EPL + SHEAR, Sersic source and light) from
 // 620 to 411 us a call, sums of their bases with the kwargs' factors applied
-// once a block (a square root and five divisions a ray less) from 391 to 351.
+// once a block (a square root and five divisions a ray less) from 391 to 351,
+// and the source's rays taken from the render (MpKeep, GradArgs::kept) to 309.
 template <typename T, int TYPE>
 constexpr int grad_waves_per_eu() {
   return (sizeof(T) == sizeof(float) && TYPE != LENSIM_NFW && TYPE != LENSIM_TNFW) ? 4 : 1;
@@ -2903,6 +2926,9 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
           if (bt) {
             px = double(AT(bt, 0));
             py = double(AT(bt, 1));
+          } else if (ga.kept) {
+            px = double(AT(gb, 0));
+            py = double(AT(gb, 1));
           } else {
             trace_ray<T, HALO, false>(m, rp, img, x, y, px, py);
           }
@@ -4122,6 +4148,10 @@ int run_grad(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int k
   } else if (bulk_keeps<T>(m, size_t(g.nx) * g.ny * (ss.on ? size_t(ss.s) * ss.s : 1))) {
     keep.beta = ws + L.beta;
   }
+  int d0, d1;
+  const bool kept = sizeof(T) == sizeof(double) && L.gbeta && m.n_bulk == 0 && fast_model<T>(m, flags, d0, d1) &&
+                    m.types[m.n_lens] == LENSIM_SERSIC_ELLIPSE;
+  if (kept) keep.beta = ws + L.gbeta;
   int rc = ss.on ? run_image_ss<T>(m, g, psf, kx, ky, edge, ss, data, params, n_img, flags, nullptr, logl, ws, L, st,
                                    gmodel, keep)
                  : run_image<T>(m, g, psf, kx, ky, edge, data, params, n_img, flags, nullptr, logl, ws, L, st, gmodel, keep);
@@ -4163,6 +4193,7 @@ int run_grad(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int k
   ga.dcoeff = reinterpret_cast<const float *>(ws + L.dcoeff);
   ga.glow = glow;
   ga.gpart = reinterpret_cast<double *>(ws + L.gpart);
+  ga.kept = kept;
   ga.gbeta = L.gbeta ? static_cast<void *>(ws + L.gbeta) : nullptr;
   ga.beta = L.beta ? static_cast<void *>(ws + L.beta) : nullptr;
   const int npix = gg.nx * gg.ny, nblk = (npix + 256 * kGradPix - 1) / (256 * kGradPix);
