@@ -2804,7 +2804,6 @@ __device__ __forceinline__ void lens_ray_grad(const ModelArgs &m, const GradArgs
                                              int k, double x, double y, double w, double *acc, const T *gb) {
   const double *pk = ga.params + (size_t(img) * m.n_prof + k) * LENSIM_NPARAM;
   CHECK_SPAN(pk, LENSIM_NPARAM * sizeof(double));
-  if constexpr (sizeof(T) == sizeof(double)) __builtin_assume(gb != nullptr);
   double axp = 0.0, ayp = 0.0;  // the other deflectors in the forward form (not needed with gb)
   if (!gb) {
     for (int j = 0; j < m.n_lens; ++j) {
