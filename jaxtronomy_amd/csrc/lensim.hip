@@ -2876,6 +2876,7 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
   CHECK_SPAN(pk, LENSIM_NPARAM * sizeof(double));
   const gm::EllKw ek = kEll ? gm::EllKw(pk[type == LENSIM_EPL ? 2 : 1], pk[type == LENSIM_EPL ? 3 : 2]) : gm::EllKw();
   std::conditional_t<kSersic, gm::SersicGrad, const double *> sersic(rd);
+  bool seen = false;  // whether the thread has a ray: without one its sums are 0 whatever the kwargs' factors are
   for (int pp = 0; pp < kGradPix; ++pp) {
   const int pix0 = (blockIdx.x * kGradPix + pp) * blockDim.x + threadIdx.x;
   const bool active = pix0 < npix;
@@ -2892,6 +2893,7 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
   const double o0 = g.o0;
   // a lens profile only matters if a source is there to be lensed
   const bool live = active && w != 0.0 && (k >= m.n_defl || m.n_source > 0) && evaluated(g, i, j);
+  seen |= live;
   for (int sy = 0; live && sy < g.s; ++sy) {
     const double oy = o0 + sy * inv_s;
     for (int sx = 0; sx < g.s; ++sx) {
@@ -2962,10 +2964,12 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
     }
   }
   }
-  if constexpr (type == LENSIM_TNFW) tnfw_grad_scale(rd, acc);
-  if constexpr (kEll && type == LENSIM_EPL) gm::epl_kw(ek, rd, pk, acc);
-  if constexpr (kEll && type != LENSIM_EPL) gm::nie_kw<type>(ek, pk, acc);
-  if constexpr (kSersic) sersic.kwargs(rd, pk, acc);
+  if (seen) {
+    if constexpr (type == LENSIM_TNFW) tnfw_grad_scale(rd, acc);
+    if constexpr (kEll && type == LENSIM_EPL) gm::epl_kw(ek, rd, pk, acc);
+    if constexpr (kEll && type != LENSIM_EPL) gm::nie_kw<type>(ek, pk, acc);
+    if constexpr (kSersic) sersic.kwargs(rd, pk, acc);
+  }
   // block sum of the 8 accumulators in a fixed order
   __shared__ double red[256 / 64][LENSIM_NPARAM];
 #pragma unroll

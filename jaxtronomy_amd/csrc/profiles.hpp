@@ -1217,10 +1217,11 @@ __device__ __forceinline__ void tnfw_ray_grad(const TnfwRec &r, const double *rd
   acc[3] -= fma(a, lx, qs * dx);
   acc[4] -= fma(a, ly, qs * dy);
 }
+// (a sum of 0 stays 0: where no ray counts, a factor that is infinite, of Rs or r_trunc 0, must not make it NaN)
 __device__ __forceinline__ void tnfw_grad_scale(const double *rd, double *acc) {
-  acc[0] *= rd[TN_IRS];
-  acc[1] *= rd[TN_A1] * rd[TN_PRE];
-  acc[2] *= rd[TN_IRT];
+  const double f[3] = {rd[TN_IRS], rd[TN_A1] * rd[TN_PRE], rd[TN_IRT]};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) acc[i] = acc[i] != 0.0 ? acc[i] * f[i] : 0.0;
 }
 
 // TNFW deflection, LensModel/Profiles/tnfw.py:67-87, :226-248, _g :329-349,

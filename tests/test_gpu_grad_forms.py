@@ -12,6 +12,7 @@ from jaxtronomy_amd.Data.imaging_data import ImageData
 from jaxtronomy_amd.Data.psf import PSF
 from jaxtronomy_amd.ImSim.image_model import ImageModel
 from jaxtronomy_amd.LensModel.lens_model import LensModel
+from jaxtronomy_amd.LensModel.lens_model_bulk import LensModelBulk
 from jaxtronomy_amd.LightModel.light_model import LightModel
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +61,33 @@ def test_gradient_vs_differences(name, lens, light, num_pix):
     for k in range(3):
         scale = np.abs(want[k]).max()
         assert scale > 0.0 and np.all(np.abs(got[k] - want[k]) <= 2e-5 * scale)
+
+
+DEGENERATE = {"EPL": dict(LENS["EPL"], e1=0.0, e2=0.0), "SIE": dict(LENS["SIE"], e1=0.0, e2=0.0),
+              "NIE": dict(LENS["NIE"], e1=0.0, e2=0.0), "NFW": LENS["NFW"],
+              "TNFW": dict(Rs=0.0, alpha_Rs=0.5, r_trunc=0.0, center_x=0.1, center_y=0.2)}
+
+
+@pytest.mark.parametrize("where", ["inline", "bulk", "planes"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_lens_without_a_source_has_no_gradient(where, precision):
+    """No ray carries the lens to the image: every kwarg's gradient is exactly 0, also where a factor of the kwargs
+    alone (of a round ellipticity, of a halo of size 0) is infinite or undefined."""
+    names = list(DEGENERATE)
+    kw = [DEGENERATE[n] for n in names]
+    z = [0.3, 0.3, 0.4, 0.5, 0.5]
+    cfg = dict(W.EPL180, numPix=9, deltaPix=0.3, supersampling=2)
+    lm = (LensModelBulk(names, precision=precision) if where == "bulk" else
+          LensModel(names, z_source=1.5, lens_redshift_list=z, multi_plane=True, precision=precision)
+          if where == "planes" else LensModel(names, precision=precision))
+    data = np.random.default_rng(0).normal(1.0, 0.1, (9, 9))
+    im = ImageModel(ImageData(**W.data_kwargs(cfg, data)), PSF("NONE"), lm, LightModel([]),
+                    lens_light_model_class=LightModel(["SERSIC_ELLIPSE"]), precision=precision,
+                    kwargs_numerics={"supersampling_factor": 2})
+    if where == "bulk":
+        params, n, m, keep = im.pack_bulk(lm.prepare_ray_shooting_kwargs(names, kw), [], [SERSIC])
+    else:
+        (params, n), m, keep = im.pack(kw, [], [SERSIC]), None, None
+    grad = im.likelihood_and_grad_batch(backend.to_device_f64(params), n, model=m)[1][0].cpu().numpy()
+    assert np.all(grad[:5] == 0.0) and np.all(np.isfinite(grad)) and np.any(grad[5] != 0.0)
+    del keep
