@@ -292,8 +292,9 @@ enum : int { TN_IRS = 2, // 1/Rs (0 for a negative Rs: X is then at its floor)
               TN_PT,     // pi tau^2 (tau^2 + 1)
               TN_DP,     // d ln(tau^2/(tau^2+1)^2) / d ln tau = 2 (1 - tau^2) / (1 + tau^2)
               TN_A1,     // 4 rho0 Rs / alpha_Rs
-              TN_IRT };  // 1 / r_trunc
-static_assert(TN_IRT < kRec, "TNFW record exceeds kRec");
+              TN_IRT,    // 1 / r_trunc
+              TN_IRG };  // 1 / Rs, of a negative Rs too
+static_assert(TN_IRG < kRec, "TNFW record exceeds kRec");
 // SHEAR   (shear.py:37-53): ra_0, dec_0 in the centre slots, gamma1, gamma2; the
 //          steps of w = theta - alpha_scaling alpha_shear(theta) (affine in theta)
 enum : int { SH_G1 = 2, SH_G2, SH_WSX, SH_WSY, SH_WRX, SH_WRY };
@@ -529,6 +530,7 @@ __device__ inline void prepare_record(int type, const double *p, double *rec, do
       rec[TN_DP] = 2.0 * (1.0 - tau2) / (1.0 + tau2);
       rec[TN_A1] = 1.0 / (Rs * (1.0 + log(1.0 / 2.0)));
       rec[TN_IRT] = 1.0 / r_trunc;
+      rec[TN_IRG] = 1.0 / Rs;
       break;
     }
     case LENSIM_SHEAR: {
@@ -1219,7 +1221,7 @@ __device__ __forceinline__ void tnfw_ray_grad(const TnfwRec &r, const double *rd
 }
 // (a sum of 0 stays 0: where no ray counts, a factor that is infinite, of Rs or r_trunc 0, must not make it NaN)
 __device__ __forceinline__ void tnfw_grad_scale(const double *rd, double *acc) {
-  const double f[3] = {rd[TN_IRS], rd[TN_A1] * rd[TN_PRE], rd[TN_IRT]};
+  const double f[3] = {rd[TN_IRG], rd[TN_A1] * rd[TN_PRE], rd[TN_IRT]};
 #pragma unroll
   for (int i = 0; i < 3; ++i) acc[i] = acc[i] != 0.0 ? acc[i] * f[i] : 0.0;
 }

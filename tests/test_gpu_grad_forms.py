@@ -91,3 +91,36 @@ def test_lens_without_a_source_has_no_gradient(where, precision):
     grad = im.likelihood_and_grad_batch(backend.to_device_f64(params), n, model=m)[1][0].cpu().numpy()
     assert np.all(grad[:5] == 0.0) and np.all(np.isfinite(grad)) and np.any(grad[5] != 0.0)
     del keep
+
+
+@pytest.mark.parametrize("where", ["inline", "bulk"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_tnfw_of_negative_radii_vs_differences(where, precision):
+    """Rs < 0 with r_trunc < 0 holds X at its floor, where alpha is still a function of Rs through rho0 and tau: alpha =
+    a (dx, dy) with one number a, so a kwarg's derivative over that by alpha_Rs is (da / d kwarg) alpha_Rs / a, here from
+    a's differences: g at X = 1e-3 cancels to 1e-6 of its terms, so a is good to 1e-9 and steps of 1e-2 leave 1e-4."""
+    kw = dict(Rs=-0.7, alpha_Rs=0.1, r_trunc=-1.9, center_x=0.05, center_y=-0.03)
+    cfg = dict(W.EPL180, numPix=9, deltaPix=0.3, supersampling=1)
+    lm = (LensModelBulk if where == "bulk" else LensModel)(["TNFW"], precision=precision)
+    data = np.random.default_rng(0).normal(1.0, 0.1, (9, 9))
+    im = ImageModel(ImageData(**W.data_kwargs(cfg, data)), PSF("NONE"), lm, LightModel(["SERSIC_ELLIPSE"]),
+                    precision=precision)
+    if where == "bulk":
+        params, n, m, keep = im.pack_bulk(lm.prepare_ray_shooting_kwargs(["TNFW"], [kw]), [SERSIC])
+    else:
+        (params, n), m, keep = im.pack([kw], [SERSIC]), None, None
+    g = im.likelihood_and_grad_batch(backend.to_device_f64(params), n, model=m)[1][0].cpu().numpy()[0]
+
+    def a(rs, rt):  # tnfw.py:226-248 with X = 0.001, up to a constant
+        x, tau = 1e-3, rt / rs
+        w, t2 = np.sqrt(tau * tau + x * x), tau * tau
+        f = np.arctanh(np.sqrt(1 - x * x)) / np.sqrt(1 - x * x)
+        return t2 / (t2 + 1)**2 * ((t2 - 1 + 2 * x * x) * f + tau * np.pi + (t2 - 1) * np.log(tau)
+                                   + w * (-np.pi + np.log(x / (tau + w)) * (t2 - 1) / tau)) / rs
+
+    h = 1e-2
+    by_rs = (a(kw["Rs"] + h, kw["r_trunc"]) - a(kw["Rs"] - h, kw["r_trunc"])) / (2 * h) / a(kw["Rs"], kw["r_trunc"])
+    by_rt = (a(kw["Rs"], kw["r_trunc"] + h) - a(kw["Rs"], kw["r_trunc"] - h)) / (2 * h) / a(kw["Rs"], kw["r_trunc"])
+    assert g[1] != 0.0
+    assert abs(g[0] / (g[1] * kw["alpha_Rs"]) - by_rs) <= 1e-3 * abs(by_rs)
+    assert abs(g[2] / (g[1] * kw["alpha_Rs"]) - by_rt) <= 1e-3 * abs(by_rt) + 1e-6
