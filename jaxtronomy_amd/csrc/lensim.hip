@@ -772,6 +772,13 @@ __device__ __forceinline__ int div_by(int n, int d, double inv_d, int &rem) {
   return q;
 }
 
+// The same for n < 2^50.
+__device__ __forceinline__ int64_t div_by64(int64_t n, int d, double inv_d, int &rem) {
+  const int64_t q = int64_t((double(n) + 0.5) * inv_d);
+  rem = int(n - q * d);
+  return q;
+}
+
 // Whether grid pixel (i, j) is evaluated (RegularGrid flux_evaluate_indexes,
 // ImSim/Numerics/grid.py:47-58: the rays of other pixels are not shot and
 // their flux is zero).
@@ -3090,19 +3097,22 @@ __device__ __forceinline__ void deflector_dalpha(const ModelArgs &m, const GradA
 // both summed five parameters over each block at every deflector: 23.5 ms for
 // 5256 deflectors and 100^2 rays, where the two steps take 0.52 and 0.28 ms.)
 
-// A ray of image img: its index on the grid, position and the weight w =
-// dlogL / d(ray flux); live: whether it has a weight and a source to hit.
+// Ray `first` + lane of image img (first + lane < the rays of the image, which
+// may be more than 2^31 in a list on one plane): its index on the grid,
+// position and the weight w = dlogL / d(ray flux); live: whether it has a weight
+// and a source to hit.
 struct GradRay {
   size_t slot;
   double x, y, w;
   bool live;
 };
 template <typename T>
-__device__ __forceinline__ GradRay grad_ray(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, int img, int rr,
-                                            bool active) {
+__device__ __forceinline__ GradRay grad_ray(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, int img,
+                                            int64_t first, int lane, bool active) {
   const int npix = g.nx * g.ny, ss = g.s * g.s;
-  int sub, i, sx;
-  const int pix = div_by(rr, ss, g.inv_ss, sub);
+  int left, sub, i, sx;
+  const int pix0 = int(div_by64(first, ss, g.inv_ss, left));
+  const int pix = pix0 + div_by(left + lane, ss, g.inv_ss, sub);
   const int j = div_by(pix, g.nx, g.inv_nx, i), sy = div_by(sub, g.s, g.inv_s, sx);
   const double ox = g.o0 + sx * g.inv_s, oy = g.o0 + sy * g.inv_s;
   GradRay r;
@@ -3169,13 +3179,13 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const MpTab tab = mp_tab(m, tab_all, img);
   if (both && bool(tab.sub) != SUB) return;  // the other instantiation's launch takes it
-  const int r_all = g.nx * g.ny * g.s * g.s;
+  const int64_t r_all = int64_t(g.nx) * g.ny * g.s * g.s;
   const int64_t cap = round_rays(per_img, tab.n), in = int64_t(blockIdx.x) * 64;
   if (in >= cap || round * cap + in >= r_all) return;
-  const int64_t rr = round * cap + in + lane;
-  const bool active = rr < r_all;
+  const int64_t first = round * cap + in;
+  const bool active = first + lane < r_all;
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
-  const GradRay ray = grad_ray<T>(m, g, ga, img, int(active ? rr : r_all - 1), active);
+  const GradRay ray = grad_ray<T>(m, g, ga, img, first, active ? lane : int(r_all - 1 - first), active);
   double4 *st = store + size_t(img) * per_img + in + lane;  // this ray's entry of run c at st[c * cap]
   if (!__any(ray.live)) {  // the same in every wave: they hold the same rays
     for (int c = wave; c < tab.n; c += nw) AT(st, c * cap) = double4{0.0, 0.0, 0.0, 0.0};
@@ -3261,13 +3271,13 @@ __global__ __launch_bounds__(64 * kBulkWaves) void bulk_adjoint_kernel(
   __shared__ WaveSumsOf<kBulkWaves> red;
   const int img = blockIdx.y, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r_all = g.nx * g.ny * g.s * g.s;
+  const int64_t r_all = int64_t(g.nx) * g.ny * g.s * g.s;
   const int64_t cap = round_rays(per_img, 1), in = int64_t(blockIdx.x) * 64;
   if (in >= cap || round * cap + in >= r_all) return;
-  const int64_t rr = round * cap + in + lane;
-  const bool active = rr < r_all;
+  const int64_t first = round * cap + in;
+  const bool active = first + lane < r_all;
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
-  const GradRay ray = grad_ray<T>(m, g, ga, img, int(active ? rr : r_all - 1), active);
+  const GradRay ray = grad_ray<T>(m, g, ga, img, first, active ? lane : int(r_all - 1 - first), active);
   double ax = 0.0, ay = 0.0;
   if (!kept && __any(ray.live)) {  // the same in every wave
     if (wave == 0)
@@ -3475,7 +3485,9 @@ int launch_defl_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, 
                      const int *tab, double *gpart_mp, double4 *store, int nblk, int n_img, hipStream_t st) {
   const size_t rays = size_t(g.nx) * g.ny * g.s * g.s;
   const DeflGradPlan p = defl_grad_plan(m, rays, n_img);
-  const dim3 grid((unsigned)((rays + 63) / 64), n_img);
+  // a round's rays (of several planes, as many as one run would leave): so a launch's threads stay below 2^32
+  const size_t most = p.n ? p.per_img : rays;
+  const dim3 grid((unsigned)(((rays < most ? rays : most) + 63) / 64), n_img);
   const dim3 dgrid((p.n + 7) / 8, n_img, p.splits);
   int sub = sub_list(m);
   if (!m.mp_n && sub == 0) sub = m.bulk_type ? int(sub_type(m.bulk_type)) : 2;  // of the bulk list alone

@@ -13,6 +13,7 @@ from jaxtronomy_amd import workloads as W
 from jaxtronomy_amd.Data.imaging_data import ImageData
 from jaxtronomy_amd.Data.psf import PSF
 from jaxtronomy_amd.ImSim.image_model import ImageModel
+from jaxtronomy_amd.LensModel.lens_model import LensModel
 from jaxtronomy_amd.LensModel.lens_model_bulk import LensModelBulk
 from jaxtronomy_amd.LightModel.light_model import LightModel
 
@@ -104,3 +105,25 @@ def test_rounds_add_up():
     assert torch.allclose(l2, l1.expand(64), rtol=1e-13, atol=0.0)
     assert float(((g2 - g1) / scale).abs().max()) < 1e-12
     del keep
+
+
+def test_more_rays_than_an_int_holds():
+    """The gradient of a list over more than 2^31 sub-rays, against the same deflector inline, whose kernels go pixel by
+    pixel: the sums of a pixel's sub-rays in another order, 2.4e9 terms rounded to 1e-16 each in blocks of at most 1e6."""
+    n, s = 4096, 12
+    cfg = dict(W.EPL180, numPix=n, deltaPix=3.2 / n, supersampling=s)
+    data = np.random.default_rng(0).normal(0.5, 0.1, (n, n))
+    halo = dict(Rs=0.6, alpha_Rs=0.4, r_trunc=1.5, center_x=0.013, center_y=0.021)
+    grads = []
+    for lm in (LensModelBulk(["TNFW"]), LensModel(["TNFW"])):
+        im = ImageModel(ImageData(**W.data_kwargs(cfg, data)), PSF("NONE"), lm, LightModel(["SERSIC_ELLIPSE"]),
+                        kwargs_numerics={"supersampling_factor": s})
+        if isinstance(lm, LensModelBulk):
+            params, b, m, keep = im.pack_bulk(lm.prepare_ray_shooting_kwargs(["TNFW"], [halo]), SOURCE)
+        else:
+            (params, b), m, keep = im.pack([halo], SOURCE), None, None
+        grads.append(im.likelihood_and_grad_batch(backend.to_device_f64(params), b, model=m)[1][0].cpu().numpy())
+        del im, keep
+        torch.cuda.empty_cache()
+    assert n * n * s * s > 2**31
+    assert np.all(np.abs(grads[0] - grads[1]) <= 1e-9 * np.abs(grads[1]).max(axis=1, keepdims=True))
