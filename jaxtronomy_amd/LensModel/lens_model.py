@@ -125,6 +125,7 @@ class LensModel(object):
                   "r2p": backend.to_device_f64(np.asarray(r2p))}
         mp = backend.LensimMultiplane()
         mp.n_planes = len(z) + 1
+        mp.max_runs = backend.plane_runs(tij, tz, r2p)
         mp.d_order = arrays["order"].data_ptr() if len(z) else None
         mp.d_T_ij = arrays["tij"].data_ptr()
         mp.d_T_z = arrays["tz"].data_ptr()

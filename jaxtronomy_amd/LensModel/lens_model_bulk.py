@@ -174,6 +174,7 @@ class LensModelBulk(object):
                   "r2p": torch.as_tensor(np.ascontiguousarray(r2p), device=dev)}
         mp = backend.LensimMultiplane()
         mp.n_planes = n + 1
+        mp.max_runs = backend.plane_runs(t_ij, t_z, r2p)
         mp.d_order = arrays["order"].data_ptr() if n else None
         mp.d_T_ij = arrays["tij"].data_ptr()
         mp.d_T_z = arrays["tz"].data_ptr()

@@ -56,7 +56,7 @@ class LensimModel(ctypes.Structure):
 class LensimMultiplane(ctypes.Structure):
     _fields_ = [
         ("n_planes", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("max_runs", ctypes.c_int32),
         ("d_order", ctypes.c_void_p),
         ("d_T_ij", ctypes.c_void_p),
         ("d_T_z", ctypes.c_void_p),
@@ -219,6 +219,21 @@ class Workspace:
         if self._buf is None or self._buf.numel() < nbytes:
             self._buf = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device())
         return self._buf
+
+
+def plane_runs(t_ij, t_z, r2p):
+    """lensim_multiplane.max_runs of plane arrays [n_planes] or [n_img, n_planes]: the
+    most runs of any image (a run: up to 64 consecutive deflector planes with
+    T_ij 0 after the first and one T_z and r2p)."""
+    t_ij, t_z, r2p = (np.asarray(a, dtype=np.float64)[..., :-1] for a in (t_ij, t_z, r2p))
+    if t_ij.shape[-1] == 0:
+        return 0
+    moved = (t_ij[..., 1:] != 0.0) | (t_z[..., 1:] != t_z[..., :-1]) | (r2p[..., 1:] != r2p[..., :-1])
+    most = 0
+    for row in np.atleast_2d(moved):
+        starts = np.concatenate(([-1], np.flatnonzero(row), [len(row)]))
+        most = max(most, int(((starts[1:] - starts[:-1] + 63) >> 6).sum()))
+    return most
 
 
 def make_model(lens_types, source_types, light_types, alpha_scaling=1.0, flux_scaling=1.0, bulk=None):

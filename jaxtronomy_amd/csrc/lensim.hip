@@ -209,6 +209,7 @@ struct ModelArgs {
   const int32_t *mp_order;
   const double *mp_tij, *mp_tz, *mp_r2p;
   int64_t mp_stride;
+  int32_t mp_runs;      // the caller's bound on the plane runs (max_runs), else the deflectors
 };
 
 __host__ __device__ inline int type_of(const ModelArgs &m, int k) {
@@ -416,29 +417,30 @@ Layout layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img, int
 // Work plan of the gradient of a bulk or multi-plane deflector list over
 // `rays` rays an image (adjoint kernels, then defl_grad_kernel).  The adjoint
 // kernels keep four doubles per ray and run: per_img of them an image, at most
-// 2^25 (1 GiB) a call as long as that holds 64 rays of every run.  The host
-// knows the number of runs only as "at most one per plane", so it launches as
-// many rounds of rays as that could take; the kernels take as many rays a
-// round as the runs there are allow, usually all in the first, and the other
-// rounds' blocks end at once.  splits: pieces a deflector's rays are cut into
-// (a partial sum each), so that about 8192 waves share the deflectors.
+// kStoreMost (1 GiB) together: `imgs` images at a time, and an image that takes
+// more by itself in `rounds` of its rays.  `runs` is the caller's bound on a
+// multi-plane model's runs (lensim_multiplane.max_runs), without one a run per
+// plane: the kernels take as many rays a round as the runs there are allow, and
+// what the plan has too many of ends at once.  splits: pieces a deflector's rays
+// of a round are cut into (a partial sum each, to which the rounds add), so that
+// about 8192 waves share the deflectors of `imgs` images.
+constexpr size_t kStoreMost = size_t(1) << 25;
 struct DeflGradPlan {
   size_t per_img;
-  int rounds, splits, n;  // n: deflectors (planes, or the bulk list)
-  int slots() const { return rounds * splits; }
+  int imgs, rounds, splits, n, runs;  // n: deflectors (planes, or the bulk list)
 };
 DeflGradPlan defl_grad_plan(const ModelArgs &m, size_t rays, int n_img) {
-  DeflGradPlan p{0, 1, 1, m.mp_n ? m.mp_n - 1 : m.n_bulk};
+  DeflGradPlan p{0, n_img, 1, 1, m.mp_n ? m.mp_n - 1 : m.n_bulk, 1};
   if (p.n == 0) return p;
-  const size_t runs = m.mp_n ? size_t(p.n) : 1, all = (rays + 63) / 64 * 64 * runs;
-  size_t share = (size_t(1) << 25) / n_img;
-  if (share < 64 * runs) share = 64 * runs;
-  p.per_img = all < share ? all : share;
-  const size_t cap = p.per_img / runs / 64 * 64;
+  if (m.mp_n) p.runs = m.mp_runs;
+  const size_t all = (rays + 63) / 64 * 64 * p.runs;
+  p.per_img = all < kStoreMost ? all : kStoreMost;
+  const size_t cap = p.per_img / p.runs / 64 * 64, fit = kStoreMost / p.per_img;
   p.rounds = int((rays + cap - 1) / cap);
-  const size_t pairs = size_t((p.n + 1) / 2) * n_img;
-  size_t sp = (8192 + pairs - 1) / pairs, most = (rays + 511) / 512;
-  p.splits = int(sp < most ? sp : most);
+  if (fit < size_t(n_img)) p.imgs = int(fit);
+  const size_t pairs = size_t((p.n + 1) / 2) * p.imgs;
+  size_t sp = (8192 + pairs - 1) / pairs, part = (rays + 511) / 512;
+  p.splits = int(sp < part ? sp : part);
   return p;
 }
 
@@ -473,9 +475,9 @@ Layout grad_layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img
   if (list && m.n_defl > 0) {
     const DeflGradPlan p = defl_grad_plan(m, rays, n_img);
     L.gpart_mp = off;
-    off = align256(off + size_t(n_img) * p.n * p.slots() * LENSIM_NPARAM * 8);
+    off = align256(off + size_t(p.imgs) * p.n * p.splits * LENSIM_NPARAM * 8);
     L.gstate = off;
-    off = align256(off + size_t(n_img) * p.per_img * 32);
+    off = align256(off + size_t(p.imgs) * p.per_img * 32);
   }
   L.gpad = L.gext = L.gchr = L.glu = off;
   if (edge) {  // extended domain (ny cs + ky - 1) x (nx cs + kx - 1)
@@ -557,6 +559,7 @@ int model_args(const lensim_model *model, ModelArgs &m) {
     m.mp_tz = mp->d_T_z;
     m.mp_r2p = mp->d_r2p;
     m.mp_stride = mp->stride;
+    m.mp_runs = mp->max_runs > 0 && mp->max_runs < m.n_defl ? mp->max_runs : m.n_defl;
     // with several planes a deflector's error moves the rays at every later
     // plane, where a strong lens magnifies it: the float form's render and
     // gradient kernels deflect the NFW family in double there too (the float
@@ -3172,10 +3175,10 @@ template <typename T, bool HALO, bool SUB>
 __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
     ModelArgs m, GridArgs g, GradArgs ga, const double *__restrict__ recd, const float *__restrict__ recf,
     const double *__restrict__ coefd, const float *__restrict__ coeff, const int *__restrict__ tab_all, bool both,
-    double4 *store, size_t per_img, int round, const double *__restrict__ all_tij,
+    double4 *store, size_t per_img, int img0, int round, bool keeps, const double *__restrict__ all_tij,
     const double *__restrict__ all_tz, const double *__restrict__ all_r2p) {
   __shared__ WaveSums red;
-  const int img = blockIdx.y, lane = threadIdx.x & 63, nw = int(blockDim.x) >> 6;
+  const int img = img0 + blockIdx.y, lane = threadIdx.x & 63, nw = int(blockDim.x) >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const MpTab tab = mp_tab(m, tab_all, img);
   if (both && bool(tab.sub) != SUB) return;  // the other instantiation's launch takes it
@@ -3186,7 +3189,7 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
   const bool active = first + lane < r_all;
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
   const GradRay ray = grad_ray<T>(m, g, ga, img, first, active ? lane : int(r_all - 1 - first), active);
-  double4 *st = store + size_t(img) * per_img + in + lane;  // this ray's entry of run c at st[c * cap]
+  double4 *st = store + size_t(blockIdx.y) * per_img + in + lane;  // this ray's entry of run c at st[c * cap]
   if (!__any(ray.live)) {  // the same in every wave: they hold the same rays
     for (int c = wave; c < tab.n; c += nw) AT(st, c * cap) = double4{0.0, 0.0, 0.0, 0.0};
     return;
@@ -3194,7 +3197,7 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
   const size_t o = size_t(img) * size_t(m.mp_stride);
   const double *tij = all_tij + o, *tzs = all_tz + o, *r2p = all_r2p + o;
   T bx = T(0), by = T(0), *b = static_cast<T *>(ga.beta) + ray.slot;
-  if (cap >= r_all) {  // the render kept the positions and beta (MpKeep)
+  if (keeps && cap >= r_all) {  // the render kept the positions and beta (MpKeep)
     if (ray.live) {
       bx = AT(b, 0);
       by = AT(b, 1);
@@ -3267,9 +3270,9 @@ template <typename T, bool HALO>
 __global__ __launch_bounds__(64 * kBulkWaves) void bulk_adjoint_kernel(
     ModelArgs m, GridArgs g, GradArgs ga, const double *__restrict__ recd, const float *__restrict__ recf,
     const double *__restrict__ coefd, const float *__restrict__ coeff, double4 *__restrict__ store, size_t per_img,
-    int round, bool kept) {
+    int img0, int round, bool kept) {
   __shared__ WaveSumsOf<kBulkWaves> red;
-  const int img = blockIdx.y, lane = threadIdx.x & 63;
+  const int img = img0 + blockIdx.y, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t r_all = int64_t(g.nx) * g.ny * g.s * g.s;
   const int64_t cap = round_rays(per_img, 1), in = int64_t(blockIdx.x) * 64;
@@ -3307,7 +3310,7 @@ __global__ __launch_bounds__(64 * kBulkWaves) void bulk_adjoint_kernel(
       AT(gb, 1) = f2.d[1];
     }
   }
-  AT(store, size_t(img) * per_img + in + lane) = double4{ray.x, ray.y, lx, ly};
+  AT(store, size_t(blockIdx.y) * per_img + in + lane) = double4{ray.x, ray.y, lx, ly};
 }
 
 // One deflector's (or, of TNFW, a pair's) sums over rays [r0, r1) of `st`: a
@@ -3324,8 +3327,9 @@ __device__ __forceinline__ void tnfw_sums(const double *const (&rd)[2], const do
   }
 }
 
-// Partial sums [img][plane or bulk index][slot][8] of lambda . d alpha /
-// d kwargs over a round's rays: a wave takes two planes' (or bulk) deflectors
+// Partial sums [img - img0][plane or bulk index][split][8] of lambda . d alpha /
+// d kwargs over a round's rays, stored by the first round, to which the others
+// add: a wave takes two planes' (or bulk) deflectors
 // q, q + 1 and one of the splits of the rays.  REST: the deflectors that are
 // not subhalos or linear (their duals' registers would cost the others waves);
 // each launch leaves the other's deflectors alone.
@@ -3337,13 +3341,15 @@ __global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g,
                                                         const float *__restrict__ coeff,
                                                         const int *__restrict__ tab_all,
                                                         const double4 *__restrict__ store, size_t per_img, int n,
-                                                        int round, int n_slots, bool both,
+                                                        int img0, int round, bool both,
                                                         double *__restrict__ gpart_mp) {
-  const int img = blockIdx.y, lane = threadIdx.x & 63;
+  const int img = img0 + blockIdx.y, lane = threadIdx.x & 63;
   if (REST && both && m.mp_n && mp_tab(m, tab_all, img).sub) return;  // no such deflector
   const int q = 2 * __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   if (q >= n) return;
-  const int nq = min(2, n - q), slot = round * int(gridDim.z) + int(blockIdx.z);
+  const int nq = min(2, n - q);
+  double *part = gpart_mp + ((size_t(blockIdx.y) * n + q) * gridDim.z + blockIdx.z) * LENSIM_NPARAM;  // of q; q + 1 after
+  const size_t next = size_t(gridDim.z) * LENSIM_NPARAM;                                             // gridDim.z splits
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
   int k[2], type[2], run[2], runs = 1;
   if (m.mp_n) {
@@ -3368,16 +3374,14 @@ __global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g,
   const int64_t n_ray = left < 0 ? 0 : (left < cap ? left : cap);
   const int64_t len = ((n_ray + 63) / 64 + gridDim.z - 1) / gridDim.z * 64;
   const int64_t r0 = min(n_ray, len * blockIdx.z), r1 = min(n_ray, r0 + len);
-  if (!REST && r0 == r1) {  // nothing of this round (REST's deflectors are stored over by its own launch, after)
-    if (lane < nq * LENSIM_NPARAM)
-      AT(gpart_mp, ((size_t(img) * n + q + lane / LENSIM_NPARAM) * n_slots + slot) * LENSIM_NPARAM +
-                       lane % LENSIM_NPARAM) = 0.0;
+  if (r0 == r1 && (!REST || round)) {  // nothing of this round (REST's deflectors are stored over by its launch, after)
+    if (!round && lane < nq * LENSIM_NPARAM) AT(part, lane / LENSIM_NPARAM * next + lane % LENSIM_NPARAM) = 0.0;
     return;
   }
   const double4 *st[2];
   const double *rd[2];
   for (int d = 0; d < 2; ++d) {
-    st[d] = store + size_t(img) * per_img + size_t(run[d < nq ? d : 0]) * cap;
+    st[d] = store + size_t(blockIdx.y) * per_img + size_t(run[d < nq ? d : 0]) * cap;
     rd[d] = rp.recd + k[d < nq ? d : 0] * kRec;
   }
   double acc[2][LENSIM_NPARAM];
@@ -3443,39 +3447,46 @@ __global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g,
       double mine = 0.0;
 #pragma unroll
       for (int i = 0; i < LENSIM_NPARAM; ++i) mine = lane == i ? v[i] : mine;
-      AT(gpart_mp, ((size_t(img) * n + q + d) * n_slots + slot) * LENSIM_NPARAM + lane) = mine;
+      AT(part, d * next + lane) = round ? AT(part, d * next + lane) + mine : mine;
     }
   }
 }
 
-// The list's partial sums added up in slot order into the first of the nblk
-// slots grad_reduce_kernel reads (the others zero).  A deflector that the
-// caller's order names on several planes gets the sum over them, one that it
-// does not name zero.
-__global__ void defl_partial_reduce(ModelArgs m, const int *__restrict__ tab_all, const double *__restrict__ gpart_mp,
-                                    int n, int n_slots, int n_img, int nblk, double *__restrict__ gpart) {
+// The list's partial sums of images img0 .. img0 + n_img - 1 added up into the
+// first of the nblk slots grad_reduce_kernel reads (the others zero): eight
+// lanes a kwarg, lane j the splits j, j + 8, ..., then the lanes' sums in pairs.
+// A deflector that the caller's order names on several planes gets the sum over
+// them, one that it does not name zero; a model of more runs than the caller's
+// bound, whose rays the plan's rounds did not all take, NaN.
+__global__ __launch_bounds__(256) void defl_partial_reduce(ModelArgs m, const int *__restrict__ tab_all,
+                                                           const double *__restrict__ gpart_mp, int n, int splits,
+                                                           int runs, int img0, int n_img, int nblk,
+                                                           double *__restrict__ gpart) {
   const int k0 = m.mp_n ? 0 : m.n_lens, nk = m.n_defl - k0;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_img * nk * LENSIM_NPARAM) return;
-  const int p = i % LENSIM_NPARAM, r = i / LENSIM_NPARAM, k = k0 + r % nk, img = r / nk;
+  const int64_t r = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (r >= int64_t(n_img) * nk) return;
+  const int p = threadIdx.x & 7, j = (threadIdx.x >> 3) & 7, li = int(r / nk), k = k0 + int(r - int64_t(li) * nk),
+            img = img0 + li;
   double v = 0.0;
   auto add = [&](int q) {
-    for (int b = 0; b < n_slots; ++b)
-      v += AT(gpart_mp, ((size_t(img) * n + q) * n_slots + b) * LENSIM_NPARAM + p);
+    for (int b = j; b < splits; b += 8) v += AT(gpart_mp, ((size_t(li) * n + q) * splits + b) * LENSIM_NPARAM + p);
   };
   if (!m.mp_n) {
     add(k - k0);
   } else {
     const MpTab tab = mp_tab(m, tab_all, img);
-    if (!tab.dup) {
+    if (tab.n > runs) {
+      v = NAN;
+    } else if (!tab.dup) {
       if (AT(tab.plane_of, k) >= 0) add(AT(tab.plane_of, k));
     } else {
       for (int q = 0; q < n; ++q)
         if ((AT(tab.who, q) & ((1 << kWhoBits) - 1)) == k) add(q);
     }
   }
+  for (int off = 8; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
   const size_t o = (size_t(img) * m.n_prof + k) * nblk;
-  for (int b = 0; b < nblk; ++b) AT(gpart, (o + b) * LENSIM_NPARAM + p) = b == 0 ? v : 0.0;
+  for (int b = j; b < nblk; b += 8) AT(gpart, (o + b) * LENSIM_NPARAM + p) = b == 0 ? v : 0.0;
 }
 
 // The gradient of the multi-plane or bulk list into ga.gpart, and beta (and
@@ -3487,41 +3498,48 @@ int launch_defl_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, 
   const DeflGradPlan p = defl_grad_plan(m, rays, n_img);
   // a round's rays (of several planes, as many as one run would leave): so a launch's threads stay below 2^32
   const size_t most = p.n ? p.per_img : rays;
-  const dim3 grid((unsigned)(((rays < most ? rays : most) + 63) / 64), n_img);
-  const dim3 dgrid((p.n + 7) / 8, n_img, p.splits);
   int sub = sub_list(m);
   if (!m.mp_n && sub == 0) sub = m.bulk_type ? int(sub_type(m.bulk_type)) : 2;  // of the bulk list alone
-  for (int r = 0; r < p.rounds; ++r) {
-    if (!m.mp_n) {
-      const bool kept = bulk_keeps<T>(m, size_t(g.nx) * g.ny);
-      bulk_adjoint_kernel<T, HALO><<<grid, kept ? 64 : 64 * kBulkWaves, 0, st>>>(
-          m, g, ga, recd, recf, ga.coefd, ga.coeff, store, p.per_img, r, kept);
-    } else {
+  // of an inline list the types are known: a launch for the kinds it holds
+  bool any_sub = m.n_bulk > 0;
+  for (int k = 0; m.mp_n && k < m.n_lens; ++k) any_sub = any_sub || sub_type(m.types[k]);
+  for (int i0 = 0; i0 < n_img; i0 += p.imgs) {
+    const int ni = n_img - i0 < p.imgs ? n_img - i0 : p.imgs;
+    const dim3 grid((unsigned)(((rays < most ? rays : most) + 63) / 64), ni);
+    const dim3 dgrid((p.n + 7) / 8, ni, p.splits);
+    for (int r = 0; r < p.rounds; ++r) {
+      if (!m.mp_n) {
+        const bool kept = bulk_keeps<T>(m, size_t(g.nx) * g.ny);
+        bulk_adjoint_kernel<T, HALO><<<grid, kept ? 64 : 64 * kBulkWaves, 0, st>>>(
+            m, g, ga, recd, recf, ga.coefd, ga.coeff, store, p.per_img, i0, r, kept);
+      } else {
 #define LENSIM_ADJOINT(H, S)                                                                                         \
   mp_adjoint_kernel<T, H, S><<<grid, 64 * mp_waves(rays, S), 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, \
-                                                                      sub == 2, store, p.per_img, r, m.mp_tij,       \
-                                                                      m.mp_tz, m.mp_r2p)
-      if (sub) LENSIM_ADJOINT(true, true);
-      if (sub != 1) LENSIM_ADJOINT(HALO, false);
+                                                                      sub == 2, store, p.per_img, i0, r,             \
+                                                                      p.imgs >= n_img, m.mp_tij, m.mp_tz, m.mp_r2p)
+        if (sub) LENSIM_ADJOINT(true, true);
+        if (sub != 1) LENSIM_ADJOINT(HALO, false);
 #undef LENSIM_ADJOINT
+      }
+      int rc = check_launch("adjoint kernel");
+      if (rc) return rc;
+      if (p.n == 0) continue;  // no deflector: beta alone
+      if (any_sub)
+        defl_grad_kernel<T, HALO, false><<<dgrid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, store,
+                                                                p.per_img, p.n, i0, r, sub == 2, gpart_mp);
+      if (sub != 1)
+        defl_grad_kernel<T, HALO, true><<<dgrid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, store,
+                                                               p.per_img, p.n, i0, r, sub == 2, gpart_mp);
+      if ((rc = check_launch("defl_grad_kernel"))) return rc;
     }
-    int rc = check_launch("adjoint kernel");
+    if (p.n == 0) continue;
+    const int64_t nw = int64_t(ni) * (m.n_defl - (m.mp_n ? 0 : m.n_lens));
+    defl_partial_reduce<<<(unsigned)((nw + 3) / 4), 256, 0, st>>>(m, tab, gpart_mp, p.n, p.splits, p.runs, i0, ni, nblk,
+                                                                  ga.gpart);
+    const int rc = check_launch("defl_partial_reduce");
     if (rc) return rc;
-    if (p.n == 0) return LENSIM_OK;  // no deflector: beta alone
-    // of an inline list the types are known: a launch for the kinds it holds
-    bool any_sub = m.n_bulk > 0 && sub != 0, any_rest = sub != 1;
-    for (int k = 0; m.mp_n && k < m.n_lens; ++k) any_sub = any_sub || sub_type(m.types[k]);
-    if (any_sub || m.n_bulk > 0)
-      defl_grad_kernel<T, HALO, false><<<dgrid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, store,
-                                                              p.per_img, p.n, r, p.slots(), sub == 2, gpart_mp);
-    if (any_rest)
-      defl_grad_kernel<T, HALO, true><<<dgrid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, store,
-                                                             p.per_img, p.n, r, p.slots(), sub == 2, gpart_mp);
-    if ((rc = check_launch("defl_grad_kernel"))) return rc;
   }
-  const int nt = n_img * (m.n_defl - (m.mp_n ? 0 : m.n_lens)) * LENSIM_NPARAM;
-  defl_partial_reduce<<<(nt + 255) / 256, 256, 0, st>>>(m, tab, gpart_mp, p.n, p.slots(), n_img, nblk, ga.gpart);
-  return check_launch("defl_partial_reduce");
+  return LENSIM_OK;
 }
 
 __global__ void grad_reduce_kernel(const double *__restrict__ gpart, int nblk, int n, double *__restrict__ grad) {
@@ -4156,10 +4174,12 @@ int run_grad(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int k
   const unsigned flags = LENSIM_IMAGE_SOURCE | LENSIM_IMAGE_LENS_LIGHT;
   MpKeep keep{};
   if (m.mp_n && m.n_source > 0) {
-    const size_t rays = size_t(g.nx) * g.ny * g.s * g.s;
-    keep.store = reinterpret_cast<double4 *>(ws + L.gstate);
-    keep.per_img = defl_grad_plan(m, rays, n_img).per_img;
-    keep.beta = ws + L.beta;
+    const DeflGradPlan p = defl_grad_plan(m, size_t(g.nx) * g.ny * g.s * g.s, n_img);
+    if (p.imgs >= n_img) {  // the store holds the whole batch
+      keep.store = reinterpret_cast<double4 *>(ws + L.gstate);
+      keep.per_img = p.per_img;
+      keep.beta = ws + L.beta;
+    }
   } else if (bulk_keeps<T>(m, size_t(g.nx) * g.ny * (ss.on ? size_t(ss.s) * ss.s : 1))) {
     keep.beta = ws + L.beta;
   }

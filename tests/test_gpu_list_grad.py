@@ -127,3 +127,41 @@ def test_more_rays_than_an_int_holds():
         torch.cuda.empty_cache()
     assert n * n * s * s > 2**31
     assert np.all(np.abs(grads[0] - grads[1]) <= 1e-9 * np.abs(grads[1]).max(axis=1, keepdims=True))
+
+
+def test_bound_on_the_plane_runs():
+    """The gradient does not depend on the bound that the caller gives on the runs, down to the runs there are; with
+    fewer the deflectors' gradients are NaN."""
+    names, kw, _ = scene(30, 0.2, False, 5)
+    z = [0.3] * 12 + [0.5] * 10 + [0.6] * 8
+    im = model(31, 2, True, np.random.default_rng(3).normal(0.5, 0.1, (31, 31)))
+    params, n, m, keep = packed(im, names, kw, z, True)
+    mp = keep[-1]["struct"]
+    assert mp.max_runs == 3
+
+    def grad():
+        return im.likelihood_and_grad_batch(backend.to_device_f64(params), n, model=m)[1]
+
+    want = grad()
+    for runs in (0, 4, 29, 1 << 20):
+        mp.max_runs = runs
+        assert torch.equal(grad(), want)
+    mp.max_runs = 2
+    got = grad()
+    assert bool(torch.isnan(got[0, :30]).all()) and torch.equal(got[0, 30:], want[0, 30:])
+
+
+def test_planes_of_one_redshift_equal_one_plane():
+    """More rays than a round's store holds for a run (2^25): several planes at one redshift against the list on one
+    plane, whose reduced deflections are the same; 3.4e7 rays' sums in another order, 1e-12 of their sizes."""
+    names, kw, _ = scene(3, 0.6, False, 5)
+    grads = []
+    for multi_plane in (False, True):
+        cfg = dict(W.EPL180, numPix=1450, deltaPix=3.2 / 1450, supersampling=4)
+        data = np.random.default_rng(0).normal(0.5, 0.1, (1450, 1450))
+        im = ImageModel(ImageData(**W.data_kwargs(cfg, data)), PSF("NONE"), LensModelBulk(UNIQUE, multi_plane=multi_plane),
+                        LightModel(["SERSIC_ELLIPSE"]), kwargs_numerics={"supersampling_factor": 4})
+        params, n, m, keep = packed(im, names, kw, [0.5] * 3, multi_plane)
+        grads.append(im.likelihood_and_grad_batch(backend.to_device_f64(params), n, model=m)[1][0].cpu().numpy())
+    scale = np.abs(grads[0]).max(axis=1, keepdims=True)
+    assert np.all(np.abs(grads[0] - grads[1]) <= 1e-9 * scale)
