@@ -422,8 +422,12 @@ Layout layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img, int
 // multi-plane model's runs (lensim_multiplane.max_runs), without one a run per
 // plane: the kernels take as many rays a round as the runs there are allow, and
 // what the plan has too many of ends at once.  splits: pieces a deflector's rays
-// of a round are cut into (a partial sum each, to which the rounds add), so that
-// about 8192 waves share the deflectors of `imgs` images.
+// of a round are cut into (a partial sum each, to which the rounds add), from 512
+// rays and so that about 2048 waves, and up to 16384 of 2048 rays, share an
+// image's deflectors.  Nothing but `imgs` depends on the batch, so a list's sums
+// on one plane have the same order in any.  The partial sums take imgs n splits
+// 64 B: with a pair of deflectors a wave at most 2 MB an image beside one sum
+// for each deflector.
 constexpr size_t kStoreMost = size_t(1) << 25;
 struct DeflGradPlan {
   size_t per_img;
@@ -438,9 +442,13 @@ DeflGradPlan defl_grad_plan(const ModelArgs &m, size_t rays, int n_img) {
   const size_t cap = p.per_img / p.runs / 64 * 64, fit = kStoreMost / p.per_img;
   p.rounds = int((rays + cap - 1) / cap);
   if (fit < size_t(n_img)) p.imgs = int(fit);
-  const size_t pairs = size_t((p.n + 1) / 2) * p.imgs;
-  size_t sp = (8192 + pairs - 1) / pairs, part = (rays + 511) / 512;
-  p.splits = int(sp < part ? sp : part);
+  const size_t pairs = size_t(p.n + 1) / 2;
+  auto over = [](size_t a, size_t b) { return (a + b - 1) / b; };
+  size_t sp = over(rays, 2048);
+  if (sp > over(16384, pairs)) sp = over(16384, pairs);
+  if (sp < over(2048, pairs)) sp = over(2048, pairs);
+  if (sp > over(rays, 512)) sp = over(rays, 512);
+  p.splits = int(sp < 2048 ? sp : 2048);
   return p;
 }
 

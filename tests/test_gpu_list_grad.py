@@ -165,3 +165,16 @@ def test_planes_of_one_redshift_equal_one_plane():
         grads.append(im.likelihood_and_grad_batch(backend.to_device_f64(params), n, model=m)[1][0].cpu().numpy())
     scale = np.abs(grads[0]).max(axis=1, keepdims=True)
     assert np.all(np.abs(grads[0] - grads[1]) <= 1e-9 * scale)
+
+
+@pytest.mark.parametrize("n_halo,num_pix", [(3, 40), (40, 61)])
+def test_list_gradient_is_the_same_in_any_batch(n_halo, num_pix):
+    """The sums' order on one plane follows the image alone."""
+    names, kw, _ = scene(n_halo, 0.3, True, 5)
+    im = model(num_pix, 1, False, np.random.default_rng(3).normal(0.5, 0.1, (num_pix, num_pix)))
+    params, n, m, keep = packed(im, names, kw, None, False)
+    alone = im.likelihood_and_grad_batch(backend.to_device_f64(params), n, model=m)
+    for b in (2, 37, 300):
+        many = im.likelihood_and_grad_batch(backend.to_device_f64(np.repeat(params, b, axis=0)), b, model=m)
+        for a, v in zip(alone, many):
+            assert torch.equal(v[0], a[0]) and torch.equal(v[-1], a[0])
