@@ -3726,9 +3726,11 @@ int launch_conv_kernel(ConvArgs c, int n_img, const T *in, const double *kf, T *
 #define LENSIM_CONV(R, H, CLS, GW) launch_conv_f64<R, H, CLS, GW>(c, n_img, in, kf, out, partial, n_tiles, st)
     if (c.kx < 10 && fits(8, 4, 1, true, kMaxLds / 2) && fits(4, 4, 1, false, kMaxLds))
       return few ? LENSIM_CONV(4, 4, 1, false) : LENSIM_CONV(8, 4, 1, true);
-    if (few && fits(4, 2, 4, false, kMaxLds)) return LENSIM_CONV(4, 2, 4, false);
-    if (fits(16, 1, 4, true, kMaxLds / 2)) return LENSIM_CONV(16, 1, 4, true);
-    if (fits(16, 2, 4, true, kMaxLds)) return LENSIM_CONV(16, 2, 4, true);
+    // (a wide flat kernel whose tall tiles do not fit stays with conv_kernel in any batch)
+    const bool one = fits(16, 1, 4, true, kMaxLds / 2), two = fits(16, 2, 4, true, kMaxLds);
+    if (few && (one || two) && fits(4, 2, 4, false, kMaxLds)) return LENSIM_CONV(4, 2, 4, false);
+    if (one) return LENSIM_CONV(16, 1, 4, true);
+    if (two) return LENSIM_CONV(16, 2, 4, true);
 #undef LENSIM_CONV
   }
   constexpr int TX = ConvTile<T>::TX;

@@ -66,3 +66,19 @@ def test_gaussian_edge_mode_vs_oracle(num_pix):
     want = O.convolve_same(flat, im.kernel, mode="edge")
     got = im.image_batch(batches(im, 1), 1)[0].cpu().numpy()
     assert np.max(np.abs(got - want)) <= 1e-12 * np.max(want)
+
+
+@pytest.mark.parametrize("ky,kx", [(33, 167), (25, 183), (11, 251), (9, 251), (201, 9), (201, 21)])
+def test_long_kernels_are_the_same_in_any_batch(ky, kx):
+    """Kernels whose tiles come near the LDS in one form and not in another: the family follows the kernel alone."""
+    rng = np.random.default_rng(kx)
+    kernel = rng.random((ky, kx))
+    kernel /= kernel.sum()
+    cfg, im = model(40, PSF("PIXEL", kernel_point_source=kernel))
+    want = O.image(W.grid_dict(cfg), ["SIE"], LENS, ["SERSIC"], SOURCE, [], [], kernel=kernel)
+    im = model(40, PSF("PIXEL", kernel_point_source=kernel), 1.01 * want)[1]
+    params = batches(im, 70)
+    many, few = im.image_batch(params, 70), im.image_batch(params[:2].contiguous(), 2)
+    assert np.max(np.abs(few[0].cpu().numpy() - want)) <= 1e-10 * np.max(want)
+    assert torch.equal(many[:2], few)
+    assert torch.equal(im.likelihood_batch(params, 70)[:2], im.likelihood_batch(params[:2].contiguous(), 2))
