@@ -82,3 +82,18 @@ def test_long_kernels_are_the_same_in_any_batch(ky, kx):
     assert np.max(np.abs(few[0].cpu().numpy() - want)) <= 1e-10 * np.max(want)
     assert torch.equal(many[:2], few)
     assert torch.equal(im.likelihood_batch(params, 70)[:2], im.likelihood_batch(params[:2].contiguous(), 2))
+
+
+@pytest.mark.parametrize("num_pix,n", [(33, 512), (50, 520), (64, 512)])
+@pytest.mark.parametrize("ky,kx", [(3, 3), (9, 9), (11, 11), (15, 15), (15, 5), (5, 15), (1, 13), (13, 9)])
+def test_small_kernels_of_a_full_chip_are_the_same_in_any_batch(ky, kx, num_pix, n):
+    """Kernels below 16 x 16 over 2048 tiles or more (conv_kernel, class by class) against a few images' tiles."""
+    kernel = np.random.default_rng(kx + 16 * ky).random((ky, kx))
+    kernel /= kernel.sum()
+    im = model(num_pix, PSF("PIXEL", kernel_point_source=kernel), np.full((num_pix, num_pix), 0.3))[1]
+    params = batches(im, n)
+    two = params[:2].contiguous()
+    assert ((num_pix + 31) // 32) ** 2 * n >= 2048
+    assert torch.equal(im.image_batch(params, n)[:2], im.image_batch(two, 2))
+    for a, b in zip(im.likelihood_and_grad_batch(params, n), im.likelihood_and_grad_batch(two, 2)):
+        assert torch.equal(a[:2], b)
