@@ -97,13 +97,14 @@ typedef enum {
  * position: T_ij is 0 after the first, T_z and r2p are equal; a redshift with
  * m deflectors makes ceil(m / 64) of them.  max_runs is the largest number of
  * runs of any image, or more; 0 (or anything outside 1 .. n_planes - 2) counts
- * a run per deflector.  lensim_loglike_grad plans its workspace and launches by
- * it: 5256 deflectors on 126 redshifts take 49 MB of workspace with it and 1 GiB
- * without for 100^2 rays.  Arrays with more runs than max_runs > 0 have NaN for
- * the deflectors' gradients. */
+ * a run per deflector.  Long runs are shared among a block's waves by it (the
+ * results do not depend on it), and lensim_loglike_grad plans its workspace and
+ * launches: 5256 deflectors on 126 redshifts take 49 MB of workspace with it and
+ * 1 GiB without for 100^2 rays.  Arrays with more runs than max_runs > 0 have NaN
+ * for the deflectors' gradients. */
 typedef struct {
   int32_t n_planes;          /* deflector planes + 1 (the source) */
-  int32_t max_runs;          /* 0, or a bound on the number of plane runs (see below) */
+  int32_t max_runs;          /* 0, or a bound on the number of plane runs (see above) */
   const int32_t *d_order;    /* [n_planes - 1] deflector index (inline lens, then bulk) of each plane */
   const double *d_T_ij;      /* [n_img][n_planes] transverse comoving distance from the previous plane */
   const double *d_T_z;       /* [n_img][n_planes] transverse comoving distance from z = 0 */

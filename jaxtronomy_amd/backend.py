@@ -225,14 +225,19 @@ def plane_runs(t_ij, t_z, r2p):
     """lensim_multiplane.max_runs of plane arrays [n_planes] or [n_img, n_planes]: the
     most runs of any image (a run: up to 64 consecutive deflector planes with
     T_ij 0 after the first and one T_z and r2p)."""
-    t_ij, t_z, r2p = (np.asarray(a, dtype=np.float64)[..., :-1] for a in (t_ij, t_z, r2p))
-    if t_ij.shape[-1] == 0:
-        return 0
-    moved = (t_ij[..., 1:] != 0.0) | (t_z[..., 1:] != t_z[..., :-1]) | (r2p[..., 1:] != r2p[..., :-1])
+    t_ij, t_z, r2p = (np.atleast_2d(np.asarray(a, dtype=np.float64)) for a in (t_ij, t_z, r2p))
+    n = t_ij.shape[1] - 1
     most = 0
-    for row in np.atleast_2d(moved):
-        starts = np.concatenate(([-1], np.flatnonzero(row), [len(row)]))
-        most = max(most, int(((starts[1:] - starts[:-1] + 63) >> 6).sum()))
+    for i in range(t_ij.shape[0] if n else 0):
+        tz, f = t_z[i], r2p[i]
+        moved = t_ij[i, 1:n] != 0.0
+        moved |= tz[1:n] != tz[:n - 1]
+        moved |= f[1:n] != f[:n - 1]
+        ends = np.flatnonzero(moved) + 1  # where the next run starts
+        runs = ends.size + 1
+        if n > 64:
+            runs = int(((np.append(ends, n) - np.append(0, ends) + 63) >> 6).sum())
+        most = max(most, runs)
     return most
 
 

@@ -21,7 +21,6 @@
 
 #include <stdarg.h>
 #include <stdio.h>
-#include <stdlib.h>
 #include <string.h>
 
 #include <mutex>
@@ -422,9 +421,10 @@ Layout layout(const ModelArgs &m, int nx, int ny, int kx, int ky, int n_img, int
 // multi-plane model's runs (lensim_multiplane.max_runs), without one a run per
 // plane: the kernels take as many rays a round as the runs there are allow, and
 // what the plan has too many of ends at once.  splits: pieces a deflector's rays
-// of a round are cut into (a partial sum each, to which the rounds add), from 512
-// rays and so that about 2048 waves, and up to 16384 of 2048 rays, share an
-// image's deflectors.  Nothing but `imgs` depends on the batch, so a list's sums
+// of a round are cut into (a partial sum each, to which the rounds add): so that
+// about 2048 waves, and up to 16384 of 2048 rays, share an image's deflectors,
+// each 512 rays or, of up to 128 splits, 64 (two deflectors and 60^2 rays 85 us a
+// call with 512, 67 with 64; 100^2 x 4 108, 102 and, of 625 splits, 113).  Nothing but `imgs` depends on the batch, so a list's sums
 // on one plane have the same order in any.  The partial sums take imgs n splits
 // 64 B: with a pair of deflectors a wave at most 2 MB an image beside one sum
 // for each deflector.
@@ -447,7 +447,8 @@ DeflGradPlan defl_grad_plan(const ModelArgs &m, size_t rays, int n_img) {
   size_t sp = over(rays, 2048);
   if (sp > over(16384, pairs)) sp = over(16384, pairs);
   if (sp < over(2048, pairs)) sp = over(2048, pairs);
-  if (sp > over(rays, 512)) sp = over(rays, 512);
+  const size_t most = over(rays, 512) > 128 ? over(rays, 512) : over(rays, 64) < 128 ? over(rays, 64) : 128;
+  if (sp > most) sp = most;
   p.splits = int(sp < 2048 ? sp : 2048);
   return p;
 }
@@ -1150,7 +1151,6 @@ __global__ __launch_bounds__(256) void block_max_kernel(const T *__restrict__ v,
   block_max_store(a, blkmax + size_t(img) * gridDim.x + blockIdx.x);
 }
 
-constexpr int kMpBlock = 64;  // rays of a block of the multi-plane kernels (a lane each)
 // What a gradient keeps of its render for the adjoint kernels, so that the
 // rays are not traced again: several planes, per ray and run the position, and
 // beta; a bulk list that render_bulk_kernel takes, or in FP64 a model that
@@ -1323,6 +1323,7 @@ __device__ __forceinline__ double wave_sum(double v) {
 // one position.  A run is up to kMpRun consecutive planes with one position,
 // T_z and reduced-to-physical factor; it is the unit the kernels below work in.
 constexpr int kMpRun = 64;
+constexpr int kMpPrep = 1024;
 
 struct MpTab {  // see mp_tab_ints
   const int *start, *run_of, *plane_of, *who;
@@ -1341,14 +1342,15 @@ __device__ __forceinline__ MpTab mp_tab(const ModelArgs &m, const int *__restric
                t[1], t[2]};
 }
 
-// The runs of each set of plane arrays, one block per set: every thread takes
-// a contiguous piece of the planes; a maximum scan over the pieces gives the
-// plane the position last changed at, and so the planes that start a run
+// The runs of one set of plane arrays, by a block of NT threads: every thread
+// takes a contiguous piece of the planes; a maximum scan over the pieces gives
+// the plane the position last changed at, and so the planes that start a run
 // (there, and every kMpRun planes after), a sum scan their numbers.
-__global__ __launch_bounds__(1024) void mp_runs_kernel(ModelArgs m, int *__restrict__ tab_all) {
-  int *tab = tab_all + size_t(blockIdx.x) * mp_tab_ints(m);
-  const size_t o = size_t(blockIdx.x) * size_t(m.mp_stride);
-  const int nd = m.mp_n - 1, t = threadIdx.x, per = (nd + 1023) / 1024;
+template <int NT>
+__device__ __forceinline__ void mp_runs_block(const ModelArgs &m, int *__restrict__ tab_all, int set) {
+  int *tab = tab_all + size_t(set) * mp_tab_ints(m);
+  const size_t o = size_t(set) * size_t(m.mp_stride);
+  const int nd = m.mp_n - 1, t = threadIdx.x, per = (nd + NT - 1) / NT;
   const int q0 = min(nd, t * per), q1 = min(nd, q0 + per);
   int *start = tab + 3, *run_of = tab + 3 + m.mp_n, *plane_of = tab + 2 + 2 * m.mp_n;
   int *who = plane_of + m.n_defl;
@@ -1356,13 +1358,13 @@ __global__ __launch_bounds__(1024) void mp_runs_kernel(ModelArgs m, int *__restr
     return q == 0 || AT(m.mp_tij, o + q) != 0.0 || AT(m.mp_tz, o + q) != AT(m.mp_tz, o + q - 1) ||
            AT(m.mp_r2p, o + q) != AT(m.mp_r2p, o + q - 1);
   };
-  __shared__ int sc[2][1024];
+  __shared__ int sc[2][NT];
   __shared__ int dup, other;
   auto scan = [&](int v, auto op) {  // inclusive, over the threads
     sc[0][t] = v;
     __syncthreads();
     int b = 0;
-    for (int d = 1; d < 1024; d <<= 1, b ^= 1) {
+    for (int d = 1; d < NT; d <<= 1, b ^= 1) {
       sc[b ^ 1][t] = t >= d ? op(sc[b][t], sc[b][t - d]) : sc[b][t];
       __syncthreads();
     }
@@ -1388,10 +1390,10 @@ __global__ __launch_bounds__(1024) void mp_runs_kernel(ModelArgs m, int *__restr
     if ((q - at) % kMpRun == 0) AT(start, idx++) = q;
     AT(run_of, q) = idx - 1;
   }
-  for (int k = t; k < m.n_defl; k += 1024) AT(plane_of, k) = -1;
+  for (int k = t; k < m.n_defl; k += NT) AT(plane_of, k) = -1;
   if (t == 0) dup = other = 0;
   __syncthreads();
-  for (int k = t; m.n_bulk > 0 && !m.bulk_type && k < m.n_bulk; k += 1024)
+  for (int k = t; m.n_bulk > 0 && !m.bulk_type && k < m.n_bulk; k += NT)
     if (!sub_type(AT(m.bulk_types, k))) other = 1;
   for (int q = q0; q < q1; ++q) {
     int k = AT(m.mp_order, q);
@@ -1402,12 +1404,15 @@ __global__ __launch_bounds__(1024) void mp_runs_kernel(ModelArgs m, int *__restr
     AT(who, q) = k | type << kWhoBits;
   }
   __syncthreads();
-  if (t == 1023) {
+  if (t == NT - 1) {
     AT(start, s.x) = nd;
     AT(tab, 0) = s.x;
     AT(tab, 1) = dup;
     AT(tab, 2) = !other;
   }
+}
+__global__ __launch_bounds__(1024) void mp_runs_kernel(ModelArgs m, int *__restrict__ tab_all) {
+  mp_runs_block<1024>(m, tab_all, blockIdx.x);
 }
 
 int launch_mp_runs(const ModelArgs &m, int *tab, int n_img, hipStream_t st) {
@@ -1415,33 +1420,17 @@ int launch_mp_runs(const ModelArgs &m, int *tab, int n_img, hipStream_t st) {
   return check_launch("mp_runs_kernel");
 }
 
-// The sums of (vx, vy) over the block's waves, lane by lane, in every wave.
-// buf alternates between consecutive calls, so that no barrier is needed before
-// the write.  Up to eight waves each read all the waves' values (in wave
-// order); sixteen would each read 16 KB of LDS that way (2000 cycles a call),
-// so there a row of 16 lanes sums one ray's values and every wave reads the
-// sums, at the price of a second barrier.
-template <int W>  // waves at most: 8 or 16
-struct WaveSumsOf {
-  double2 part[2][W][65];  // rows of 65: the 16 values of a ray lie on distinct banks
-  double2 sum[W == 16 ? 2 : 1][64];
+// The sums of (vx, vy) over the block's waves (eight at most), lane by lane and
+// in wave order, in every wave.  buf alternates between consecutive calls, so
+// that no barrier is needed before the write.
+constexpr int kSumWaves = 8;
+struct WaveSums {
+  double2 part[2][kSumWaves][64];
 };
-using WaveSums = WaveSumsOf<16>;
-template <int W>
-__device__ __forceinline__ void across_waves(WaveSumsOf<W> &red, int buf, int nw, double &vx, double &vy) {
+__device__ __forceinline__ void across_waves(WaveSums &red, int buf, int nw, double &vx, double &vy) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   red.part[buf][wave][lane] = double2{vx, vy};
   __syncthreads();
-  if (W == 16 && nw == 16) {
-    const int ray = threadIdx.x >> 4, w = threadIdx.x & 15;
-    const double2 v = red.part[buf][w][ray];
-    const double2 s{row_sum(v.x), row_sum(v.y)};
-    if (w == 0) red.sum[buf][ray] = s;
-    __syncthreads();
-    vx = red.sum[buf][lane].x;
-    vy = red.sum[buf][lane].y;
-    return;
-  }
   vx = vy = 0.0;
   for (int w = 0; w < nw; ++w) {
     const double2 v = red.part[buf][w][lane];
@@ -1450,23 +1439,119 @@ __device__ __forceinline__ void across_waves(WaveSumsOf<W> &red, int buf, int nw
   }
 }
 
+// Classes that a run's deflectors are summed in (every classes-th of them, then
+// the classes): their number follows the image's rays and the list's length
+// alone, and with it the order of the sums, whatever launch does them
+// (mp_launch).  Measured: a line of sight of 5256 0.46 ms with 16, 0.52 with 8 for
+// 100^2 rays, 2.95 with 8, 4.2 with 16 for 400^2; 48 halos on 8 planes 10% more
+// with 4 than with 8 at 100^2 x 4 rays, the same or up to 30% less at 180^2 x 9;
+// 8 halos on 2 planes, 30 on 10 4 to 10% less.  Past 2^28 rays two, which keeps a
+// launch's threads below 2^32.
+__host__ __device__ inline int mp_classes(int n_defl, int64_t n_ray, bool sub) {
+  if (n_ray > (int64_t(1) << 28)) return 2;
+  if (n_defl >= 1024) return sub && n_ray < 65536 ? 16 : 8;
+  return n_defl > 32 && n_ray < 24576 ? 8 : 4;
+}
+
+// A wave of a multi-plane kernel and the 64 rays it holds.  The waves of a block
+// share their rays and take a class of a run each; SOLO: a block is one wave, which takes
+// the classes in turn, without a barrier.
+template <bool SOLO>
+struct MpWave {
+  int wave, nw, classes;
+  __device__ __forceinline__ explicit MpWave(int classes)
+      : wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)), nw(int(blockDim.x) >> 6), classes(classes) {}
+  __device__ __forceinline__ bool lead() const { return SOLO || wave == 0; }  // loads, adds and stores for the rays
+  __device__ __forceinline__ void barrier() const {
+    if constexpr (!SOLO) __syncthreads();
+  }
+};
+template <bool SOLO>
+struct MpRed {
+  double2 part[2][16][65];  // rows of 65: the 16 values of a ray lie on distinct banks
+  double2 sum[2][64];
+};
+template <>
+struct MpRed<true> {};
+
+// (vx, vy): the sum over a run's `len` members of what one(q, vx, vy) adds for
+// member q, in every wave that holds the rays.  buf alternates between
+// consecutive calls, so that no barrier is needed before the write.  Up to eight
+// classes are added in class order, each wave reading all of them; sixteen in
+// the order of row_sum (the quads of classes in pairs, (Q0 + Q3) + (Q2 + Q1)):
+// sixteen waves would each read 16 KB of LDS (2000 cycles a call), so there a
+// row of 16 lanes sums one ray's values and every wave reads the sums, at the
+// price of a second barrier.
+template <bool SUB, typename F>
+__device__ __forceinline__ void run_sum(const MpWave<false> &w, MpRed<false> &red, int buf, int len, double &vx, double &vy,
+                                        F one) {
+  const int lane = threadIdx.x & 63;
+  vx = vy = 0.0;
+  for (int q = w.wave; q < len; q += w.nw) one(q, vx, vy);
+  red.part[buf][w.wave][lane] = double2{vx, vy};
+  __syncthreads();
+  if (SUB && w.nw == 16) {
+    const int ray = threadIdx.x >> 4, c = threadIdx.x & 15;
+    const double2 v = red.part[buf][c][ray];
+    const double2 s{row_sum(v.x), row_sum(v.y)};
+    if (c == 0) red.sum[buf][ray] = s;
+    __syncthreads();
+    vx = red.sum[buf][lane].x;
+    vy = red.sum[buf][lane].y;
+    return;
+  }
+  vx = vy = 0.0;
+  for (int c = 0; c < w.nw; ++c) {
+    const double2 v = red.part[buf][c][lane];
+    vx += v.x;
+    vy += v.y;
+  }
+}
+// (Up to three members: their sum in order is that of either tree.)
+template <bool SUB, typename F>
+__device__ __forceinline__ void run_sum(const MpWave<true> &w, MpRed<true> &, int, int len, double &vx, double &vy, F one) {
+  const bool tree = SUB && w.classes == 16 && len > 3;
+  const int nt = tree ? 16 : min(len, w.classes);
+  double ax = 0.0, ay = 0.0, bx = 0.0, by = 0.0, dx = 0.0, dy = 0.0;  // a pair, a quad, Q0 + Q3
+  vx = vy = 0.0;
+  for (int t = 0; t < nt; ++t) {
+    const int c = !tree ? t : (t < 4 ? t : (t < 8 ? t + 8 : (t < 12 ? t : t - 8)));
+    double sx = 0.0, sy = 0.0;
+    for (int q = c; q < len; q += w.classes) one(q, sx, sy);
+    if (!tree) {
+      vx += sx;
+      vy += sy;
+      continue;
+    }
+    ax = t & 1 ? ax + sx : sx;
+    ay = t & 1 ? ay + sy : sy;
+    if (!(t & 1)) continue;
+    bx = t & 2 ? bx + ax : ax;
+    by = t & 2 ? by + ay : ay;
+    if (t == 3) dx = bx, dy = by;
+    if (t == 7) dx += bx, dy += by;
+    if (t == 11) vx = bx, vy = by;
+    if (t == 15) vx = dx + (vx + bx), vy = dy + (vy + by);
+  }
+}
+
 // Multi-plane ray tracing (MultiPlaneBulk.ray_shooting,
-// LensModel/MultiPlane/multi_plane_bulk.py:152-212) of 64 rays, one per lane,
-// by the whole block: each of its waves holds the same rays and takes every
-// nw-th deflector of a run, and the waves' sums meet in LDS once per run.  The
-// deflector is then the same for all lanes of a wave (its record comes by
-// scalar loads), 1 / T_z is taken once per run, and the chain of
-// record loads and deflections a ray waits for is nw times shorter: one lane
-// per ray left 400^2 rays at 2.4 waves per SIMD, waiting on memory for most of
-// a deflector's 1100 cycles.  Every thread of the block reaches this call.
+// LensModel/MultiPlane/multi_plane_bulk.py:152-212) of 64 rays, one per lane.
+// A run's deflectors are the same for all lanes of a wave (a record comes by
+// scalar loads) and 1 / T_z is taken once per run.  Shared by the block's waves,
+// the chain of record loads and deflections a ray waits for is as many times
+// shorter as the runs are long: one lane per ray left 400^2 rays through 5256
+// deflectors at 2.4 waves per SIMD, waiting on memory for most of a deflector's
+// 1100 cycles.  Runs of a deflector or two, or rays enough to fill the chip,
+// gain nothing by it and pay a barrier per run: solo (mp_shape).  Every thread
+// of a block that shares reaches this call.
 // each(c, x, y): run c's position, for callers that keep it.
-template <typename T, bool HALO, bool DBL, bool DBL_TNFW, bool SUB, typename F>
+template <typename T, bool HALO, bool DBL, bool DBL_TNFW, bool SUB, bool SOLO, typename F>
 __device__ __forceinline__ void block_trace(const ModelArgs &m, const RecPtrs<T> &rp, const MpTab &tab,
                                             const double *__restrict__ tij, const double *__restrict__ tzs,
                                             const double *__restrict__ r2p, int img, double x, double y,
-                                            WaveSums &red, double &bx, double &by, F each) {
-  const int lane = threadIdx.x & 63, nw = int(blockDim.x) >> 6;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+                                            const MpWave<SOLO> &w, MpRed<SOLO> &red, double &bx, double &by, F each) {
+  const int lane = threadIdx.x & 63;
   double angx = x, angy = y, px = 0.0, py = 0.0;
   // the deflectors of a run, a lane each, loaded one run ahead
   auto members = [&](int p0, int p1) { return p0 + lane < p1 ? AT(tab.who, p0 + lane) : 0; };
@@ -1481,12 +1566,11 @@ __device__ __forceinline__ void block_trace(const ModelArgs &m, const RecPtrs<T>
     py = fma(angy, dt, py);
     const double xr = px * itz, yr = py * itz;
     each(c, xr, yr);
-    double ax = 0.0, ay = 0.0;
-    for (int q = wave; q < p1 - p0; q += nw) {
+    double ax, ay;
+    run_sum<SUB>(w, red, c & 1, p1 - p0, ax, ay, [&](int q, double &sx, double &sy) {
       const int k = __builtin_amdgcn_readlane(ks, q);
-      deflect_one<T, HALO, DBL, DBL_TNFW, SUB>(m, rp, img, k & ((1 << kWhoBits) - 1), k >> kWhoBits, xr, yr, ax, ay);
-    }
-    across_waves(red, c & 1, nw, ax, ay);
+      deflect_one<T, HALO, DBL, DBL_TNFW, SUB>(m, rp, img, k & ((1 << kWhoBits) - 1), k >> kWhoBits, xr, yr, sx, sy);
+    });
     angx = fma(-ax, f, angx);
     angy = fma(-ay, f, angy);
     p0 = p1;
@@ -1507,41 +1591,65 @@ __device__ __forceinline__ void block_trace(const ModelArgs &m, const RecPtrs<T>
   const size_t mp_o = size_t(img) * size_t((m).mp_stride);              \
   const double *tij = (m).mp_tij + mp_o, *tzs = (m).mp_tz + mp_o, *r2p = (m).mp_r2p + mp_o
 
-// Waves per block for n rays an image: enough that a launch of one image
-// puts four or more waves on each SIMD where its deflectors allow it, and no
-// more, since a run is cut into as many pieces.  It depends on the image
-// alone (not on the batch), as the order of the sums does.  Measured on the
-// line of sight (400^2 rays): 3.42 ms a call with 8 waves, 3.50 with 4, 4.16
-// with 6; 100^2 rays render in 0.49 ms with 16.  Past 2^28 rays two, which keeps a launch's
-// threads below 2^32.
-int mp_waves(size_t n_ray, bool sub) {
-  if (n_ray > (size_t(1) << 28)) return 2;
-  return sub && n_ray < 65536 ? 16 : 8;
+// A launch over `some` of n_ray rays of n_img images: a wave per class, or solo.
+// Sharing gains where the runs are long and the chip is not full: solo are lists
+// of less than two deflectors a run (by the caller's bound, at least a run per
+// deflector without one), and from 4096 waves of rays (16 a CU; 2048 for lists
+// whose types take twice the registers) runs of less than four turns of the
+// classes.  Against a wave per class, and one lane per ray or quad over the whole
+// list before (us a call, FP64 images): seven deflectors on seven planes, 16 of
+// 180^2 x 9 rays 342, 2740, 335; 16 halos on one plane, one of 100^2 x 4 rays
+// 87, 37, 46, 32 of them 185, 225, 257; 40 of several types on 5 planes 16 of
+// 180^2 x 9 2000, 3880, 2450.
+struct MpLaunch {
+  bool solo;
+  unsigned threads;
+  dim3 grid;
+};
+MpLaunch mp_launch(const ModelArgs &m, size_t n_ray, size_t some, int n_img, bool sub) {
+  const int classes = mp_classes(m.n_defl, int64_t(n_ray), sub);
+  const size_t groups = (some + 63) / 64, all = groups * n_img;
+  MpLaunch l;
+  l.solo = m.n_defl < 2 * m.mp_runs || (all >= 2048 && !sub) ||
+           (all >= 4096 && m.n_defl < 4 * int64_t(classes) * m.mp_runs);
+  l.threads = l.solo ? 64 : 64 * classes;
+  l.grid = dim3((unsigned)groups, n_img);
+  return l;
 }
 
-template <typename T, bool HALO, bool DBL, bool SUB>
-__global__ __launch_bounds__(SUB ? 1024 : 512) void raytrace_mp_kernel(ModelArgs m, const double *__restrict__ recd,
+// Threads a block of a multi-plane kernel may have.
+constexpr int mp_threads_most(bool sub, bool solo) { return solo ? 64 : (sub ? 1024 : 512); }
+// Waves per SIMD the solo render is held to (its FP64 form without halos keeps
+// three so, as render_kernel's; the others would spill or have them anyway).
+template <typename T>
+constexpr int mp_render_waves(bool halo, bool solo) {
+  return sizeof(T) == sizeof(double) && !halo && solo ? 3 : 1;
+}
+
+template <typename T, bool HALO, bool DBL, bool SUB, bool SOLO>
+__global__ __launch_bounds__(mp_threads_most(SUB, SOLO)) void raytrace_mp_kernel(ModelArgs m, const double *__restrict__ recd,
                                                            const float *__restrict__ recf,
                                                            const double *__restrict__ coefd,
                                                            const float *__restrict__ coeff,
                                                            const int *__restrict__ tab_all,
                                                            const double *__restrict__ xs,
                                                            const double *__restrict__ ys, int64_t n_ray,
-                                                           int64_t first, bool both, double *__restrict__ bx,
-                                                           double *__restrict__ by) {
-  __shared__ WaveSums red;
+                                                           int64_t first, bool both,
+                                                           double *__restrict__ bx, double *__restrict__ by) {
+  __shared__ MpRed<SOLO> red;
   const int img = blockIdx.y;
-  const int64_t ray0 = first + int64_t(blockIdx.x) * kMpBlock + (threadIdx.x & 63);
+  const int64_t ray0 = first + int64_t(blockIdx.x) * 64 + (threadIdx.x & 63);
   const bool active = ray0 < n_ray;
   const int64_t ray = active ? ray0 : n_ray - 1;  // lanes past the end follow the last ray
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
   const MpTab tab = mp_tab(m, tab_all, img);
   if (both && bool(tab.sub) != SUB) return;  // the other instantiation's launch takes it
+  const MpWave<SOLO> w(mp_classes(m.n_defl, n_ray, SUB));
   LENSIM_MP_ARRAYS(m, img);
   double tx, ty;
-  block_trace<T, HALO, DBL, false, SUB>(m, rp, tab, tij, tzs, r2p, img, AT(xs, ray), AT(ys, ray), red, tx,
-                                        ty, [](int, double, double) {});
-  if (active && threadIdx.x < 64) {
+  block_trace<T, HALO, DBL, false, SUB, SOLO>(m, rp, tab, tij, tzs, r2p, img, AT(xs, ray), AT(ys, ray), w, red, tx, ty,
+                                              [](int, double, double) {});
+  if (active && w.lead()) {
     AT(bx, size_t(img) * n_ray + ray) = tx;
     AT(by, size_t(img) * n_ray + ray) = ty;
   }
@@ -1555,17 +1663,18 @@ __device__ __forceinline__ int64_t round_rays(size_t per_img, int runs) {
 
 // render_kernel for several planes: the block's waves walk the sub-rays of its
 // 64 pixels together (block_trace); the first wave adds the light and stores.
-template <typename T, bool HALO, bool DBL, bool SUB>
-__global__ __launch_bounds__(SUB ? 1024 : 512) void render_mp_kernel(ModelArgs m, GridArgs g, const double *__restrict__ recd,
+template <typename T, bool HALO, bool DBL, bool SUB, bool SOLO>
+__global__ __launch_bounds__(mp_threads_most(SUB, SOLO))
+__attribute__((amdgpu_waves_per_eu(mp_render_waves<T>(HALO, SOLO)))) void render_mp_kernel(ModelArgs m, GridArgs g, const double *__restrict__ recd,
                                                          const float *__restrict__ recf,
                                                          const double *__restrict__ coefd,
                                                          const float *__restrict__ coeff,
                                                          const int *__restrict__ tab_all, unsigned flags, bool both,
                                                          MpKeep keep, T *__restrict__ out) {
-  __shared__ WaveSums red;
+  __shared__ MpRed<SOLO> red;
   const int img = blockIdx.y;
   const int npix = g.nx * g.ny;
-  const int pix0 = blockIdx.x * kMpBlock + (threadIdx.x & 63);
+  const int pix0 = int(blockIdx.x * 64) + int(threadIdx.x & 63);
   const bool active = pix0 < npix;
   const int pix = active ? pix0 : npix - 1;
   int i;
@@ -1573,6 +1682,7 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void render_mp_kernel(ModelArgs m
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
   const MpTab tab = mp_tab(m, tab_all, img);
   if (both && bool(tab.sub) != SUB) return;  // the other instantiation's launch takes it
+  const MpWave<SOLO> w(mp_classes(m.n_defl, npix, SUB));
   LENSIM_MP_ARRAYS(m, img);
   const double ra_c = i * g.m00 + j * g.m01 + g.ra0;
   const double dec_c = i * g.m10 + j * g.m11 + g.dec0;
@@ -1581,9 +1691,9 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void render_mp_kernel(ModelArgs m
   const int k_src0 = m.n_defl, k_src1 = m.n_defl + m.n_source, k_l1 = m.n_prof;
   double acc = 0.0;
   const bool eval = active && evaluated(g, i, j);
-  const bool any = __any(eval);  // the same in every wave: they hold the same pixels
+  const bool any = __any(eval);  // the same in every wave that holds the pixels
   const int64_t cap = keep.store ? round_rays(keep.per_img, tab.n) : 0;
-  const bool keeps = active && threadIdx.x < 64 && cap >= int64_t(npix) * g.s * g.s;
+  const bool keeps = active && w.lead() && cap >= int64_t(npix) * g.s * g.s;
   for (int sy = 0; any && sy < g.s; ++sy) {
     const double oy = g.o0 + sy * g.inv_s;
     for (int sx = 0; sx < g.s; ++sx) {
@@ -1592,10 +1702,10 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void render_mp_kernel(ModelArgs m
       const double y = dec_c + g.m10 * ox + g.m11 * oy;
       double bx = x, by = y;
       if (do_src) {
-        __syncthreads();  // the last sub-ray's sums are read
+        w.barrier();  // the last sub-ray's sums are read
         const size_t ray = size_t(pix) * (g.s * g.s) + size_t(sy * g.s + sx);
-        block_trace<T, HALO, DBL, DBL, SUB>(
-            m, rp, tab, tij, tzs, r2p, img, x, y, red, bx, by, [&](int c, double xr, double yr) {
+        block_trace<T, HALO, DBL, DBL, SUB, SOLO>(
+            m, rp, tab, tij, tzs, r2p, img, x, y, w, red, bx, by, [&](int c, double xr, double yr) {
               if (keeps) AT(keep.store, size_t(img) * keep.per_img + ray + size_t(c) * cap) = double4{xr, yr, 0.0, 0.0};
             });
         if (keeps && keep.beta) {
@@ -1604,14 +1714,14 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void render_mp_kernel(ModelArgs m
           AT(b, 1) = T(by);
         }
       }
-      if (eval && threadIdx.x < 64) {
+      if (eval && w.lead()) {
         if (do_src) acc += light_sum<T>(m, rp, k_src0, k_src1, bx, by);
         if (do_light) acc += light_sum<T>(m, rp, k_src1, k_l1, x, y);
       }
     }
   }
   const T v = T(acc * (g.scale * m.flux_scaling));
-  if (active && threadIdx.x < 64) AT(out, size_t(img) * npix + pix) = v;
+  if (active && w.lead()) AT(out, size_t(img) * npix + pix) = v;
 }
 
 // Whether every deflector is a subhalo or linear (add_deflection's SUB): 1
@@ -1629,11 +1739,15 @@ int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, 
                      const float *coeff, const int *tab, unsigned flags, const MpKeep &keep, T *out, int n_img,
                      hipStream_t st) {
   const size_t npix = size_t(g.nx) * g.ny;
-  const dim3 grid((unsigned)((npix + kMpBlock - 1) / kMpBlock), n_img);
   const int sub = sub_list(m);
-#define LENSIM_RENDER(H, D, S)                                                                                \
-  render_mp_kernel<T, H, D, S><<<grid, 64 * mp_waves(npix, S), 0, st>>>(m, g, recd, recf, coefd, coeff, tab, \
-                                                                       flags, sub == 2, keep, out)
+  auto launch = [&](auto kernel, const MpLaunch &l) {
+    kernel<<<l.grid, l.threads, 0, st>>>(m, g, recd, recf, coefd, coeff, tab, flags, sub == 2, keep, out);
+  };
+#define LENSIM_RENDER(H, D, S)                                                                          \
+  do {                                                                                                  \
+    const MpLaunch l = mp_launch(m, npix, npix, n_img, S);                                              \
+    launch(l.solo ? &render_mp_kernel<T, H, D, S, true> : &render_mp_kernel<T, H, D, S, false>, l);     \
+  } while (0)
   // the float form deflects SIE / NIE and the NFW family in double
   constexpr bool kF32 = sizeof(T) == sizeof(float);
   if (sub) LENSIM_RENDER(true, kF32, true);
@@ -1660,7 +1774,7 @@ __global__ __launch_bounds__(512) void render_bulk_kernel(ModelArgs m, GridArgs 
                                                           const double *__restrict__ coefd,
                                                           const float *__restrict__ coeff, unsigned flags,
                                                           T *__restrict__ beta, T *__restrict__ out) {
-  __shared__ WaveSumsOf<8> red;
+  __shared__ WaveSums red;
   const int img = blockIdx.y, nw = blockDim.x >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int npix = g.nx * g.ny;
@@ -1750,10 +1864,14 @@ int launch_raytrace_mp(const ModelArgs &m, const double *recd, const float *recf
   constexpr int64_t kPiece = int64_t(1) << 28;
   for (int64_t r0 = 0; r0 < n_ray; r0 += kPiece) {
     const int64_t nr = n_ray - r0 < kPiece ? n_ray - r0 : kPiece;
-    const dim3 grid((unsigned)((nr + kMpBlock - 1) / kMpBlock), n_img);
-#define LENSIM_TRACE(H, D, S)                                                                              \
-  raytrace_mp_kernel<T, H, D, S><<<grid, 64 * mp_waves(size_t(n_ray), S), 0, st>>>(                        \
-      m, recd, recf, coefd, coeff, tab, x, y, n_ray, r0, sub == 2, bx, by)
+    auto launch = [&](auto kernel, const MpLaunch &l) {
+      kernel<<<l.grid, l.threads, 0, st>>>(m, recd, recf, coefd, coeff, tab, x, y, n_ray, r0, sub == 2, bx, by);
+    };
+#define LENSIM_TRACE(H, D, S)                                                                           \
+  do {                                                                                                  \
+    const MpLaunch l = mp_launch(m, size_t(n_ray), size_t(nr), n_img, S);                               \
+    launch(l.solo ? &raytrace_mp_kernel<T, H, D, S, true> : &raytrace_mp_kernel<T, H, D, S, false>, l); \
+  } while (0)
     // the float form keeps the float TNFW of a list without SIE / NIE or NFW
     // (rays within 2e-6 of FP64); those deflect in double (see nie_defl)
     if (sub) LENSIM_TRACE(true, false, true);
@@ -1832,6 +1950,15 @@ __device__ __forceinline__ double chi2_pixel(const ConvArgs &c, size_t p, T mode
   return chi;
 }
 
+// The chi^2 partial of 32 x 16 pixels, tile (txi, ty) of the image, by a wave: v
+// is lane l's sum of eight consecutive rows of column l % 32, in row order.
+__device__ __forceinline__ void tile_partial(const ConvArgs &c, double v, int lane, int img, int txi, int ty,
+                                             double *partial) {
+  v = wave_sum(v);
+  const int n = c.n_tiles_x * ((c.ny + 15) >> 4);
+  if (lane == 0 && 16 * ty < c.ny) AT(partial, size_t(img) * n + ty * c.n_tiles_x + txi) = v;
+}
+
 // out[y][x] = sum_{a,c} in[y - cy + a][x - cx + c] * Kf[a][c]  (Kf = flipped kernel).
 // Block = TX columns x (TY / kWin) row groups; each thread computes kWin
 // consecutive rows of one column from a register window that slides down the
@@ -1840,7 +1967,10 @@ __device__ __forceinline__ double chi2_pixel(const ConvArgs &c, size_t p, T mode
 // blocks than CUs: there each step's scalar loads of the weights would miss
 // the caches in turn (the kernel was just written by another launch), one
 // memory latency per step.
-template <typename T, int TY, bool LW>
+// CLS: 0, or conv_f64_kernel's classes of kernel columns for the same bits as
+// its (the columns class by class, the classes' sums in order) and its chi^2
+// partials.
+template <typename T, int TY, bool LW, int CLS>
 __global__ __launch_bounds__(256) void conv_kernel(ConvArgs c, const T *__restrict__ in,
                                                    const double *__restrict__ kt, T *__restrict__ out,
                                                    double *__restrict__ partial) {
@@ -1897,9 +2027,9 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs c, const T *__restri
   __syncthreads();
   const int lx = tid % TX, tg = tid / TX;
   // float64 accumulation in both forms (full-rate FMA on CDNA4)
-  double acc[kWin];
+  double acc[kWin], sum[kWin];  // sum: of the classes before
 #pragma unroll
-  for (int r = 0; r < kWin; ++r) acc[r] = 0.0;
+  for (int r = 0; r < kWin; ++r) acc[r] = sum[r] = 0.0;
   // steps t = (kernel column cc, row chunk ch) flattened; the window of step
   // t + 1 is loaded while step t is computed
   const T *colbase = tile + lx * THp + tg * kWin;
@@ -1911,9 +2041,15 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs c, const T *__restri
   for (int jj = 0; jj < kWin; ++jj) w[jj] = LW ? wl[jj] : kt[jj];
   int cc = 0, ch = 0;
   for (int t = 0; t < nsteps; ++t) {
+    bool next_class = false;
     if (++ch == nch) {
       ch = 0;
-      ++cc;
+      if (CLS > 1) {
+        next_class = cc + CLS >= c.kx;
+        cc = next_class ? cc % CLS + 1 : cc + CLS;
+      } else {
+        ++cc;
+      }
     }
     // next step's weights and window are requested before this step's FMAs
     // (the compiler still waits for them before the FMAs: the weights are
@@ -1924,9 +2060,9 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs c, const T *__restri
     if (t + 1 < nsteps) {
       if constexpr (LW) {
 #pragma unroll
-        for (int jj = 0; jj < kWin; ++jj) wn[jj] = wl[(t + 1) * kWin + jj];
+        for (int jj = 0; jj < kWin; ++jj) wn[jj] = wl[cc * kyp + ch * kWin + jj];
       } else {
-        const double *kw = kt + (t + 1) * kWin;  // = kt + cc * kyp + ch * kWin
+        const double *kw = kt + cc * kyp + ch * kWin;
 #pragma unroll
         for (int jj = 0; jj < kWin; ++jj) wn[jj] = kw[jj];
       }
@@ -1943,6 +2079,13 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs c, const T *__restri
     for (int q = 0; q < 2 * kWin - 1; ++q) buf[q] = double(nb[q]);
 #pragma unroll
     for (int jj = 0; jj < kWin; ++jj) w[jj] = wn[jj];
+    if (next_class) {
+#pragma unroll
+      for (int r = 0; r < kWin; ++r) {
+        sum[r] += acc[r];
+        acc[r] = 0.0;
+      }
+    }
   }
   const int x = x0 + lx;
   double chi = 0.0;
@@ -1952,14 +2095,16 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs c, const T *__restri
       const int y = y0 + tg * kWin + r;
       if (y < c.ny) {
         const size_t p = size_t(y) * c.nx + x;
-        const T m = T(acc[r]);
+        const T m = T(CLS > 1 ? sum[r] : acc[r]);
         if (out) AT(out, size_t(img) * c.nx * c.ny + p) = m;
         if (partial) chi += chi2_pixel<T>(c, p, m, img);
         if (c.gout) AT(static_cast<T *>(c.gout), size_t(img) * c.nx * c.ny + p) = T(dlogl_dm(c, p, double(m), img));
       }
     }
   }
-  if (partial) {
+  if (partial && CLS) {
+    tile_partial(c, chi, tid & 63, img, txi, (y0 >> 4) + (tid >> 6), partial);
+  } else if (partial) {
     // wave reduction then one value per wave through LDS (fixed order)
     for (int off = 32; off > 0; off >>= 1) chi += __shfl_xor(chi, off, 64);
     __syncthreads();
@@ -2136,7 +2281,7 @@ __global__ __launch_bounds__(64 * CLS * H) void conv_f64_kernel(ConvArgs c, int 
     double m = acc[i];
     if constexpr (CLS > 1) {
       const double *s = tile + (wave / CLS * CLS * R + r) * 64 + lane;
-      m = (s[0] + s[R * 64]) + (s[2 * R * 64] + s[3 * R * 64]);
+      m = ((s[0] + s[R * 64]) + s[2 * R * 64]) + s[3 * R * 64];
     }
     chi[i] = 0.0;
     if (x < c.nx && y < c.ny) {
@@ -2152,13 +2297,10 @@ __global__ __launch_bounds__(64 * CLS * H) void conv_f64_kernel(ConvArgs c, int 
     for (int i = 0; i < R / CLS; ++i) tile[(row0 + cls + CLS * i) * 32 + lx] = chi[i];
     __syncthreads();
     for (int q = wave; q < R * H / 8; q += CLS * H) {
-      const int ty = (y0 >> 4) + q;
       double v = 0.0;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v += tile[q * 512 + i * 64 + lane];
-      v = wave_sum(v);
-      const int n = c.n_tiles_x * ((c.ny + 15) >> 4);
-      if (lane == 0 && 16 * ty < c.ny) AT(partial, size_t(img) * n + ty * c.n_tiles_x + txi) = v;
+      for (int i = 0; i < 8; ++i) v += tile[(q * 16 + (lane >> 5) * 8 + i) * 32 + lx];
+      tile_partial(c, v, lane, img, txi, (y0 >> 4) + q, partial);
     }
   }
 }
@@ -2231,18 +2373,23 @@ int psf_job_blocks(const PsfJob &pj) {
   return 0;
 }
 
-// Blocks [0, nb_prep): one thread per (image, profile) record; the rest: the PSF job.
+// Blocks [0, nb_prep): one thread per (image, profile) record; [nb_prep, nb_prep
+// + nb_runs): a set of plane runs each; the rest: the PSF job.
 __global__ __launch_bounds__(256) void prep_psf_kernel(ModelArgs m, const double *__restrict__ params, int n_img,
                                                        double *__restrict__ recd, float *__restrict__ recf,
                                                        double *__restrict__ coefd, float *__restrict__ coeff,
                                                        double *__restrict__ dcoefd, float *__restrict__ dcoeff,
-                                                       PsfJob pj, int nb_prep) {
+                                                       PsfJob pj, int *__restrict__ tab, int nb_prep, int nb_runs) {
   if (int(blockIdx.x) < nb_prep) {
     const int idx = blockIdx.x * 256 + threadIdx.x;
     if (idx < n_img * m.n_prof) prep_one(m, params, n_img, idx, recd, recf, coefd, coeff, dcoefd, dcoeff);
     return;
   }
-  const int b = blockIdx.x - nb_prep;
+  if (int(blockIdx.x) < nb_prep + nb_runs) {
+    mp_runs_block<256>(m, tab, blockIdx.x - nb_prep);
+    return;
+  }
+  const int b = blockIdx.x - nb_prep - nb_runs;
   if (pj.mode == 2) {
     psf_mfma_prep_block(pj.k, pj.kx, pj.ky, pj.nks, pj.n_steps, pj.hdr, pj.frag, b);
   } else {
@@ -3179,18 +3326,18 @@ __device__ __forceinline__ void adjoint_one(const ModelArgs &m, const GradArgs &
 // share position and lambda: gA does not change where T is 0).  Each ray's beta
 // is stored too, for the source profiles' launches.  Bound by the runs' serial chain at few rays
 // (a barrier and the deflectors' records per run), by the vector ALU at many.
-template <typename T, bool HALO, bool SUB>
-__global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
+template <typename T, bool HALO, bool SUB, bool SOLO>
+__global__ __launch_bounds__(mp_threads_most(SUB, SOLO)) void mp_adjoint_kernel(
     ModelArgs m, GridArgs g, GradArgs ga, const double *__restrict__ recd, const float *__restrict__ recf,
     const double *__restrict__ coefd, const float *__restrict__ coeff, const int *__restrict__ tab_all, bool both,
     double4 *store, size_t per_img, int img0, int round, bool keeps, const double *__restrict__ all_tij,
     const double *__restrict__ all_tz, const double *__restrict__ all_r2p) {
-  __shared__ WaveSums red;
-  const int img = img0 + blockIdx.y, lane = threadIdx.x & 63, nw = int(blockDim.x) >> 6;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ MpRed<SOLO> red;
+  const int img = img0 + blockIdx.y, lane = threadIdx.x & 63;
   const MpTab tab = mp_tab(m, tab_all, img);
   if (both && bool(tab.sub) != SUB) return;  // the other instantiation's launch takes it
   const int64_t r_all = int64_t(g.nx) * g.ny * g.s * g.s;
+  const MpWave<SOLO> w(mp_classes(m.n_defl, r_all, SUB));
   const int64_t cap = round_rays(per_img, tab.n), in = int64_t(blockIdx.x) * 64;
   if (in >= cap || round * cap + in >= r_all) return;
   const int64_t first = round * cap + in;
@@ -3198,8 +3345,8 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
   const RecPtrs<T> rp = rec_ptrs<T>(m, recd, recf, coefd, coeff, img);
   const GradRay ray = grad_ray<T>(m, g, ga, img, first, active ? lane : int(r_all - 1 - first), active);
   double4 *st = store + size_t(blockIdx.y) * per_img + in + lane;  // this ray's entry of run c at st[c * cap]
-  if (!__any(ray.live)) {  // the same in every wave: they hold the same rays
-    for (int c = wave; c < tab.n; c += nw) AT(st, c * cap) = double4{0.0, 0.0, 0.0, 0.0};
+  if (!__any(ray.live)) {  // the same in every wave that holds the rays
+    for (int c = SOLO ? 0 : w.wave; c < tab.n; c += SOLO ? 1 : w.nw) AT(st, c * cap) = double4{0.0, 0.0, 0.0, 0.0};
     return;
   }
   const size_t o = size_t(img) * size_t(m.mp_stride);
@@ -3212,13 +3359,13 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
     }
   } else {
     double bxd, byd;
-    block_trace<T, HALO, true, true, SUB>(m, rp, tab, tij, tzs, r2p, img, ray.x, ray.y, red, bxd, byd,
+    block_trace<T, HALO, true, true, SUB, SOLO>(m, rp, tab, tij, tzs, r2p, img, ray.x, ray.y, w, red, bxd, byd,
                                           [&](int c, double x, double y) {
-                                            if (wave == 0) AT(st, c * cap) = double4{x, y, 0.0, 0.0};
+                                            if (w.lead()) AT(st, c * cap) = double4{x, y, 0.0, 0.0};
                                           });
     bx = T(bxd);
     by = T(byd);
-    if (ray.live && wave == 0) {
+    if (ray.live && w.lead()) {
       AT(b, 0) = bx;
       AT(b, 1) = by;
     }
@@ -3234,7 +3381,7 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
     gAx = dt * gPx;
     gAy = dt * gPy;
   }
-  __syncthreads();  // the positions are stored, the last sums read
+  w.barrier();  // the positions are stored, the last sums read
   auto members = [&](int p0, int p1) { return p0 + lane < p1 ? AT(tab.who, p0 + lane) : 0; };
   int c = tab.n - 1, p0 = AT(tab.start, c), p1 = AT(tab.start, c + 1);
   int ks = members(p0, p1);
@@ -3246,13 +3393,12 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
     const double4 at_next = AT(st, cn * cap);
     const double dt_next = AT(tij, q0), tz_next = AT(tzs, q0), f_next = AT(r2p, q0);
     const double lx = -f * gAx, ly = -f * gAy;
-    double jx = 0.0, jy = 0.0;
-    for (int q = wave; q < p1 - p0; q += nw) {
+    double jx, jy;
+    if (w.lead()) AT(st, c * cap) = double4{at.x, at.y, ray.live ? lx : 0.0, ray.live ? ly : 0.0};
+    run_sum<SUB>(w, red, c & 1, p1 - p0, jx, jy, [&](int q, double &sx, double &sy) {
       const int k = __builtin_amdgcn_readlane(ks, q);
-      adjoint_one<T, HALO, SUB>(m, ga, rp, img, k & ((1 << kWhoBits) - 1), k >> kWhoBits, at.x, at.y, lx, ly, jx, jy);
-    }
-    if (wave == 0) AT(st, c * cap) = double4{at.x, at.y, ray.live ? lx : 0.0, ray.live ? ly : 0.0};
-    across_waves(red, c & 1, nw, jx, jy);
+      adjoint_one<T, HALO, SUB>(m, ga, rp, img, k & ((1 << kWhoBits) - 1), k >> kWhoBits, at.x, at.y, lx, ly, sx, sy);
+    });
     gPx = fma(jx, itz, gPx);
     gPy = fma(jy, itz, gPy);
     gAx = fma(dt, gPx, gAx);
@@ -3273,13 +3419,13 @@ __global__ __launch_bounds__(SUB ? 1024 : 512) void mp_adjoint_kernel(
 // inline deflectors too); kept: the render kept beta, and the block is one
 // wave.  Stores (x, y, l), beta, and dS/dbeta for the inline
 // deflectors' launches.
-constexpr int kBulkWaves = 8;
+constexpr int kBulkWaves = kSumWaves;
 template <typename T, bool HALO>
 __global__ __launch_bounds__(64 * kBulkWaves) void bulk_adjoint_kernel(
     ModelArgs m, GridArgs g, GradArgs ga, const double *__restrict__ recd, const float *__restrict__ recf,
     const double *__restrict__ coefd, const float *__restrict__ coeff, double4 *__restrict__ store, size_t per_img,
     int img0, int round, bool kept) {
-  __shared__ WaveSumsOf<kBulkWaves> red;
+  __shared__ WaveSums red;
   const int img = img0 + blockIdx.y, lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t r_all = int64_t(g.nx) * g.ny * g.s * g.s;
@@ -3338,10 +3484,11 @@ __device__ __forceinline__ void tnfw_sums(const double *const (&rd)[2], const do
 // Partial sums [img - img0][plane or bulk index][split][8] of lambda . d alpha /
 // d kwargs over a round's rays, stored by the first round, to which the others
 // add: a wave takes two planes' (or bulk) deflectors
-// q, q + 1 and one of the splits of the rays.  REST: the deflectors that are
-// not subhalos or linear (their duals' registers would cost the others waves);
-// each launch leaves the other's deflectors alone.
-template <typename T, bool HALO, bool REST>
+// q, q + 1 and one of the splits of the rays.  SUBS: the subhalos and linear
+// deflectors; REST: the others, whose duals' registers would cost those waves.
+// A launch of one kind leaves the other's deflectors alone; a short list's two
+// kinds go in one launch (4 us less a call).
+template <typename T, bool HALO, bool SUBS, bool REST>
 __global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
                                                         const double *__restrict__ recd,
                                                         const float *__restrict__ recf,
@@ -3352,7 +3499,7 @@ __global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g,
                                                         int img0, int round, bool both,
                                                         double *__restrict__ gpart_mp) {
   const int img = img0 + blockIdx.y, lane = threadIdx.x & 63;
-  if (REST && both && m.mp_n && mp_tab(m, tab_all, img).sub) return;  // no such deflector
+  if (!SUBS && both && m.mp_n && mp_tab(m, tab_all, img).sub) return;  // no such deflector
   const int q = 2 * __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   if (q >= n) return;
   const int nq = min(2, n - q);
@@ -3382,7 +3529,7 @@ __global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g,
   const int64_t n_ray = left < 0 ? 0 : (left < cap ? left : cap);
   const int64_t len = ((n_ray + 63) / 64 + gridDim.z - 1) / gridDim.z * 64;
   const int64_t r0 = min(n_ray, len * blockIdx.z), r1 = min(n_ray, r0 + len);
-  if (r0 == r1 && (!REST || round)) {  // nothing of this round (REST's deflectors are stored over by its launch, after)
+  if (r0 == r1 && (SUBS || round)) {  // nothing of this round (REST's deflectors are stored over by its launch, after)
     if (!round && lane < nq * LENSIM_NPARAM) AT(part, lane / LENSIM_NPARAM * next + lane % LENSIM_NPARAM) = 0.0;
     return;
   }
@@ -3398,19 +3545,19 @@ __global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g,
 #pragma unroll
     for (int i = 0; i < LENSIM_NPARAM; ++i) acc[d][i] = 0.0;
   const bool pair = nq == 2 && type[0] == LENSIM_TNFW && type[1] == LENSIM_TNFW && run[0] == run[1];
-  if (!REST && pair) {
+  if (SUBS && pair) {
     if constexpr (HALO) tnfw_sums<2>(rd, st[0], r0, r1, lane, acc);
   } else {
     for (int d = 0; d < nq; ++d) {
       double a[2][LENSIM_NPARAM];
 #pragma unroll
       for (int i = 0; i < LENSIM_NPARAM; ++i) a[0][i] = 0.0;
-      if (!REST && type[d] == LENSIM_TNFW) {
+      if (SUBS && type[d] == LENSIM_TNFW) {
         if constexpr (HALO) {
           const double *const r[2] = {rd[d], rd[d]};
           tnfw_sums<1>(r, st[d], r0, r1, lane, a);
         }
-      } else if (!REST && (type[d] == LENSIM_CONVERGENCE || type[d] == LENSIM_SHEAR)) {
+      } else if (SUBS && (type[d] == LENSIM_CONVERGENCE || type[d] == LENSIM_SHEAR)) {
         const double cx = rd[d][R_CX], cy = rd[d][R_CY], c2 = rd[d][2], c3 = rd[d][3];
         const bool conv = type[d] == LENSIM_CONVERGENCE;
         for (int64_t r = r0 + lane; r < r1; r += 64) {
@@ -3446,7 +3593,7 @@ __global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g,
     }
   }
   for (int d = 0; d < nq; ++d) {
-    if (REST == sub_type(type[d])) continue;
+    if (sub_type(type[d]) ? !SUBS : !REST) continue;
     double v[LENSIM_NPARAM];
 #pragma unroll
     for (int i = 0; i < LENSIM_NPARAM; ++i) v[i] = wave_sum(d == 0 ? acc[0][i] : acc[1][i]);
@@ -3460,27 +3607,20 @@ __global__ __launch_bounds__(256) void defl_grad_kernel(ModelArgs m, GridArgs g,
   }
 }
 
-// The list's partial sums of images img0 .. img0 + n_img - 1 added up into the
-// first of the nblk slots grad_reduce_kernel reads (the others zero): eight
-// lanes a kwarg, lane j the splits j, j + 8, ..., then the lanes' sums in pairs.
-// A deflector that the caller's order names on several planes gets the sum over
+// A kwarg p of the list's deflector k of image img, summed over its splits
+// (gpart_mp: image li of the part of the batch that it holds): lane j of eight
+// takes the splits j, j + 8, ..., then the lanes' sums are added in pairs.  A
+// deflector that the caller's order names on several planes gets the sum over
 // them, one that it does not name zero; a model of more runs than the caller's
 // bound, whose rays the plan's rounds did not all take, NaN.
-__global__ __launch_bounds__(256) void defl_partial_reduce(ModelArgs m, const int *__restrict__ tab_all,
-                                                           const double *__restrict__ gpart_mp, int n, int splits,
-                                                           int runs, int img0, int n_img, int nblk,
-                                                           double *__restrict__ gpart) {
-  const int k0 = m.mp_n ? 0 : m.n_lens, nk = m.n_defl - k0;
-  const int64_t r = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (r >= int64_t(n_img) * nk) return;
-  const int p = threadIdx.x & 7, j = (threadIdx.x >> 3) & 7, li = int(r / nk), k = k0 + int(r - int64_t(li) * nk),
-            img = img0 + li;
+__device__ __forceinline__ double list_sum(const ModelArgs &m, const int *tab_all, const double *gpart_mp, int n,
+                                           int splits, int runs, int li, int img, int k, int p, int j) {
   double v = 0.0;
   auto add = [&](int q) {
     for (int b = j; b < splits; b += 8) v += AT(gpart_mp, ((size_t(li) * n + q) * splits + b) * LENSIM_NPARAM + p);
   };
   if (!m.mp_n) {
-    add(k - k0);
+    add(k - m.n_lens);
   } else {
     const MpTab tab = mp_tab(m, tab_all, img);
     if (tab.n > runs) {
@@ -3493,7 +3633,21 @@ __global__ __launch_bounds__(256) void defl_partial_reduce(ModelArgs m, const in
     }
   }
   for (int off = 8; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
-  const size_t o = (size_t(img) * m.n_prof + k) * nblk;
+  return v;
+}
+
+// The list's sums of images img0 .. img0 + n_img - 1 (a part of the batch) into
+// the first of the nblk slots grad_reduce_kernel reads, the others zero.
+__global__ __launch_bounds__(256) void defl_partial_reduce(ModelArgs m, const int *__restrict__ tab_all,
+                                                           const double *__restrict__ gpart_mp, int n, int splits,
+                                                           int runs, int img0, int n_img, int nblk,
+                                                           double *__restrict__ gpart) {
+  const int k0 = m.mp_n ? 0 : m.n_lens, nk = m.n_defl - k0;
+  const int64_t r = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (r >= int64_t(n_img) * nk) return;
+  const int p = threadIdx.x & 7, j = (threadIdx.x >> 3) & 7, li = int(r / nk), k = k0 + int(r - int64_t(li) * nk);
+  const double v = list_sum(m, tab_all, gpart_mp, n, splits, runs, li, img0 + li, k, p, j);
+  const size_t o = (size_t(img0 + li) * m.n_prof + k) * nblk;
   for (int b = j; b < nblk; b += 8) AT(gpart, (o + b) * LENSIM_NPARAM + p) = b == 0 ? v : 0.0;
 }
 
@@ -3505,7 +3659,7 @@ int launch_defl_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, 
   const size_t rays = size_t(g.nx) * g.ny * g.s * g.s;
   const DeflGradPlan p = defl_grad_plan(m, rays, n_img);
   // a round's rays (of several planes, as many as one run would leave): so a launch's threads stay below 2^32
-  const size_t most = p.n ? p.per_img : rays;
+  const size_t some = p.n && p.per_img < rays ? p.per_img : rays;
   int sub = sub_list(m);
   if (!m.mp_n && sub == 0) sub = m.bulk_type ? int(sub_type(m.bulk_type)) : 2;  // of the bulk list alone
   // of an inline list the types are known: a launch for the kinds it holds
@@ -3513,7 +3667,7 @@ int launch_defl_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, 
   for (int k = 0; m.mp_n && k < m.n_lens; ++k) any_sub = any_sub || sub_type(m.types[k]);
   for (int i0 = 0; i0 < n_img; i0 += p.imgs) {
     const int ni = n_img - i0 < p.imgs ? n_img - i0 : p.imgs;
-    const dim3 grid((unsigned)(((rays < most ? rays : most) + 63) / 64), ni);
+    const dim3 grid((unsigned)((some + 63) / 64), ni);
     const dim3 dgrid((p.n + 7) / 8, ni, p.splits);
     for (int r = 0; r < p.rounds; ++r) {
       if (!m.mp_n) {
@@ -3521,10 +3675,15 @@ int launch_defl_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, 
         bulk_adjoint_kernel<T, HALO><<<grid, kept ? 64 : 64 * kBulkWaves, 0, st>>>(
             m, g, ga, recd, recf, ga.coefd, ga.coeff, store, p.per_img, i0, r, kept);
       } else {
-#define LENSIM_ADJOINT(H, S)                                                                                         \
-  mp_adjoint_kernel<T, H, S><<<grid, 64 * mp_waves(rays, S), 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, \
-                                                                      sub == 2, store, p.per_img, i0, r,             \
-                                                                      p.imgs >= n_img, m.mp_tij, m.mp_tz, m.mp_r2p)
+        auto launch = [&](auto kernel, const MpLaunch &l) {
+          kernel<<<l.grid, l.threads, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, sub == 2, store, p.per_img,
+                                               i0, r, p.imgs >= n_img, m.mp_tij, m.mp_tz, m.mp_r2p);
+        };
+#define LENSIM_ADJOINT(H, S)                                                                          \
+  do {                                                                                                \
+    const MpLaunch l = mp_launch(m, rays, some, ni, S);                                               \
+    launch(l.solo ? &mp_adjoint_kernel<T, H, S, true> : &mp_adjoint_kernel<T, H, S, false>, l);       \
+  } while (0)
         if (sub) LENSIM_ADJOINT(true, true);
         if (sub != 1) LENSIM_ADJOINT(HALO, false);
 #undef LENSIM_ADJOINT
@@ -3532,15 +3691,20 @@ int launch_defl_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, 
       int rc = check_launch("adjoint kernel");
       if (rc) return rc;
       if (p.n == 0) continue;  // no deflector: beta alone
-      if (any_sub)
-        defl_grad_kernel<T, HALO, false><<<dgrid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, store,
-                                                                p.per_img, p.n, i0, r, sub == 2, gpart_mp);
-      if (sub != 1)
-        defl_grad_kernel<T, HALO, true><<<dgrid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, store,
-                                                               p.per_img, p.n, i0, r, sub == 2, gpart_mp);
+      auto sums = [&](auto kernel) {
+        kernel<<<dgrid, 256, 0, st>>>(m, g, ga, recd, recf, ga.coefd, ga.coeff, tab, store, p.per_img, p.n, i0, r,
+                                      sub == 2, gpart_mp);
+      };
+      const bool rest = sub != 1;
+      if (any_sub && rest && p.n <= 64) {
+        sums(&defl_grad_kernel<T, HALO, true, true>);
+      } else {
+        if (any_sub) sums(&defl_grad_kernel<T, HALO, true, false>);
+        if (rest) sums(&defl_grad_kernel<T, HALO, false, true>);
+      }
       if ((rc = check_launch("defl_grad_kernel"))) return rc;
     }
-    if (p.n == 0) continue;
+    if (p.n == 0 || p.imgs >= n_img) continue;  // (grad_reduce_kernel adds up the batch's sums)
     const int64_t nw = int64_t(ni) * (m.n_defl - (m.mp_n ? 0 : m.n_lens));
     defl_partial_reduce<<<(unsigned)((nw + 3) / 4), 256, 0, st>>>(m, tab, gpart_mp, p.n, p.splits, p.runs, i0, ni, nblk,
                                                                   ga.gpart);
@@ -3550,10 +3714,27 @@ int launch_defl_grad(const ModelArgs &m, const GridArgs &g, const GradArgs &ga, 
   return LENSIM_OK;
 }
 
-__global__ void grad_reduce_kernel(const double *__restrict__ gpart, int nblk, int n, double *__restrict__ grad) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;  // (img * n_prof + k) * 8 + q
-  if (idx >= n) return;
-  const int q = idx % LENSIM_NPARAM, ik = idx / LENSIM_NPARAM;
+// The gradient from the profiles' partials, a thread each; the first
+// list_blocks blocks: that of the list's deflectors from their splits, a wave
+// each (0: they are in gpart, or there is no list).
+__global__ __launch_bounds__(256) void grad_reduce_kernel(ModelArgs m, const int *__restrict__ tab_all,
+                                                          const double *__restrict__ gpart_mp, DeflGradPlan pl,
+                                                          int list_blocks, int n_img,
+                                                          const double *__restrict__ gpart, int nblk,
+                                                          double *__restrict__ grad) {
+  const int k0 = m.mp_n ? 0 : m.n_lens, nk = m.n_defl - k0;
+  if (int(blockIdx.x) < list_blocks) {
+    const int64_t r = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (r >= int64_t(n_img) * nk) return;
+    const int p = threadIdx.x & 7, j = (threadIdx.x >> 3) & 7, img = int(r / nk), k = k0 + int(r - int64_t(img) * nk);
+    const double v = list_sum(m, tab_all, gpart_mp, pl.n, pl.splits, pl.runs, img, img, k, p, j);
+    if (j == 0) AT(grad, (size_t(img) * m.n_prof + k) * LENSIM_NPARAM + p) = v;
+    return;
+  }
+  const int idx = (blockIdx.x - list_blocks) * 256 + threadIdx.x;  // (img * n_prof + k) * 8 + q
+  if (idx >= n_img * m.n_prof * LENSIM_NPARAM) return;
+  const int q = idx % LENSIM_NPARAM, ik = idx / LENSIM_NPARAM, k = ik % m.n_prof;
+  if (list_blocks && k >= k0 && k < m.n_defl) return;
   double s = 0.0;
   for (int b = 0; b < nblk; ++b) s += AT(gpart, (size_t(ik) * nblk + b) * LENSIM_NPARAM + q);
   AT(grad, idx) = s;
@@ -3680,15 +3861,15 @@ size_t conv_smem(int kx, int kyp, int ty = ConvTile<T>::TY) {
 // to *n_tiles): 64-row tiles where their LDS fits (four waves a block, a
 // smaller share of halo rows), 32-row tiles otherwise.  FP64 images go to
 // conv_f64_kernel as long as its tile fits the LDS.
-template <typename T, int TY, bool LW>
+template <typename T, int TY, bool LW, int CLS = 0>
 int launch_conv_tile(const ConvArgs &c, dim3 grid, size_t smem, const T *in, const double *kf, T *out,
                      double *partial, hipStream_t st) {
   if (smem > 65536) {  // dynamic LDS beyond 64 KB needs the kernel attribute raised first
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&conv_kernel<T, TY, LW>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&conv_kernel<T, TY, LW, CLS>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, int(smem));
     if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(conv_kernel)");
   }
-  conv_kernel<T, TY, LW><<<grid, ConvTile<T>::TX * TY / kWin, smem, st>>>(c, in, kf, out, partial);
+  conv_kernel<T, TY, LW, CLS><<<grid, ConvTile<T>::TX * TY / kWin, smem, st>>>(c, in, kf, out, partial);
   return check_launch("conv_kernel");
 }
 
@@ -3712,20 +3893,33 @@ template <typename T>
 int launch_conv_kernel(ConvArgs c, int n_img, const T *in, const double *kf, T *out, double *partial,
                        int *n_tiles, hipStream_t st) {
   if constexpr (sizeof(T) == sizeof(double)) {
-    // conv_f64_kernel by the number of 32 x 32 tiles (fewer than CUs: short
-    // tiles, weights in LDS) and its LDS; classes of kernel columns by the
-    // kernel alone, so that an image's sums are the same in any batch: below
-    // ten columns the split's barriers cost more than the work it shares (5 x
-    // 5, 64 images of 180^2, 57.5 against 67.7 us a call; 11 x 11 73 in both,
-    // one image of 60^2 19.4 against 21.5).  One block of 82 KB LDS or more
-    // fills a CU: there two row groups of waves (81 x 81, 743 against 918 us).
-    const bool few = size_t((c.nx + 31) / 32) * ((c.ny + 31) / 32) * n_img < 256;
+    // Classes of kernel columns by the kernel alone, so that an image's sums are
+    // the same in any batch: below ten columns the split's barriers cost more
+    // than the work it shares (5 x 5, 64 images of 180^2, 57.5 against 67.7 us a
+    // call; one image of 60^2 with 11 x 11 19.4 with, 21.5 without).  The shape
+    // by the number of 32 x 32 tiles and the LDS: with fewer tiles than CUs short
+    // ones, weights in LDS; from 2048 tiles (eight a CU) kernels below 16 x 16 go
+    // to conv_kernel in the same order, whose waves hold fewer registers (64
+    // images of 180^2 with 15 x 15 74.6 against 80.4 us a call, 128 120.8 against
+    // 145; at 1024 tiles, 256 of 60^2, 46.5 against 43.9).  One block of 82 KB
+    // LDS or more fills a CU: there two row groups of waves (81 x 81, 743 against
+    // 918 us).
+    const size_t tiles = size_t((c.nx + 31) / 32) * ((c.ny + 31) / 32) * n_img;
+    const bool few = tiles < 256;
     auto fits = [&](int r, int h, int cls, bool gw, size_t lds) {
       return conv_f64_smem(c.kx, c.ky, r, h, cls, gw) <= lds;
     };
+    if (c.kx < 16 && c.ky < 16 && tiles >= 2048) {
+      c.n_tiles_x = (c.nx + 31) / 32;
+      *n_tiles = c.n_tiles_x * ((c.ny + 15) / 16);
+      const dim3 grid(c.n_tiles_x * ((c.ny + 63) / 64), n_img);
+      const size_t smem = conv_smem<T>(c.kx, c.kyp, 64);
+      return c.kx < 10 ? launch_conv_tile<T, 64, false, 1>(c, grid, smem, in, kf, out, partial, st)
+                       : launch_conv_tile<T, 64, false, 4>(c, grid, smem, in, kf, out, partial, st);
+    }
 #define LENSIM_CONV(R, H, CLS, GW) launch_conv_f64<R, H, CLS, GW>(c, n_img, in, kf, out, partial, n_tiles, st)
     if (c.kx < 10 && fits(8, 4, 1, true, kMaxLds / 2) && fits(4, 4, 1, false, kMaxLds))
-      return few ? LENSIM_CONV(4, 4, 1, false) : LENSIM_CONV(8, 4, 1, true);
+      return LENSIM_CONV(4, 4, 1, false);
     // (a wide flat kernel whose tall tiles do not fit stays with conv_kernel in any batch)
     const bool one = fits(16, 1, 4, true, kMaxLds / 2), two = fits(16, 2, 4, true, kMaxLds);
     if (few && (one || two) && fits(4, 2, 4, false, kMaxLds)) return LENSIM_CONV(4, 2, 4, false);
@@ -3825,18 +4019,22 @@ struct ConvChoice {
   }
 };
 
-// The records (with EPL coefficients' derivatives when dc) and the PSF
-// preparation in one launch; the plane runs of a multi-plane model in another.
+// The records (with EPL coefficients' derivatives when dc), the PSF
+// preparation and the runs of up to kMpPrep planes in one launch (4 us less a call
+// of a few deflectors); the runs of more, which want a block's 1024 threads, in
+// another.
 int launch_prep_psf(const ModelArgs &m, const double *params, int n_img, const PsfJob &pj, bool dc, unsigned char *ws,
                     const Layout &L, hipStream_t st) {
   const int nb_prep = (n_img * m.n_prof + 255) / 256;
-  prep_psf_kernel<<<nb_prep + psf_job_blocks(pj), 256, 0, st>>>(
+  const int nb_runs = m.mp_n > 0 && m.mp_n <= kMpPrep ? int(mp_tab_sets(m, n_img)) : 0;
+  int *tab = reinterpret_cast<int *>(ws + L.mp_tab);
+  prep_psf_kernel<<<nb_prep + nb_runs + psf_job_blocks(pj), 256, 0, st>>>(
       m, params, n_img, reinterpret_cast<double *>(ws + L.recd), reinterpret_cast<float *>(ws + L.recf),
       reinterpret_cast<double *>(ws + L.coefd), reinterpret_cast<float *>(ws + L.coeff),
       dc ? reinterpret_cast<double *>(ws + L.dcoefd) : nullptr, dc ? reinterpret_cast<float *>(ws + L.dcoeff) : nullptr,
-      pj, nb_prep);
+      pj, tab, nb_prep, nb_runs);
   int rc = check_launch("prep_psf_kernel");
-  if (!rc && m.mp_n) rc = launch_mp_runs(m, reinterpret_cast<int *>(ws + L.mp_tab), n_img, st);
+  if (!rc && m.mp_n > 0 && !nb_runs) rc = launch_mp_runs(m, tab, n_img, st);
   return rc;
 }
 
@@ -4265,7 +4463,12 @@ int run_grad(const ModelArgs &m, const GridArgs &g, const lensim_psf *psf, int k
     if (rc) return rc;
   }
   const int n = n_img * m.n_prof * LENSIM_NPARAM;
-  grad_reduce_kernel<<<(n + 255) / 256, 256, 0, st>>>(ga.gpart, nblk, n, grad);
+  const DeflGradPlan pl = defl_grad_plan(m, size_t(gg.nx) * gg.ny * gg.s * gg.s, n_img);
+  const int64_t rows = pl.n && pl.imgs >= n_img ? int64_t(n_img) * (m.n_defl - (m.mp_n ? 0 : m.n_lens)) : 0;
+  const int list_blocks = int((rows + 3) / 4);
+  grad_reduce_kernel<<<list_blocks + (n + 255) / 256, 256, 0, st>>>(
+      m, reinterpret_cast<const int *>(ws + L.mp_tab), reinterpret_cast<const double *>(ws + L.gpart_mp), pl, list_blocks,
+      n_img, ga.gpart, nblk, grad);
   return check_launch("grad_reduce_kernel");
 }
 
@@ -4897,7 +5100,10 @@ int lensim_raytrace(const lensim_model *model, const double *d_params, int32_t n
   cr.add(d_beta_y, size_t(n_img) * size_t(n_ray) * sizeof(double));
   cr.add(ws, L.total);
   if ((rc = cr.begin(st))) return rc;
-  if ((rc = launch_prep(m, d_params, n_img, w, L, st))) return cr.end(st, rc);
+  const bool runs_in_prep = m.mp_n > 0 && m.mp_n <= kMpPrep;
+  rc = runs_in_prep ? launch_prep_psf(m, d_params, n_img, PsfJob{}, false, w, L, st)
+                    : launch_prep(m, d_params, n_img, w, L, st);
+  if (rc) return cr.end(st, rc);
   dim3 grid((unsigned)((n_ray + 255) / 256), n_img);
   const double *recd = reinterpret_cast<const double *>(w + L.recd);
   const float *recf = reinterpret_cast<const float *>(w + L.recf);
@@ -4905,7 +5111,7 @@ int lensim_raytrace(const lensim_model *model, const double *d_params, int32_t n
   const float *coeff = reinterpret_cast<const float *>(w + L.coeff);
   if (m.mp_n) {
     int *tab = reinterpret_cast<int *>(w + L.mp_tab);
-    if ((rc = launch_mp_runs(m, tab, n_img, st))) return cr.end(st, rc);
+    if (!runs_in_prep && (rc = launch_mp_runs(m, tab, n_img, st))) return cr.end(st, rc);
     rc = precision == LENSIM_FP64 ? launch_raytrace_mp<double>(m, recd, recf, coefd, coeff, tab, d_x, d_y, n_ray, n_img,
                                                                d_beta_x, d_beta_y, st)
                                   : launch_raytrace_mp<float>(m, recd, recf, coefd, coeff, tab, d_x, d_y, n_ray, n_img,

@@ -4,8 +4,15 @@ the oracle's plane scan."""
 
 import numpy as np
 import pytest
+import torch
 
+from jaxtronomy_amd import backend
+from jaxtronomy_amd import workloads as W
+from jaxtronomy_amd.Data.imaging_data import ImageData
+from jaxtronomy_amd.Data.psf import PSF
+from jaxtronomy_amd.ImSim.image_model import ImageModel
 from jaxtronomy_amd.LensModel.lens_model_bulk import LensModelBulk
+from jaxtronomy_amd.LightModel.light_model import LightModel
 from oracle import lensim_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -70,3 +77,33 @@ def test_two_models_with_their_own_distances():
         sx, sy = lm.ray_shooting(x, y, rs)
         assert np.array_equal(bx[i].cpu().numpy(), sx.cpu().numpy())
         assert np.array_equal(by[i].cpu().numpy(), sy.cpu().numpy())
+
+
+@pytest.mark.parametrize("counts,with_sie,n_img", [((16,), False, 70), ((3, 3, 2), False, 70), ((20, 20), False, 70),
+                                                   ((55,) * 20, False, 70), ((3, 2, 1), True, 40), ((30, 40), True, 40),
+                                                   ((1, 1, 1, 1), True, 40)])
+def test_same_bits_alone_and_in_a_batch_that_fills_the_chip(counts, with_sie, n_img):
+    """4, 8 and 16 classes shared by a block's waves (one image) and in turn in one wave (many): images, likelihoods
+    and gradients."""
+    names, kw, z = scene(counts, with_sie, 9)
+    cfg = dict(W.EPL180, numPix=64, deltaPix=0.1, supersampling=1)
+    data = np.random.default_rng(0).normal(0.5, 0.1, (64, 64))
+    lm = LensModelBulk(UNIQUE, multi_plane=True)
+    im = ImageModel(ImageData(**W.data_kwargs(cfg, data)), PSF("NONE"), lm, LightModel(["SERSIC"]))
+    rs = lm.prepare_ray_shooting_kwargs(names, kw, z_source=5.0, lens_redshift_list=z)
+    params, n, m, keep = im.pack_bulk(rs, [dict(amp=20.0, R_sersic=0.4, n_sersic=1.5, center_x=0.05, center_y=0.03)])
+    many = np.repeat(params, n_img, axis=0)
+    many[:, 0, 0] *= 1.0 + 1e-3 * np.arange(n_img)
+    many = backend.to_device_f64(many)
+    two = many[:2].contiguous()
+    for call in (im.image_batch, im.likelihood_batch):
+        assert torch.equal(call(many, n_img, model=m)[:2], call(two, 2, model=m))
+    for a, b in zip(im.likelihood_and_grad_batch(many, n_img, model=m), im.likelihood_and_grad_batch(two, 2, model=m)):
+        assert torch.equal(a[:2], b)
+    x, y = np.meshgrid(np.linspace(-3, 3, 520), np.linspace(-3, 3, 520))  # 4225 waves of rays
+    bx, by = lm.ray_shooting(x, y, rs)
+    for i in (0, 519):  # as one image of as many rays, whose order is the same, in another launch
+        sx, sy = lm.ray_shooting(np.vstack([x[i:i + 1]] * 2), np.vstack([y[i:i + 1]] * 2), rs)
+        scale = float((bx[i] - sx[0]).abs().max()), float((by[i] - sy[0]).abs().max())
+        assert max(scale) <= 1e-12
+    del keep
