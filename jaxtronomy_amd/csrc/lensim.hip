@@ -1166,7 +1166,7 @@ int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, 
                      const float *coeff, const int *tab, unsigned flags, const MpKeep &keep, T *out, int n_img,
                      hipStream_t st);
 
-int bulk_waves(const ModelArgs &m, size_t npix);
+int bulk_classes(const ModelArgs &m, size_t npix);
 template <typename T>
 int launch_render_bulk(const ModelArgs &m, const GridArgs &g, const double *recd, const float *recf,
                        const double *coefd, const float *coeff, unsigned flags, const MpKeep &keep, T *out, int n_img,
@@ -1210,7 +1210,7 @@ int launch_render(const ModelArgs &m, const GridArgs &g, const double *recd, con
   const dim3 rgrid((g.nx * g.ny + 255) / 256, n_img);
   int d0, d1;
   const bool fast = fast_model<T>(m, flags, d0, d1);
-  const bool share = !m.mp_n && (flags & LENSIM_IMAGE_SOURCE) && bulk_waves(m, size_t(g.nx) * g.ny) > 1;
+  const bool share = !m.mp_n && (flags & LENSIM_IMAGE_SOURCE) && bulk_classes(m, size_t(g.nx) * g.ny) > 1;
   if (m.mp_n || share) {  // the block maxima for the MFMA convolution follow from the image in a second launch
     int rc = share ? launch_render_bulk<T>(m, g, recd, recf, coefd, coeff, flags, keep, out, n_img, st)
                    : launch_render_mp<T>(m, g, recd, recf, coefd, coeff, tab, flags, keep, out, n_img, st);
@@ -1425,7 +1425,7 @@ int launch_mp_runs(const ModelArgs &m, int *tab, int n_img, hipStream_t st) {
 // that no barrier is needed before the write.
 constexpr int kSumWaves = 8;
 struct WaveSums {
-  double2 part[2][kSumWaves][64];
+  double2 part[2][kSumWaves][65];  // (rows of 64 measured 2% slower on 16 images of 300^2 and 1000 subhalos)
 };
 __device__ __forceinline__ void across_waves(WaveSums &red, int buf, int nw, double &vx, double &vy) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1767,14 +1767,19 @@ int launch_render_mp(const ModelArgs &m, const GridArgs &g, const double *recd, 
 // A lane per pixel alone leaves 4 images of 100^2 at less than one wave per
 // SIMD, each waiting out 200 deflectors' latency four times over (479 us; 275
 // so, and the adjoint kernel's 204 us of deflections fall away with the beta
-// kept here: a gradient 989 -> 605 us).  beta: see MpKeep.
-template <typename T, bool HALO, bool DBL>
-__global__ __launch_bounds__(512) void render_bulk_kernel(ModelArgs m, GridArgs g, const double *__restrict__ recd,
+// kept here: a gradient 989 -> 605 us).  Where the pixels fill the chip by
+// themselves the shared form idles seven waves of eight through the light and
+// waits at its barriers (64 halos, 128 images of 150^2 in mixed form 2.2 -> 2.9
+// ms against render_kernel):
+// SOLO: a block is one wave, which takes the classes in turn and adds them in the
+// same order (2.1 ms).  beta: see MpKeep.
+template <typename T, bool HALO, bool DBL, bool SOLO>
+__global__ __launch_bounds__(SOLO ? 64 : 512) void render_bulk_kernel(ModelArgs m, GridArgs g, const double *__restrict__ recd,
                                                           const float *__restrict__ recf,
                                                           const double *__restrict__ coefd,
                                                           const float *__restrict__ coeff, unsigned flags,
-                                                          T *__restrict__ beta, T *__restrict__ out) {
-  __shared__ WaveSums red;
+                                                          int classes, T *__restrict__ beta, T *__restrict__ out) {
+  __shared__ std::conditional_t<SOLO, char, WaveSums> red;
   const int img = blockIdx.y, nw = blockDim.x >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int npix = g.nx * g.ny;
@@ -1800,8 +1805,20 @@ __global__ __launch_bounds__(512) void render_bulk_kernel(ModelArgs m, GridArgs 
     double ax = 0.0, ay = 0.0;
     if (wave == 0)
       for (int k = 0; k < m.n_lens; ++k) deflect_one<T, HALO, DBL>(m, rp, img, k, m.types[k], x, y, ax, ay);
-    deflect_bulk<T, HALO, DBL>(m, rp, x, y, ax, ay, wave, nw);
-    across_waves(red, r & 1, nw, ax, ay);
+    if constexpr (SOLO) {
+      double tx = 0.0, ty = 0.0;
+      for (int c = 0; c < classes; ++c) {
+        deflect_bulk<T, HALO, DBL>(m, rp, x, y, ax, ay, c, classes);
+        tx += ax;
+        ty += ay;
+        ax = ay = 0.0;
+      }
+      ax = tx;
+      ay = ty;
+    } else {
+      deflect_bulk<T, HALO, DBL>(m, rp, x, y, ax, ay, wave, nw);
+      across_waves(red, r & 1, nw, ax, ay);
+    }
     if (wave == 0 && eval) {
       const double bx = x - ax * m.alpha_scaling, by = y - ay * m.alpha_scaling;
       if (beta) {
@@ -1816,13 +1833,14 @@ __global__ __launch_bounds__(512) void render_bulk_kernel(ModelArgs m, GridArgs 
   if (active && wave == 0) AT(out, size_t(img) * npix + pix) = T(acc * (g.scale * m.flux_scaling));
 }
 
-// Waves that share a bulk list's pixels (render_bulk_kernel), 1 for
-// render_kernel: enough for one image to put four waves on each SIMD while
-// each takes eight deflectors or more.  It depends on the image alone (not on
-// the batch), as the order of the sums does.  Measured with 1 / 2 / 4 / 8
-// waves: 16 mixed images of 300^2 and 1000 subhalos 21.8 / 21.5 / 20.95 / 22.2
-// ms a call, 4 gradients of 100^2 and 200 in FP64 1010 / 684 / 605 / 604 us.
-int bulk_waves(const ModelArgs &m, size_t npix) {
+// Classes that a bulk list is summed in (every classes-th deflector, then the
+// classes) by render_bulk_kernel, 1 for render_kernel: as many waves for one
+// image as put four on each SIMD while each takes eight deflectors or more.
+// They depend on the image alone (not on the batch), as the order of the sums
+// does.  Measured with 1 / 2 / 4 / 8 waves: 16 mixed images of 300^2 and 1000
+// subhalos 21.8 / 21.5 / 20.95 / 22.2 ms a call, 4 gradients of 100^2 and 200 in
+// FP64 1010 / 684 / 605 / 604 us.
+int bulk_classes(const ModelArgs &m, size_t npix) {
   int nw = 1;
   while (m.mp_n == 0 && m.n_source > 0 && nw < 8 && npix * nw < 64 * 4096 && m.n_bulk >= 16 * nw) nw *= 2;
   return nw;
@@ -1832,7 +1850,7 @@ int bulk_waves(const ModelArgs &m, size_t npix) {
 // not where the float form renders in double what the adjoint takes in float.
 template <typename T>
 bool bulk_keeps(const ModelArgs &m, size_t npix) {
-  return bulk_waves(m, npix) > 1 && (sizeof(T) == sizeof(double) || !m.has_nie_nfw);
+  return bulk_classes(m, npix) > 1 && (sizeof(T) == sizeof(double) || !m.has_nie_nfw);
 }
 
 template <typename T>
@@ -1841,9 +1859,22 @@ int launch_render_bulk(const ModelArgs &m, const GridArgs &g, const double *recd
                        hipStream_t st) {
   const size_t npix = size_t(g.nx) * g.ny;
   const dim3 grid((unsigned)((npix + 63) / 64), n_img);
-#define LENSIM_RENDER(H, D)                                                                               \
-  render_bulk_kernel<T, H, D><<<grid, 64 * bulk_waves(m, npix), 0, st>>>(m, g, recd, recf, coefd, coeff, \
-                                                                         flags, static_cast<T *>(keep.beta), out)
+  const int classes = bulk_classes(m, npix);
+  // Solo where the pixels' waves alone are one and a half times what the chip
+  // holds (2 a SIMD of the forms that deflect in double, 4 of the float one; of
+  // the float form's long lists, whose last waves leave the chip idle longer,
+  // eight times).  Shared against solo: 64 halos in FP64, 16 images of 100^2 x 4
+  // rays 350, 372 us, 32 of them 677, 562, 128 of 150^2 5530, 4120; in mixed form
+  // 223, 273, 407, 417, 2910, 2140; 1000 in mixed form, 16 of 300^2 x 9 30.2, 30.9
+  // ms, 128 of 150^2 x 4 33.7, 30.9.
+  const size_t waves = (npix + 63) / 64 * n_img;
+  const bool dbl = sizeof(T) == sizeof(double) || m.has_nie_nfw;
+  const bool solo = waves >= (dbl ? 3072 : (m.n_bulk < 512 ? 6144 : 32768));
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, solo ? 64 : 64 * classes, 0, st>>>(m, g, recd, recf, coefd, coeff, flags, classes,
+                                                      static_cast<T *>(keep.beta), out);
+  };
+#define LENSIM_RENDER(H, D) launch(solo ? &render_bulk_kernel<T, H, D, true> : &render_bulk_kernel<T, H, D, false>)
   constexpr bool kF32 = sizeof(T) == sizeof(float);  // as render_kernel's
   if (kF32 && m.has_nie_nfw && m.has_halo) LENSIM_RENDER(true, kF32);
   else if (kF32 && m.has_nie_nfw) LENSIM_RENDER(false, kF32);
