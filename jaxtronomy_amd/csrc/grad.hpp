@@ -41,15 +41,6 @@ __device__ __forceinline__ bool is_nan(const S &x) {
   return v != v;
 }
 
-// Util/param_util.py:88-100
-template <typename T, typename S>
-__device__ __forceinline__ void phi_q(const S &e1, const S &e2, S &phi, S &q) {
-  phi = atan2(e2, e1) * T(0.5);
-  S c = sqrt(e1 * e1 + e2 * e2);
-  c = fmin(c, T(0.9999));
-  q = (T(1) - c) / (T(1) + c);
-}
-
 // Sum_{n<N} c_n(t) w^n (quadratic-division form; see real_poly_at_complex)
 template <typename T, typename S>
 __device__ __forceinline__ void series_g(const T *__restrict__ c, const T *__restrict__ dc, int n, const S &t,
@@ -118,7 +109,7 @@ __device__ __forceinline__ void series_g(const T *__restrict__ c, const T *__res
 
 // EPL, LensModel/Profiles/epl.py:109-124, :178-200, :364-394.  p: theta_E,
 // gamma, e1, e2, center_x, center_y.  nser: series length (from the value of f).
-// q, cs, sn: the axis ratio and cos / sin of the orientation (from the record, or phi_q).
+// q, cs, sn: the axis ratio and cos / sin of the orientation (from the record).
 template <typename T, typename S>
 __device__ __forceinline__ void epl_g_geo(const S *p, const S &q, const S &cs, const S &sn,
                                           const T *__restrict__ c, const T *__restrict__ dc, int nser, const S &x,
@@ -161,14 +152,6 @@ __device__ __forceinline__ void epl_g_geo(const S *p, const S &q, const S &cs, c
   ay = ay + (fr * sn + fi * cs);
 }
 
-template <typename T, typename S>
-__device__ void epl_g(const S *p, const T *__restrict__ c, const T *__restrict__ dc, int nser, const S &x,
-                      const S &y, S &ax, S &ay) {
-  S phi, q;
-  phi_q<T>(p[2], p[3], phi, q);
-  epl_g_geo<T>(p, q, cos(phi), sin(phi), c, dc, nser, x, y, ax, ay);
-}
-
 // NIE / SIE, LensModel/Profiles/nie.py:86-107, :182-200, :280-295, from the
 // axis ratio q and the orientation's cos / sin (cs, sn).
 template <typename T, typename S>
@@ -189,41 +172,16 @@ __device__ __forceinline__ void nie_g_geo(const S &theta_E, const S &q, const S 
   ay = ay + (fx * sn + fy * cs);
 }
 
-// p: theta_E, e1, e2, s_scale, center_x, center_y (SIE: s_scale = 1e-10, centre at p[3..4]).
+// A linear deflector from its raw slot.
 template <typename T, typename S>
-__device__ void nie_g(const S &theta_E, const S &e1, const S &e2, const S &s_scale, const S &cx, const S &cy,
-                      const S &x, const S &y, S &ax, S &ay) {
-  S phi, q;
-  phi_q<T>(e1, e2, phi, q);
-  nie_g_geo<T>(theta_E, q, cos(phi), sin(phi), s_scale, cx, cy, x, y, ax, ay);
-}
-
-// One deflector from its raw slot.
-template <typename T, typename S>
-__device__ __forceinline__ void defl_g(int type, const S *p, const T *c, const T *dc, int nser, const S &x,
-                                       const S &y, S &ax, S &ay) {
-  switch (type) {
-    case LENSIM_EPL:
-      epl_g<T>(p, c, dc, nser, x, y, ax, ay);
-      break;
-    case LENSIM_SIE:
-      nie_g<T>(p[0], p[1], p[2], lift(T(0.0000000001), x), p[3], p[4], x, y, ax, ay);
-      break;
-    case LENSIM_NIE:
-      nie_g<T>(p[0], p[1], p[2], p[3], p[4], p[5], x, y, ax, ay);
-      break;
-    case LENSIM_SHEAR: {
-      const S dx = x - p[2], dy = y - p[3];
-      ax = ax + (p[0] * dx + p[1] * dy);
-      ay = ay + (p[1] * dx - p[0] * dy);
-      break;
-    }
-    case LENSIM_CONVERGENCE:  // convergence.py:34-46; p: kappa, ra_0, dec_0
-      ax = ax + p[0] * (x - p[1]);
-      ay = ay + p[0] * (y - p[2]);
-      break;
-    default:
-      break;
+__device__ __forceinline__ void defl_g(int type, const S *p, const S &x, const S &y, S &ax, S &ay) {
+  if (type == LENSIM_SHEAR) {
+    const S dx = x - p[2], dy = y - p[3];
+    ax = ax + (p[0] * dx + p[1] * dy);
+    ay = ay + (p[1] * dx - p[0] * dy);
+  } else if (type == LENSIM_CONVERGENCE) {  // convergence.py:34-46; p: kappa, ra_0, dec_0
+    ax = ax + p[0] * (x - p[1]);
+    ay = ay + p[0] * (y - p[2]);
   }
 }
 

@@ -2672,7 +2672,7 @@ struct GradArgs {
   double *gpart;          // [n_img][n_prof][nblk][8]
   void *gbeta;            // [n_img][ny][nx][s][s][2] dS/dbeta of the sources' sum, compute type, or NULL
   bool kept;              // gbeta holds beta (from the render) until the source's launch puts dS/dbeta there
-  void *beta;             // same shape: beta (bulk and multi-plane lists, by the adjoint kernels), or NULL
+  void *beta;             // same shape: beta (bulk and multi-plane lists, by the render or the adjoint kernels), or NULL
 };
 
 // A light profile's flux and its derivatives in its own kwargs (the N seeds
@@ -2727,8 +2727,12 @@ __device__ __forceinline__ gm::Dual<T, 2> sources_at(const ModelArgs &m, const G
 // gb: this ray's dS/dbeta of the sources' sum (two values), when the model
 // has inline lenses and sources: the first source's launch writes it, the lens
 // launches (which run after it) read it instead of deflecting by the other
-// deflectors and evaluating the sources again.  bt: this ray's beta, where an
-// adjoint kernel stored it (and gb) before.
+// deflectors and evaluating the sources again.  bt: this ray's beta, where the
+// render or an adjoint kernel stored it (and an adjoint kernel gb) before.
+// A lens with a live ray always has gb.  The float forms of ray_grad and
+// lens_ray_grad keep the branch without it all the same: with it gone the
+// compiler contracts the arithmetic of the other one differently, and the mixed
+// gradient moves by 2.7e-8 of itself.
 template <typename T, int N, bool HALO>
 __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga, const RecPtrs<T> &rp, int img,
                                          int k, int type, double x, double y, double w, double *acc, T *gb,
@@ -2744,20 +2748,7 @@ __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga,
   if (k < m.n_lens && gb) {
     // d flux = dS/dbeta . d beta, d beta = -alpha_scaling d alpha_k
     S ax = S(T(0)), ay = S(T(0));
-    const int e = m.epl_index[k];
-    const size_t co = (e >= 0) ? (size_t(img) * m.n_epl + e) * LENSIM_EPL_NMAX : 0;
-    int nser = 1;
-    if (type == LENSIM_EPL)
-      nser = int(sizeof(T) == sizeof(float) ? rp.recd[k * kRec + EPL_NF] : rp.recd[k * kRec + EPL_NMAX]);
-    const T *c = sizeof(T) == sizeof(float) ? reinterpret_cast<const T *>(ga.coeff + co)
-                                            : reinterpret_cast<const T *>(ga.coefd + co);
-    const T *dc = sizeof(T) == sizeof(float) ? reinterpret_cast<const T *>(ga.dcoeff + co)
-                                             : reinterpret_cast<const T *>(ga.dcoefd + co);
-    if (e >= 0) {
-      CHECK_SPAN(c, LENSIM_EPL_NMAX * sizeof(T));
-      CHECK_SPAN(dc, LENSIM_EPL_NMAX * sizeof(T));
-    }
-    gm::defl_g<T, S>(type, ps, c, dc, nser, S(T(x)), S(T(y)), ax, ay);
+    gm::defl_g<T, S>(type, ps, S(T(x)), S(T(y)), ax, ay);
     const T gx = AT(gb, 0), gy = AT(gb, 1), as = T(m.alpha_scaling);
 #pragma unroll
     for (int i = 0; i < N; ++i) acc[i] += w * double(-as * (gx * ax.d[i] + gy * ay.d[i]));
@@ -2775,21 +2766,8 @@ __device__ __forceinline__ void ray_grad(const ModelArgs &m, const GradArgs &ga,
     }
     deflect_bulk<T, HALO>(m, rp, x, y, axp, ayp);
     S ax = S(T(axp)), ay = S(T(ayp));
-    const int e = m.epl_index[k];
-    const size_t co = (e >= 0) ? (size_t(img) * m.n_epl + e) * LENSIM_EPL_NMAX : 0;
-    int nser = 1;
-    if (type == LENSIM_EPL)
-      nser = int(sizeof(T) == sizeof(float) ? rp.recd[k * kRec + EPL_NF] : rp.recd[k * kRec + EPL_NMAX]);
-    const T *c = sizeof(T) == sizeof(float) ? reinterpret_cast<const T *>(ga.coeff + co)
-                                            : reinterpret_cast<const T *>(ga.coefd + co);
-    const T *dc = sizeof(T) == sizeof(float) ? reinterpret_cast<const T *>(ga.dcoeff + co)
-                                             : reinterpret_cast<const T *>(ga.dcoefd + co);
-    if (e >= 0) {
-      CHECK_SPAN(c, LENSIM_EPL_NMAX * sizeof(T));
-      CHECK_SPAN(dc, LENSIM_EPL_NMAX * sizeof(T));
-    }
     const S xs = S(T(x)), ys = S(T(y));
-    gm::defl_g<T, S>(type, ps, c, dc, nser, xs, ys, ax, ay);
+    gm::defl_g<T, S>(type, ps, xs, ys, ax, ay);
     const S bx = xs - ax * T(m.alpha_scaling), by = ys - ay * T(m.alpha_scaling);
     // the sources' gradient in beta, chained into this deflector's kwargs:
     // d flux = dS/dbeta_x d beta_x + dS/dbeta_y d beta_y
@@ -2882,11 +2860,8 @@ __device__ __forceinline__ void epl_dalpha(const ModelArgs &m, const GradArgs &g
   for (int i = 0; i < LENSIM_NPARAM; ++i) ps[i] = i == 1 ? S::seed(T(pk[1]), 0) : S(T(pk[i]));
   const int e = m.epl_index[k];
   const size_t co = (size_t(img) * m.n_epl + e) * LENSIM_EPL_NMAX;
-  const int nser = int(sizeof(T) == sizeof(float) ? rp.recd[k * kRec + EPL_NF] : rp.recd[k * kRec + EPL_NMAX]);
-  const T *c = sizeof(T) == sizeof(float) ? reinterpret_cast<const T *>(ga.coeff + co)
-                                          : reinterpret_cast<const T *>(ga.coefd + co);
-  const T *dc = sizeof(T) == sizeof(float) ? reinterpret_cast<const T *>(ga.dcoeff + co)
-                                           : reinterpret_cast<const T *>(ga.dcoefd + co);
+  const int nser = int(rp.recd[k * kRec + EPL_NF]);  // the float form
+  const T *c = reinterpret_cast<const T *>(ga.coeff + co), *dc = reinterpret_cast<const T *>(ga.dcoeff + co);
   CHECK_SPAN(c, LENSIM_EPL_NMAX * sizeof(T));
   CHECK_SPAN(dc, LENSIM_EPL_NMAX * sizeof(T));
   // q, cos phi and sin phi from the record, not per ray
@@ -3097,7 +3072,7 @@ grad_kernel(ModelArgs m, GridArgs g, GradArgs ga,
       const double x = ra_c + g.m00 * ox + g.m01 * oy;
       const double y = dec_c + g.m10 * ox + g.m11 * oy;
       // this ray's slots: dS/dbeta, written by the first source's launch (or an adjoint kernel) and read by
-      // the inline lens launches; beta, written by an adjoint kernel and read by the source launches
+      // the inline lens launches; beta, written by the render or an adjoint kernel and read by the source launches
       const size_t slot = ((size_t(img) * npix + pix) * size_t(g.s * g.s) + size_t(sy * g.s + sx)) * 2;
       T *gb = (gbeta && (k < m.n_lens || k == m.n_defl)) ? gbeta + slot : nullptr;
       const T *bt = (ga.beta && k >= m.n_defl && k < m.n_defl + m.n_source) ? static_cast<const T *>(ga.beta) + slot
