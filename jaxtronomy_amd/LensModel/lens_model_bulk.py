@@ -154,10 +154,12 @@ class LensModelBulk(object):
         return {"all_kwargs": all_kwargs, "index_list": np.array(index_list), "T_ij_list": np.array(T_ij),
                 "T_z_list": np.array(T_z), "reduced2physical_factor": np.array(r2p)}
 
-    def multiplane_arrays(self, ray_shooting_kwargs, order):
+    def multiplane_arrays(self, ray_shooting_kwargs, order, rays_only=False):
         """Device arrays of the lensim_multiplane descriptor: the n deflector planes
         (packed deflector index of each, in the dict's plane order) plus the
-        source plane; trailing NULL planes (fillers, zero distance) are dropped."""
+        source plane; trailing NULL planes (fillers, zero distance) are dropped.
+        rays_only: for ray shooting, whose launch takes max_runs as a hint alone (the
+        planes that are apart in the first image, where a bound takes 30 us for 5000)."""
         idx = np.asarray(ray_shooting_kwargs["index_list"], dtype=int)
         n_unique = len(self.unique_lens_model_list)
         real = np.nonzero(idx < n_unique)[0]
@@ -174,7 +176,8 @@ class LensModelBulk(object):
                   "r2p": torch.as_tensor(np.ascontiguousarray(r2p), device=dev)}
         mp = backend.LensimMultiplane()
         mp.n_planes = n + 1
-        mp.max_runs = backend.plane_runs(t_ij, t_z, r2p)
+        mp.max_runs = (1 + n // 64 + int(np.count_nonzero(t_ij[0, 1:n] != 0.0)) if rays_only
+                       else backend.plane_runs(t_ij, t_z, r2p))
         mp.d_order = arrays["order"].data_ptr() if n else None
         mp.d_T_ij = arrays["tij"].data_ptr()
         mp.d_T_z = arrays["tz"].data_ptr()
@@ -261,7 +264,7 @@ class LensModelBulk(object):
         return out
 
     def _model(self, inline_types, bulk_types, source_types=(), light_types=(), flux_scaling=1.0,
-               ray_shooting_kwargs=None):
+               ray_shooting_kwargs=None, rays_only=False):
         """lensim_model of a pack() result (call right after pack: the plane order
         of a multi-plane model comes from it) and the device arrays to keep alive."""
         d_types = None
@@ -279,7 +282,7 @@ class LensModelBulk(object):
         if self.multi_plane:
             if ray_shooting_kwargs is None or "T_ij_list" not in ray_shooting_kwargs:
                 raise ValueError("multi-plane models need the ray_shooting_kwargs of prepare_ray_shooting_kwargs")
-            mp, arrays = self.multiplane_arrays(ray_shooting_kwargs, self._plane_order)
+            mp, arrays = self.multiplane_arrays(ray_shooting_kwargs, self._plane_order, rays_only)
             m.multiplane = ctypes.addressof(mp)
             keep.append(arrays)
         return m, keep  # keep the device arrays alive while m is used
@@ -288,7 +291,7 @@ class LensModelBulk(object):
         """LensModelBulk.ray_shooting, lens_model_bulk.py:113-128."""
         lib = backend.lib()
         n_img, it, ip, bt, bp = self.pack(ray_shooting_kwargs)
-        m, keep = self._model(it, bt, ray_shooting_kwargs=ray_shooting_kwargs)
+        m, keep = self._model(it, bt, ray_shooting_kwargs=ray_shooting_kwargs, rays_only=True)
         params = backend.to_device_f64(np.concatenate([ip, bp], axis=1))
         xt = backend.to_device_f64(x)
         yt = backend.to_device_f64(y)

@@ -1486,9 +1486,10 @@ template <bool SUB, typename F>
 __device__ __forceinline__ void run_sum(const MpWave<false> &w, MpRed<false> &red, int buf, int len, double &vx, double &vy,
                                         F one) {
   const int lane = threadIdx.x & 63;
-  vx = vy = 0.0;
-  for (int q = w.wave; q < len; q += w.nw) one(q, vx, vy);
-  red.part[buf][w.wave][lane] = double2{vx, vy};
+  double ax = 0.0, ay = 0.0;
+  for (int q = w.wave; q < len; q += w.nw) one(q, ax, ay);
+  // (by the lane's own index: by w.wave rays of 1828 halos over 202^2 took 662 us for 652)
+  red.part[buf][threadIdx.x >> 6][lane] = double2{ax, ay};
   __syncthreads();
   if (SUB && w.nw == 16) {
     const int ray = threadIdx.x >> 4, c = threadIdx.x & 15;
