@@ -3905,18 +3905,18 @@ int launch_conv_kernel(ConvArgs c, int n_img, const T *in, const double *kf, T *
     // than the work it shares (5 x 5, 64 images of 180^2, 57.5 against 67.7 us a
     // call; one image of 60^2 with 11 x 11 19.4 with, 21.5 without).  The shape
     // by the number of 32 x 32 tiles and the LDS: with fewer tiles than CUs short
-    // ones, weights in LDS; from 2048 tiles (eight a CU) kernels below 16 x 16 go
+    // ones, weights in LDS; from eight a CU (2048 tiles) kernels below 16 x 16 go
     // to conv_kernel in the same order, whose waves hold fewer registers (64
     // images of 180^2 with 15 x 15 74.6 against 80.4 us a call, 128 120.8 against
     // 145; at 1024 tiles, 256 of 60^2, 46.5 against 43.9).  One block of 82 KB
     // LDS or more fills a CU: there two row groups of waves (81 x 81, 743 against
     // 918 us).
     const size_t tiles = size_t((c.nx + 31) / 32) * ((c.ny + 31) / 32) * n_img;
-    const bool few = tiles < 256;
+    const bool few = tiles < size_t(cu_count());
     auto fits = [&](int r, int h, int cls, bool gw, size_t lds) {
       return conv_f64_smem(c.kx, c.ky, r, h, cls, gw) <= lds;
     };
-    if (c.kx < 16 && c.ky < 16 && tiles >= 2048) {
+    if (c.kx < 16 && c.ky < 16 && tiles >= 8 * size_t(cu_count())) {
       c.n_tiles_x = (c.nx + 31) / 32;
       *n_tiles = c.n_tiles_x * ((c.ny + 15) / 16);
       const dim3 grid(c.n_tiles_x * ((c.ny + 63) / 64), n_img);
