@@ -6,9 +6,8 @@ buffers; selected by LENSIM_CHECKED=1 or backend.use_checked()).
 hipcc cross-compiles without a GPU.  Packed-FP32 instructions are disabled on
 purpose (-target-feature -packed-fp32-ops); the host pass warns that it does
 not know that feature, which is harmless.  Matrix-core results stay in vector
-registers (-amdgpu-mfma-vgpr-form): with accumulation registers the compiler
-copied the float64 convolution's accumulators between the two register files
-on every loop iteration.
+registers (-amdgpu-mfma-vgpr-form): the convolution folds its float sums into
+float64 every few kernel rows, which vector instructions do.
 """
 
 import os

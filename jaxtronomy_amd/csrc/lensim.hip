@@ -3260,7 +3260,7 @@ __device__ __forceinline__ void deflector_dalpha(const ModelArgs &m, const GradA
 // planes) holds no parameter sums, and those are taken with a lane per ray, in
 // registers, with one wave sum per deflector at the end.  (One kernel that did
 // both summed five parameters over each block at every deflector: 23.5 ms for
-// 5256 deflectors and 100^2 rays, where the two steps take 0.52 and 0.28 ms.)
+// 5256 deflectors and 100^2 rays, where the two steps take 0.50 and 0.26 ms.)
 
 // Ray `first` + lane of image img (first + lane < the rays of the image, which
 // may be more than 2^31 in a list on one plane): its index on the grid,
